@@ -606,7 +606,173 @@ struct AdjBar {
 
 __device__ inline double *bpl(const AdjArgs &a, const AdjBar &B, int p) { return B.bw + (long)p * a.b.nnn; }
 
-// Transposed Jacobian of the face flux against Hb, one Dual pass per input.
+// The transposed products below are reverse sweeps written out by hand: the
+// values of the flux are formed once and its operations walked backwards,
+// about four flux evaluations, where a Dual pass per input took 31 (or 18)
+// evaluations of more than twice the work each.
+//
+// tau (xx xy xz yy yz zz of t) times S
+__device__ inline void tau_s(const double t[9], const double s[3], double r[3]) {
+  r[0] = t[0] * s[0] + t[1] * s[1] + t[2] * s[2];
+  r[1] = t[1] * s[0] + t[3] * s[1] + t[4] * s[2];
+  r[2] = t[2] * s[0] + t[4] * s[1] + t[5] * s[2];
+}
+
+__device__ inline double dot3(const double a[3], const double b[3]) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
+
+// The viscous part -(tau S) . (w, u) - q . S of a flux against the adjoint
+// (w, f4) of its momentum and energy: tb (9) of the stresses and the heat
+// flux, sb += of S.  y = -(w + f4 u) is the adjoint of tau S.
+__device__ inline void visc_vjp(const double w[3], double f4, const double u[3], const double t[9], const double s[3],
+                                double tb[9], double sb[3]) {
+  double y[3];
+#pragma unroll
+  for (int x = 0; x < 3; x++) y[x] = -(w[x] + f4 * u[x]);
+  tb[0] = y[0] * s[0];
+  tb[1] = y[0] * s[1] + y[1] * s[0];
+  tb[2] = y[0] * s[2] + y[2] * s[0];
+  tb[3] = y[1] * s[1];
+  tb[4] = y[1] * s[2] + y[2] * s[1];
+  tb[5] = y[2] * s[2];
+  double ty[3];
+  tau_s(t, y, ty);
+#pragma unroll
+  for (int x = 0; x < 3; x++) {
+    tb[6 + x] = -f4 * s[x];
+    sb[x] += ty[x] - f4 * t[6 + x];
+  }
+}
+
+// Adjoint of roe_face_t: fb of f (5) to Lb, Rb (5 each), tlb, trb (9 each)
+// and sb (3).  The dissipation P |Lambda| Q dW is taken in its wave form:
+// with the Roe averages u, h, c, the mean density r, the jumps dr, dp, du
+// and dn = du . n,
+//   a0 = |un| (dr - dp/c^2),  a1, a2 = |un +- c| (dp +- r c dn) / (2 c^2),
+//   D = ( a0 + a1 + a2,
+//         (a0 + a1 + a2) u + |un| r (du - n dn) + (a1 - a2) c n,
+//         a0 u^2/2 + |un| r (u . du - un dn) + (a1 + a2) h + (a1 - a2) c un ),
+// the same function of L, R and S, since dp = gam1 (u^2/2 drho - u . dm +
+// dE) holds for the Roe averages of any two states.
+__device__ __forceinline__ void roe_face_vjp(const APhys &ph, const double s[3], const double L[5], const double R[5],
+                                             const double tl[9], const double tr[9], const double fb[5], double Lb[5],
+                                             double Rb[5], double tlb[9], double trb[9], double sb[3]) {
+#pragma clang fp contract(fast)
+  const double gam1 = ph.gam1, gg = ph.gam / ph.gam1;
+  const double *w = fb + 1;  // adjoint of the momentum flux
+  const double f4 = fb[4];
+  const double A = ::sqrt(dot3(s, s)), iA = 1. / A;
+  const double n[3] = {s[0] * iA, s[1] * iA, s[2] * iA};
+  const double irl = 1. / L[0], irr = 1. / R[0];
+  const double *uL = L + 1, *uR = R + 1;
+  const double hL = gg * L[4] * irl + 0.5 * dot3(uL, uL), hR = gg * R[4] * irr + 0.5 * dot3(uR, uR);
+  const double gd = ::sqrt(R[0] * irl), g1 = 1. / (1. + gd), g2 = gd * g1, r = L[0] * gd;
+  double u[3], du[3];
+#pragma unroll
+  for (int x = 0; x < 3; x++) {
+    u[x] = g1 * uL[x] + g2 * uR[x];
+    du[x] = uR[x] - uL[x];
+  }
+  const double h = g1 * hL + g2 * hR, k = 0.5 * dot3(u, u), c = ::sqrt(gam1 * (h - k)), ic = 1. / c, ic2 = ic * ic;
+  const double vn = dot3(u, n), dn = dot3(du, n), dr = R[0] - L[0], dp = R[4] - L[4];
+  const double e0 = vn < 0. ? -1. : 1., e1 = vn + c < 0. ? -1. : 1., e2 = vn - c < 0. ? -1. : 1.;
+  const double l0 = e0 * vn, l1 = e1 * (vn + c), l2 = e2 * (vn - c);
+  const double p0 = dr - dp * ic2, p1 = 0.5 * ic2 * (dp + r * c * dn), p2 = 0.5 * ic2 * (dp - r * c * dn);
+  const double a0 = l0 * p0, a1 = l1 * p1, a2 = l2 * p2, sh = l0 * r, a12 = a1 - a2, udu = dot3(u, du);
+  // D and its adjoint -A fb
+  const double D0 = a0 + a1 + a2;
+  double fD = fb[0] * D0 + f4 * (a0 * k + sh * (udu - vn * dn) + (a1 + a2) * h + a12 * c * vn);
+#pragma unroll
+  for (int x = 0; x < 3; x++) fD += w[x] * (D0 * u[x] + sh * (du[x] - n[x] * dn) + a12 * c * n[x]);
+  const double d4 = -A * f4;
+  double dv[3] = {-A * w[0], -A * w[1], -A * w[2]};
+  const double dvn = dot3(dv, n), t0 = -A * fb[0] + dot3(dv, u);
+  const double a12b = c * (dvn + d4 * vn), a0b = t0 + d4 * k, a1b = t0 + d4 * h + a12b, a2b = t0 + d4 * h - a12b;
+  const double shb = dot3(dv, du) - dvn * dn + d4 * (udu - vn * dn);
+  double cb = a12 * (dvn + d4 * vn), vnb = d4 * (a12 * c - sh * dn), dnb = -sh * (dvn + d4 * vn);
+  double hb = d4 * (a1 + a2), kb = d4 * a0;
+  double ub[3], dub[3], nb[3];
+#pragma unroll
+  for (int x = 0; x < 3; x++) {
+    ub[x] = D0 * dv[x] + d4 * sh * du[x];
+    dub[x] = sh * (dv[x] + d4 * u[x]);
+    nb[x] = (a12 * c - sh * dn) * dv[x];
+  }
+  // wave strengths
+  const double p0b = a0b * l0, p1b = a1b * l1, p2b = a2b * l2;
+  const double l0b = a0b * p0 + shb * r, l1b = a1b * p1, l2b = a2b * p2;
+  double rb = shb * l0;
+  const double dpb = ic2 * (0.5 * (p1b + p2b) - p0b), zb = 0.5 * ic2 * (p1b - p2b);
+  double c2b = ic2 * (p0b * dp * ic2 - p1b * p1 - p2b * p2);
+  rb += zb * c * dn;
+  cb += zb * r * dn;
+  dnb += zb * r * c;
+  vnb += e0 * l0b + e1 * l1b + e2 * l2b;
+  cb += e1 * l1b - e2 * l2b;
+  c2b += 0.5 * ic * cb;
+  hb += gam1 * c2b;
+  kb -= gam1 * c2b;
+#pragma unroll
+  for (int x = 0; x < 3; x++) {
+    ub[x] += kb * u[x] + vnb * n[x];
+    nb[x] += vnb * u[x] + dnb * du[x];
+    dub[x] += dnb * n[x];
+  }
+  // averages
+  const double gdb = (dot3(ub, du) + hb * (hR - hL)) * g1 * g1;
+  Lb[0] = -p0b + 0.5 * rb * r * irl - 0.5 * gdb * gd * irl;
+  Rb[0] = p0b + 0.5 * rb * r * irr + 0.5 * gdb * gd * irr;
+  Lb[4] = -dpb;
+  Rb[4] = dpb;
+  // physical fluxes F(L) + F(R): m = rho u . S, (m, m u + p S, m h)
+  const double nbn = dot3(nb, n);
+#pragma unroll
+  for (int x = 0; x < 3; x++) sb[x] = (nb[x] - n[x] * nbn) * iA - fD * n[x];
+#pragma unroll
+  for (int side = 0; side < 2; side++) {
+    const double *q = side ? R : L, *uq = side ? uR : uL, *t = side ? tr : tl;
+    double *qb = side ? Rb : Lb, *tb = side ? trb : tlb;
+    const double ir = side ? irr : irl, hq = side ? hR : hL, gq_ = side ? g2 : g1, sg = side ? 1. : -1.;
+    const double un = dot3(uq, s), m = q[0] * un;
+    const double mb = fb[0] + dot3(w, uq) + f4 * hq, hqb = f4 * m + gq_ * hb;
+    double ts[3];
+    tau_s(t, s, ts);
+    qb[0] += mb * un - hqb * gg * q[4] * ir * ir;
+    qb[4] += dot3(w, s) + hqb * gg * ir;
+    const double unb = mb * q[0];
+#pragma unroll
+    for (int x = 0; x < 3; x++) {
+      qb[1 + x] = sg * dub[x] + gq_ * ub[x] + m * w[x] - f4 * ts[x] + unb * s[x] + hqb * uq[x];
+      sb[x] += unb * uq[x] + (q[4] - ph.pinfl) * w[x];
+    }
+    visc_vjp(w, f4, uq, t, s, tb, sb);
+  }
+}
+
+// Adjoint of phys_flux_t: with u = m / rho and U = u . S the flux is
+// (rho U, m U + (p - pinfl) S - tau S, (E + p - pinfl) U - u . tau S - q . S)
+__device__ __forceinline__ void phys_flux_vjp(const APhys &ph, const double v[5], double p, const double t[9],
+                                              const double s[3], const double fb[5], double vb[5], double &pb,
+                                              double tb[9], double sb[3]) {
+#pragma clang fp contract(fast)
+  const double *w = fb + 1;
+  const double f4 = fb[4], ir = 1. / v[0];
+  const double u[3] = {v[1] * ir, v[2] * ir, v[3] * ir};
+  const double U = dot3(u, s), Ub = fb[0] * v[0] + dot3(w, v + 1) + f4 * (v[4] + p - ph.pinfl);
+  double ts[3], ub[3];
+  tau_s(t, s, ts);
+  pb = dot3(w, s) + f4 * U;
+  vb[4] = f4 * U;
+#pragma unroll
+  for (int x = 0; x < 3; x++) {
+    ub[x] = Ub * s[x] - f4 * ts[x];
+    vb[1 + x] = U * w[x] + ub[x] * ir;
+    sb[x] = Ub * u[x] + (p - ph.pinfl) * w[x];
+  }
+  vb[0] = fb[0] * U - dot3(ub, u) * ir;
+  visc_vjp(w, f4, u, t, s, tb, sb);
+}
+
+// Transposed Jacobian of the face flux against Hb.
 __global__ void __launch_bounds__(128) k_adjb_faces(AdjArgs a, AdjBar B, int d) {
   int c[3];
   if (!face_of(a.b, d, blockIdx.x * 128L + threadIdx.x, c)) return;
@@ -615,50 +781,26 @@ __global__ void __launch_bounds__(128) k_adjb_faces(AdjArgs a, AdjBar B, int d) 
   int al = c[d], a1 = b.lo(d), a2 = b.hi(d);
   const double *ub = B.ub;
   const long ldv = a.ldv;
-  double s[3];
+  double s[3], sb[3];
 #pragma unroll
   for (int cc = 0; cc < 3; cc++) s[cc] = load_sn<double>(a, m, d, cc);
-  double sb[3] = {0., 0., 0.};
   if (al > a1 && al < a2) {
     // u(m) has -H(m), u(m-inc) has +H(m); H = 0.5 f
     double fb[5];
 #pragma unroll
     for (int e = 0; e < 5; e++) fb[e] = 0.5 * (ub[e * ldv + n - inc] - ub[e * ldv + n]);
-    double q[4][5], L[5], R[5], tl[9], tr[9];
+    double L[5], R[5], Lb[5], Rb[5], tl[9], tr[9], tlb[9], trb[9];
 #pragma unroll
     for (int e = 0; e < 5; e++) {
       const double *qp = a.ws + (long)(P_Q + e) * b.nnn;
-#pragma unroll
-      for (int k = 0; k < 4; k++) q[k][e] = qp[m + (k - 2) * inc];
-      muscl_lr(a.muscl, a.xk, q[0][e], q[1][e], q[2][e], q[3][e], L[e], R[e]);
+      muscl_lr(a.muscl, a.xk, qp[m - 2 * inc], qp[m - inc], qp[m], qp[m + inc], L[e], R[e]);
     }
 #pragma unroll
     for (int x = 0; x < 9; x++) {
       tl[x] = a.ws[(long)(P_TQ + x) * b.nnn + m - inc];
       tr[x] = a.ws[(long)(P_TQ + x) * b.nnn + m];
     }
-    double xb[31];
-#pragma unroll 1
-    for (int k = 0; k < 31; k++) {
-      Dual sD[3], LD[5], RD[5], tlD[9], trD[9], fD[5];
-#pragma unroll
-      for (int x = 0; x < 3; x++) sD[x] = mk(s[x], k == 28 + x);
-#pragma unroll
-      for (int x = 0; x < 5; x++) {
-        LD[x] = mk(L[x], k == x);
-        RD[x] = mk(R[x], k == 5 + x);
-      }
-#pragma unroll
-      for (int x = 0; x < 9; x++) {
-        tlD[x] = mk(tl[x], k == 10 + x);
-        trD[x] = mk(tr[x], k == 19 + x);
-      }
-      roe_face_t(a.ph, sD, LD, RD, tlD, trD, fD);
-      double acc = 0.;
-#pragma unroll
-      for (int e = 0; e < 5; e++) acc += fb[e] * fD[e].d;
-      xb[k] = acc;
-    }
+    roe_face_vjp(a.ph, s, L, R, tl, tr, fb, Lb, Rb, tlb, trb, sb);
     // MUSCL: L = cl0 q0 + cl1 q1 + cl2 q2, R = cr1 q1 + cr2 q2 + cr3 q3
     const double c4 = 0.25 * a.muscl;
     const double cl0 = -c4 * (1. - a.xk), cl1 = 1. + c4 * ((1. - a.xk) - (1. + a.xk)), cl2 = c4 * (1. + a.xk);
@@ -666,55 +808,34 @@ __global__ void __launch_bounds__(128) k_adjb_faces(AdjArgs a, AdjBar B, int d) 
 #pragma unroll
     for (int e = 0; e < 5; e++) {
       double *qb = bpl(a, B, B_Q + e);
-      double Lb = xb[e], Rb = xb[5 + e];
-      atomicAdd(qb + m - 2 * inc, cl0 * Lb);
-      atomicAdd(qb + m - inc, cl1 * Lb + cr1 * Rb);
-      atomicAdd(qb + m, cl2 * Lb + cr2 * Rb);
-      atomicAdd(qb + m + inc, cr3 * Rb);
+      atomicAdd(qb + m - 2 * inc, cl0 * Lb[e]);
+      atomicAdd(qb + m - inc, cl1 * Lb[e] + cr1 * Rb[e]);
+      atomicAdd(qb + m, cl2 * Lb[e] + cr2 * Rb[e]);
+      atomicAdd(qb + m + inc, cr3 * Rb[e]);
     }
 #pragma unroll
     for (int x = 0; x < 9; x++) {
-      atomicAdd(bpl(a, B, B_TQ + x) + m - inc, xb[10 + x]);
-      atomicAdd(bpl(a, B, B_TQ + x) + m, xb[19 + x]);
+      atomicAdd(bpl(a, B, B_TQ + x) + m - inc, tlb[x]);
+      atomicAdd(bpl(a, B, B_TQ + x) + m, trb[x]);
     }
-#pragma unroll
-    for (int x = 0; x < 3; x++) sb[x] = xb[28 + x];
   } else {
     bool lo = al == a1;
     long mg = lo ? m - inc : m;
     double hb[5];
 #pragma unroll
     for (int e = 0; e < 5; e++) hb[e] = lo ? -ub[e * ldv + n] : ub[e * ldv + n - inc];
-    double w[5], t[9], p = a.ws[(long)(P_Q + 4) * b.nnn + mg];
+    double w[5], t[9], wb[5], tb[9], pb, p = a.ws[(long)(P_Q + 4) * b.nnn + mg];
 #pragma unroll
     for (int e = 0; e < 5; e++) w[e] = a.ws[(long)(P_W + e) * b.nnn + mg];
 #pragma unroll
     for (int x = 0; x < 9; x++) t[x] = a.ws[(long)(P_TQ + x) * b.nnn + mg];
-    double xb[18];
-#pragma unroll 1
-    for (int k = 0; k < 18; k++) {
-      Dual wD[5], tD[9], sD[3], fD[5];
-#pragma unroll
-      for (int x = 0; x < 5; x++) wD[x] = mk(w[x], k == x);
-      Dual pD = mk(p, k == 5);
-#pragma unroll
-      for (int x = 0; x < 9; x++) tD[x] = mk(t[x], k == 6 + x);
-#pragma unroll
-      for (int x = 0; x < 3; x++) sD[x] = mk(s[x], k == 15 + x);
-      phys_flux_t(a.ph, wD, pD, tD, sD, fD);
-      double acc = 0.;
-#pragma unroll
-      for (int e = 0; e < 5; e++) acc += hb[e] * fD[e].d;
-      xb[k] = acc;
-    }
+    phys_flux_vjp(a.ph, w, p, t, s, hb, wb, pb, tb, sb);
     // one writer per ghost for W and p; stresses of the ghost through TQB
 #pragma unroll
-    for (int e = 0; e < 5; e++) atomicAdd(bpl(a, B, B_W + e) + mg, xb[e]);
-    atomicAdd(bpl(a, B, B_Q + 4) + mg, xb[5]);
+    for (int e = 0; e < 5; e++) atomicAdd(bpl(a, B, B_W + e) + mg, wb[e]);
+    atomicAdd(bpl(a, B, B_Q + 4) + mg, pb);
 #pragma unroll
-    for (int x = 0; x < 9; x++) atomicAdd(bpl(a, B, B_TQ + x) + mg, xb[6 + x]);
-#pragma unroll
-    for (int x = 0; x < 3; x++) sb[x] = xb[15 + x];
+    for (int x = 0; x < 9; x++) atomicAdd(bpl(a, B, B_TQ + x) + mg, tb[x]);
   }
 #pragma unroll
   for (int cc = 0; cc < 3; cc++) atomicAdd(B.snb + ((long)cc * 3 + d) * b.nnn + m, sb[cc]);
