@@ -14,12 +14,12 @@
 //
 // Every piece of the residual is written once, templated on the scalar:
 // double gives the values, Dual (value, tangent) gives exact directional
-// derivatives.  The JVP runs the chain on Dual planes.  The VJP walks the
-// chain backwards; where a piece is nonlinear (the face fluxes, the ghost
-// rules, the thermodynamics, the stresses) the transposed product of its
-// local Jacobian with the incoming adjoint is formed from one Dual pass per
-// input of that piece, so it is exact to rounding, and the adjoints are
-// scattered to the cells with FP64 atomic adds.
+// derivatives.  The JVP runs the chain on Dual planes.  The VJP forms the
+// values and walks the chain backwards with hand-written reverse sweeps of
+// the face fluxes, the stresses, the gradients and the thermodynamics (the
+// ghost rules: one Dual pass per input).  Its passes gather: a face's
+// adjoints are stored at the face and summed by the cells that use them, so
+// that only the ghost rules, a surface, scatter with FP64 atomic adds.
 //
 // Arithmetic restates oracle_flux.c / oracle_visc.c (sch_roe.f90:322-578,
 // zpres.f90:66-79, zvismo.f90:90-104, clpara.f90:44-58, clnrd.f90:60-134,
@@ -311,10 +311,9 @@ __device__ void phys_flux_t(const APhys &ph, const T w[5], T p, const T t[9], co
 // ---------------------------------------------------------------------------
 // Workspace planes (block-local index m, nnn entries each; JVP tangents in a
 // second set).  Q: primitive state of every real and ghost cell; TT: T;
-// MU: mu of the real cells; W: conservative ghost state; G: raw Green-Gauss
-// sums (12); C0: gradient scale; TQ: stresses and heat flux (9); H: face
-// fluxes (3 directions x 5).
-constexpr int P_Q = 0, P_TT = 5, P_MU = 6, P_W = 7, P_G = 12, P_C0 = 24, P_TQ = 25, P_H = 34, NPLANE = 49;
+// MU: mu of the real cells; W: conservative ghost state; TQ: stresses and
+// heat flux (9); H: face fluxes (3 directions x 5, JVP only).
+constexpr int P_Q = 0, P_TT = 5, P_MU = 6, P_W = 7, P_TQ = 12, P_H = 21, NPLANE = 36, NVPLANE = 21;
 
 struct AdjArgs {
   Blk b;
@@ -434,9 +433,9 @@ __device__ inline T gq(const AdjArgs &a, int q, long m) {
   return q < 3 ? plane<T>(a, P_Q + 1 + q)[m] : plane<T>(a, P_TT)[m];
 }
 
-// Raw Green-Gauss sums of one real cell in zgrad2's accumulation order
+// Green-Gauss sums of one real cell in zgrad2's accumulation order
 // (directions k, j, i; per direction the interior low face, the interior
-// high face, then the boundary faces) and the scale.
+// high face, then the boundary faces), scaled, and the stresses from them.
 template <typename T>
 __global__ void __launch_bounds__(256) k_adj_grad(AdjArgs a) {
   int c[3];
@@ -487,22 +486,11 @@ __global__ void __launch_bounds__(256) k_adj_grad(AdjArgs a) {
       }
     }
   }
+  const T c0 = grad_scale(ldx<T>(a.vol, a.vold, m + b.npc));
+  T tq[9];
 #pragma unroll
-  for (int x = 0; x < 12; x++) wplane<T>(a, P_G + x).set(m, G[x]);
-  long n = m + b.npc;
-  wplane<T>(a, P_C0).set(m, grad_scale(ldx<T>(a.vol, a.vold, n)));
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_adj_tq(AdjArgs a) {
-  int c[3];
-  if (!real_cell(a.b, blockIdx.x * 256L + threadIdx.x, c)) return;
-  long m = a.b.idx(c[0], c[1], c[2]) - a.b.npc;
-  T g[12], tq[9];
-  T c0 = plane<T>(a, P_C0)[m];
-#pragma unroll
-  for (int x = 0; x < 12; x++) g[x] = plane<T>(a, P_G + x)[m] * c0;
-  stresses(a.ph, g, plane<T>(a, P_MU)[m], tq);
+  for (int x = 0; x < 12; x++) G[x] = G[x] * c0;
+  stresses(a.ph, G, plane<T>(a, P_MU)[m], tq);
 #pragma unroll
   for (int x = 0; x < 9; x++) wplane<T>(a, P_TQ + x).set(m, tq[x]);
 }
@@ -593,10 +581,13 @@ __global__ void __launch_bounds__(256) k_adj_gather(AdjArgs a, double *u, double
 }
 
 // ---------------------------------------------------------------------------
-// adjoint pieces.  Adjoint planes (block-local, nnn each): QB primitive
-// state (5), WB conservative ghost state (5), VB gradient quantities u, v,
-// w, T (4), TQB stresses (9), GB raw gradient sums (12), MUB mu.
-constexpr int B_Q = 0, B_W = 5, B_V = 10, B_TQ = 14, B_G = 23, B_MU = 35, NBPLANE = 36;
+// adjoint pieces.  Adjoint planes (block-local, nnn each): F the left and
+// right MUSCL states of every face (3 directions x (5 + 5), zero on boundary
+// faces), W the conservative ghost state and its pressure (5 + 1), V the
+// gradient quantities u, v, w, T of the ghosts (4), G the raw gradient sums
+// (the nine distinct ones: the adjoint of the velocity gradient is
+// symmetric), MU mu.
+constexpr int B_F = 0, B_W = 30, B_V = 36, B_G = 40, B_MU = 49, NBPLANE = 50;
 
 struct AdjBar {
   double *bw;                 // adjoint planes
@@ -621,30 +612,16 @@ __device__ inline void tau_s(const double t[9], const double s[3], double r[3]) 
 __device__ inline double dot3(const double a[3], const double b[3]) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
 
 // The viscous part -(tau S) . (w, u) - q . S of a flux against the adjoint
-// (w, f4) of its momentum and energy: tb (9) of the stresses and the heat
-// flux, sb += of S.  y = -(w + f4 u) is the adjoint of tau S.
-__device__ inline void visc_vjp(const double w[3], double f4, const double u[3], const double t[9], const double s[3],
-                                double tb[9], double sb[3]) {
-  double y[3];
-#pragma unroll
-  for (int x = 0; x < 3; x++) y[x] = -(w[x] + f4 * u[x]);
-  tb[0] = y[0] * s[0];
-  tb[1] = y[0] * s[1] + y[1] * s[0];
-  tb[2] = y[0] * s[2] + y[2] * s[0];
-  tb[3] = y[1] * s[1];
-  tb[4] = y[1] * s[2] + y[2] * s[1];
-  tb[5] = y[2] * s[2];
+// (w, f4) of its momentum and energy: sb += its adjoint of S.
+__device__ inline void visc_sb(const double w[3], double f4, const double u[3], const double t[9], double sb[3]) {
+  const double y[3] = {-(w[0] + f4 * u[0]), -(w[1] + f4 * u[1]), -(w[2] + f4 * u[2])};
   double ty[3];
   tau_s(t, y, ty);
 #pragma unroll
-  for (int x = 0; x < 3; x++) {
-    tb[6 + x] = -f4 * s[x];
-    sb[x] += ty[x] - f4 * t[6 + x];
-  }
+  for (int x = 0; x < 3; x++) sb[x] += ty[x] - f4 * t[6 + x];
 }
 
-// Adjoint of roe_face_t: fb of f (5) to Lb, Rb (5 each), tlb, trb (9 each)
-// and sb (3).  The dissipation P |Lambda| Q dW is taken in its wave form:
+// Adjoint of roe_face_t: fb of f (5) to Lb, Rb (5 each) and sb (3).  The dissipation P |Lambda| Q dW is taken in its wave form:
 // with the Roe averages u, h, c, the mean density r, the jumps dr, dp, du
 // and dn = du . n,
 //   a0 = |un| (dr - dp/c^2),  a1, a2 = |un +- c| (dp +- r c dn) / (2 c^2),
@@ -655,7 +632,7 @@ __device__ inline void visc_vjp(const double w[3], double f4, const double u[3],
 // dE) holds for the Roe averages of any two states.
 __device__ __forceinline__ void roe_face_vjp(const APhys &ph, const double s[3], const double L[5], const double R[5],
                                              const double tl[9], const double tr[9], const double fb[5], double Lb[5],
-                                             double Rb[5], double tlb[9], double trb[9], double sb[3]) {
+                                             double Rb[5], double sb[3]) {
 #pragma clang fp contract(fast)
   const double gam1 = ph.gam1, gg = ph.gam / ph.gam1;
   const double *w = fb + 1;  // adjoint of the momentum flux
@@ -730,7 +707,7 @@ __device__ __forceinline__ void roe_face_vjp(const APhys &ph, const double s[3],
 #pragma unroll
   for (int side = 0; side < 2; side++) {
     const double *q = side ? R : L, *uq = side ? uR : uL, *t = side ? tr : tl;
-    double *qb = side ? Rb : Lb, *tb = side ? trb : tlb;
+    double *qb = side ? Rb : Lb;
     const double ir = side ? irr : irl, hq = side ? hR : hL, gq_ = side ? g2 : g1, sg = side ? 1. : -1.;
     const double un = dot3(uq, s), m = q[0] * un;
     const double mb = fb[0] + dot3(w, uq) + f4 * hq, hqb = f4 * m + gq_ * hb;
@@ -744,7 +721,7 @@ __device__ __forceinline__ void roe_face_vjp(const APhys &ph, const double s[3],
       qb[1 + x] = sg * dub[x] + gq_ * ub[x] + m * w[x] - f4 * ts[x] + unb * s[x] + hqb * uq[x];
       sb[x] += unb * uq[x] + (q[4] - ph.pinfl) * w[x];
     }
-    visc_vjp(w, f4, uq, t, s, tb, sb);
+    visc_sb(w, f4, uq, t, sb);
   }
 }
 
@@ -752,7 +729,7 @@ __device__ __forceinline__ void roe_face_vjp(const APhys &ph, const double s[3],
 // (rho U, m U + (p - pinfl) S - tau S, (E + p - pinfl) U - u . tau S - q . S)
 __device__ __forceinline__ void phys_flux_vjp(const APhys &ph, const double v[5], double p, const double t[9],
                                               const double s[3], const double fb[5], double vb[5], double &pb,
-                                              double tb[9], double sb[3]) {
+                                              double sb[3]) {
 #pragma clang fp contract(fast)
   const double *w = fb + 1;
   const double f4 = fb[4], ir = 1. / v[0];
@@ -769,237 +746,301 @@ __device__ __forceinline__ void phys_flux_vjp(const APhys &ph, const double v[5]
     sb[x] = Ub * u[x] + (p - ph.pinfl) * w[x];
   }
   vb[0] = fb[0] * U - dot3(ub, u) * ir;
-  visc_vjp(w, f4, u, t, s, tb, sb);
+  visc_sb(w, f4, u, t, sb);
 }
 
-// Transposed Jacobian of the face flux against Hb.
-__global__ void __launch_bounds__(128) k_adjb_faces(AdjArgs a, AdjBar B, int d) {
+// MUSCL: L = cl0 q0 + cl1 q1 + cl2 q2, R = cr1 q1 + cr2 q2 + cr3 q3
+struct MusclW {
+  double l0, l1, l2, r1, r2, r3;
+};
+__device__ inline MusclW muscl_w(const AdjArgs &a) {
+  const double c4 = 0.25 * a.muscl, m = c4 * (1. - a.xk), p = c4 * (1. + a.xk);
+  return {-m, 1. + (m - p), p, p, 1. - (p - m), -m};
+}
+
+// Transposed Jacobian of every face's flux, the three directions in one
+// launch (nb0, nb1: workgroups of the first two): adjoints of the MUSCL
+// states, of the ghost state on boundary faces, and the metric's.  One
+// writer per entry.  The stresses' adjoints are gathered by k_adjb_tq.
+__global__ void __launch_bounds__(128) k_adjb_faces(AdjArgs a, AdjBar B, unsigned nb0, unsigned nb1) {
+  const int d = blockIdx.x < nb0 ? 0 : (blockIdx.x < nb0 + nb1 ? 1 : 2);
+  const long blk = blockIdx.x - (d == 0 ? 0 : (d == 1 ? nb0 : nb0 + nb1));
   int c[3];
-  if (!face_of(a.b, d, blockIdx.x * 128L + threadIdx.x, c)) return;
+  if (!face_of(a.b, d, blk * 128L + threadIdx.x, c)) return;
   const Blk &b = a.b;
-  long inc = b.inc(d), m = b.idx(c[0], c[1], c[2]) - b.npc, n = m + b.npc;
-  int al = c[d], a1 = b.lo(d), a2 = b.hi(d);
+  const long inc = b.inc(d), m = b.idx(c[0], c[1], c[2]) - b.npc, n = m + b.npc, nnn = b.nnn, ldv = a.ldv;
+  const int al = c[d], a1 = b.lo(d), a2 = b.hi(d);
   const double *ub = B.ub;
-  const long ldv = a.ldv;
   double s[3], sb[3];
 #pragma unroll
   for (int cc = 0; cc < 3; cc++) s[cc] = load_sn<double>(a, m, d, cc);
+  double Lb[5] = {0., 0., 0., 0., 0.}, Rb[5] = {0., 0., 0., 0., 0.};
   if (al > a1 && al < a2) {
     // u(m) has -H(m), u(m-inc) has +H(m); H = 0.5 f
-    double fb[5];
+    double fb[5], L[5], R[5], tl[9], tr[9];
 #pragma unroll
     for (int e = 0; e < 5; e++) fb[e] = 0.5 * (ub[e * ldv + n - inc] - ub[e * ldv + n]);
-    double L[5], R[5], Lb[5], Rb[5], tl[9], tr[9], tlb[9], trb[9];
 #pragma unroll
     for (int e = 0; e < 5; e++) {
-      const double *qp = a.ws + (long)(P_Q + e) * b.nnn;
+      const double *qp = a.ws + (P_Q + e) * nnn;
       muscl_lr(a.muscl, a.xk, qp[m - 2 * inc], qp[m - inc], qp[m], qp[m + inc], L[e], R[e]);
     }
 #pragma unroll
     for (int x = 0; x < 9; x++) {
-      tl[x] = a.ws[(long)(P_TQ + x) * b.nnn + m - inc];
-      tr[x] = a.ws[(long)(P_TQ + x) * b.nnn + m];
+      tl[x] = a.ws[(P_TQ + x) * nnn + m - inc];
+      tr[x] = a.ws[(P_TQ + x) * nnn + m];
     }
-    roe_face_vjp(a.ph, s, L, R, tl, tr, fb, Lb, Rb, tlb, trb, sb);
-    // MUSCL: L = cl0 q0 + cl1 q1 + cl2 q2, R = cr1 q1 + cr2 q2 + cr3 q3
-    const double c4 = 0.25 * a.muscl;
-    const double cl0 = -c4 * (1. - a.xk), cl1 = 1. + c4 * ((1. - a.xk) - (1. + a.xk)), cl2 = c4 * (1. + a.xk);
-    const double cr1 = c4 * (1. + a.xk), cr2 = 1. - c4 * ((1. + a.xk) - (1. - a.xk)), cr3 = -c4 * (1. - a.xk);
-#pragma unroll
-    for (int e = 0; e < 5; e++) {
-      double *qb = bpl(a, B, B_Q + e);
-      atomicAdd(qb + m - 2 * inc, cl0 * Lb[e]);
-      atomicAdd(qb + m - inc, cl1 * Lb[e] + cr1 * Rb[e]);
-      atomicAdd(qb + m, cl2 * Lb[e] + cr2 * Rb[e]);
-      atomicAdd(qb + m + inc, cr3 * Rb[e]);
-    }
-#pragma unroll
-    for (int x = 0; x < 9; x++) {
-      atomicAdd(bpl(a, B, B_TQ + x) + m - inc, tlb[x]);
-      atomicAdd(bpl(a, B, B_TQ + x) + m, trb[x]);
-    }
+    roe_face_vjp(a.ph, s, L, R, tl, tr, fb, Lb, Rb, sb);
   } else {
-    bool lo = al == a1;
-    long mg = lo ? m - inc : m;
-    double hb[5];
+    const bool lo = al == a1;
+    const long mg = lo ? m - inc : m;
+    double hb[5], w[5], t[9], wb[5], pb, p = a.ws[(P_Q + 4) * nnn + mg];
 #pragma unroll
     for (int e = 0; e < 5; e++) hb[e] = lo ? -ub[e * ldv + n] : ub[e * ldv + n - inc];
-    double w[5], t[9], wb[5], tb[9], pb, p = a.ws[(long)(P_Q + 4) * b.nnn + mg];
 #pragma unroll
-    for (int e = 0; e < 5; e++) w[e] = a.ws[(long)(P_W + e) * b.nnn + mg];
+    for (int e = 0; e < 5; e++) w[e] = a.ws[(P_W + e) * nnn + mg];
 #pragma unroll
-    for (int x = 0; x < 9; x++) t[x] = a.ws[(long)(P_TQ + x) * b.nnn + mg];
-    phys_flux_vjp(a.ph, w, p, t, s, hb, wb, pb, tb, sb);
-    // one writer per ghost for W and p; stresses of the ghost through TQB
+    for (int x = 0; x < 9; x++) t[x] = a.ws[(P_TQ + x) * nnn + mg];
+    phys_flux_vjp(a.ph, w, p, t, s, hb, wb, pb, sb);
 #pragma unroll
-    for (int e = 0; e < 5; e++) atomicAdd(bpl(a, B, B_W + e) + mg, wb[e]);
-    atomicAdd(bpl(a, B, B_Q + 4) + mg, pb);
-#pragma unroll
-    for (int x = 0; x < 9; x++) atomicAdd(bpl(a, B, B_TQ + x) + mg, tb[x]);
+    for (int e = 0; e < 5; e++) bpl(a, B, B_W + e)[mg] = wb[e];
+    bpl(a, B, B_W + 5)[mg] = pb;
   }
 #pragma unroll
-  for (int cc = 0; cc < 3; cc++) atomicAdd(B.snb + ((long)cc * 3 + d) * b.nnn + m, sb[cc]);
-}
-
-// ghost stresses were copies of the adjacent cell
-__global__ void __launch_bounds__(256) k_adjb_tq_ghost(AdjArgs a, AdjBar B, long nf, const int64_t *__restrict__ g,
-                                                       const int64_t *__restrict__ in) {
-  long f = blockIdx.x * 256L + threadIdx.x;
-  if (f >= nf) return;
-  long mg = g[f] - a.b.npc, mi = in[f] - a.b.npc;
-#pragma unroll
-  for (int x = 0; x < 9; x++) atomicAdd(bpl(a, B, B_TQ + x) + mi, bpl(a, B, B_TQ + x)[mg]);
-}
-
-// stresses of a real cell: adjoints of the raw gradient sums, of mu and of
-// vol (through the scale), one Dual pass per input (12 sums, mu, vol)
-__global__ void __launch_bounds__(128) k_adjb_tq(AdjArgs a, AdjBar B) {
-  int c[3];
-  if (!real_cell(a.b, blockIdx.x * 128L + threadIdx.x, c)) return;
-  const Blk &b = a.b;
-  long m = b.idx(c[0], c[1], c[2]) - b.npc, n = m + b.npc;
-  double G[12], tb[9], mu = a.ws[(long)P_MU * b.nnn + m], vol = a.vol[n];
-#pragma unroll
-  for (int x = 0; x < 12; x++) G[x] = a.ws[(long)(P_G + x) * b.nnn + m];
-#pragma unroll
-  for (int x = 0; x < 9; x++) tb[x] = bpl(a, B, B_TQ + x)[m];
-#pragma unroll 1
-  for (int k = 0; k < 14; k++) {
-    Dual g[12], tq[9];
-    Dual c0 = grad_scale(mk(vol, k == 13));
-#pragma unroll
-    for (int x = 0; x < 12; x++) g[x] = mk(G[x], k == x) * c0;
-    stresses(a.ph, g, mk(mu, k == 12), tq);
-    double acc = 0.;
-#pragma unroll
-    for (int x = 0; x < 9; x++) acc += tb[x] * tq[x].d;
-    if (k < 12)
-      bpl(a, B, B_G + k)[m] = acc;
-    else if (k == 12)
-      bpl(a, B, B_MU)[m] = acc;
-    else
-      B.volb[n] += acc;
+  for (int e = 0; e < 5; e++) {
+    bpl(a, B, B_F + 10 * d + e)[m] = Lb[e];
+    bpl(a, B, B_F + 10 * d + 5 + e)[m] = Rb[e];
   }
+#pragma unroll
+  for (int cc = 0; cc < 3; cc++) B.snb[((long)cc * 3 + d) * nnn + m] = sb[cc];
 }
 
-// Green-Gauss sums of one face, transposed: adjoints of the face's
-// quantities (both cells, or twice the ghost) and of its metric
-__global__ void __launch_bounds__(256) k_adjb_grad(AdjArgs a, AdjBar B, int d) {
+// Stresses of a real cell: their adjoints gathered from the cell's six faces
+// (a boundary face's ghost holds a copy of the cell's stresses), then those
+// of the raw gradient sums, of mu and of vol.  A face's flux has
+// -(tau S) . (w, u) - q . S against its adjoint (w, f4), with u the velocity
+// of the cell's side: y = -(w + f4 u) is the adjoint of tau S.
+__global__ void __launch_bounds__(256) k_adjb_tq(AdjArgs a, AdjBar B) {
+#pragma clang fp contract(fast)
   int c[3];
-  if (!face_of(a.b, d, blockIdx.x * 256L + threadIdx.x, c)) return;
+  if (!real_cell(a.b, blockIdx.x * 256L + threadIdx.x, c)) return;
   const Blk &b = a.b;
-  long inc = b.inc(d), m = b.idx(c[0], c[1], c[2]) - b.npc;
-  int al = c[d], a1 = b.lo(d), a2 = b.hi(d);
-  double s[3], sb[3] = {0., 0., 0.};
+  const long m = b.idx(c[0], c[1], c[2]) - b.npc, n = m + b.npc, nnn = b.nnn, ldv = a.ldv;
+  const double *Q = a.ws + (P_Q + 1) * nnn, *W = a.ws + P_W * nnn;
+  const double c4m = 0.25 * a.muscl * (1. - a.xk), c4p = 0.25 * a.muscl * (1. + a.xk);
+  double ub0[4], u0[3], tb[9];
 #pragma unroll
-  for (int cc = 0; cc < 3; cc++) s[cc] = load_sn<double>(a, m, d, cc);
-  if (al > a1 && al < a2) {
+  for (int e = 0; e < 4; e++) ub0[e] = B.ub[(e + 1) * ldv + n];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      double fv = gq<double>(a, q, m) + gq<double>(a, q, m - inc), fvb = 0.;
+  for (int x = 0; x < 3; x++) u0[x] = Q[x * nnn + m];
 #pragma unroll
-      for (int cc = 0; cc < 3; cc++) {
-        const double *gb = bpl(a, B, B_G + 3 * q + cc);
-        double tb = gb[m - inc] - gb[m];
-        fvb += tb * s[cc];
-        sb[cc] += tb * fv;
-      }
-      atomicAdd(bpl(a, B, B_V + q) + m, fvb);
-      atomicAdd(bpl(a, B, B_V + q) + m - inc, fvb);
+  for (int x = 0; x < 9; x++) tb[x] = 0.;
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const long inc = b.inc(d);
+    const bool bnd[2] = {c[d] == b.lo(d), c[d] == b.hi(d) - 1};
+    double um[2][3];  // velocities of the neighbours below and above
+#pragma unroll
+    for (int x = 0; x < 3; x++) {
+      um[0][x] = Q[x * nnn + m - inc];
+      um[1][x] = Q[x * nnn + m + inc];
     }
-  } else {
-    bool lo = al == a1;
-    long mg = lo ? m - inc : m, mr = lo ? m : m - inc;
-    double sgn = lo ? -1. : 1.;
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      double gv = gq<double>(a, q, mg), gvb = 0.;
+    for (int side = 0; side < 2; side++) {
+      const long off = side ? inc : -inc;
+      const double sg = side ? 1. : -1.;
+      double s[3], w[4], u[3];
 #pragma unroll
-      for (int cc = 0; cc < 3; cc++) {
-        double tb = sgn * bpl(a, B, B_G + 3 * q + cc)[mr];
-        gvb += tb * s[cc] * 2.;
-        sb[cc] += tb * 2. * gv;
+      for (int x = 0; x < 3; x++) s[x] = load_sn<double>(a, side ? m + inc : m, d, x);
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        w[e] = bnd[side] ? sg * ub0[e] : 0.5 * sg * (ub0[e] - B.ub[(e + 1) * ldv + n + off]);
+      if (bnd[side]) {
+        const double ir = 1. / W[m + off];
+#pragma unroll
+        for (int x = 0; x < 3; x++) u[x] = W[(x + 1) * nnn + m + off] * ir;
+      } else {
+        // the MUSCL state of the cell's side: extrapolated toward the face
+#pragma unroll
+        for (int x = 0; x < 3; x++) u[x] = u0[x] + c4m * (u0[x] - um[1 - side][x]) + c4p * (um[side][x] - u0[x]);
       }
-      atomicAdd(bpl(a, B, B_V + q) + mg, gvb);
+      double y[3];
+#pragma unroll
+      for (int x = 0; x < 3; x++) y[x] = -(w[x] + w[3] * u[x]);
+      tb[0] += y[0] * s[0];
+      tb[1] += y[0] * s[1] + y[1] * s[0];
+      tb[2] += y[0] * s[2] + y[2] * s[0];
+      tb[3] += y[1] * s[1];
+      tb[4] += y[1] * s[2] + y[2] * s[1];
+      tb[5] += y[2] * s[2];
+#pragma unroll
+      for (int x = 0; x < 3; x++) tb[6 + x] -= w[3] * s[x];
     }
   }
+  // tq is linear in mu and in the scale c0 of the gradients
+  const double mu = a.ws[P_MU * nnn + m], vol = a.vol[n], c0 = grad_scale(vol);
+  double tt = 0.;
 #pragma unroll
-  for (int cc = 0; cc < 3; cc++) atomicAdd(B.snb + ((long)cc * 3 + d) * b.nnn + m, sb[cc]);
+  for (int x = 0; x < 9; x++) tt += tb[x] * a.ws[(P_TQ + x) * nnn + m];
+  bpl(a, B, B_MU)[m] = tt / mu;
+  B.volb[n] = signbit(vol) ? 0. : -tt / (vol + DBL_MIN);
+  const double mc = mu * c0, m3 = 2. / 3. * mc, kq = a.ph.cp * (mu / a.ph.pr) * c0;
+  const double g[9] = {m3 * (2. * tb[0] - tb[3] - tb[5]), mc * tb[1], mc * tb[2],
+                       m3 * (2. * tb[3] - tb[0] - tb[5]), mc * tb[4], m3 * (2. * tb[5] - tb[0] - tb[3]),
+                       kq * tb[6], kq * tb[7], kq * tb[8]};
+#pragma unroll
+  for (int x = 0; x < 9; x++) bpl(a, B, B_G + x)[m] = g[x];
 }
 
-// ghost rules transposed: adjoints of the ghost's W, q and T onto the
-// adjacent cell's conservative state, one Dual pass per input
+// plane (from B_G) of the adjoint of d(quantity q)/d(x_cc)
+__device__ inline constexpr int g_plane(int q, int cc) {
+  return q == 3 ? 6 + cc : (q + cc == 0 ? 0 : (q == cc ? (q == 1 ? 3 : 5) : q + cc + (q + cc == 3 ? 1 : 0)));
+}
+static_assert(g_plane(0, 1) == 1 && g_plane(2, 0) == 2 && g_plane(1, 1) == 3 && g_plane(1, 2) == 4 && g_plane(2, 2) == 5,
+              "xx xy xz yy yz zz");
+
+// Real cells, the last pass over them: the Green-Gauss sums of the cell's six
+// faces transposed (onto its own u, v, w, T; onto a boundary face's ghost;
+// onto the metrics of its low faces and of the block's high faces), the MUSCL
+// states' adjoints of the faces that reach the cell, and the thermodynamics
+// onto the conservative state.
+__global__ void __launch_bounds__(256) k_adjb_cells(AdjArgs a, AdjBar B) {
+#pragma clang fp contract(fast)
+  int c[3];
+  if (!real_cell(a.b, blockIdx.x * 256L + threadIdx.x, c)) return;
+  const Blk &b = a.b;
+  const long n = b.idx(c[0], c[1], c[2]), m = n - b.npc, nnn = b.nnn;
+  const MusclW mw = muscl_w(a);
+  double g0[9], q0[4], vb[4] = {0., 0., 0., 0.}, qb[5] = {0., 0., 0., 0., 0.};
+#pragma unroll
+  for (int x = 0; x < 9; x++) g0[x] = bpl(a, B, B_G + x)[m];
+#pragma unroll
+  for (int q = 0; q < 4; q++) q0[q] = gq<double>(a, q, m);
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const long inc = b.inc(d);
+    const int al = c[d], a1 = b.lo(d), a2 = b.hi(d);
+#pragma unroll
+    for (int side = 0; side < 2; side++) {
+      const bool bnd = side ? al == a2 - 1 : al == a1;
+      const long off = side ? inc : -inc, mf = side ? m + inc : m;
+      double s[3], t[9], sb[3] = {0., 0., 0.};
+#pragma unroll
+      for (int x = 0; x < 3; x++) s[x] = load_sn<double>(a, mf, d, x);
+      // adjoint of the face sums: low cell's less high cell's
+#pragma unroll
+      for (int x = 0; x < 9; x++) {
+        const double gn = bnd ? 0. : bpl(a, B, B_G + x)[m + off];
+        t[x] = side ? g0[x] - gn : gn - g0[x];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        double f = 0.;
+#pragma unroll
+        for (int x = 0; x < 3; x++) f += t[g_plane(q, x)] * s[x];
+        if (bnd) bpl(a, B, B_V + q)[m + off] = 2. * f;
+        else vb[q] += f;
+        if (side == 0 || bnd) {
+          const double fv = bnd ? 2. * gq<double>(a, q, m + off) : q0[q] + gq<double>(a, q, m + off);
+#pragma unroll
+          for (int x = 0; x < 3; x++) sb[x] += t[g_plane(q, x)] * fv;
+        }
+      }
+      if (side == 0 || bnd) {
+#pragma unroll
+        for (int x = 0; x < 3; x++) B.snb[((long)x * 3 + d) * nnn + mf] += sb[x];
+      }
+    }
+    // the cell is q1 of its high face, q2 of its low face, q0 of the face
+    // after the high one and q3 of the face before the low one
+#pragma unroll
+    for (int e = 0; e < 5; e++) {
+      const double *Lb = bpl(a, B, B_F + 10 * d + e), *Rb = Lb + 5 * nnn;
+      double r = mw.l2 * Lb[m] + mw.r2 * Rb[m] + mw.l1 * Lb[m + inc] + mw.r1 * Rb[m + inc];
+      if (al + 2 < a2) r += mw.l0 * Lb[m + 2 * inc];
+      if (al - 1 > a1) r += mw.r3 * Rb[m - inc];
+      qb[e] += r;
+    }
+  }
+  double w[5];
+  load_v(a, n, w);
+  const double ir = 1. / w[0], T = q0[3];
+  double Tb = vb[3];
+  if (a.ph.iflu == 1) Tb += bpl(a, B, B_MU)[m] * a.ws[P_MU * nnn + m] * (1.5 / T - 1. / (T + a.ph.asuth));
+  const double pb = qb[4] + Tb * a.ph.gam * ir, ep = a.ph.gam1 * pb;
+  double r0 = qb[0] - Tb * T * ir;
+#pragma unroll
+  for (int x = 0; x < 3; x++) {
+    const double xb = qb[1 + x] + vb[x];
+    B.vb[(1 + x) * a.ldv + n] = (xb - ep * w[1 + x]) * ir;
+    r0 -= (xb - 0.5 * ep * w[1 + x]) * q0[x] * ir;
+  }
+  B.vb[n] = r0;
+  B.vb[4 * a.ldv + n] = ep;
+}
+
+// Ghost rules transposed: adjoints of the ghost's W, q and T onto the
+// adjacent cell's conservative state, one Dual pass and one thread per input.
 template <int FAR>
 __global__ void __launch_bounds__(128) k_adjb_ghost(AdjArgs a, AdjBar B, long nf, const int64_t *__restrict__ g,
                                                     const int64_t *__restrict__ in, const double *__restrict__ nrm) {
-  long f = blockIdx.x * 128L + threadIdx.x;
-  if (f >= nf) return;
+  const long t = blockIdx.x * 128L + threadIdx.x;
+  if (t >= 5 * nf) return;
+  const long f = t % nf;
+  const int k = (int)(t / nf);
   const Blk &b = a.b;
-  long mg = g[f] - b.npc, ni = in[f];
+  const long mg = g[f] - b.npc, ni = in[f], nnn = b.nnn;
+  // the direction the ghost lies in, and the interior face whose MUSCL
+  // states reach it (where the block has one)
+  const int c[3] = {b.id1 + (int)(mg % b.nid), b.jd1 + (int)((mg / b.nid) % (b.nijd / b.nid)),
+                    b.kd1 + (int)(mg / b.nijd)};
+  const int d = (c[2] < b.k1 || c[2] >= b.k2) ? 2 : ((c[1] < b.j1 || c[1] >= b.j2) ? 1 : 0);
+  const bool lo = c[d] < b.lo(d);
+  const long inc = b.inc(d);
+  const MusclW mw = muscl_w(a);
   double wb[5], qb[5], tb;
 #pragma unroll
   for (int e = 0; e < 5; e++) {
+    const double *Lb = bpl(a, B, B_F + 10 * d + e), *Rb = Lb + 5 * nnn;
     wb[e] = bpl(a, B, B_W + e)[mg];
-    qb[e] = bpl(a, B, B_Q + e)[mg];
+    qb[e] = lo ? mw.l0 * Lb[mg + 2 * inc] : mw.r3 * Rb[mg - inc];
   }
+  qb[4] += bpl(a, B, B_W + 5)[mg];
 #pragma unroll
   for (int q = 0; q < 3; q++) qb[1 + q] += bpl(a, B, B_V + q)[mg];
   tb = bpl(a, B, B_V + 3)[mg];
   double vi[5];
   load_v(a, ni, vi);
-#pragma unroll 1
-  for (int k = 0; k < 5; k++) {
-    Dual vD[5], wg[5], qg[5], tg;
+  Dual vD[5], wg[5], qg[5], tg;
 #pragma unroll
-    for (int x = 0; x < 5; x++) vD[x] = mk(vi[x], k == x);
-    if (FAR)
-      far_ghost(a.ph, a.w0, nrm[f], nrm[nf + f], nrm[2 * nf + f], vD, wg, qg, tg);
-    else
-      wall_ghost(a.ph, vD, wg, qg, tg);
-    double acc = tb * tg.d;
+  for (int x = 0; x < 5; x++) vD[x] = mk(vi[x], k == x);
+  if (FAR)
+    far_ghost(a.ph, a.w0, nrm[f], nrm[nf + f], nrm[2 * nf + f], vD, wg, qg, tg);
+  else
+    wall_ghost(a.ph, vD, wg, qg, tg);
+  double acc = tb * tg.d;
 #pragma unroll
-    for (int e = 0; e < 5; e++) acc += wb[e] * wg[e].d + qb[e] * qg[e].d;
-    atomicAdd(B.vb + k * a.ldv + ni, acc);
-  }
+  for (int e = 0; e < 5; e++) acc += wb[e] * wg[e].d + qb[e] * qg[e].d;
+  atomicAdd(B.vb + k * a.ldv + ni, acc);
 }
 
-// real cells: primitive state, T and mu onto the conservative state
-__global__ void __launch_bounds__(128) k_adjb_thermo(AdjArgs a, AdjBar B) {
-  int c[3];
-  if (!real_cell(a.b, blockIdx.x * 128L + threadIdx.x, c)) return;
-  const Blk &b = a.b;
-  long n = b.idx(c[0], c[1], c[2]), m = n - b.npc;
-  double qb[5], tb = bpl(a, B, B_V + 3)[m], mub = bpl(a, B, B_MU)[m];
+// the entries of vb, snb and volb that no pass writes: snb of every entry
+// (the face pass writes the faces), vb and volb of the ghosts
+__global__ void __launch_bounds__(256) k_adjb_clear(Blk b, long ldv, double *vb, double *snb, double *volb) {
+  const long m = blockIdx.x * 256L + threadIdx.x;
+  if (m >= b.nnn) return;
 #pragma unroll
-  for (int e = 0; e < 5; e++) qb[e] = bpl(a, B, B_Q + e)[m];
+  for (int x = 0; x < 9; x++) snb[x * b.nnn + m] = 0.;
+  if (b.real(b.id1 + (int)(m % b.nid), b.jd1 + (int)((m / b.nid) % (b.nijd / b.nid)), b.kd1 + (int)(m / b.nijd)))
+    return;
 #pragma unroll
-  for (int q = 0; q < 3; q++) qb[1 + q] += bpl(a, B, B_V + q)[m];
-  double w[5];
-  load_v(a, n, w);
-#pragma unroll 1
-  for (int k = 0; k < 5; k++) {
-    Dual wD[5], p, tt, mu;
-#pragma unroll
-    for (int x = 0; x < 5; x++) wD[x] = mk(w[x], k == x);
-    thermo(a.ph, wD, p, tt, mu);
-    Dual q[5] = {wD[0], wD[1] / wD[0], wD[2] / wD[0], wD[3] / wD[0], p};
-    double acc = tb * tt.d + mub * mu.d;
-#pragma unroll
-    for (int e = 0; e < 5; e++) acc += qb[e] * q[e].d;
-    B.vb[k * a.ldv + n] += acc;
-  }
+  for (int e = 0; e < 5; e++) vb[e * ldv + b.npc + m] = 0.;
+  volb[b.npc + m] = 0.;
 }
 
 __global__ void k_adj_zero(double *p, long cnt) {
   long i = blockIdx.x * 256L + threadIdx.x;
   if (i < cnt) p[i] = 0.;
-}
-
-// np planes of leading dimension ld, entries off .. off+cnt-1
-__global__ void k_adj_zero_planes(double *p, long ld, int np, long off, long cnt) {
-  long i = blockIdx.x * 256L + threadIdx.x;
-  if (i >= cnt * np) return;
-  p[(i / cnt) * ld + off + i % cnt] = 0.;
 }
 
 // ---------------------------------------------------------------------------
@@ -1142,7 +1183,6 @@ void forward_chain(const AdjArgs &a, long nwall, const int64_t *wg, const int64_
   if (nwall) hipLaunchKernelGGL((k_adj_ghost<T, 0>), dim3(nblk(nwall, 256)), dim3(256), 0, st, a, nwall, wg, wi, fn);
   if (nfar) hipLaunchKernelGGL((k_adj_ghost<T, 1>), dim3(nblk(nfar, 256)), dim3(256), 0, st, a, nfar, fg, fi, fn);
   hipLaunchKernelGGL(k_adj_grad<T>, dim3(nblk(ncell, 256)), dim3(256), 0, st, a);
-  hipLaunchKernelGGL(k_adj_tq<T>, dim3(nblk(ncell, 256)), dim3(256), 0, st, a);
   if (nwall) hipLaunchKernelGGL(k_adj_tq_ghost<T>, dim3(nblk(nwall, 256)), dim3(256), 0, st, a, nwall, wg, wi);
   if (nfar) hipLaunchKernelGGL(k_adj_tq_ghost<T>, dim3(nblk(nfar, 256)), dim3(256), 0, st, a, nfar, fg, fi);
 }
@@ -1203,42 +1243,32 @@ extern "C" int codens_adj_residual_vjp(const codens_block *cb, const codens_phys
     return CODENS_EINVAL;
   }
   long nnn = a.b.nnn;
-  double *ws = (double *)codens_workspace(sizeof(double) * (NPLANE + NBPLANE) * nnn, 8);
+  double *ws = (double *)codens_workspace(sizeof(double) * (NVPLANE + NBPLANE) * nnn, 8);
   if (!ws) {
     codens_set_error("%s: workspace allocation failed", what);
     return CODENS_EHIP;
   }
   hipStream_t st = (hipStream_t)stream;
   a.ws = ws;
-  AdjBar B{ws + NPLANE * nnn, ubar, vbar, snbar, volbar};
-  hipLaunchKernelGGL(k_adj_zero, dim3(nblk((NPLANE + NBPLANE) * nnn, 256)), dim3(256), 0, st, ws,
-                     (NPLANE + NBPLANE) * nnn);
-  // results are overwritten on the block's entries
-  hipLaunchKernelGGL(k_adj_zero_planes, dim3(nblk(5 * nnn, 256)), dim3(256), 0, st, vbar, (long)ldv, 5,
-                     (long)a.b.npc, nnn);
-  hipLaunchKernelGGL(k_adj_zero, dim3(nblk(9 * nnn, 256)), dim3(256), 0, st, snbar, 9 * nnn);
-  hipLaunchKernelGGL(k_adj_zero_planes, dim3(nblk(nnn, 256)), dim3(256), 0, st, volbar, nnn, 1, (long)a.b.npc,
-                     nnn);
+  AdjBar B{ws + NVPLANE * nnn, ubar, vbar, snbar, volbar};
+  const Blk &b = a.b;
+  const long ni = b.i2 - b.i1, nj = b.j2 - b.j1, nk = b.k2 - b.k1, ncell = ni * nj * nk;
+  // every plane entry that is read is written before, except a ghost that
+  // neither list names
+  if (nwall + nfar < 2 * (ni * nj + nj * nk + ni * nk))
+    hipLaunchKernelGGL(k_adj_zero, dim3(nblk(NVPLANE * nnn, 256)), dim3(256), 0, st, ws, NVPLANE * nnn);
+  hipLaunchKernelGGL(k_adjb_clear, dim3(nblk(nnn, 256)), dim3(256), 0, st, b, (long)ldv, vbar, snbar, volbar);
   forward_chain<double>(a, nwall, wall_ghost, wall_inner, nfar, far_ghost, far_inner, far_nrm, st);
-  long ncell = (long)(a.b.i2 - a.b.i1) * (a.b.j2 - a.b.j1) * (a.b.k2 - a.b.k1);
-  for (int d = 0; d < 3; d++)
-    hipLaunchKernelGGL(k_adjb_faces, dim3(nblk(nfaces(a.b, d), 128)), dim3(128), 0, st, a, B, d);
+  const unsigned nf0 = nblk(nfaces(b, 0), 128), nf1 = nblk(nfaces(b, 1), 128), nf2 = nblk(nfaces(b, 2), 128);
+  hipLaunchKernelGGL(k_adjb_faces, dim3(nf0 + nf1 + nf2), dim3(128), 0, st, a, B, nf0, nf1);
+  hipLaunchKernelGGL(k_adjb_tq, dim3(nblk(ncell, 256)), dim3(256), 0, st, a, B);
+  hipLaunchKernelGGL(k_adjb_cells, dim3(nblk(ncell, 256)), dim3(256), 0, st, a, B);
   if (nwall)
-    hipLaunchKernelGGL(k_adjb_tq_ghost, dim3(nblk(nwall, 256)), dim3(256), 0, st, a, B, (long)nwall, wall_ghost,
-                       wall_inner);
-  if (nfar)
-    hipLaunchKernelGGL(k_adjb_tq_ghost, dim3(nblk(nfar, 256)), dim3(256), 0, st, a, B, (long)nfar, far_ghost,
-                       far_inner);
-  hipLaunchKernelGGL(k_adjb_tq, dim3(nblk(ncell, 128)), dim3(128), 0, st, a, B);
-  for (int d = 0; d < 3; d++)
-    hipLaunchKernelGGL(k_adjb_grad, dim3(nblk(nfaces(a.b, d), 256)), dim3(256), 0, st, a, B, d);
-  if (nwall)
-    hipLaunchKernelGGL(k_adjb_ghost<0>, dim3(nblk(nwall, 128)), dim3(128), 0, st, a, B, (long)nwall, wall_ghost,
+    hipLaunchKernelGGL(k_adjb_ghost<0>, dim3(nblk(5 * nwall, 128)), dim3(128), 0, st, a, B, (long)nwall, wall_ghost,
                        wall_inner, far_nrm);
   if (nfar)
-    hipLaunchKernelGGL(k_adjb_ghost<1>, dim3(nblk(nfar, 128)), dim3(128), 0, st, a, B, (long)nfar, far_ghost,
+    hipLaunchKernelGGL(k_adjb_ghost<1>, dim3(nblk(5 * nfar, 128)), dim3(128), 0, st, a, B, (long)nfar, far_ghost,
                        far_inner, far_nrm);
-  hipLaunchKernelGGL(k_adjb_thermo, dim3(nblk(ncell, 128)), dim3(128), 0, st, a, B);
   return codens_check_launch(what);
 }
 
