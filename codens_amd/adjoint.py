@@ -147,7 +147,7 @@ class AdjointProblem:
         """(snbar, volbar) -> adjoint of the wall displacements, at the nodes
         xyz (with their ghost layer) the metrics were formed from."""
         nnn = self.b.nnn
-        bars = [torch.zeros(nnn, dtype=torch.float64, device="cuda") for _ in range(3)]
+        bars = [torch.empty(nnn, dtype=torch.float64, device="cuda") for _ in range(3)]
         abi.adj_metric_vjp(self.blk, *xyz, self.sg, snbar.contiguous(), volbar.contiguous(), *bars)
         yb = _fold_ghost_nodes(self.b, bars[1].view(self.b.nkd, self.b.njd, self.b.nid))
         return yb.reshape(-1)[self.wall_local]
@@ -157,13 +157,14 @@ class AdjointProblem:
         """u(v) of the production kernels (real cells; zero elsewhere)."""
         S = self.S
         S.v.copy_(v)
+        S.u = torch.zeros_like(S.v)  # the caller's: sch_roe writes the real cells and zeroes the ghosts
         S.sn_blk = [sn_blk.contiguous()]
         S.vol = vol.contiguous()
         S.thermo()
         S.ghosts()
         S.stresses()
         S.residual()
-        return S.u[:5] * self.real
+        return S.u[:5]
 
     def jvp(self, v, sn_blk, vol, vd, snd, vold):
         z = lambda t, like: torch.zeros_like(like) if t is None else t.contiguous()
@@ -173,13 +174,14 @@ class AdjointProblem:
         return u, ud
 
     def vjp(self, v, sn_blk, vol, ubar):
-        vb = torch.zeros_like(v)
-        snb = torch.zeros_like(sn_blk)
-        volb = torch.zeros_like(vol)
-        ub = torch.zeros((5, v.shape[-1]), dtype=torch.float64, device="cuda")
-        ub.copy_(ubar[:5] * self.real)
+        # the call overwrites every entry of a one-block layout (planes past
+        # the fifth aside) and reads ubar on the real cells only
+        vb = torch.empty_like(v, memory_format=torch.contiguous_format)
+        vb[5:] = 0.
+        snb = torch.empty_like(sn_blk, memory_format=torch.contiguous_format)
+        volb = torch.empty_like(vol, memory_format=torch.contiguous_format)
         abi.adj_residual_vjp(self.blk, self.ph, self.sc, v.contiguous(), sn_blk.contiguous(), vol.contiguous(),
-                             self.winf, self.bcs, ub, vb[:5] if v.shape[0] > 5 else vb, snb, volb)
+                             self.winf, self.bcs, ubar[:5].contiguous(), vb[:5], snb, volb)
         return vb, snb, volb
 
     # -- the step and the objective -----------------------------------------
@@ -189,7 +191,7 @@ class AdjointProblem:
         v = v0
         for a in RK_ALPHA:
             u = Residual.apply(v, sn_blk, vol, self)
-            v = v0 - a * c * u
+            v = torch.addcmul(v0, c, u, value=-a)
         return v
 
     def objective(self, v, sn_blk):

@@ -1051,101 +1051,63 @@ struct MArgs {
   const double *x, *y, *z;
   double sg[3];
   double *xb, *yb, *zb;
-  long nid, njd, nkd;
 };
 
-// storage offset of node (i, j, k) counted from the block's first entry
-__device__ inline long nodeo(const MArgs &M, long i, long j, long k) { return i + M.nid * (j + M.njd * k); }
-
-__device__ inline void corner_ofs(int d, int q, int &di, int &dj, int &dk) {
-  // svol.f90 face corners: k faces (0,0,0)(1,0,0)(0,1,0)(1,1,0); j faces
-  // (0,0,0)(1,0,0)(0,0,1)(1,0,1); i faces (0,0,0)(0,1,0)(0,0,1)(0,1,1)
-  const int K[4][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {1, 1, 0}};
-  const int J[4][3] = {{0, 0, 0}, {1, 0, 0}, {0, 0, 1}, {1, 0, 1}};
-  const int I[4][3] = {{0, 0, 0}, {0, 1, 0}, {0, 0, 1}, {0, 1, 1}};
-  const int(*T)[3] = d == 2 ? K : (d == 1 ? J : I);
-  di = T[q][0]; dj = T[q][1]; dk = T[q][2];
-}
-
-// the two half-diagonals of a face: d1 = P(e1) - P(0), d2 = P(e2) - P(e3)
-__device__ inline void diag_ofs(int d, int e[3][3]) {
-  if (d == 2) {
-    int t[3][3] = {{1, 1, 0}, {0, 1, 0}, {1, 0, 0}};
-    for (int a = 0; a < 3; a++) for (int c = 0; c < 3; c++) e[a][c] = t[a][c];
-  } else if (d == 1) {
-    int t[3][3] = {{1, 0, 1}, {0, 0, 1}, {1, 0, 0}};
-    for (int a = 0; a < 3; a++) for (int c = 0; c < 3; c++) e[a][c] = t[a][c];
-  } else {
-    int t[3][3] = {{0, 1, 1}, {0, 0, 1}, {0, 1, 0}};
-    for (int a = 0; a < 3; a++) for (int c = 0; c < 3; c++) e[a][c] = t[a][c];
+// One node: the faces it is a corner of (four per direction), each with its
+// metric sn = sg d1 x d2 (d1, d2 the half-diagonals P(pq) - P(0) and P(q) -
+// P(p), p < q the face's own directions) and its part of the volumes, the
+// face sum (P(0) + P(p) + P(q) + P(pq)) . sn with weight 1/12 in the cell
+// below and -1/12 in the one above, transposed onto the node.  Every face is
+// formed by its four corners instead of scattered to them: 60 operations
+// against 24 atomic adds.
+__global__ void __launch_bounds__(256) k_madj_nodes(MArgs M, const double *__restrict__ snb,
+                                                    const double *__restrict__ volb) {
+  const Blk &b = M.b;
+  const long o = blockIdx.x * 256L + threadIdx.x, nnn = b.nnn;
+  if (o >= nnn) return;
+  const int nn[3] = {(int)b.nid, (int)(b.nijd / b.nid), (int)(nnn / b.nijd)};
+  const int c[3] = {(int)(o % b.nid), (int)((o / b.nid) % nn[1]), (int)(o / b.nijd)};
+  const double *P[3] = {M.x + b.npc, M.y + b.npc, M.z + b.npc};
+  double nb[3] = {0., 0., 0.};
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const int p = d == 0 ? 1 : 0, q = d == 2 ? 1 : 2;
+    const long id = b.inc(d), ip = b.inc(p), iq = b.inc(q);
+#pragma unroll
+    for (int corner = 0; corner < 4; corner++) {  // the node is P(0), P(p), P(q), P(pq) of the face
+      const int cp = corner & 1, cq = corner >> 1;
+      const int fp = c[p] - cp, fq = c[q] - cq;
+      if (fp < 0 || fq < 0 || fp >= nn[p] - 1 || fq >= nn[q] - 1) continue;
+      const long f = o - cp * ip - cq * iq;
+      double d1[3], d2[3], cs[3];
+#pragma unroll
+      for (int x = 0; x < 3; x++) {
+        const double p0 = P[x][f], p1 = P[x][f + ip], p2 = P[x][f + iq], p3 = P[x][f + ip + iq];
+        d1[x] = p3 - p0;
+        d2[x] = p2 - p1;
+        cs[x] = ((p0 + p1) + p2) + p3;
+      }
+      double fb = 0.;  // adjoint of the face sum
+      if (c[d] > 0) fb += volb[b.npc + f - id];
+      if (c[d] < nn[d] - 1) fb -= volb[b.npc + f];
+      fb *= 0.25 / 3.;
+      double tb[3];
+#pragma unroll
+      for (int x = 0; x < 3; x++) tb[x] = M.sg[d] * (snb[((long)x * 3 + d) * nnn + f] + fb * cs[x]);
+      const double sgn = M.sg[d] * fb;
+#pragma unroll
+      for (int x = 0; x < 3; x++) {
+        const int y = (x + 1) % 3, z = (x + 2) % 3;
+        const double sn = d1[y] * d2[z] - d1[z] * d2[y];
+        // d1b = d2 x tb on P(pq) - P(0); d2b = tb x d1 on P(q) - P(p)
+        const double e = cp == cq ? d2[y] * tb[z] - d2[z] * tb[y] : tb[y] * d1[z] - tb[z] * d1[y];
+        nb[x] += sgn * sn + (cq ? e : -e);
+      }
+    }
   }
-}
-
-// volume adjoints onto the six face sums of each cell: vol = (1/12) x
-// (s_i(i+1) - s_i(i) + s_j(j+1) - s_j(j) + s_k(k+1) - s_k(k))
-__global__ void __launch_bounds__(256) k_madj_vol(MArgs M, const double *__restrict__ volb, double *fsb) {
-  long t = blockIdx.x * 256L + threadIdx.x;
-  long nc = (M.nid - 1) * (M.njd - 1) * (M.nkd - 1);
-  if (t >= nc) return;
-  long i = t % (M.nid - 1), j = (t / (M.nid - 1)) % (M.njd - 1), k = t / ((M.nid - 1) * (M.njd - 1));
-  long o = nodeo(M, i, j, k), nnn = M.b.nnn;
-  double vb = volb[M.b.npc + o] * (0.25 / 3.);
-  atomicAdd(fsb + o + 1, vb);
-  atomicAdd(fsb + o, -vb);
-  atomicAdd(fsb + nnn + o + M.nid, vb);
-  atomicAdd(fsb + nnn + o, -vb);
-  atomicAdd(fsb + 2 * nnn + o + M.nid * M.njd, vb);
-  atomicAdd(fsb + 2 * nnn + o, -vb);
-}
-
-// one face of direction d: face sum and cross product transposed onto the
-// nodes (snb: the metric adjoint, 9 x nnn, block-local)
-__global__ void __launch_bounds__(256) k_madj_face(MArgs M, int d, const double *__restrict__ snb,
-                                                   const double *__restrict__ fsb) {
-  long t = blockIdx.x * 256L + threadIdx.x;
-  long n0 = M.nid - (d != 0), n1 = M.njd - (d != 1), n2 = M.nkd - (d != 2);
-  if (t >= n0 * n1 * n2) return;
-  long i = t % n0, j = (t / n0) % n1, k = t / (n0 * n1);
-  long o = nodeo(M, i, j, k), nnn = M.b.nnn;
-  const double *P[3] = {M.x + M.b.npc, M.y + M.b.npc, M.z + M.b.npc};
-  double *PB[3] = {M.xb, M.yb, M.zb};
-  // sn of this face from the nodes
-  int e[3][3];
-  diag_ofs(d, e);
-  long oe1 = nodeo(M, i + e[0][0], j + e[0][1], k + e[0][2]);
-  long oe2 = nodeo(M, i + e[1][0], j + e[1][1], k + e[1][2]);
-  long oe3 = nodeo(M, i + e[2][0], j + e[2][1], k + e[2][2]);
-  double d1[3], d2[3];
-  for (int c = 0; c < 3; c++) {
-    d1[c] = P[c][oe1] - P[c][o];
-    d2[c] = P[c][oe2] - P[c][oe3];
-  }
-  double sn[3] = {M.sg[d] * (d1[1] * d2[2] - d1[2] * d2[1]), M.sg[d] * (d1[2] * d2[0] - d1[0] * d2[2]),
-                  M.sg[d] * (d1[0] * d2[1] - d1[1] * d2[0])};
-  // face sum fs = sum_c (P0 + P1 + P2 + P3)_c sn_c
-  double fb = fsb[(long)d * nnn + o];
-  double snbar[3];
-  long oc[4];
-  for (int q = 0; q < 4; q++) {
-    int di, dj, dk;
-    corner_ofs(d, q, di, dj, dk);
-    oc[q] = nodeo(M, i + di, j + dj, k + dk);
-  }
-  for (int c = 0; c < 3; c++) {
-    double cs = ((P[c][oc[0]] + P[c][oc[1]]) + P[c][oc[2]]) + P[c][oc[3]];
-    snbar[c] = snb[((long)c * 3 + d) * nnn + o] + fb * cs;
-    for (int q = 0; q < 4; q++) atomicAdd(PB[c] + oc[q], fb * sn[c]);
-  }
-  // sn = sg (d1 x d2): d1b = d2 x tb, d2b = tb x d1 with tb = sg snbar
-  double tb[3] = {M.sg[d] * snbar[0], M.sg[d] * snbar[1], M.sg[d] * snbar[2]};
-  double d1b[3] = {d2[1] * tb[2] - d2[2] * tb[1], d2[2] * tb[0] - d2[0] * tb[2], d2[0] * tb[1] - d2[1] * tb[0]};
-  double d2b[3] = {tb[1] * d1[2] - tb[2] * d1[1], tb[2] * d1[0] - tb[0] * d1[2], tb[0] * d1[1] - tb[1] * d1[0]};
-  for (int c = 0; c < 3; c++) {
-    atomicAdd(PB[c] + oe1, d1b[c]);
-    atomicAdd(PB[c] + o, -d1b[c]);
-    atomicAdd(PB[c] + oe2, d2b[c]);
-    atomicAdd(PB[c] + oe3, -d2b[c]);
-  }
+  M.xb[o] = nb[0];
+  M.yb[o] = nb[1];
+  M.zb[o] = nb[2];
 }
 
 inline unsigned nblk(long n, int t) { return (unsigned)((n + t - 1) / t); }
@@ -1287,21 +1249,6 @@ extern "C" int codens_adj_metric_vjp(const codens_block *cb, const double *x, co
   M.x = x; M.y = y; M.z = z;
   for (int d = 0; d < 3; d++) M.sg[d] = sg3[d];
   M.xb = xbar; M.yb = ybar; M.zb = zbar;
-  M.nid = M.b.nid; M.njd = M.b.nijd / M.b.nid; M.nkd = M.b.nnn / M.b.nijd;
-  long nnn = M.b.nnn;
-  double *fsb = (double *)codens_workspace(sizeof(double) * 3 * nnn, 9);
-  if (!fsb) {
-    codens_set_error("%s: workspace allocation failed", what);
-    return CODENS_EHIP;
-  }
-  hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_adj_zero, dim3(nblk(3 * nnn, 256)), dim3(256), 0, st, fsb, 3 * nnn);
-  for (double *pb : {xbar, ybar, zbar}) hipLaunchKernelGGL(k_adj_zero, dim3(nblk(nnn, 256)), dim3(256), 0, st, pb, nnn);
-  long nc = (M.nid - 1) * (M.njd - 1) * (M.nkd - 1);
-  hipLaunchKernelGGL(k_madj_vol, dim3(nblk(nc, 256)), dim3(256), 0, st, M, volbar, fsb);
-  for (int d = 0; d < 3; d++) {
-    long nf = (M.nid - (d != 0)) * (M.njd - (d != 1)) * (M.nkd - (d != 2));
-    hipLaunchKernelGGL(k_madj_face, dim3(nblk(nf, 256)), dim3(256), 0, st, M, d, snbar, fsb);
-  }
+  hipLaunchKernelGGL(k_madj_nodes, dim3(nblk(M.b.nnn, 256)), dim3(256), 0, (hipStream_t)stream, M, snbar, volbar);
   return codens_check_launch(what);
 }
