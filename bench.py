@@ -24,9 +24,10 @@ tests/golden/converged_wall_32x16x8.npz), FP64 implicit phase and FP32
 defect correction; `value` is the FP32 run's cell-updates/s to the drop.
 
 Prints one JSON line: Mcell-updates/s, the roofline of the dominant kernel
-(implimf_sweep: 264 algorithmic bytes per real cell per launch) measured with
-HIP events on the launch stream, and the reference Fortran build timed on the
-host on a bounded sample of the same workload.
+(implimf_sweep2, two sub-iterations in one pass, or implimf_sweep: 264
+algorithmic bytes per real cell per launch) measured with HIP events on the
+launch stream, and the reference Fortran build timed on the host on a bounded
+sample of the same workload.
 """
 import argparse
 import json
@@ -41,8 +42,9 @@ SWEEP_BYTES_PER_CELL = 8 * (5 + 5 + 5 + 9 + 1 + 3 + 5)  # u, v, d_in, sn, diag, 
 # Memory traffic of one sweep launch on the 256x128x64 workload: 2.0 x FETCH_SIZE
 # + 1.0 x WRITE_SIZE (factors from a 512 MiB device copy in the same run),
 # 658,503 KiB = 674.3 MB against 553.6 MB algorithmic (64x4 tiles)
-# (profiles/traffic_wall_ns_256x128x64.md).
-SWEEP_TRAFFIC_BYTES = 658503 * 1024
+# (profiles/traffic_wall_ns_256x128x64.md); of two sub-iterations in one
+# launch 645,000 KiB, with the same factors.
+SWEEP_TRAFFIC_BYTES = {"implimf_sweep": 658503 * 1024, "implimf_sweep2": 645000 * 1024}
 HBM_PEAK_GBS = 8000.0
 
 
@@ -90,10 +92,10 @@ def cpu_allcores(case, stages, sample=None):
 
 
 # kernels (or launch groups) timed with HIP events on the launch stream
-TIMED_KERNELS = ("implimf_sweep", "implimf_sweep1", "implimf_coef", "implimf_update", "implimf32_sweep",
-                 "implimf32_sweep1", "implimf32_coef", "implimf32_update", "roe_prim", "roe_limiter_chain",
-                 "roe_face_flux", "roe_gather", "roe_fused", "roe_zero_ghost", "zvisqc", "chronos", "zpres",
-                 "zvismo")
+TIMED_KERNELS = ("implimf_sweep", "implimf_sweep2", "implimf_sweep1", "implimf_coef", "implimf_update",
+                 "implimf32_sweep", "implimf32_sweep1", "implimf32_coef", "implimf32_update", "roe_prim",
+                 "roe_limiter_chain", "roe_face_flux", "roe_gather", "roe_fused", "roe_zero_ghost", "zvisqc",
+                 "chronos", "zpres", "zvismo")
 
 
 def main():
@@ -188,11 +190,21 @@ def main():
     sweep_name = "implimf32_sweep" if fp32 else "implimf_sweep"
     sweep_bytes = SWEEP_BYTES_PER_CELL // 2 if fp32 else SWEEP_BYTES_PER_CELL  # the same 33 values in FP32
     n_timing = max(3, args.steps // 4)
+    # the launches of two sub-iterations at once, where there are any: each
+    # moves what one sub-iteration's does, so that passes over the cells, not
+    # sub-iterations, make the bytes
+    sw2 = kern.get("implimf_sweep2")
     sw = kern.get(sweep_name, {"avg_us": float("nan"), "launches": nblk * (case.lmax - 1) * n_timing})
     # bytes of all sweep launches over their summed time: the timing stages
     # sweep every cell lmax-1 times, in one launch per block and
     # sub-iteration, or one per sub-iteration when the blocks are batched
-    cells_per_launch = ncell * (case.lmax - 1) * n_timing / sw["launches"]
+    if sw2:
+        singles = kern[sweep_name]["launches"] if sweep_name in kern else 0
+        passes = sw2["launches"] / (singles + 2 * sw2["launches"]) * (case.lmax - 1) * n_timing
+        sweep_name, sw = "implimf_sweep2", sw2
+    else:
+        passes = (case.lmax - 1) * n_timing
+    cells_per_launch = ncell * passes / sw["launches"]
     achieved = sweep_bytes * cells_per_launch / (sw["avg_us"] * 1e-6) / 1e9
     out = {
         "metric": "Mcell-updates/s per implicit iter to 1e-8 residual drop; % of HBM roofline",
@@ -215,7 +227,7 @@ def main():
                        if nblk == 1 else "per block")},
         "roofline": {"bound": "hbm", "kernel": sweep_name, "achieved": round(achieved, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": SWEEP_TRAFFIC_BYTES if (ci, cj, ck) == (256, 128, 64) and not fp32 and not multi
+                     "traffic": SWEEP_TRAFFIC_BYTES.get(sweep_name) if (ci, cj, ck) == (256, 128, 64) and not multi
                      else None,
                      "bytes_per_cell": sweep_bytes,
                      "avg_us": round(sw["avg_us"], 2), "cells_per_launch": round(cells_per_launch)},

@@ -186,6 +186,23 @@ __device__ __forceinline__ int tab_find(const E *__restrict__ tab, int nb, int p
   return lo;
 }
 
+// A block from a table, whose loads the compiler does not know to be uniform,
+// in scalar registers.
+__device__ __forceinline__ long uniform_long(long x) {
+  const unsigned lo = __builtin_amdgcn_readfirstlane((int)x), hi = __builtin_amdgcn_readfirstlane((int)(x >> 32));
+  return (long)(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ Blk uniform_blk(const Blk &t) {
+  Blk b;
+  b.npc = uniform_long(t.npc); b.nid = uniform_long(t.nid); b.nijd = uniform_long(t.nijd); b.nnn = uniform_long(t.nnn);
+  b.id1 = __builtin_amdgcn_readfirstlane(t.id1); b.jd1 = __builtin_amdgcn_readfirstlane(t.jd1);
+  b.kd1 = __builtin_amdgcn_readfirstlane(t.kd1);
+  b.i1 = __builtin_amdgcn_readfirstlane(t.i1); b.i2 = __builtin_amdgcn_readfirstlane(t.i2);
+  b.j1 = __builtin_amdgcn_readfirstlane(t.j1); b.j2 = __builtin_amdgcn_readfirstlane(t.j2);
+  b.k1 = __builtin_amdgcn_readfirstlane(t.k1); b.k2 = __builtin_amdgcn_readfirstlane(t.k2);
+  return b;
+}
+
 // workgroup wg's tile within its block's own grid
 template <typename E>
 __device__ __forceinline__ dim3 tab_tile(const E &e, int pass, unsigned wg) {

@@ -4,7 +4,9 @@
 // sub-iterations.  Here every sub-iteration is one kernel that re-derives dF
 // of a cell and of its six neighbours from v and the previous increment d:
 // per sub-iteration a cell moves u, v, d_old, sn, diag, coefe and d_new through
-// HBM (33 doubles) instead of also streaming nine dF arrays in and out.
+// HBM (33 doubles) instead of also streaming nine dF arrays in and out.  In
+// FP64, on all but small blocks, two sub-iterations share that pass
+// (k_impl_sweep2).
 // Because every read of d and dF in a sub-iteration sees the previous
 // sub-iteration's values (implimf_3d.f90:230-431), the cells are independent
 // and any traversal order gives the reference's result.
@@ -622,6 +624,342 @@ __global__ void __launch_bounds__(TXS *TYS) SW_ATTR k_impl_sweep_tiled(Blk b, Ph
 #include "sweep_tile.inc"
 }
 
+// plane-relative load: base is uniform (the plane's first entry), off the
+// cell's 32-bit byte offset in the plane, so that the address is a scalar base
+// and one register (a plane of more than 2^29 entries would take a block of
+// more than 2^31).  The empty asm keeps the compiler from folding the uniform
+// part into per-thread 64-bit addresses.
+template <typename T>
+using GPtr = __attribute__((address_space(1))) T *;
+template <typename T>
+__device__ __forceinline__ GPtr<T> gp(T *base, unsigned off) {
+  uint64_t p = (uint64_t)base;
+  asm("" : "+s"(p));
+  return (GPtr<T>)((GPtr<char>)p + off);
+}
+template <typename T>
+__device__ __forceinline__ T ldp(const T *base, unsigned off) {
+  return *gp(base, off);
+}
+// Hides an offset's value from the loop optimiser, which would otherwise keep
+// a 64-bit address per array and thread in registers and advance them all.
+__device__ __forceinline__ unsigned opaque(unsigned x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// ---------------------------------------------------------------------------
+// Two sub-iterations A and B in one pass over the operands, which are most of
+// a sub-iteration's traffic (33 doubles per cell, of which the increments are
+// ten).  A workgroup's 32 x 16 threads each own a cell; A is right on all but
+// the outermost ring, B on all but two, so the tile writes 28 x 12 cells.
+// Marching k, plane k of A gives plane k - 1 of B its last part, so that B
+// uses the operands of plane k right after A, and carries five sums and a
+// reciprocal per cell to the next plane.  A's and B's 14-vectors of a plane lie
+// in LDS buffers of their own; a wave holds two rows.
+//
+// Every cell's operations are those of sweep_tile.inc in the same order, the
+// fused multiply-adds that the compiler forms there written out, so that a
+// pair gives the bits of two single sweeps (the minmod chains turn a change of
+// the last bit of the state into 1e-7 of the next residual).  The term of an
+// i face is formed by the cell above it and passed down a lane.
+//
+// One workgroup per CU (135 KB of LDS, 236 registers, two waves per SIMD).  On
+// 256 x 128 x 64 a pair takes 190 us and moves 660 MB, against 2 x 125 us for
+// single sweeps of 674 MB each, at 5.4 TB/s, what a large copy reaches; a pair's
+// waves issue or wait for arithmetic and LDS half of the time.  With workgroup barriers in place of
+// the flags below it took 225 us, with the i and j faces' operands loaded at
+// the top of their plane instead of during the plane below 199 us.
+constexpr int S2_TX = 32, S2_TY = 16, S2_NC = S2_TX * S2_TY, S2_OX = S2_TX - 4, S2_OY = S2_TY - 4;
+constexpr int S2_STASH = 5, S2_LDS = (28 + S2_STASH) * S2_NC;
+constexpr int S2_KS = 16;  // k planes per workgroup in the all-blocks launch
+
+// the value of the lane above
+__device__ __forceinline__ double lane_above(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x130 /* wave_shl:1 */, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x130, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// dflux with its fused multiply-adds written out
+__device__ __forceinline__ void dflux_q(const Phys &ph, const double V[5], const double D[5], double q[14]) {
+#pragma clang fp contract(off)
+  const double w0 = V[0] + D[0], w1 = V[1] + D[1], w2 = V[2] + D[2], w3 = V[3] + D[3], w4 = V[4] + D[4];
+  const double ri = 1. / w0, r0 = 1. / V[0];
+  const double u = w1 * ri, v = w2 * ri, w = w3 * ri;
+  const double kn = fma(w, w, fma(u, u, v * v));
+  const double xn = fma(-(0.5 * w0), kn, w4) - ph.pinfl, pn = ph.gam1 * xn;
+  const double a = V[1] * r0, b = V[2] * r0, c = V[3] * r0;
+  const double k0 = fma(V[3], c, fma(V[1], a, V[2] * b));
+  const double x0 = fma(-0.5, k0, V[4]) - ph.pinfl, p = ph.gam1 * x0;
+  const double e5 = fma(ph.gam1, x0, V[4]) - ph.pinfl, en = fma(ph.gam1, xn, w4) - ph.pinfl;
+  const double wu = w0 * u, wv = w0 * v;
+  q[0] = D[1]; q[1] = D[2]; q[2] = D[3];
+  q[3] = fma(w0, u * u, pn) - fma(V[1], a, p);
+  q[4] = fma(wu, v, -(V[2] * a));
+  q[5] = fma(wu, w, -(V[3] * a));
+  q[6] = fma(w0, v * v, pn) - fma(V[2], b, p);
+  q[7] = fma(wv, w, -(V[3] * b));
+  q[8] = fma(w0, w * w, pn) - fma(V[3], c, p);
+  q[9] = fma(u, en, -(e5 * a));
+  q[10] = fma(v, en, -(e5 * b));
+  q[11] = fma(w, en, -(e5 * c));
+  q[12] = D[0];
+  q[13] = D[4];
+}
+
+// Twice q_tn, with its fused multiply-adds written out: component by
+// component, q of the other cell taken by get(c).  The half is exact and goes
+// into the fused multiply-add that uses the term.  Of the first two products
+// of component e the first is the fused one, or the second if e is in SECOND.
+// The compiler fuses the second one in the all-blocks kernel's k faces and
+// nowhere else: in K_FACE on the upper face of a plane (which the plane above
+// takes over), in K_FIRST on the lower face of the first plane of a slab.
+constexpr int K_FACE = 1 << 2 | 1 << 3 | 1 << 4, K_FIRST = 1 << 1;
+template <int SECOND = 0, class Get>
+__device__ __forceinline__ void tn2_fma(const double A[14], const double s[3], double tn[5], Get get) {
+#pragma clang fp contract(off)
+  constexpr int C[5][3] = {{0, 1, 2}, {3, 4, 5}, {4, 6, 7}, {5, 7, 8}, {9, 10, 11}};
+  double x[12];
+#pragma unroll
+  for (int c = 0; c < 12; c++) x[c] = A[c] + get(c);
+#pragma unroll
+  for (int e = 0; e < 5; e++) {
+    const double a = x[C[e][0]], b = x[C[e][1]];
+    tn[e] = fma(x[C[e][2]], s[2], SECOND >> e & 1 ? fma(b, s[1], a * s[0]) : fma(a, s[0], b * s[1]));
+  }
+}
+
+// component of q that holds d of equation e
+__device__ __forceinline__ constexpr int q_comp(int e) { return e == 0 ? 12 : (e == 4 ? 13 : e - 1); }
+
+// BATCH: with the bits of the all-blocks launch's single sweeps
+template <bool FF, bool BATCH>
+__device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int nty, int ks, const Phys &ph,
+                                            const double *__restrict__ u, const double *__restrict__ ff,
+                                            const double *__restrict__ v, long ldv, const double *__restrict__ sn,
+                                            const double *__restrict__ coefe, const double *__restrict__ diag,
+                                            const DView dold, const DView dnew, double *sx, volatile int *flag) {
+#pragma clang fp contract(off)
+  const int bx = lg % ntx, by = (lg / ntx) % nty, bz = lg / (ntx * nty);
+  const int t = threadIdx.x, tx = t % S2_TX, ty = t / S2_TX;
+  const int i = b.i1 + bx * S2_OX - 2 + tx, j = b.j1 + by * S2_OY - 2 + ty;
+  const int kb = b.k1 + bz * ks, ke = min(kb + ks, b.k2);
+  const int ka = max(kb - 1, b.k1), kz = min(ke, b.k2 - 1);  // planes of A
+  const bool own = i >= b.i1 && i < b.i2 && j >= b.j1 && j < b.j2;
+  const bool out = own && tx >= 2 && tx < S2_TX - 2 && ty >= 2 && ty < S2_TY - 2;
+  const bool ireal = i + 1 < b.i2, jreal = j + 1 < b.j2;
+  // offset in a plane of this thread's cell, or of the nearest cell whose low
+  // faces exist (the first ghost past the real cells closes their last face)
+  auto plane = [&](int x, int y) { return ((unsigned)(x - b.id1) + (unsigned)(y - b.jd1) * (unsigned)b.nid) * 8u; };
+  const unsigned pl0 = plane(min(max(i, b.i1), b.i2), min(max(j, b.j1), b.j2 - 1));
+  // LDS slots of the neighbours (the thread's own at the tile's edge, where
+  // the result is not used)
+  const int tl = max(t - 1, 0), tr = min(t + 1, S2_NC - 1), td = max(t - S2_TX, tx), tu = min(t + S2_TX, S2_NC - S2_TX + tx);
+  double *const qA = sx, *const qB = sx + 14 * S2_NC, *const stash = sx + 28 * S2_NC + t;
+  auto st = [&](int x) -> double & { return stash[x * S2_NC]; };  // V of the plane
+  const long nnn = b.nnn, nijd = b.nijd;
+  constexpr int KF = BATCH ? K_FACE : 0, K1 = BATCH ? K_FIRST : 0;
+  auto first = [&](int k) { return (k - b.k1) % SW_KS == 0; };  // of a slab of the single sweeps
+  double qn[14], tkA[5], base[5], skl[3], ckl, rdb = 0.;  // qn: q of A's next plane
+  long mk = (long)(ka - b.kd1) * nijd;
+  auto load_vd = [&](long m, unsigned off, double V[5], double D[5]) {
+#pragma unroll
+    for (int e = 0; e < 5; e++) {
+      V[e] = ldp(v + (e * ldv + b.npc + m), off);
+      D[e] = ldp(dold.p + (e * dold.ld + (b.npc - dold.off) + m), off);
+    }
+  };
+  // own slots start as the plane below A's first: q of A there, zero of B
+  {
+    const unsigned pl = opaque(pl0);
+    double V[5], D[5], q[14];
+#pragma unroll
+    for (int c = 0; c < 14; c++) q[c] = qn[c] = 0.;
+#pragma unroll
+    for (int c = 0; c < 3; c++) skl[c] = ldp(sn + ((c * 3 + 2) * nnn + mk), pl);
+    ckl = ldp(coefe + (2 * nnn + mk), pl);
+    if (own && ka > b.k1) {
+      load_vd(mk - nijd, pl, V, D);
+      dflux_q(ph, V, D, q);
+    }
+    if (own) {
+      load_vd(mk, pl, V, D);
+      dflux_q(ph, V, D, qn);
+#pragma unroll
+      for (int e = 0; e < 5; e++) st(e) = V[e];
+    }
+    auto below = [&](int c) { return q[c]; };
+    if (BATCH && !first(ka)) tn2_fma<KF>(qn, skl, tkA, below);
+    else tn2_fma<K1>(qn, skl, tkA, below);
+#pragma unroll
+    for (int c = 0; c < 14; c++) {
+      qA[c * S2_NC + t] = q[c];
+      qB[c * S2_NC + t] = 0.;
+    }
+#pragma unroll
+    for (int e = 0; e < 5; e++) base[e] = 0.;
+  }
+  // A wave takes rows from the waves below and above it only, so it waits for
+  // those two to have written theirs instead of at a workgroup barrier: the
+  // waves of a SIMD then drift apart and one computes while the other waits
+  // for its loads.  Every wave runs the same number of phases and raises its
+  // flag in each before it waits, so every wait ends.  A row is overwritten
+  // only after its readers have raised the flag of the following phase.
+  const int wv = __builtin_amdgcn_readfirstlane(t / 64);
+  int phase = 0;
+  auto meet = [&]() {
+    phase++;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    flag[wv] = phase;
+    if (wv > 0) while (flag[wv - 1] < phase) __builtin_amdgcn_s_sleep(0);
+    if (wv < S2_NC / 64 - 1) while (flag[wv + 1] < phase) __builtin_amdgcn_s_sleep(0);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+  struct IJ {
+    double sil[3], sjl[3], sjh[3], cil, cih, cjl, cjh;
+  } o, on;
+  auto load_ij = [&](long m, unsigned pl, IJ &o) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      o.sil[c] = ldp(sn + (c * 3 * nnn + m), pl);
+      o.sjl[c] = ldp(sn + ((c * 3 + 1) * nnn + m), pl);
+      o.sjh[c] = ldp(sn + ((c * 3 + 1) * nnn + m + b.nid), pl);
+    }
+    o.cil = ldp(coefe + m, pl);
+    o.cih = ldp(coefe + m, pl + 8u);
+    o.cjl = ldp(coefe + (nnn + m), pl);
+    o.cjh = ldp(coefe + (nnn + m + b.nid), pl);
+  };
+  load_ij(mk, opaque(pl0), o);
+  for (int k = ka; k <= kz; k++, mk += nijd) {
+    const bool kreal = k + 1 < b.k2;
+    const unsigned pl = opaque(pl0);
+    // the loads of the plane but its i and j faces', which came with the plane
+    // below
+    double skh[3], uu[5], fv[5] = {0., 0., 0., 0., 0.}, Vn[5], Dn[5];
+#pragma unroll
+    for (int c = 0; c < 3; c++) skh[c] = ldp(sn + ((c * 3 + 2) * nnn + mk + nijd), pl);
+    const double ckh = kreal ? ldp(coefe + (2 * nnn + mk + nijd), pl) : 0.;
+    const double dg = ldp(diag + mk, pl);
+#pragma unroll
+    for (int e = 0; e < 5; e++) uu[e] = ldp(u + (e * ldv + b.npc + mk), pl);
+    if constexpr (FF) {
+#pragma unroll
+      for (int e = 0; e < 5; e++) fv[e] = ldp(ff + (e * ldv + b.npc + mk), pl);
+    }
+    if (own && kreal) load_vd(mk + nijd, pl, Vn, Dn);
+    double q[14], w[5], tn[5], dlo[5], dhi[5];
+    // the i and j faces and the lower k face of the plane's cell, its q in
+    // buffer Q: w = -u - ff + ... as sweep_tile.inc sums it
+    auto faces = [&](const double *Q, const double tk[5]) {
+      tn2_fma(q, o.sil, tn, [&](int c) { return Q[c * S2_NC + tl]; });
+#pragma unroll
+      for (int e = 0; e < 5; e++) {
+        const double th = lane_above(tn[e]);
+        w[e] = fma(o.cil, Q[q_comp(e) * S2_NC + tl], fma(0.5, tn[e], -uu[e] - fv[e]));
+        if (ireal) w[e] = fma(o.cih, Q[q_comp(e) * S2_NC + tr], w[e]);
+        w[e] = fma(-0.5, th, w[e]);
+      }
+      tn2_fma(q, o.sjl, tn, [&](int c) { return Q[c * S2_NC + td]; });
+#pragma unroll
+      for (int e = 0; e < 5; e++) {
+        w[e] = fma(o.cjl, Q[q_comp(e) * S2_NC + td], fma(0.5, tn[e], w[e]));
+        if (jreal) w[e] = fma(o.cjh, Q[q_comp(e) * S2_NC + tu], w[e]);
+      }
+      tn2_fma(q, o.sjh, tn, [&](int c) { return Q[c * S2_NC + tu]; });
+#pragma unroll
+      for (int e = 0; e < 5; e++) w[e] = fma(ckl, dlo[e], fma(0.5, tk[e], fma(-0.5, tn[e], w[e])));
+    };
+    // A on plane k
+#pragma unroll
+    for (int e = 0; e < 5; e++) dlo[e] = qA[q_comp(e) * S2_NC + t];  // of the plane below
+#pragma unroll
+    for (int c = 0; c < 14; c++) {
+      q[c] = qn[c];
+      qA[c * S2_NC + t] = q[c];
+      qn[c] = 0.;
+    }
+    meet();
+    faces(qA, tkA);
+    // the plane above, the face between and what its increment adds
+    if (own && kreal) dflux_q(ph, Vn, Dn, qn);
+    auto here = [&](int c) { return q[c]; };
+    tn2_fma<KF>(qn, skh, tkA, here);
+#pragma unroll
+    for (int e = 0; e < 5; e++) {
+      if (kreal) w[e] = fma(ckh, qn[q_comp(e)], w[e]);
+      w[e] = fma(-0.5, tkA[e], w[e]);
+    }
+    if (BATCH && first(k + 1)) tn2_fma<K1>(qn, skh, tkA, here);
+    const double rd = 1. / dg;
+#pragma unroll
+    for (int e = 0; e < 5; e++) dhi[e] = w[e] * rd;  // A's increment
+#pragma unroll
+    for (int c = 0; c < 14; c++) q[c] = 0.;
+    if (own) {
+      double V[5];
+#pragma unroll
+      for (int e = 0; e < 5; e++) V[e] = st(e);
+      dflux_q(ph, V, dhi, q);
+      if (kreal) {
+#pragma unroll
+        for (int e = 0; e < 5; e++) st(e) = Vn[e];
+      }
+    }
+    // B: plane k - 1 is complete with the face to plane k
+    double tk[5];
+    auto belowB = [&](int c) { return qB[c * S2_NC + t]; };
+    tn2_fma<KF>(q, skl, tk, belowB);
+#pragma unroll
+    for (int e = 0; e < 5; e++) {
+      dlo[e] = qB[q_comp(e) * S2_NC + t];
+      dhi[e] = fma(-0.5, tk[e], fma(ckl, dhi[e], base[e])) * rdb;
+    }
+    if (BATCH && first(k)) tn2_fma<K1>(q, skl, tk, belowB);
+    if (out && k > kb) {
+#pragma unroll
+      for (int e = 0; e < 5; e++) *gp(dnew.p + (e * dnew.ld + (b.npc - dnew.off) + mk - nijd), pl) = dhi[e];
+    }
+#pragma unroll
+    for (int c = 0; c < 14; c++) qB[c * S2_NC + t] = q[c];
+    load_ij(mk + nijd, pl, on);  // of the plane above (a ghost's past the last: not used)
+    meet();
+    faces(qB, tk);
+    o = on;
+#pragma unroll
+    for (int e = 0; e < 5; e++) base[e] = w[e];
+    rdb = rd;
+    ckl = ckh;
+#pragma unroll
+    for (int c = 0; c < 3; c++) skl[c] = skh[c];
+  }
+  if (out && ke == b.k2) {  // the block's last plane: its upper face is a ghost's
+    double q[14], tk[5];
+#pragma unroll
+    for (int c = 0; c < 14; c++) q[c] = qB[c * S2_NC + t];
+    tn2_fma<KF>(q, skl, tk, [&](int) { return 0.; });
+#pragma unroll
+    for (int e = 0; e < 5; e++)
+      *gp(dnew.p + (e * dnew.ld + (b.npc - dnew.off) + mk - nijd), opaque(pl0)) =
+          fma(-0.5, tk[e], base[e]) * rdb;
+  }
+}
+
+template <bool FF>
+__global__ void __launch_bounds__(S2_NC) __attribute__((amdgpu_waves_per_eu(2)))
+k_impl_sweep2(Blk b, Phys ph, int ntx, int nty, int ks, const double *__restrict__ u, const double *__restrict__ ff,
+              const double *__restrict__ v, long ldv, const double *__restrict__ sn, const double *__restrict__ coefe,
+              const double *__restrict__ diag, DView dold, DView dnew, int rev) {
+  __shared__ double sx[S2_LDS];
+  __shared__ int flag[S2_NC / 64];
+  if (threadIdx.x < S2_NC / 64) flag[threadIdx.x] = 0;
+  __syncthreads();
+  unsigned lg = xcd_linear();
+  if (rev) lg = gridDim.x - 1 - lg;
+  sweep2_body<FF, false>(b, (int)lg, ntx, nty, ks, ph, u, ff, v, ldv, sn, coefe, diag, dold, dnew, sx, flag);
+}
+
 // ---------------------------------------------------------------------------
 // Tile shape of the tiled sub-iteration, per block shape: 64 x 4, 32 x 8 or
 // 16 x 16, all of 256 threads.  Every cell's arithmetic is the same in all,
@@ -689,6 +1027,51 @@ void launch_sweep(int tile, const Blk &b, hipStream_t st, Phys ph, int ityprk, c
   }
 }
 
+// The two-sub-iteration kernel on a block: its tiles, and the slab depth with
+// the fewest steps over the rounds of one workgroup per compute unit (a slab
+// of ks planes takes ks + 2 steps and about one more to start).
+struct Pair {
+  int ntx, nty, ks;
+  long wgs, steps;  // workgroups; steps of one after another on a compute unit
+};
+Pair pair_of(const Blk &b) {
+  const int nz = b.k2 - b.k1, ncu = codens_resident_workgroups(1);
+  Pair p{(b.i2 - b.i1 + S2_OX - 1) / S2_OX, (b.j2 - b.j1 + S2_OY - 1) / S2_OY, 1, 0, 0};
+  for (int ks = 1; ks <= nz; ks++) {
+    const long w = (long)p.ntx * p.nty * ((nz + ks - 1) / ks);
+    const long c = (w + ncu - 1) / ncu * (std::min(ks + 2, nz) + 1);
+    if (ks == 1 || c < p.steps) { p.ks = ks; p.wgs = w; p.steps = c; }
+  }
+  return p;
+}
+
+// Whether a block's sub-iterations run in pairs: the modelled time (us) of a
+// pair against that of two single sweeps.  Measured on MI355X: a step of the
+// pair kernel takes 5.5 us, a step of a single sweep 3.4 us while few of the
+// chip's 512 workgroup places are taken and 6.8 us when all are.  Two singles
+// / a pair: 256 x 128 x 64 250 / 190 us, 200 x 120 x 100 370 / 207, 128 x 128
+// x 32 60 / 60, 75 x 61 x 43 45 / 39, 32 x 16 x 8 14 / 19.  In FP32 the sweeps
+// are bound by their arithmetic, of which a pair has half as much again (its
+// tile's rings): singles.
+constexpr double PAIR_STEP = 5.5, ONE_STEP = 6.8;
+bool pair_model(const Blk &b) {
+  const int tile = tile_model(b), tx = tile_tx(tile), ty = tile_ty(tile), nz = b.k2 - b.k1;
+  const long txy = (long)((b.i2 - b.i1 + tx - 1) / tx) * ((b.j2 - b.j1 + ty - 1) / ty);
+  const int ks = slab_depth(txy, nz, SW_KS);
+  const double fill = txy * ((nz + ks - 1) / ks) / 512.;
+  const double one = std::max(1., fill) * (ks + 1) * 0.5 * ONE_STEP * (1. + std::min(1., fill));
+  return PAIR_STEP * pair_of(b).steps < 2. * one;
+}
+
+// two sub-iterations in -> out
+void launch_sweep2(const Blk &b, hipStream_t st, Phys ph, int ityprk, const double *u, const double *ff,
+                   const double *v, long ldv, const double *sn, const double *coefe, const double *diag, DView in,
+                   DView out, int rev) {
+  const Pair p = pair_of(b);
+  hipLaunchKernelGGL(ityprk ? k_impl_sweep2<true> : k_impl_sweep2<false>, dim3((unsigned)p.wgs), dim3(S2_NC), 0, st, b,
+                     ph, p.ntx, p.nty, p.ks, u, ff, v, ldv, sn, coefe, diag, in, out, rev);
+}
+
 template <bool EU, typename T>
 int pick_tile(const Blk &b, hipStream_t st, Phys ph, int ityprk, const T *u, const T *ff, const T *v, long ldv,
               const double *ps, const T *sn, const T *coefe, const T *diag, TView<T> in, TView<T> out) {
@@ -730,6 +1113,20 @@ int pick_tile(const Blk &b, hipStream_t st, Phys ph, int ityprk, const T *u, con
   return pick;
 }
 }  // namespace
+
+// Launches of lmx sub-iterations: the first (from d = 0), singles, pairs
+struct SweepPlan {
+  int single, pairs, n;
+};
+static SweepPlan sweep_plan(int lmx, bool pairs) {
+  const int rest = lmx > 1 ? lmx - 1 : 0, np = pairs ? rest / 2 : 0;
+  return {rest - 2 * np, np, lmx > 0 ? 1 + rest - np : 0};
+}
+
+static int forced_tile() {
+  std::lock_guard<std::mutex> lk(g_tile_mu);
+  return g_tile_mode;
+}
 
 // tile of a block without timing anything: the forced mode, the choice
 // already timed for its shape, or the model's
@@ -842,29 +1239,35 @@ static int implimf_common(bool eu, const codens_block *cb, const codens_phys *cp
   DView A = {d, (long)ldv, 0}, B = {W, b.nnn, b.npc};
   int tile = 0;
   // sub-iteration 1 starts from d = 0: d = -u/diag (k_impl_sweep1); the
-  // others are tiled sweeps, alternate ones in reverse tile order
-  for (int s = 1; s <= lmx; s++) {
-    DView out = ((lmx - s) % 2 == 0) ? A : B;
-    DView in = ((lmx - s) % 2 == 0) ? B : A;
-    const double *fx = ityprk ? ff : u;
-    if (s == 1) {
+  // others run in pairs, one left over on its own, alternate launches in
+  // reverse tile order; a forced tile shape, the Euler form, or a block where
+  // pairs do not pay (pair_model), runs them one by one.  The launches
+  // alternate between the two buffers, the last one landing in d.
+  const SweepPlan plan = sweep_plan(lmx, !eu && forced_tile() < 0 && pair_model(b));
+  const double *fx = ityprk ? ff : u, *psx = eu ? ps : v;
+  for (int s = 0; s < plan.n; s++) {
+    DView out = ((plan.n - 1 - s) % 2 == 0) ? A : B;
+    DView in = ((plan.n - 1 - s) % 2 == 0) ? B : A;
+    if (s == 0) {
       CodensTimed _tm(tname("implimf_sweep1"), st);
       hipLaunchKernelGGL(k_impl_sweep1<double>, g, t, 0, st, b, (int)ityprk, u, fx, (long)ldv, diag, out);
-    } else {
-      const double *psx = eu ? ps : v;
-      if (s == 2 && fixed)
+    } else if (s <= plan.single) {
+      if (s == 1 && fixed)
         tile = known_tile(b, eu, (int)sizeof(double));
-      else if (s == 2)
+      else if (s == 1)
         tile = eu ? pick_tile<true, double>(b, st, ph, (int)ityprk, u, fx, v, (long)ldv, psx, sn, coefe, diag, in, out)
                   : pick_tile<false, double>(b, st, ph, (int)ityprk, u, fx, v, (long)ldv, psx, sn, coefe, diag, in,
                                              out);
       CodensTimed _tm(tname("implimf_sweep"), st);
       if (eu)
         launch_sweep<true, double>(tile, b, st, ph, (int)ityprk, u, fx, v, (long)ldv, psx, sn, coefe, diag, in, out,
-                                   s % 2 == 0);
+                                   s % 2);
       else
         launch_sweep<false, double>(tile, b, st, ph, (int)ityprk, u, fx, v, (long)ldv, psx, sn, coefe, diag, in, out,
-                                    s % 2 == 0);
+                                    s % 2);
+    } else {
+      CodensTimed _tm(tname("implimf_sweep2"), st);
+      launch_sweep2(b, st, ph, (int)ityprk, u, fx, v, (long)ldv, sn, coefe, diag, in, out, s % 2);
     }
   }
   {
@@ -891,14 +1294,14 @@ int codens_implimf_3d_with(const codens_block *b, const codens_phys *ph, const d
 // diagonal and ping-pong increment (9 planes of nnn) start at 9 npc of the
 // workspace.  The sub-iterations of small blocks then share the chip instead
 // of each filling a few CUs.
-enum { IB_ZERO, IB_CELL, IB_SWEEP, IB_COEF, IB_N };
+enum { IB_ZERO, IB_CELL, IB_SWEEP, IB_COEF, IB_SWEEP2, IB_N };
 
 struct ImplEnt {
   Blk b;
   unsigned start[IB_N];         // first workgroup of this block, per pass
   unsigned gx[IB_N], gy[IB_N];  // this block's grid, per pass
   int tile;                     // sub-iteration tile shape of this block (0: 64 x 4, 1: 32 x 8)
-  int ks_coef, ks_sweep;        // k planes per workgroup
+  int ks_coef, ks_sweep, ks_sweep2;  // k planes per workgroup
 };
 
 __global__ void __launch_bounds__(256) k_zero5_batch(const ImplEnt *__restrict__ tab, int nb, double *d, long ldv) {
@@ -962,6 +1365,25 @@ __global__ void __launch_bounds__(SW_TX *SW_TY) k_impl_sweep_batch(const ImplEnt
                                             c + 3 * b.nnn, out_d ? B : A, out_d ? A : B, sq);
 }
 
+// two sub-iterations of every block
+template <bool FF>
+__global__ void __launch_bounds__(S2_NC) __attribute__((amdgpu_waves_per_eu(2)))
+k_impl_sweep2_batch(const ImplEnt *__restrict__ tab, int nb, Phys ph, const double *__restrict__ u,
+                    const double *__restrict__ ff, const double *__restrict__ v, long ldv,
+                    const double *__restrict__ sn_all, double *ws, double *d, int out_d, int rev) {
+  __shared__ double sx[S2_LDS];
+  __shared__ int flag[S2_NC / 64];
+  if (threadIdx.x < S2_NC / 64) flag[threadIdx.x] = 0;
+  __syncthreads();
+  const unsigned wg = rev ? gridDim.x - 1 - xcd_linear() : xcd_linear();
+  const ImplEnt &E = tab[tab_find(tab, nb, IB_SWEEP2, wg)];
+  const Blk b = uniform_blk(E.b);
+  double *c = ws + 9 * b.npc;
+  DView A = {d, ldv, 0}, B = {c + 4 * b.nnn, b.nnn, b.npc};
+  sweep2_body<FF, true>(b, (int)(wg - E.start[IB_SWEEP2]), (int)E.gx[IB_SWEEP2], (int)E.gy[IB_SWEEP2], E.ks_sweep2, ph, u, ff,
+                  v, ldv, sn_all + 9 * b.npc, c, c + 3 * b.nnn, out_d ? B : A, out_d ? A : B, sx, flag);
+}
+
 __global__ void __launch_bounds__(TX *TY) k_impl_update_batch(const ImplEnt *__restrict__ tab, int nb, double *v,
                                                               long ldv, const double *__restrict__ d, int nvar) {
   const unsigned wg = xcd_linear();
@@ -985,6 +1407,8 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
   std::vector<int32_t> key;
   std::vector<std::pair<long, long>> span(nblk);
   unsigned tot[IB_N] = {0};
+  double one = 0., two = 0.;
+  auto slabs = [](int nz, int ks) { return (nz + ks - 1) / ks; };
   for (int l = 0; l < nblk; l++) {
     int rc = codens_check_block(&blocks[l], what);
     if (rc) return rc;
@@ -1007,11 +1431,19 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
     // the same values at any slab depth
     E.ks_coef = CK_KS;
     E.ks_sweep = SW_KS;
+    const int nz = b.k2 - b.k1, ns2 = slabs(nz, S2_KS);
+    const unsigned n2x = (b.i2 - b.i1 + S2_OX - 1) / S2_OX, n2y = (b.j2 - b.j1 + S2_OY - 1) / S2_OY;
+    E.ks_sweep2 = slabs(nz, ns2);  // even slabs of at most S2_KS planes
+    // pairs or singles, for all blocks alike: the steps of each on a chip that
+    // is full, as in pair_model
+    one += ONE_STEP / 512. * ntx * nty * slabs(nz, SW_KS) * (SW_KS + 1);
+    two += PAIR_STEP / 256. * n2x * n2y * slabs(nz, E.ks_sweep2) * (E.ks_sweep2 + 3);
     const unsigned nkz = (unsigned)((b.k2 - b.k1 + E.ks_sweep - 1) / E.ks_sweep);
     unsigned g[IB_N][3] = {{(unsigned)((b.nnn + 255) / 256), 1, 1},
                            {cg.x, cg.y, cg.z},
                            {ntx, nty, nkz},
-                           {cg.x, cg.y, (unsigned)((b.k2 - b.k1 + E.ks_coef - 1) / E.ks_coef)}};
+                           {cg.x, cg.y, (unsigned)((b.k2 - b.k1 + E.ks_coef - 1) / E.ks_coef)},
+                           {n2x, n2y, (unsigned)slabs(nz, E.ks_sweep2)}};
     for (int p = 0; p < IB_N; p++) {
       E.start[p] = tot[p];
       E.gx[p] = g[p][0];
@@ -1027,6 +1459,7 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
     }
   }
   const long tot_n = span[nblk - 1].second;
+  const bool pairs = forced_tile() < 0 && two < 2. * one;
   for (int l = 0; l < nblk; l++) key.push_back(ent[l].tile);
   ImplEnt *tab = (ImplEnt *)codens_device_table(1, key, ent.data(), sizeof(ImplEnt) * nblk, st, what);
   if (!tab) return CODENS_EHIP;
@@ -1045,16 +1478,23 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
     hipLaunchKernelGGL(k_impl_coef_batch, dim3(tot[IB_COEF]), dim3(TX, TY), 0, st, ct, nb, ph, (const double *)v,
                        (long)ldv, mu, mut, dt, vol, cson, sn_all, dtpas, (int)kfmg, ws);
   }
-  for (int s = 1; s <= lmx; s++) {
-    int out_d = (lmx - s) % 2 == 0;
-    if (s == 1) {
+  // the launches of implimf_common: sub-iteration 1, singles, then pairs
+  const SweepPlan plan = sweep_plan(lmx, pairs);
+  for (int s = 0; s < plan.n; s++) {
+    const int out_d = (plan.n - 1 - s) % 2 == 0;
+    if (s == 0) {
       CodensTimed _tm("implimf_sweep1", st);
       hipLaunchKernelGGL(k_impl_sweep1_batch, dim3(tot[IB_CELL]), dim3(TX, TY), 0, st, ct, nb, (int)ityprk, u, fx,
                          (long)ldv, ws, d, out_d);
-    } else {
+    } else if (s <= plan.single) {
       CodensTimed _tm("implimf_sweep", st);
       hipLaunchKernelGGL(k_impl_sweep_batch, dim3(tot[IB_SWEEP]), dim3(SW_TX * SW_TY), 0, st, ct, nb, ph,
-                         (int)ityprk, u, fx, (const double *)v, (long)ldv, sn_all, ws, d, out_d, s % 2 == 0);
+                         (int)ityprk, u, fx, (const double *)v, (long)ldv, sn_all, ws, d, out_d, s % 2);
+    } else {
+      CodensTimed _tm("implimf_sweep2", st);
+      hipLaunchKernelGGL(ityprk ? k_impl_sweep2_batch<true> : k_impl_sweep2_batch<false>, dim3(tot[IB_SWEEP2]),
+                         dim3(S2_NC), 0, st, ct, nb, ph, u, fx, (const double *)v, (long)ldv, sn_all, ws, d, out_d,
+                         s % 2);
     }
   }
   {

@@ -420,7 +420,8 @@ int codens_sumsq_rate(const codens_block *blocks, int32_t nb, const double *a, c
  * solve.f90:487-515): when enabled, every launch of the main kernels is
  * bracketed by HIP events on its own stream.  Names: "zpres", "chronos",
  * "zvisqc", "roe_limiter_chain", "roe_face_flux", "roe_gather",
- * "implimf_coef", "implimf_sweep", "implimf_update", "sch_expli", "rk_stage".
+ * "implimf_coef", "implimf_sweep", "implimf_sweep2" (two sub-iterations in
+ * one launch), "implimf_update", "sch_expli", "rk_stage".
  * codens_timing_read synchronises on the recorded events and returns the
  * summed duration and launch count of one kernel; reset != 0 clears it. */
 int codens_timing_enable(int32_t on);
@@ -617,7 +618,9 @@ int codens_workspace_set(int32_t set);
  * 64 x 4, 1 forces 32 x 8, 2 forces 16 x 16 (the all-blocks entry points
  * hold the first two: there a forced 16 x 16 takes the lane model's choice
  * between them: launched lanes times each shape's measured time per lane).
- * All give identical results.  *previous (may be NULL) receives the mode in
+ * In mode -1 the FP64 sub-iterations of codens_implimf_3d run two to a
+ * launch, one left over alone, on blocks where that is modelled faster; a
+ * forced shape runs every one alone.  All give identical results.  *previous (may be NULL) receives the mode in
  * force before the call. */
 int codens_sweep_tile(int32_t mode, int32_t *previous);
 
