@@ -20,45 +20,42 @@ using namespace codens;
   c[2] = (b).k1 + xb.z;                              \
   if (c[0] >= (b).i2 || c[1] >= (b).j2) return;
 
-// Workspace of the implicit phase, block-local index m: rv, diag, the half
-// normal velocities u1..u3 and coefficients of the faces, the elimination
-// coefficients alpha, beta6, beta7 (line-major), the increments dw6, dw7, and
-// the line systems of the current sweep (line-major).
+// Workspace of the implicit phase: the half normal velocities uf and the
+// coefficients ce of the faces of the three directions, the increments dw6,
+// dw7, the right-hand sides r6, r7 of the current sweep's lines (overwritten by
+// the eliminated ones), and of the lines of each direction the coefficient lc,
+// the elimination coefficients al and the denominators den.  Entries of the i
+// lines are line-major, all others at the block-local index m.
 struct ImpliWs {
-  double *rv, *cd, *uf, *ce, *al, *b6, *b7, *dw6, *dw7;
-  double *la, *lb, *lc, *l6, *l7;  // line-major coefficients and right-hand sides of one sweep
+  double *uf, *ce, *dw6, *dw7, *r6, *r7, *lc, *al, *den;
+  double *cd;  // the cells' diagonal, read before dw6 is written
 };
 
-// the 18 planes of nnn of a block's workspace starting at ws
+constexpr int IMPLI_PLANES = 19;
+
+// the planes of nnn of a block's workspace starting at ws
 __host__ __device__ inline ImpliWs impli_ws(double *ws, long nnn) {
-  return ImpliWs{ws,           ws + nnn,      ws + 2 * nnn,  ws + 5 * nnn,  ws + 8 * nnn,
-                 ws + 9 * nnn, ws + 10 * nnn, ws + 11 * nnn, ws + 12 * nnn, ws + 13 * nnn,
-                 ws + 14 * nnn, ws + 15 * nnn, ws + 16 * nnn, ws + 17 * nnn};
+  return ImpliWs{ws,           ws + 3 * nnn,  ws + 6 * nnn,  ws + 7 * nnn,  ws + 8 * nnn,
+                 ws + 9 * nnn, ws + 10 * nnn, ws + 13 * nnn, ws + 16 * nnn, ws + 6 * nnn};
 }
 
-// impli2_eqt_3d.f90:113-122: rv and the diagonal's own part
-__device__ __forceinline__ void cells_body(const Blk &b, dim3 tile, const double *__restrict__ v,
-                                           const double *__restrict__ mu, const double *__restrict__ mut,
-                                           const double *__restrict__ dt, const double *__restrict__ vol,
-                                           const double *__restrict__ cfke, double cmt, const ImpliWs &w) {
-  REAL3_AT(b, tile)
-  long n = b.idx(c[0], c[1], c[2]), m = n - b.npc;
-  w.rv[m] = (mu[n] + mut[n] / cmt) / v[n];
-  w.cd[m] = vol[n] / dt[n] + cfke[n] * vol[n];
+// x / d, y = rcp64(d): the steps of the compiler's division after its
+// reciprocal, so that quotients of one divisor share that; zeros, infinities
+// and NaN as there
+__device__ __forceinline__ double div_rcp(double x, double d, double y) {
+  const double q = x * y;
+  return __builtin_amdgcn_div_fixup(fma(fma(-d, q, x), y, q), d, x);
 }
 
-__global__ void __launch_bounds__(TX *TY) k_impli2_cells(Blk b, const double *__restrict__ v, long ldv,
-                                                         const double *__restrict__ mu,
-                                                         const double *__restrict__ mut,
-                                                         const double *__restrict__ dt,
-                                                         const double *__restrict__ vol,
-                                                         const double *__restrict__ cfke, double cmt, ImpliWs w) {
-  cells_body(b, xcd_block(), v, mu, mut, dt, vol, cfke, cmt, w);
-}
-
-// impli2_eqt_3d.f90:126-208: coefficients of every face i1..i2 (resp. j, k)
+// impli2_eqt_3d.f90:113-208: coefficients of every face i1..i2 (resp. j, k)
 // of the real transverse range; the launch covers the cells up to i2, j2, k2.
+// rv = (mu + mut/cmt)/rho of the two cells (zero of a ghost, as in the
+// reference's cleared array) is formed here, its divisions and the velocities'
+// sharing one reciprocal per cell.  22 planes through memory, 3.6 TB/s: 42 us on
+// 130 x 96 x 66, where a pass of its own for rv and one that cleared the work
+// arrays took 29 us more.
 __device__ __forceinline__ void faces_body(const Blk &b, dim3 xb, const double *__restrict__ v, long ldv,
+                                           const double *__restrict__ mu, const double *__restrict__ mut, double cmt,
                                            const double *__restrict__ sn, const double *__restrict__ vol,
                                            const ImpliWs &w) {
   int c[3];
@@ -66,111 +63,158 @@ __device__ __forceinline__ void faces_body(const Blk &b, dim3 xb, const double *
   c[1] = b.j1 + xb.y * TY + threadIdx.y;
   c[2] = b.k1 + xb.z;
   if (c[0] > b.i2 || c[1] > b.j2) return;
-  long n = b.idx(c[0], c[1], c[2]), m = n - b.npc;
+  const double yc = rcp64(cmt);
+  auto cell = [&](long n, bool real, double q[4]) {
+    const double r = v[n], y = rcp64(r);
+#pragma unroll
+    for (int e = 0; e < 3; e++) q[e] = div_rcp(v[(1 + e) * ldv + n], r, y);
+    q[3] = real ? div_rcp(mu[n] + div_rcp(mut[n], cmt, yc), r, y) : 0.;
+  };
+  const long n = b.idx(c[0], c[1], c[2]), m = n - b.npc;
+  double q[4];
+  cell(n, c[0] < b.i2 && c[1] < b.j2 && c[2] < b.k2, q);
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     bool ok = true;
 #pragma unroll
     for (int x = 0; x < 3; x++) ok = ok && c[x] <= b.hi(x) - (x == d ? 0 : 1);
     if (!ok) continue;
-    long inc = b.inc(d);
+    const long inc = b.inc(d);
     double s1 = snv(sn, b.nnn, m, d, 0), s2 = snv(sn, b.nnn, m, d, 1), s3 = snv(sn, b.nnn, m, d, 2);
     double cnds = s1 * s1 + s2 * s2 + s3 * s3;
-    double uu = 0.5 * (v[ldv + n] / v[n] + v[ldv + n - inc] / v[n - inc]);
-    double vv = 0.5 * (v[2 * ldv + n] / v[n] + v[2 * ldv + n - inc] / v[n - inc]);
-    double ww = 0.5 * (v[3 * ldv + n] / v[n] + v[3 * ldv + n - inc] / v[n - inc]);
+    double l[4];
+    cell(n - inc, c[d] > b.lo(d), l);
+    double uu = 0.5 * (q[0] + l[0]), vv = 0.5 * (q[1] + l[1]), ww = 0.5 * (q[2] + l[2]);
     double uf = 0.5 * (uu * s1 + vv * s2 + ww * s3);
     w.uf[d * b.nnn + m] = uf;
-    w.ce[d * b.nnn + m] = fabs(uf) + (w.rv[m] + w.rv[m - inc]) * cnds / (vol[n] + vol[n - inc]);
+    w.ce[d * b.nnn + m] = fabs(uf) + (q[3] + l[3]) * cnds / (vol[n] + vol[n - inc]);
   }
 }
 
 __global__ void __launch_bounds__(TX *TY) k_impli2_faces(Blk b, const double *__restrict__ v, long ldv,
+                                                         const double *__restrict__ mu,
+                                                         const double *__restrict__ mut, double cmt,
                                                          const double *__restrict__ sn,
                                                          const double *__restrict__ vol, ImpliWs w) {
-  faces_body(b, xcd_block(), v, ldv, sn, vol, w);
+  faces_body(b, xcd_block(), v, ldv, mu, mut, cmt, sn, vol, w);
 }
-
-// impli2_eqt_3d.f90:210-220
-__device__ __forceinline__ void diag_body(const Blk &b, dim3 tile, const ImpliWs &w) {
-  REAL3_AT(b, tile)
-  long m = b.idx(c[0], c[1], c[2]) - b.npc, nnn = b.nnn;
-  const double *ce = w.ce;
-  w.cd[m] = w.cd[m] + ce[m] + ce[m + 1] + ce[nnn + m] + ce[nnn + m + b.nid] + ce[2 * nnn + m] +
-            ce[2 * nnn + m + b.nijd];
-}
-
-__global__ void __launch_bounds__(TX *TY) k_impli2_diag(Blk b, ImpliWs w) { diag_body(b, xcd_block(), w); }
 
 // One sweep along direction d (impli2_eqt_3d.f90:238-275, 292-329, 346-383)
-// in two launches.
+// solves a a-b-c system per grid line for both equations.  The coefficients do
+// not change between sweeps, so the part of the elimination that is theirs
+// (al, den) is done once for all directions (k_impli2_elim), next to each
+// other in one launch as each is a serial chain per line.  A sweep is then
 //
-// k_impli2_rhs, over all real cells: the line system's coefficients a, b, c
-// and the right-hand sides of both equations, whose transverse terms read
-// the previous sweep's increments only, so every cell is independent.  They
-// go to a line-major layout, entry (a - lo_d) * nl + line with the line index
-// (c_p - lo_p) + (c_q - lo_q) * n_p, so that the recursion below reads
-// consecutive lines at consecutive addresses.  Tiles are 16 x 16 cells of one
-// k plane; for i lines the tile is transposed through LDS, so that both the
-// reads (i fastest) and the writes (j fastest) move 128-byte runs.
+// k_impli2_rhs, over all real cells: the right-hand sides, whose transverse
+// terms read the previous sweep's increments only (those of ghosts are zero;
+// before the first sweep all are, and k_impli2_diag writes the right-hand
+// sides, -u).
 //
-// k_impli2_line, one thread per line: the elimination from the high end of
-// the line (recursion values zero beyond the last real cell, as the
-// reference's zeroed arrays give) and then the substitution from the low
-// end, which writes the increments dw6, dw7.  The coefficients do not depend
-// on the recursion, so eight steps' loads are issued ahead of their
-// arithmetic.
+// k_impli2_line, one lane per line and equation: the elimination of the
+// right-hand side from the high end of the line (recursion values zero beyond
+// the last real cell, as the reference's zeroed arrays give) and the
+// substitution from the low end, which writes the increments, or at the last
+// sweep adds them to v (impli2_eqt_3d.f90:406-416).
+//
+// Lines of j and k are neighbours in i, so their entries lie at the cells' own
+// index.  The lines of i are kept line-major, entry (i - i1) * nl + line with
+// the line index (j - j1) + (k - k1) * nj, so that the recursions read
+// consecutive lines at consecutive addresses; the kernels over cells transpose
+// tiles of 16 x 16 cells through LDS for them, so that both sides move
+// 128-byte runs.
+//
+// On 130 x 96 x 66 the elimination of the coefficients takes 25 us (its 18
+// planes move at 4.8 TB/s), a sweep's right-hand sides 13 us (5 TB/s) and its
+// recursions 19 to 25 us (0.15 to 0.3 us per step of a line, two equations of
+// 32 lines per wave, as few lines as there are then spread over more SIMDs);
+// with the coefficients formed and eliminated again in every sweep, one lane
+// for both equations and the loads a batch of eight steps ahead the two took
+// 20 and 40 us.  The whole phase 454 -> 290 us.
 constexpr int RT = 16;
+
+// writes val[e] of cell c = (i, j, k) of this thread's tile to the line-major
+// arrays out[e] (i lines)
+template <int N>
+__device__ __forceinline__ void put_i_lines(const Blk &b, dim3 xb, const double val[N], double *const out[N]) {
+  __shared__ double sh[N][RT][RT + 1];
+  const int tx = threadIdx.x % RT, ty = threadIdx.x / RT;
+#pragma unroll
+  for (int e = 0; e < N; e++) sh[e][ty][tx] = val[e];
+  __syncthreads();
+  const long nj = b.j2 - b.j1, nl = nj * (b.k2 - b.k1);
+  const int i = b.i1 + xb.x * RT + ty, j = b.j1 + xb.y * RT + tx;
+  if (i < b.i2 && j < b.j2) {
+    const long L = (long)(i - b.i1) * nl + (j - b.j1) + (long)xb.z * nj;
+#pragma unroll
+    for (int e = 0; e < N; e++) out[e][L] = sh[e][tx][ty];
+  }
+}
+
+// impli2_eqt_3d.f90:113-122, 210-220: the cells' diagonal, the coefficients a,
+// b, c of the i lines (a and b where k_impli2_elim leaves al and den) and the
+// right-hand sides of the first sweep
+__device__ __forceinline__ void diag_body(const Blk &b, dim3 xb, const double *__restrict__ dt,
+                                          const double *__restrict__ vol, const double *__restrict__ cfke,
+                                          const double *__restrict__ u, long ldv, const ImpliWs &w) {
+  const int i = b.i1 + xb.x * RT + threadIdx.x % RT, j = b.j1 + xb.y * RT + threadIdx.x / RT;
+  double val[5] = {0., 0., 0., 0., 0.};
+  if (i < b.i2 && j < b.j2) {
+    const long n = b.idx(i, j, b.k1 + xb.z), m = n - b.npc, nnn = b.nnn;
+    const double *__restrict__ ce = w.ce, *__restrict__ uf = w.uf;
+    const double c0 = ce[m], c1 = ce[m + 1], u0 = uf[m], u1 = uf[m + 1];
+    double cd = vol[n] / dt[n] + cfke[n] * vol[n];
+    cd = cd + c0 + c1 + ce[nnn + m] + ce[nnn + m + b.nid] + ce[2 * nnn + m] + ce[2 * nnn + m + b.nijd];
+    w.cd[m] = cd;
+    val[0] = c0 + u0;
+    val[1] = cd + u1 - u0;
+    val[2] = -c1 + u1;
+    val[3] = -u[5 * ldv + n];
+    val[4] = -u[6 * ldv + n];
+  }
+  double *const out[5] = {w.al, w.den, w.lc, w.r6, w.r7};
+  put_i_lines<5>(b, xb, val, out);
+}
+
+__global__ void __launch_bounds__(RT *RT) k_impli2_diag(Blk b, const double *__restrict__ dt,
+                                                        const double *__restrict__ vol,
+                                                        const double *__restrict__ cfke,
+                                                        const double *__restrict__ u, long ldv, ImpliWs w) {
+  diag_body(b, xcd_block(), dt, vol, cfke, u, ldv, w);
+}
 
 __device__ __forceinline__ void rhs_body(const Blk &b, dim3 xb, int d, const double *__restrict__ u, long ldv,
                                          const ImpliWs &w) {
-  __shared__ double sh[5][RT][RT + 1];
-  const int tx = threadIdx.x % RT, ty = threadIdx.x / RT;
   const int p = d == 0 ? 1 : 0, q = d == 2 ? 1 : 2;
-  const long np_ = b.hi(p) - b.lo(p), nl = np_ * (b.hi(q) - b.lo(q));
   int c[3];
-  c[0] = b.i1 + xb.x * RT + tx;
-  c[1] = b.j1 + xb.y * RT + ty;
+  c[0] = b.i1 + xb.x * RT + threadIdx.x % RT;
+  c[1] = b.j1 + xb.y * RT + threadIdx.x / RT;
   c[2] = b.k1 + xb.z;
   const bool in = c[0] < b.i2 && c[1] < b.j2;
-  double val[5] = {0., 0., 0., 0., 0.};
+  double val[2] = {0., 0.};
   if (in) {
-    const long inc = b.inc(d), ip = b.inc(p), iq = b.inc(q), nnn = b.nnn;
+    const long ip = b.inc(p), iq = b.inc(q), nnn = b.nnn;
     const long n = b.idx(c[0], c[1], c[2]), m = n - b.npc;
-    const double *__restrict__ uD = w.uf + d * nnn, *__restrict__ uP = w.uf + p * nnn;
-    const double *__restrict__ uQ = w.uf + q * nnn;
-    const double *__restrict__ cD = w.ce + d * nnn, *__restrict__ cP = w.ce + p * nnn;
-    const double *__restrict__ cQ = w.ce + q * nnn;
-    const double *__restrict__ w6 = w.dw6, *__restrict__ w7 = w.dw7;
+    const double *__restrict__ uP = w.uf + p * nnn, *__restrict__ uQ = w.uf + q * nnn;
+    const double *__restrict__ cP = w.ce + p * nnn, *__restrict__ cQ = w.ce + q * nnn;
+    const bool lp = c[p] > b.lo(p), hp = c[p] + 1 < b.hi(p), lq = c[q] > b.lo(q), hq = c[q] + 1 < b.hi(q);
     double td = -uP[m + ip] + uP[m] - uQ[m + iq] + uQ[m];
     double tpp = cP[m + ip] - uP[m + ip], tmp_ = cP[m] + uP[m];
     double tpq = cQ[m + iq] - uQ[m + iq], tmq = cQ[m] + uQ[m];
-    val[3] = -u[5 * ldv + n] + td * w6[m] + tmp_ * w6[m - ip] + tpp * w6[m + ip] + tmq * w6[m - iq] +
-             tpq * w6[m + iq];
-    val[4] = -u[6 * ldv + n] + td * w7[m] + tmp_ * w7[m - ip] + tpp * w7[m + ip] + tmq * w7[m - iq] +
-             tpq * w7[m + iq];
-    val[0] = cD[m] + uD[m];
-    val[1] = w.cd[m] + uD[m + inc] - uD[m];
-    val[2] = -cD[m + inc] + uD[m + inc];
-  }
-  double *const out[5] = {w.la, w.lb, w.lc, w.l6, w.l7};
-  if (d != 0) {
-    if (in) {
-      const long L = (long)(c[d] - b.lo(d)) * nl + (c[p] - b.lo(p)) + (long)(c[q] - b.lo(q)) * np_;
 #pragma unroll
-      for (int e = 0; e < 5; e++) out[e][L] = val[e];
+    for (int e = 0; e < 2; e++) {
+      const double *__restrict__ dw = e == 0 ? w.dw6 : w.dw7;
+      const double wl = lp ? dw[m - ip] : 0., wh = hp ? dw[m + ip] : 0.;
+      const double ql = lq ? dw[m - iq] : 0., qh = hq ? dw[m + iq] : 0.;
+      val[e] = -u[(5 + e) * ldv + n] + td * dw[m] + tmp_ * wl + tpp * wh + tmq * ql + tpq * qh;
     }
-    return;
+    if (d != 0) {
+      w.r6[m] = val[0];
+      w.r7[m] = val[1];
+    }
   }
-#pragma unroll
-  for (int e = 0; e < 5; e++) sh[e][ty][tx] = val[e];
-  __syncthreads();
-  // i lines: p = j, q = k; thread (tx, ty) writes cell (i0 + ty, j0 + tx)
-  const int i = b.i1 + xb.x * RT + ty, j = b.j1 + xb.y * RT + tx;
-  if (i < b.i2 && j < b.j2) {
-    const long L = (long)(i - b.i1) * nl + (j - b.j1) + (long)(c[2] - b.k1) * np_;
-#pragma unroll
-    for (int e = 0; e < 5; e++) out[e][L] = sh[e][tx][ty];
+  if (d == 0) {
+    double *const out[2] = {w.r6, w.r7};
+    put_i_lines<2>(b, xb, val, out);
   }
 }
 
@@ -179,130 +223,167 @@ __global__ void __launch_bounds__(RT *RT) k_impli2_rhs(Blk b, int d, const doubl
   rhs_body(b, xcd_block(), d, u, ldv, w);
 }
 
-constexpr int LU = 8;  // recursion steps per batch of loads
-
-// The two recursions of one line, each software-pipelined: the loads of the
-// next LU steps are issued before the arithmetic of the current LU steps, so
-// one memory round trip covers 2 x LU steps of the serial chain.
-__device__ __forceinline__ void line_body(const Blk &b, int d, long t, const ImpliWs &w) {
+// Line t of direction d: its length, the cell's index of its first entry and
+// the step from one to the next, and the same for the arrays of the lines.
+struct Line {
+  int nd;
+  long m0, inc, at, step;
+  bool ok;
+};
+__device__ __forceinline__ Line line_of(const Blk &b, int d, long t) {
   const int p = d == 0 ? 1 : 0, q = d == 2 ? 1 : 2;
   const long np_ = b.hi(p) - b.lo(p), nl = np_ * (b.hi(q) - b.lo(q));
-  if (t >= nl) return;
-  const int nd = b.hi(d) - b.lo(d), nb = nd / LU;
-  const double *A = w.la + t, *B = w.lb + t, *C = w.lc + t, *R6 = w.l6 + t, *R7 = w.l7 + t;
-  double *AL = w.al + t, *B6 = w.b6 + t, *B7 = w.b7 + t;
-  // elimination from the high end: steps a = nd-1, nd-2, ...
-  double al1 = 0., b61 = 0., b71 = 0.;  // values at the next face up the line
-  double ai[LU], bi[LU], ci[LU], r6[LU], r7[LU];
-  if (nb > 0) {
-#pragma unroll
-    for (int x = 0; x < LU; x++) {
-      const long L = (long)(nd - 1 - x) * nl;
-      ai[x] = A[L]; bi[x] = B[L]; ci[x] = C[L]; r6[x] = R6[L]; r7[x] = R7[L];
-    }
-  }
-  for (int bt = 0; bt < nb; bt++) {
-    const int a = nd - 1 - bt * LU;
-    double an[LU], bn[LU], cn[LU], sn6[LU], sn7[LU];
-    if (bt + 1 < nb) {
-#pragma unroll
-      for (int x = 0; x < LU; x++) {
-        const long L = (long)(a - LU - x) * nl;
-        an[x] = A[L]; bn[x] = B[L]; cn[x] = C[L]; sn6[x] = R6[L]; sn7[x] = R7[L];
-      }
-    }
-#pragma unroll
-    for (int x = 0; x < LU; x++) {
-      const long L = (long)(a - x) * nl;
-      double den = bi[x] + ci[x] * al1;
-      al1 = ai[x] / den;
-      b61 = (r6[x] - ci[x] * b61) / den;
-      b71 = (r7[x] - ci[x] * b71) / den;
-      AL[L] = al1; B6[L] = b61; B7[L] = b71;
-    }
-#pragma unroll
-    for (int x = 0; x < LU; x++) {
-      ai[x] = an[x]; bi[x] = bn[x]; ci[x] = cn[x]; r6[x] = sn6[x]; r7[x] = sn7[x];
-    }
-  }
-  for (int a = nd - 1 - nb * LU; a >= 0; a--) {
-    const long L = (long)a * nl;
-    double c0 = C[L];
-    double den = B[L] + c0 * al1;
-    al1 = A[L] / den;
-    b61 = (R6[L] - c0 * b61) / den;
-    b71 = (R7[L] - c0 * b71) / den;
-    AL[L] = al1; B6[L] = b61; B7[L] = b71;
-  }
-  // substitution from the low end: steps a = 0, 1, ...  (same thread wrote
-  // AL, B6, B7 above, so its own loads see those values)
+  Line l;
+  l.ok = t < nl;
   int c[3];
   c[p] = b.lo(p) + (int)(t % np_);
   c[q] = b.lo(q) + (int)(t / np_);
   c[d] = b.lo(d);
-  const long inc = b.inc(d);
-  const long m0 = b.idx(c[0], c[1], c[2]) - b.npc;
-  double *dw6 = w.dw6, *dw7 = w.dw7;
-  double w6 = 0., w7 = 0.;  // increments of the ghost cell below the line
-  double xa[LU], x6[LU], x7[LU];
-  if (nb > 0) {
+  l.nd = b.hi(d) - b.lo(d);
+  l.m0 = b.idx(c[0], c[1], c[2]) - b.npc;
+  l.inc = b.inc(d);
+  l.at = d == 0 ? t : l.m0;
+  l.step = d == 0 ? nl : l.inc;
+  return l;
+}
+
+// The recursions run at the latency of their loads unless those are far ahead:
+// each keeps the operands of its next LU steps in registers and loads a step's
+// operands where it has used those of the step LU before.  LU steps' loads
+// and stores are near the 63 that a wave can have in flight.
+constexpr int LU = 15;
+
+// The coefficients' elimination from the high end of a line.
+template <bool I>
+__device__ __forceinline__ void elim_body(const Blk &b, int d, long t, const ImpliWs &w) {
+  const Line l = line_of(b, d, t);
+  if (!l.ok) return;
+  const long nnn = b.nnn;
+  double *const al = w.al + d * nnn + l.at, *const den = w.den + d * nnn + l.at, *const lc = w.lc + d * nnn + l.at;
+  const double *const uD = w.uf + d * nnn + l.m0, *const cD = w.ce + d * nnn + l.m0, *const cd = w.cd + l.m0;
+  double al1 = 0., uh = 0., ch = 0.;  // al, uD and cD of the next cell up the line
+  if (!I) {
+    uh = uD[l.nd * l.inc];
+    ch = cD[l.nd * l.inc];
+  }
+  double x[LU][3];
+  auto load = [&](double z[3], int a) {
+    const long i = max(a, 0);
+    if (I) {
+      z[0] = al[i * l.step]; z[1] = den[i * l.step]; z[2] = lc[i * l.step];
+    } else {
+      z[0] = uD[i * l.inc]; z[1] = cD[i * l.inc]; z[2] = cd[i * l.inc];
+    }
+  };
+  auto run = [&](const double z[3], int a) {
+    const long i = a * l.step;
+    double A = z[0], B = z[1], C = z[2];
+    if (!I) {
+      A = z[1] + z[0];
+      B = z[2] + uh - z[0];
+      C = -ch + uh;
+      uh = z[0];
+      ch = z[1];
+      lc[i] = C;
+    }
+    const double dn = B + C * al1;
+    al1 = div_rcp(A, dn, rcp64(dn));
+    al[i] = al1;
+    den[i] = dn;
+  };
 #pragma unroll
-    for (int x = 0; x < LU; x++) {
-      const long L = (long)x * nl;
-      xa[x] = AL[L]; x6[x] = B6[L]; x7[x] = B7[L];
+  for (int s = 0; s < LU; s++) load(x[s], l.nd - 1 - s);
+  int a = l.nd - 1;
+  for (; a >= LU - 1; a -= LU) {
+#pragma unroll
+    for (int s = 0; s < LU; s++) {
+      run(x[s], a - s);
+      load(x[s], a - s - LU);
     }
   }
-  for (int bt = 0; bt < nb; bt++) {
-    const int a = bt * LU;
-    double ya[LU], y6[LU], y7[LU];
-    if (bt + 1 < nb) {
 #pragma unroll
-      for (int x = 0; x < LU; x++) {
-        const long L = (long)(a + LU + x) * nl;
-        ya[x] = AL[L]; y6[x] = B6[L]; y7[x] = B7[L];
+  for (int s = 0; s < LU - 1; s++)
+    if (a - s >= 0) run(x[s], a - s);
+}
+
+__host__ __device__ inline long n_lines(const Blk &b, int d) {
+  const int p = d == 0 ? 1 : 0, q = d == 2 ? 1 : 2;
+  return (long)(b.hi(p) - b.lo(p)) * (b.hi(q) - b.lo(q));
+}
+
+__global__ void __launch_bounds__(64) k_impli2_elim(Blk b, ImpliWs w) {
+  const int d = blockIdx.y;
+  if (d == 0) elim_body<true>(b, 0, blockIdx.x * 64L + threadIdx.x, w);
+  else elim_body<false>(b, d, blockIdx.x * 64L + threadIdx.x, w);
+}
+
+// The two recursions of a line for one equation: lanes 0..31 of a wave are 32
+// lines of the first, lanes 32..63 of the second.
+constexpr int LINES = 32;  // lines per wave
+template <bool LAST>
+__device__ __forceinline__ void line_body(const Blk &b, int d, long t0, double *v, long ldv, const ImpliWs &w) {
+  const int eq = threadIdx.x / LINES;
+  const Line l = line_of(b, d, t0 + threadIdx.x % LINES);
+  if (!l.ok) return;
+  const long nnn = b.nnn;
+  double *const R = (eq ? w.r7 : w.r6) + l.at;
+  const double *const al = w.al + d * nnn + l.at, *const den = w.den + d * nnn + l.at;
+  const double *const lc = w.lc + d * nnn + l.at;
+  {
+    double x[LU][3], b1 = 0.;
+    auto load = [&](double z[3], int a) {
+      const long j = max(a, 0) * l.step;
+      z[0] = R[j]; z[1] = den[j]; z[2] = lc[j];
+    };
+    auto run = [&](const double z[3], int a) {
+      b1 = div_rcp(z[0] - z[2] * b1, z[1], rcp64(z[1]));
+      R[a * l.step] = b1;
+    };
+#pragma unroll
+    for (int s = 0; s < LU; s++) load(x[s], l.nd - 1 - s);
+    int a = l.nd - 1;
+    for (; a >= LU - 1; a -= LU) {
+#pragma unroll
+      for (int s = 0; s < LU; s++) {
+        run(x[s], a - s);
+        load(x[s], a - s - LU);
       }
     }
 #pragma unroll
-    for (int x = 0; x < LU; x++) {
-      w6 = xa[x] * w6 + x6[x];
-      w7 = xa[x] * w7 + x7[x];
-      const long m = m0 + (long)(a + x) * inc;
-      dw6[m] = w6;
-      dw7[m] = w7;
-    }
+    for (int s = 0; s < LU - 1; s++)
+      if (a - s >= 0) run(x[s], a - s);
+  }
+  // substitution from the low end (the same lane wrote R above, so its own
+  // loads see those values)
+  double *const out = LAST ? v + (5 + eq) * ldv + b.npc + l.m0 : (eq ? w.dw7 : w.dw6) + l.m0;
+  double x[LU][3], wl = 0.;  // wl: increment of the cell below, zero of the ghost
+  auto load = [&](double z[3], int a) {
+    const long i = min(a, l.nd - 1);
+    z[0] = al[i * l.step]; z[1] = R[i * l.step];
+    if (LAST) z[2] = out[i * l.inc];
+  };
+  auto run = [&](const double z[3], int a) {
+    wl = z[0] * wl + z[1];
+    out[a * l.inc] = LAST ? z[2] + wl : wl;
+  };
 #pragma unroll
-    for (int x = 0; x < LU; x++) {
-      xa[x] = ya[x]; x6[x] = y6[x]; x7[x] = y7[x];
+  for (int s = 0; s < LU; s++) load(x[s], s);
+  int a = 0;
+  for (; a + LU <= l.nd; a += LU) {
+#pragma unroll
+    for (int s = 0; s < LU; s++) {
+      run(x[s], a + s);
+      load(x[s], a + s + LU);
     }
   }
-  for (int a = nb * LU; a < nd; a++) {
-    const long L = (long)a * nl;
-    w6 = AL[L] * w6 + B6[L];
-    w7 = AL[L] * w7 + B7[L];
-    dw6[m0 + (long)a * inc] = w6;
-    dw7[m0 + (long)a * inc] = w7;
-  }
+#pragma unroll
+  for (int s = 0; s < LU - 1; s++)
+    if (a + s < l.nd) run(x[s], a + s);
 }
 
-__global__ void __launch_bounds__(64) k_impli2_line(Blk b, int d, ImpliWs w) {
-  line_body(b, d, blockIdx.x * 64L + threadIdx.x, w);
-}
-
-// :406-416
-__device__ __forceinline__ void impli2_update_body(const Blk &b, dim3 tile, double *v, long ldv, const ImpliWs &w) {
-  REAL3_AT(b, tile)
-  long n = b.idx(c[0], c[1], c[2]), m = n - b.npc;
-  v[5 * ldv + n] = v[5 * ldv + n] + w.dw6[m];
-  v[6 * ldv + n] = v[6 * ldv + n] + w.dw7[m];
-}
-
-__global__ void __launch_bounds__(TX *TY) k_impli2_update(Blk b, double *v, long ldv, ImpliWs w) {
-  impli2_update_body(b, xcd_block(), v, ldv, w);
-}
-
-__global__ void k_zero_n(double *p, long cnt) {
-  long i = blockIdx.x * 256L + threadIdx.x;
-  if (i < cnt) p[i] = 0.;
+template <bool LAST>
+__global__ void __launch_bounds__(64) k_impli2_line(Blk b, int d, double *v, long ldv, ImpliWs w) {
+  line_body<LAST>(b, d, blockIdx.x * (long)LINES, v, ldv, w);
 }
 
 extern "C" int codens_impli2_eqt_3d(const codens_block *cb, const double *u, int64_t ldv, const double *dt,
@@ -316,43 +397,37 @@ extern "C" int codens_impli2_eqt_3d(const codens_block *cb, const double *u, int
   }
   Blk b = make_blk(cb);
   hipStream_t st = (hipStream_t)stream;
-  long nnn = b.nnn;
-  double *ws = (double *)codens_workspace(sizeof(double) * 18 * nnn, 3);
+  double *ws = (double *)codens_workspace(sizeof(double) * IMPLI_PLANES * b.nnn, 3);
   if (!ws) {
     codens_set_error("codens_impli2_eqt_3d: workspace allocation failed");
     return CODENS_EHIP;
   }
-  ImpliWs w = impli_ws(ws, nnn);
+  ImpliWs w = impli_ws(ws, b.nnn);
   CodensTimed _tm("impli2_eqt_3d", st);
-  // rv, the face arrays and the increments start at zero (ghost entries stay)
-  hipLaunchKernelGGL(k_zero_n, dim3((unsigned)((13 * nnn + 255) / 256)), dim3(256), 0, st, ws, 13 * nnn);
-  dim3 g = cell_grid(b), t(TX, TY);
-  hipLaunchKernelGGL(k_impli2_cells, g, t, 0, st, b, v, (long)ldv, mu, mut, dt, vol, cfke, cmt, w);
   dim3 gf((b.i2 - b.i1 + 1 + TX - 1) / TX, (b.j2 - b.j1 + 1 + TY - 1) / TY, b.k2 - b.k1 + 1);
-  hipLaunchKernelGGL(k_impli2_faces, gf, t, 0, st, b, v, (long)ldv, sn, vol, w);
-  hipLaunchKernelGGL(k_impli2_diag, g, t, 0, st, b, w);
+  hipLaunchKernelGGL(k_impli2_faces, gf, dim3(TX, TY), 0, st, b, v, (long)ldv, mu, mut, cmt, sn, vol, w);
   dim3 gr((b.i2 - b.i1 + RT - 1) / RT, (b.j2 - b.j1 + RT - 1) / RT, b.k2 - b.k1);
-  for (int d = 0; d < 3; d++) {
-    int p = d == 0 ? 1 : 0, q = d == 2 ? 1 : 2;
-    int nl = (b.hi(p) - b.lo(p)) * (b.hi(q) - b.lo(q));
-    for (int sweep = 0; sweep < 2; sweep++) {
-      hipLaunchKernelGGL(k_impli2_rhs, gr, dim3(RT * RT), 0, st, b, d, u, (long)ldv, w);
-      hipLaunchKernelGGL(k_impli2_line, dim3((nl + 63) / 64), dim3(64), 0, st, b, d, w);
-    }
+  hipLaunchKernelGGL(k_impli2_diag, gr, dim3(RT * RT), 0, st, b, dt, vol, cfke, u, (long)ldv, w);
+  const long most = std::max(n_lines(b, 0), std::max(n_lines(b, 1), n_lines(b, 2)));
+  hipLaunchKernelGGL(k_impli2_elim, dim3((unsigned)((most + 63) / 64), 3), dim3(64), 0, st, b, w);
+  for (int s = 0; s < 6; s++) {
+    const int d = s / 2;
+    if (s > 0) hipLaunchKernelGGL(k_impli2_rhs, gr, dim3(RT * RT), 0, st, b, d, u, (long)ldv, w);
+    hipLaunchKernelGGL(s == 5 ? k_impli2_line<true> : k_impli2_line<false>,
+                       dim3((unsigned)((n_lines(b, d) + LINES - 1) / LINES)), dim3(64), 0, st, b, d, v, (long)ldv, w);
   }
-  hipLaunchKernelGGL(k_impli2_update, g, t, 0, st, b, v, (long)ldv, w);
   return codens_check_launch("codens_impli2_eqt_3d");
 }
 
 // ---------------------------------------------------------------------------
-// impli2_eqt_3d for all blocks of a layout: each pass of the phase (zero,
-// cells, faces, diagonal, and per sweep the line systems and the line
-// recursions, then the update) is one flattened launch over every block,
-// with a device table of the blocks' extents and first workgroups per pass.
-// Block l's 18-plane workspace starts at 18 npc.  The line recursion is a
-// serial chain per line, so a launch takes about the time of its longest
-// line: one launch over the lines of all blocks replaces one per block.
-enum { TB_ZERO, TB_CELL, TB_FACE, TB_RHS, TB_LINE0, TB_LINE1, TB_LINE2, TB_N };
+// impli2_eqt_3d for all blocks of a layout: each pass of the phase (faces,
+// diagonal, coefficients' elimination, and per sweep the right-hand sides and
+// the line recursions) is one flattened launch over every block, with a device
+// table of the blocks' extents and first workgroups per pass.  Block l's
+// workspace starts at IMPLI_PLANES npc.  The line recursion is a serial chain
+// per line, so a launch takes about the time of its longest line: one launch
+// over the lines of all blocks replaces one per block.
+enum { TB_FACE, TB_RHS, TB_ELIM0, TB_ELIM1, TB_ELIM2, TB_LINE0, TB_LINE1, TB_LINE2, TB_N };
 
 struct TurbEnt {
   Blk b;
@@ -360,64 +435,58 @@ struct TurbEnt {
   unsigned gx[TB_N], gy[TB_N];  // this block's grid, per pass
 };
 
-__global__ void __launch_bounds__(256) k_impli2_zero_batch(const TurbEnt *__restrict__ tab, int nb, double *ws) {
-  const TurbEnt &E = tab[tab_find(tab, nb, TB_ZERO, blockIdx.x)];
-  const long i = (blockIdx.x - E.start[TB_ZERO]) * 256L + threadIdx.x;
-  if (i < 13 * E.b.nnn) ws[18 * E.b.npc + i] = 0.;
-}
-
-__global__ void __launch_bounds__(TX *TY) k_impli2_cells_batch(const TurbEnt *__restrict__ tab, int nb,
-                                                               const double *__restrict__ v,
-                                                               const double *__restrict__ mu,
-                                                               const double *__restrict__ mut,
-                                                               const double *__restrict__ dt,
-                                                               const double *__restrict__ vol,
-                                                               const double *__restrict__ cfke, double cmt,
-                                                               double *ws) {
-  const unsigned wg = xcd_linear();
-  const TurbEnt &E = tab[tab_find(tab, nb, TB_CELL, wg)];
-  const Blk b = E.b;
-  cells_body(b, tab_tile(E, TB_CELL, wg), v, mu, mut, dt, vol, cfke, cmt, impli_ws(ws + 18 * b.npc, b.nnn));
-}
-
 __global__ void __launch_bounds__(TX *TY) k_impli2_faces_batch(const TurbEnt *__restrict__ tab, int nb,
                                                                const double *__restrict__ v, long ldv,
+                                                               const double *__restrict__ mu,
+                                                               const double *__restrict__ mut, double cmt,
                                                                const double *__restrict__ sn_all,
                                                                const double *__restrict__ vol, double *ws) {
   const unsigned wg = xcd_linear();
   const TurbEnt &E = tab[tab_find(tab, nb, TB_FACE, wg)];
-  const Blk b = E.b;
-  faces_body(b, tab_tile(E, TB_FACE, wg), v, ldv, sn_all + 9 * b.npc, vol, impli_ws(ws + 18 * b.npc, b.nnn));
+  const Blk b = uniform_blk(E.b);
+  faces_body(b, tab_tile(E, TB_FACE, wg), v, ldv, mu, mut, cmt, sn_all + 9 * b.npc, vol,
+             impli_ws(ws + IMPLI_PLANES * b.npc, b.nnn));
 }
 
-__global__ void __launch_bounds__(TX *TY) k_impli2_diag_batch(const TurbEnt *__restrict__ tab, int nb, double *ws) {
+__global__ void __launch_bounds__(RT *RT) k_impli2_diag_batch(const TurbEnt *__restrict__ tab, int nb,
+                                                              const double *__restrict__ dt,
+                                                              const double *__restrict__ vol,
+                                                              const double *__restrict__ cfke,
+                                                              const double *__restrict__ u, long ldv, double *ws) {
   const unsigned wg = xcd_linear();
-  const TurbEnt &E = tab[tab_find(tab, nb, TB_CELL, wg)];
-  const Blk b = E.b;
-  diag_body(b, tab_tile(E, TB_CELL, wg), impli_ws(ws + 18 * b.npc, b.nnn));
+  const TurbEnt &E = tab[tab_find(tab, nb, TB_RHS, wg)];
+  const Blk b = uniform_blk(E.b);
+  diag_body(b, tab_tile(E, TB_RHS, wg), dt, vol, cfke, u, ldv, impli_ws(ws + IMPLI_PLANES * b.npc, b.nnn));
+}
+
+__global__ void __launch_bounds__(64) k_impli2_elim_batch(const TurbEnt *__restrict__ tab, int nb, double *ws) {
+  const int d = blockIdx.y;
+  const unsigned wg = blockIdx.x;
+  const TurbEnt &L = tab[nb - 1];
+  if (wg >= L.start[TB_ELIM0 + d] + L.gx[TB_ELIM0 + d]) return;  // the grid is that of the direction with most
+  const TurbEnt &E = tab[tab_find(tab, nb, TB_ELIM0 + d, wg)];
+  const Blk b = uniform_blk(E.b);
+  const long t = (wg - E.start[TB_ELIM0 + d]) * 64L + threadIdx.x;
+  const ImpliWs w = impli_ws(ws + IMPLI_PLANES * b.npc, b.nnn);
+  if (d == 0) elim_body<true>(b, 0, t, w);
+  else elim_body<false>(b, d, t, w);
 }
 
 __global__ void __launch_bounds__(RT *RT) k_impli2_rhs_batch(const TurbEnt *__restrict__ tab, int nb, int d,
                                                              const double *__restrict__ u, long ldv, double *ws) {
   const unsigned wg = xcd_linear();
   const TurbEnt &E = tab[tab_find(tab, nb, TB_RHS, wg)];
-  const Blk b = E.b;
-  rhs_body(b, tab_tile(E, TB_RHS, wg), d, u, ldv, impli_ws(ws + 18 * b.npc, b.nnn));
+  const Blk b = uniform_blk(E.b);
+  rhs_body(b, tab_tile(E, TB_RHS, wg), d, u, ldv, impli_ws(ws + IMPLI_PLANES * b.npc, b.nnn));
 }
 
-__global__ void __launch_bounds__(64) k_impli2_line_batch(const TurbEnt *__restrict__ tab, int nb, int d,
-                                                          double *ws) {
+template <bool LAST>
+__global__ void __launch_bounds__(64) k_impli2_line_batch(const TurbEnt *__restrict__ tab, int nb, int d, double *v,
+                                                          long ldv, double *ws) {
   const TurbEnt &E = tab[tab_find(tab, nb, TB_LINE0 + d, blockIdx.x)];
-  const Blk b = E.b;
-  line_body(b, d, (blockIdx.x - E.start[TB_LINE0 + d]) * 64L + threadIdx.x, impli_ws(ws + 18 * b.npc, b.nnn));
-}
-
-__global__ void __launch_bounds__(TX *TY) k_impli2_update_batch(const TurbEnt *__restrict__ tab, int nb, double *v,
-                                                                long ldv, double *ws) {
-  const unsigned wg = xcd_linear();
-  const TurbEnt &E = tab[tab_find(tab, nb, TB_CELL, wg)];
-  const Blk b = E.b;
-  impli2_update_body(b, tab_tile(E, TB_CELL, wg), v, ldv, impli_ws(ws + 18 * b.npc, b.nnn));
+  const Blk b = uniform_blk(E.b);
+  line_body<LAST>(b, d, (blockIdx.x - E.start[TB_LINE0 + d]) * (long)LINES, v, ldv,
+                  impli_ws(ws + IMPLI_PLANES * b.npc, b.nnn));
 }
 
 extern "C" int codens_impli2_eqt_3d_batch(int32_t nblk, const codens_block *blocks, const double *u, int64_t ldv,
@@ -444,14 +513,15 @@ extern "C" int codens_impli2_eqt_3d_batch(int32_t nblk, const codens_block *bloc
     TurbEnt &E = ent[l];
     E.b = b;
     const unsigned ni = b.i2 - b.i1, nj = b.j2 - b.j1, nk = b.k2 - b.k1;
-    dim3 cg = cell_grid(b);
-    unsigned g[TB_N][3] = {{(unsigned)((13 * b.nnn + 255) / 256), 1, 1},
-                           {cg.x, cg.y, cg.z},
-                           {(ni + 1 + TX - 1) / TX, (nj + 1 + TY - 1) / TY, nk + 1},
+    auto waves = [&](int d, int per) { return (unsigned)((n_lines(b, d) + per - 1) / per); };
+    unsigned g[TB_N][3] = {{(ni + 1 + TX - 1) / TX, (nj + 1 + TY - 1) / TY, nk + 1},
                            {(ni + RT - 1) / RT, (nj + RT - 1) / RT, nk},
-                           {(nj * nk + 63) / 64, 1, 1},
-                           {(ni * nk + 63) / 64, 1, 1},
-                           {(ni * nj + 63) / 64, 1, 1}};
+                           {waves(0, 64), 1, 1},
+                           {waves(1, 64), 1, 1},
+                           {waves(2, 64), 1, 1},
+                           {waves(0, LINES), 1, 1},
+                           {waves(1, LINES), 1, 1},
+                           {waves(2, LINES), 1, 1}};
     for (int p = 0; p < TB_N; p++) {
       E.start[p] = tot[p];
       E.gx[p] = g[p][0];
@@ -469,7 +539,7 @@ extern "C" int codens_impli2_eqt_3d_batch(int32_t nblk, const codens_block *bloc
   const long tot_n = span[nblk - 1].second;
   TurbEnt *tab = (TurbEnt *)codens_device_table(2, key, ent.data(), sizeof(TurbEnt) * nblk, st, what);
   if (!tab) return CODENS_EHIP;
-  double *ws = (double *)codens_workspace(sizeof(double) * 18 * tot_n, 3);
+  double *ws = (double *)codens_workspace(sizeof(double) * IMPLI_PLANES * tot_n, 3);
   if (!ws) {
     codens_set_error("%s: workspace allocation failed", what);
     return CODENS_EHIP;
@@ -477,20 +547,18 @@ extern "C" int codens_impli2_eqt_3d_batch(int32_t nblk, const codens_block *bloc
   const TurbEnt *ct = tab;
   const int nb = nblk;
   CodensTimed _tm("impli2_eqt_3d", st);
-  hipLaunchKernelGGL(k_impli2_zero_batch, dim3(tot[TB_ZERO]), dim3(256), 0, st, ct, nb, ws);
-  dim3 t(TX, TY);
-  hipLaunchKernelGGL(k_impli2_cells_batch, dim3(tot[TB_CELL]), t, 0, st, ct, nb, (const double *)v, mu, mut, dt, vol,
-                     cfke, cmt, ws);
-  hipLaunchKernelGGL(k_impli2_faces_batch, dim3(tot[TB_FACE]), t, 0, st, ct, nb, (const double *)v, (long)ldv,
-                     sn_all, vol, ws);
-  hipLaunchKernelGGL(k_impli2_diag_batch, dim3(tot[TB_CELL]), t, 0, st, ct, nb, ws);
-  for (int d = 0; d < 3; d++) {
-    for (int sweep = 0; sweep < 2; sweep++) {
-      hipLaunchKernelGGL(k_impli2_rhs_batch, dim3(tot[TB_RHS]), dim3(RT * RT), 0, st, ct, nb, d, u, (long)ldv, ws);
-      hipLaunchKernelGGL(k_impli2_line_batch, dim3(tot[TB_LINE0 + d]), dim3(64), 0, st, ct, nb, d, ws);
-    }
+  hipLaunchKernelGGL(k_impli2_faces_batch, dim3(tot[TB_FACE]), dim3(TX, TY), 0, st, ct, nb, (const double *)v,
+                     (long)ldv, mu, mut, cmt, sn_all, vol, ws);
+  hipLaunchKernelGGL(k_impli2_diag_batch, dim3(tot[TB_RHS]), dim3(RT * RT), 0, st, ct, nb, dt, vol, cfke, u,
+                     (long)ldv, ws);
+  hipLaunchKernelGGL(k_impli2_elim_batch, dim3(std::max(tot[TB_ELIM0], std::max(tot[TB_ELIM1], tot[TB_ELIM2])), 3),
+                     dim3(64), 0, st, ct, nb, ws);
+  for (int s = 0; s < 6; s++) {
+    const int d = s / 2;
+    if (s > 0) hipLaunchKernelGGL(k_impli2_rhs_batch, dim3(tot[TB_RHS]), dim3(RT * RT), 0, st, ct, nb, d, u, (long)ldv, ws);
+    hipLaunchKernelGGL(s == 5 ? k_impli2_line_batch<true> : k_impli2_line_batch<false>, dim3(tot[TB_LINE0 + d]),
+                       dim3(64), 0, st, ct, nb, d, v, (long)ldv, ws);
   }
-  hipLaunchKernelGGL(k_impli2_update_batch, dim3(tot[TB_CELL]), t, 0, st, ct, nb, v, (long)ldv, ws);
   return codens_check_launch(what);
 }
 
