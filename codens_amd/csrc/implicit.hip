@@ -171,8 +171,35 @@ __device__ inline void face_tn(const DFlux &A, const DFlux &B, double s1, double
   c[2] = (b).k1 + xb.z;                        \
   if (c[0] >= (b).i2 || c[1] >= (b).j2) return;
 
-__device__ inline double rv_of(const Phys &ph, const double *mu, const double *mut, double rinv, long n) {
-  return ph.gam * (mu[n] / ph.pr + mut[n] / ph.prt) * rinv;
+// plane-relative load: base is uniform (the plane's first entry), off the
+// cell's 32-bit byte offset in the plane, so that the address is a scalar base
+// and one register (a plane of more than 2^29 entries would take a block of
+// more than 2^31).  The empty asm keeps the compiler from folding the uniform
+// part into per-thread 64-bit addresses.
+template <typename T>
+using GPtr = __attribute__((address_space(1))) T *;
+template <typename T>
+__device__ __forceinline__ GPtr<T> gp(T *base, unsigned off) {
+  uint64_t p = (uint64_t)base;
+  asm("" : "+s"(p));
+  return (GPtr<T>)((GPtr<char>)p + off);
+}
+template <typename T>
+__device__ __forceinline__ T ldp(const T *base, unsigned off) {
+  return *gp(base, off);
+}
+// Hides an offset's value from the loop optimiser, which would otherwise keep
+// a 64-bit address per array and thread in registers and advance them all.
+__device__ __forceinline__ unsigned opaque(unsigned x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// Workgroup barrier that orders only the LDS traffic of the plane exchange.
+__device__ inline void lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // implimf_3d.f90:113-224: spectral-radius coefficients of the faces and the
@@ -191,7 +218,15 @@ __device__ inline double rv_of(const Phys &ph, const double *mu, const double *m
 // coefficients move by ~1e-16 relative).  A cell's diagonal adds its six
 // faces in the order of implimf_3d.f90:206-215 (i low, i high, j low, j high,
 // k low, k high) and is complete once the next plane has evaluated the k face
-// above it.  Every global load of a plane is issued before its first barrier.
+// above it.
+//
+// Bound by memory: on 200 x 120 x 100 117 us, 3.8 TB/s of the 23 planes that it
+// cannot do without, where loads one after another behind the divisions that
+// used the first of them, per-thread 64-bit addresses (127 registers) and
+// slabs of 8 in two rounds, the second half empty, took 133 us; 75 x 61 x 43
+// 19 -> 14 us.  With the FP32 copies 157 us on 256 x 128 x 64, where the
+// coefficients in FP64 (90 us) and a pass that rounded them and the operands
+// (119 us) read them twice.
 constexpr int CK_KS = 8;
 constexpr int CK_PL = (TX + 2) * (TY + 2);
 
@@ -199,20 +234,24 @@ struct CoefCell {  // the per-cell operands of a face coefficient
   double u, v, w, c, rv, vol;
 };
 
-__device__ __forceinline__ CoefCell coef_cell(const Blk &b, const Phys &ph, const double *__restrict__ v, long ldv,
-                                              const double *__restrict__ mu, const double *__restrict__ mut,
-                                              const double *__restrict__ vol, const double *__restrict__ cson,
-                                              int i, int j, int k) {
-  long n = b.idx(i, j, k);
-  double r = 1.0 / v[n];
-  CoefCell q;
-  q.u = v[ldv + n] * r;
-  q.v = v[2 * ldv + n] * r;
-  q.w = v[3 * ldv + n] * r;
-  q.c = cson[n];
-  q.rv = b.real(i, j, k) ? rv_of(ph, mu, mut, r, n) : 0.;
-  q.vol = vol[n];
-  return q;
+// what they are made of, at byte offset off of the plane whose first storage
+// entry is n0
+struct CoefRaw {
+  double r, m1, m2, m3, c, mu, mut, vol;
+};
+
+__device__ __forceinline__ CoefRaw coef_load(const double *__restrict__ v, long ldv, const double *__restrict__ mu,
+                                             const double *__restrict__ mut, const double *__restrict__ vol,
+                                             const double *__restrict__ cson, long n0, unsigned off) {
+  return CoefRaw{ldp(v + n0, off),    ldp(v + (ldv + n0), off), ldp(v + (2 * ldv + n0), off),
+                 ldp(v + (3 * ldv + n0), off), ldp(cson + n0, off), ldp(mu + n0, off),
+                 ldp(mut + n0, off),  ldp(vol + n0, off)};
+}
+
+__device__ __forceinline__ CoefCell coef_cell(const Phys &ph, const CoefRaw &x, bool real) {
+  const double r = 1.0 / x.r;
+  return CoefCell{x.m1 * r, x.m2 * r, x.m3 * r, x.c,
+                  real ? ph.gam * (x.mu / ph.pr + x.mut / ph.prt) * r : 0., x.vol};
 }
 
 // coefficient of the face between cells lo and hi (normal s of the face)
@@ -232,14 +271,24 @@ struct CoefLds {
   double CI[(TX + 1) * TY], CJ[TX * (TY + 1)];
 };
 
-// the tile xb (x, y: TX x TY columns, z: CK_KS-plane slab) of block b
+// FP32 copies of the sub-iterations' operands, written next to the
+// coefficients (block-local planes of nnn)
+struct F32Copies {
+  const double *u, *ff;  // ff: null if not used
+  float *vF, *uF, *fF, *snF;
+};
+
+// the tile xb (x, y: TX x TY columns, z: CK_KS-plane slab) of block b.  T =
+// float rounds the coefficients and copies the operands to FP32 on the way:
+// they are the ones that this pass reads, u excepted.
+template <typename T>
 __device__ __forceinline__ void coef_tiled_body(const Blk &b, dim3 xb, const Phys &ph, const double *__restrict__ v,
                                                 long ldv, const double *__restrict__ mu,
                                                 const double *__restrict__ mut, const double *__restrict__ dt,
                                                 const double *__restrict__ vol, const double *__restrict__ cson,
                                                 const double *__restrict__ sn, double dtpas, int kfmg,
-                                                double *__restrict__ coefe, double *__restrict__ diag, int ks,
-                                                CoefLds &S) {
+                                                T *__restrict__ coefe, T *__restrict__ diag, int ks, CoefLds &S,
+                                                const F32Copies &F) {
 #pragma clang fp contract(off)
   auto &L = S.L;
   double *CI = S.CI, *CJ = S.CJ;
@@ -266,10 +315,19 @@ __device__ __forceinline__ void coef_tiled_body(const Blk &b, dim3 xb, const Phy
   const int id2 = b.id1 + (int)b.nid - 1, jd2 = b.jd1 + (int)(b.nijd / b.nid) - 1;
   const bool rneed = ring && ri >= b.id1 && ri <= id2 && rj >= b.jd1 && rj <= jd2;
   const int slot = (ty + 1) * (TX + 2) + (tx + 1);
+  // byte offsets in a plane of the own cell (clamped to the cells whose faces
+  // are evaluated), the ring cell and the ring thread's high face; the
+  // index in the block of the plane's first cell
+  auto plane = [&](int x, int y) { return ((unsigned)(x - b.id1) + (unsigned)(y - b.jd1) * (unsigned)b.nid) * 8u; };
+  const unsigned po = plane(min(i, b.i2), min(j, b.j2)), pr = rneed ? plane(ri, rj) : 0u;
+  long mk = (long)(kb - 1 - b.kd1) * b.nijd;
+  auto sn3 = [&](int d, unsigned off, double s[3]) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) s[c] = ldp(sn + ((3 * c + d) * b.nnn + mk), off);
+  };
   CoefCell below{}, cur{};
-  if (own) below = coef_cell(b, ph, v, ldv, mu, mut, vol, cson, i, j, kb - 1);
+  below = coef_cell(ph, coef_load(v, ldv, mu, mut, vol, cson, b.npc + mk, po), kb > b.k1);
   double part = 0.;  // the diagonal of the cell below, all but its k high face
-  long mb = -1;
   // the tile's high face of a ring thread: i face at i0+TX of row j0+t
   // (t < TY), j face at j0+TY of column i0+t-TY (TY <= t < TY + TX), where it
   // bounds a real cell of the tile; its LDS slot and CI/CJ entry
@@ -285,29 +343,32 @@ __device__ __forceinline__ void coef_tiled_body(const Blk &b, dim3 xb, const Phy
   // j < j2, up to the block's high boundary face i = i2), the low j face
   // likewise
   const bool fi = i <= b.i2 && j < b.j2, fj = i < b.i2 && j <= b.j2;
+  const unsigned pf = hdir >= 0 ? plane(hfi, hfj) : 0u;
+  const double *sf = sn + (hdir == 1 ? b.nnn : 0L) + pf / 8;  // the high face's normal in plane 0
   for (int k = kb; k <= ke; k++) {
     const bool top = k == ke;  // the k face above the slab's last plane only
-    // every global load of the plane, issued before its first barrier so
-    // that their latencies overlap
-    if (load) cur = coef_cell(b, ph, v, ldv, mu, mut, vol, cson, i, j, k);
-    CoefCell rq{};
+    mk += b.nijd;
+    // every global load of the plane, issued before any is used so that their
+    // latencies overlap (offsets are clamped into the plane, so that all
+    // threads load; what a thread does not need it does not use)
+    const long nk = b.npc + mk;
+    const CoefRaw xo = coef_load(v, ldv, mu, mut, vol, cson, nk, po);
+    CoefRaw xr{1., 0., 0., 0., 0., 0., 0., 0.};
+    double sk[3], si[3] = {0., 0., 0.}, sj[3] = {0., 0., 0.}, sh[3] = {0., 0., 0.}, dtn = 1.;
+    sn3(2, po, sk);
+    if (!top) {
+      sn3(0, po, si);
+      sn3(1, po, sj);
+      dtn = ldp(dt + nk, po);
+      if (ring) {
+        xr = coef_load(v, ldv, mu, mut, vol, cson, nk, pr);
+#pragma unroll
+        for (int c = 0; c < 3; c++) sh[c] = sf[(3 * c * b.nnn + mk)];
+      }
+    }
+    cur = coef_cell(ph, xo, own && k < b.k2);
     const bool rl = !top && rneed;
-    if (rl) rq = coef_cell(b, ph, v, ldv, mu, mut, vol, cson, ri, rj, k);
-    long m = -1;
-    double sk0 = 0., sk1 = 0., sk2 = 0., dtn = 1.;
-    if (own) {
-      m = b.idx(i, j, k) - b.npc;
-      sk0 = snv(sn, b.nnn, m, 2, 0); sk1 = snv(sn, b.nnn, m, 2, 1); sk2 = snv(sn, b.nnn, m, 2, 2);
-      if (!top) dtn = dt[m + b.npc];
-    }
-    const long mo = b.idx(min(i, b.i2), min(j, b.j2), k) - b.npc;
-    double si0 = 0., si1 = 0., si2 = 0., sj0 = 0., sj1 = 0., sj2 = 0., sh0 = 0., sh1 = 0., sh2 = 0.;
-    if (!top && fi) { si0 = snv(sn, b.nnn, mo, 0, 0); si1 = snv(sn, b.nnn, mo, 0, 1); si2 = snv(sn, b.nnn, mo, 0, 2); }
-    if (!top && fj) { sj0 = snv(sn, b.nnn, mo, 1, 0); sj1 = snv(sn, b.nnn, mo, 1, 1); sj2 = snv(sn, b.nnn, mo, 1, 2); }
-    if (!top && hdir >= 0) {
-      long mf = b.idx(hfi, hfj, k) - b.npc;
-      sh0 = snv(sn, b.nnn, mf, hdir, 0); sh1 = snv(sn, b.nnn, mf, hdir, 1); sh2 = snv(sn, b.nnn, mf, hdir, 2);
-    }
+    const CoefCell rq = coef_cell(ph, xr, b.real(ri, rj, k));
     if (!top) {
       if (load) {
         L[0][slot] = cur.u; L[1][slot] = cur.v; L[2][slot] = cur.w;
@@ -318,14 +379,26 @@ __device__ __forceinline__ void coef_tiled_body(const Blk &b, dim3 xb, const Phy
         L[3][rslot] = rq.c; L[4][rslot] = rq.rv; L[5][rslot] = rq.vol;
       }
     }
-    __syncthreads();
+    lds_sync();
+    constexpr bool F32 = sizeof(T) == sizeof(float);
+    double cv[F32 ? 5 : 1], cu[F32 ? 5 : 1], cf[F32 ? 5 : 1];
+    if constexpr (F32) {  // their latency overlaps the faces
+      if (own && !top) {
+#pragma unroll
+        for (int e = 0; e < 5; e++) {
+          cv[e] = ldp(v + (e * ldv + nk), po);
+          cu[e] = ldp(F.u + (e * ldv + nk), po);
+          if (F.ff) cf[e] = ldp(F.ff + (e * ldv + nk), po);
+        }
+      }
+    }
     double ckl = 0.;
     if (own) {
-      ckl = coef_face(cur, below, sk0, sk1, sk2);
-      if (mb >= 0) {  // the cell below is complete
+      ckl = coef_face(cur, below, sk[0], sk[1], sk[2]);
+      if (k > kb) {  // the cell below is complete
         double dg = part + ckl;
         if (kfmg == 3) dg = dg + 1.5 * below.vol / dtpas;
-        diag[mb] = dg;
+        *gp(diag + (mk - b.nijd), po / (8 / sizeof(T))) = (T)dg;
       }
     }
     if (!top) {
@@ -334,37 +407,75 @@ __device__ __forceinline__ void coef_tiled_body(const Blk &b, dim3 xb, const Phy
         q.u = L[0][s]; q.v = L[1][s]; q.w = L[2][s]; q.c = L[3][s]; q.rv = L[4][s]; q.vol = L[5][s];
         return q;
       };
-      if (fi) CI[ty * (TX + 1) + tx] = coef_face(lds(slot), lds(slot - 1), si0, si1, si2);
-      if (fj) CJ[ty * TX + tx] = coef_face(lds(slot), lds(slot - (TX + 2)), sj0, sj1, sj2);
-      if (hdir == 0) CI[hc] = coef_face(lds(hs), lds(hs - 1), sh0, sh1, sh2);
-      else if (hdir == 1) CJ[hc] = coef_face(lds(hs), lds(hs - (TX + 2)), sh0, sh1, sh2);
+      if (fi) CI[ty * (TX + 1) + tx] = coef_face(lds(slot), lds(slot - 1), si[0], si[1], si[2]);
+      if (fj) CJ[ty * TX + tx] = coef_face(lds(slot), lds(slot - (TX + 2)), sj[0], sj[1], sj[2]);
+      if (hdir == 0) CI[hc] = coef_face(lds(hs), lds(hs - 1), sh[0], sh[1], sh[2]);
+      else if (hdir == 1) CJ[hc] = coef_face(lds(hs), lds(hs - (TX + 2)), sh[0], sh[1], sh[2]);
     }
-    __syncthreads();
+    if constexpr (F32) {
+      auto put_sn = [&](int d, unsigned off, const double x[3]) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) *gp(F.snF + ((3 * c + d) * b.nnn + mk), off / 2) = (float)x[c];
+      };
+      // the low faces of real cells and the block's high boundary faces
+      if (own && (!top || ke == b.k2)) put_sn(2, po, sk);
+      if (!top && fi) put_sn(0, po, si);
+      if (!top && fj) put_sn(1, po, sj);
+      if (!top && hdir == 0 && hfi == b.i2) put_sn(0, pf, sh);
+      if (!top && hdir == 1 && hfj == b.j2) put_sn(1, pf, sh);
+    }
+    lds_sync();
+    if constexpr (F32) {
+      if (own && !top) {
+#pragma unroll
+        for (int e = 0; e < 5; e++) {
+          *gp(F.vF + (e * b.nnn + mk), po / 2) = (float)cv[e];
+          *gp(F.uF + (e * b.nnn + mk), po / 2) = (float)cu[e];
+          if (F.ff) *gp(F.fF + (e * b.nnn + mk), po / 2) = (float)cf[e];
+        }
+      }
+    }
     if (!top && own) {
       double c0 = CI[ty * (TX + 1) + tx], c1 = CI[ty * (TX + 1) + tx + 1];
       double c2 = CJ[ty * TX + tx], c3 = CJ[(ty + 1) * TX + tx];
-      coefe[m] = c0;
-      coefe[b.nnn + m] = c2;
-      coefe[2 * b.nnn + m] = ckl;
+      const unsigned pt = po / (8 / sizeof(T));
+      *gp(coefe + mk, pt) = (T)c0;
+      *gp(coefe + (b.nnn + mk), pt) = (T)c2;
+      *gp(coefe + (2 * b.nnn + mk), pt) = (T)ckl;
       part = cur.vol / dtn;
       part = part + c0 + c1 + c2 + c3 + ckl;
-      mb = m;
     }
     below = cur;
   }
 }
 
-__global__ void __launch_bounds__(TX *TY) k_impl_coef_tiled(Blk b, Phys ph, const double *__restrict__ v, long ldv,
+template <typename T>
+__global__ void __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(4, 4)))
+k_impl_coef_tiled(Blk b, Phys ph, const double *__restrict__ v, long ldv,
                                                             const double *__restrict__ mu,
                                                             const double *__restrict__ mut,
                                                             const double *__restrict__ dt,
                                                             const double *__restrict__ vol,
                                                             const double *__restrict__ cson,
                                                             const double *__restrict__ sn, double dtpas, int kfmg,
-                                                            double *__restrict__ coefe, double *__restrict__ diag,
-                                                            int ks) {
+                                                            T *__restrict__ coefe, T *__restrict__ diag, int ks,
+                                                            F32Copies F) {
   __shared__ CoefLds S;
-  coef_tiled_body(b, xcd_block(), ph, v, ldv, mu, mut, dt, vol, cson, sn, dtpas, kfmg, coefe, diag, ks, S);
+  coef_tiled_body<T>(b, xcd_block(), ph, v, ldv, mu, mut, dt, vol, cson, sn, dtpas, kfmg, coefe, diag, ks, S, F);
+}
+
+// Slab depth of k_impl_coef_tiled on the tiles g.x x g.y: of four workgroups
+// per compute unit, the fewest steps over their rounds (a slab of ks planes
+// takes ks + 1)
+static int coef_slab(const Blk &b, dim3 g) {
+  const int nz = b.k2 - b.k1, places = codens_resident_workgroups(4);
+  int ks = 1;
+  long best = 0;
+  for (int x = 1; x <= nz; x++) {
+    const long c = ((long)g.x * g.y * ((nz + x - 1) / x) + places - 1) / places * (x + 1);
+    if (x == 1 || c < best) { ks = x; best = c; }
+  }
+  return ks;
 }
 
 // implimf_eu.f90:124-170: coefficients of the Euler implicit phase,
@@ -573,13 +684,6 @@ __device__ inline T lds_d(const T *a, int e) {
   return e == 0 ? a[12 * P] : (e == 4 ? a[13 * P] : a[(e - 1) * P]);
 }
 
-// Workgroup barrier that orders only the LDS traffic of the plane exchange.
-__device__ inline void lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 #ifdef CODENS_SW_WAVES
 #define SW_ATTR __attribute__((amdgpu_waves_per_eu(CODENS_SW_WAVES, CODENS_SW_WAVES)))
 #else
@@ -622,30 +726,6 @@ __global__ void __launch_bounds__(TXS *TYS) SW_ATTR k_impl_sweep_tiled(Blk b, Ph
   int lg = (nwg % 8 == 0) ? (hw % 8) * (nwg / 8) + hw / 8 : hw;
   if (rev) lg = nwg - 1 - lg;
 #include "sweep_tile.inc"
-}
-
-// plane-relative load: base is uniform (the plane's first entry), off the
-// cell's 32-bit byte offset in the plane, so that the address is a scalar base
-// and one register (a plane of more than 2^29 entries would take a block of
-// more than 2^31).  The empty asm keeps the compiler from folding the uniform
-// part into per-thread 64-bit addresses.
-template <typename T>
-using GPtr = __attribute__((address_space(1))) T *;
-template <typename T>
-__device__ __forceinline__ GPtr<T> gp(T *base, unsigned off) {
-  uint64_t p = (uint64_t)base;
-  asm("" : "+s"(p));
-  return (GPtr<T>)((GPtr<char>)p + off);
-}
-template <typename T>
-__device__ __forceinline__ T ldp(const T *base, unsigned off) {
-  return *gp(base, off);
-}
-// Hides an offset's value from the loop optimiser, which would otherwise keep
-// a 64-bit address per array and thread in registers and advance them all.
-__device__ __forceinline__ unsigned opaque(unsigned x) {
-  asm volatile("" : "+v"(x));
-  return x;
 }
 
 // ---------------------------------------------------------------------------
@@ -1230,10 +1310,10 @@ static int implimf_common(bool eu, const codens_block *cb, const codens_phys *cp
       hipLaunchKernelGGL(k_impl_coef_eu, g, t, 0, st, b, v, (long)ldv, dt, vol, cson, sn,
                          kfmg == 3 ? 1.5 / dt1min : 0., coefe, diag);
     } else {
-      const int ks = slab_depth((long)g.x * g.y, b.k2 - b.k1, CK_KS);
+      const int ks = coef_slab(b, g);
       dim3 gc(g.x, g.y, (unsigned)((b.k2 - b.k1 + ks - 1) / ks));
-      hipLaunchKernelGGL(k_impl_coef_tiled, gc, t, 0, st, b, ph, v, (long)ldv, mu, mut, dt, vol, cson, sn, dtpas,
-                         (int)kfmg, coefe, diag, ks);
+      hipLaunchKernelGGL(k_impl_coef_tiled<double>, gc, t, 0, st, b, ph, v, (long)ldv, mu, mut, dt, vol, cson, sn,
+                         dtpas, (int)kfmg, coefe, diag, ks, F32Copies{});
     }
   }
   DView A = {d, (long)ldv, 0}, B = {W, b.nnn, b.npc};
@@ -1324,10 +1404,10 @@ __global__ void __launch_bounds__(TX *TY) k_impl_coef_batch(const ImplEnt *__res
   __shared__ CoefLds S;
   const unsigned wg = xcd_linear();
   const ImplEnt &E = tab[tab_find(tab, nb, IB_COEF, wg)];
-  const Blk b = E.b;
+  const Blk b = uniform_blk(E.b);
   double *c = ws + 9 * b.npc;
-  coef_tiled_body(b, tab_tile(E, IB_COEF, wg), ph, v, ldv, mu, mut, dt, vol, cson, sn_all + 9 * b.npc, dtpas, kfmg,
-                  c, c + 3 * b.nnn, E.ks_coef, S);
+  coef_tiled_body<double>(b, tab_tile(E, IB_COEF, wg), ph, v, ldv, mu, mut, dt, vol, cson, sn_all + 9 * b.npc, dtpas,
+                          kfmg, c, c + 3 * b.nnn, E.ks_coef, S, F32Copies{});
 }
 
 __global__ void __launch_bounds__(TX *TY) k_impl_sweep1_batch(const ImplEnt *__restrict__ tab, int nb, int ityprk,
@@ -1506,29 +1586,7 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
 }
 
 // ---------------------------------------------------------------------------
-// FP32 defect-correction form.  np planes of a source (stride lds, storage
-// entries npc .. npc+nnn-1) rounded to float planes of stride nnn.
-struct F32Src {
-  const double *src;  // entry npc + m of plane e at src[e * lds + npc + m]
-  long lds, npc;
-  int np;
-  float *dst;  // plane e at dst[e * nnn + m]
-};
-struct F32Set {
-  F32Src s[5];
-  int n;
-};
-
-// up to five such conversions in one launch (one pass over the block's
-// entries)
-__global__ void __launch_bounds__(256) k_to_f32_set(long nnn, F32Set set) {
-  long m = blockIdx.x * 256L + threadIdx.x;
-  if (m >= nnn) return;
-  for (int q = 0; q < set.n; q++) {
-    const F32Src &c = set.s[q];
-    for (int e = 0; e < c.np; e++) c.dst[e * nnn + m] = (float)c.src[e * c.lds + c.npc + m];
-  }
-}
+// FP32 defect-correction form
 
 // d = the FP32 increment widened to FP64, v += d (real cells)
 __global__ void __launch_bounds__(TX *TY) k_impl_update_f32(Blk b, double *v, long ldv, double *d,
@@ -1559,10 +1617,9 @@ extern "C" int codens_implimf_3d_f32(const codens_block *cb, const codens_phys *
   Phys ph = make_phys(cp);
   hipStream_t st = (hipStream_t)stream;
   const long nnn = b.nnn;
-  double *ws = (double *)codens_workspace(sizeof(double) * 4 * nnn, 2);
   // float planes: v 5, u 5, ff 5, sn 9, coefe 3 + diag 1, two increments 5 + 5
   float *wf = (float *)codens_workspace(sizeof(float) * 38 * nnn, 6);
-  if (!ws || !wf) {
+  if (!wf) {
     codens_set_error("%s: workspace allocation failed", what);
     return CODENS_EHIP;
   }
@@ -1575,17 +1632,10 @@ extern "C" int codens_implimf_3d_f32(const codens_block *cb, const codens_phys *
   dim3 g = cell_grid(b), t(TX, TY);
   {
     CodensTimed _tm("implimf32_coef", st);
-    const int ks = slab_depth((long)g.x * g.y, b.k2 - b.k1, CK_KS);
+    const int ks = coef_slab(b, g);
     dim3 gc(g.x, g.y, (unsigned)((b.k2 - b.k1 + ks - 1) / ks));
-    hipLaunchKernelGGL(k_impl_coef_tiled, gc, t, 0, st, b, ph, v, (long)ldv, mu, mut, dt, vol, cson, sn, dtpas,
-                       (int)kfmg, ws, ws + 3 * nnn, ks);
-    F32Set set{};
-    set.s[set.n++] = F32Src{(const double *)ws, nnn, 0L, 4, cF};
-    set.s[set.n++] = F32Src{v, (long)ldv, (long)b.npc, 5, vF};
-    set.s[set.n++] = F32Src{u, (long)ldv, (long)b.npc, 5, uF};
-    if (ityprk) set.s[set.n++] = F32Src{ff, (long)ldv, (long)b.npc, 5, fF};
-    set.s[set.n++] = F32Src{sn, nnn, 0L, 9, snF};
-    hipLaunchKernelGGL(k_to_f32_set, g1, t1, 0, st, nnn, set);
+    hipLaunchKernelGGL(k_impl_coef_tiled<float>, gc, t, 0, st, b, ph, v, (long)ldv, mu, mut, dt, vol, cson, sn, dtpas,
+                       (int)kfmg, cF, dgF, ks, F32Copies{u, ityprk ? ff : nullptr, vF, uF, fF, snF});
   }
   // storage-indexed views of the block-local float planes (entry n at n - npc)
   const float *vS = vF - b.npc, *uS = uF - b.npc, *fS = fF - b.npc;
