@@ -101,21 +101,6 @@ void *codens_workspace(size_t bytes, int slot) {
   return s.p;
 }
 
-__global__ void __launch_bounds__(256) k_zero_shell(codens::Blk b, long n0, long n1, double *p, long ld, int np) {
-  const codens::Shell s = codens::make_shell(b);
-  long t = blockIdx.x * 256L + threadIdx.x;
-  if (t >= s.na + s.nb + s.nc) return;
-  long n = codens::shell_entry(b, s, t);
-  if (n < n0 || n > n1) return;
-  for (int e = 0; e < np; e++) p[e * ld + n] = 0.;
-}
-
-void codens_zero_shell(const codens::Blk &b, long n0, long n1, double *p, long ld, int np, hipStream_t st) {
-  long cnt = codens::shell_count(b);
-  if (cnt > 0)
-    hipLaunchKernelGGL(k_zero_shell, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st, b, n0, n1, p, ld, np);
-}
-
 namespace {
 std::map<std::pair<int, int>, unsigned *> g_queue;  // (device, workspace set) -> 2 counters
 }  // namespace

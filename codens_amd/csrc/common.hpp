@@ -81,14 +81,16 @@ constexpr int TX = 64, TY = 4;
 // With rev, each XCD runs its share in reverse order: a kernel that follows
 // one over the same arrays then begins on the data that kernel touched last,
 // still in the last-level cache.
-__device__ inline dim3 xcd_block(bool rev = false) {
-  unsigned gx = gridDim.x, gy = gridDim.y, nwg = gx * gy * gridDim.z;
+// nz is the number of z layers that take part.
+__device__ inline dim3 xcd_block(bool rev, unsigned nz) {
+  unsigned gx = gridDim.x, gy = gridDim.y, nwg = gx * gy * nz;
   unsigned hw = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
   unsigned x = hw % 8u, q = nwg / 8u, r = nwg % 8u;
   unsigned lg = x * q + (x < r ? x : r) + hw / 8u;
   if (rev) lg = nwg - 1 - lg;
   return dim3(lg % gx, (lg / gx) % gy, lg / (gx * gy));
 }
+__device__ inline dim3 xcd_block(bool rev = false) { return xcd_block(rev, gridDim.z); }
 
 inline dim3 cell_grid(const Blk &b) {
   int nx = b.i2 - b.i1, ny = b.j2 - b.j1, nz = b.k2 - b.k1;
@@ -148,6 +150,37 @@ __host__ __device__ inline long shell_entry(const Blk &b, const Shell &s, long t
   return b.npc + lk * s.nijd + lj * s.nid + li;
 }
 
+// Clearing the ghosts within the launch that writes the real cells: the grid
+// (x, y, z0) of 256-thread workgroups gets layers beyond z0 (with_shell) whose
+// workgroups clear SHELL_PER entries a thread (shell_layers), instead of a
+// launch of their own, which takes 3.4 us on the smallest block and 5.9 us on
+// 256 x 128 x 64.  They start last and are left out of the order that
+// xcd_block(z0) deals: dealt with the others they all fell to one XCD, and the
+// fused residual of 256 x 128 x 64, whose workgroups fill the chip twice, took
+// 490 us instead of 370.
+constexpr int SHELL_PER = 4;
+inline dim3 with_shell(const Blk &b, dim3 g) {
+  const long per = 256L * SHELL_PER * g.x * g.y;
+  g.z += (unsigned)((shell_count(b) + per - 1) / per);
+  return g;
+}
+__device__ __forceinline__ void shell_entries(const Blk &b, long wg, long n0, long n1, double *p, long ld, int np) {
+  const Shell s = make_shell(b);
+  const long cnt = s.na + s.nb + s.nc, t0 = wg * 256L * SHELL_PER + threadIdx.x + threadIdx.y * blockDim.x;
+  for (int x = 0; x < SHELL_PER; x++) {
+    const long t = t0 + x * 256L;
+    if (t >= cnt) return;
+    const long n = shell_entry(b, s, t);
+    if (n < n0 || n > n1) continue;
+    for (int e = 0; e < np; e++) p[e * ld + n] = 0.;
+  }
+}
+__device__ __forceinline__ bool shell_layers(const Blk &b, int z0, long n0, long n1, double *p, long ld, int np) {
+  if ((int)blockIdx.z < z0) return false;
+  shell_entries(b, ((long)(blockIdx.z - z0) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x, n0, n1, p, ld, np);
+  return true;
+}
+
 // k planes per workgroup of a k-marching kernel: kmax, halved until the
 // grid of tiles_xy i-j tiles has at least 512 workgroups (two per compute
 // unit of MI355X's 256) or the slab is one plane.  A deeper slab re-reads
@@ -169,10 +202,11 @@ inline int slab_depth(long tiles_xy, int nz, int kmax) {
 // block's first workgroup in the launch and its own grid (x, y; z follows).
 // Linear workgroup index, remapped so that each XCD owns a contiguous run
 // of the launch (neighbouring tiles of a block share its L2).
-__device__ __forceinline__ unsigned xcd_linear() {
-  unsigned nwg = gridDim.x, hw = blockIdx.x, x = hw % 8u, q = nwg / 8u, r = nwg % 8u;
+__device__ __forceinline__ unsigned xcd_linear(unsigned nwg) {
+  unsigned hw = blockIdx.x, x = hw % 8u, q = nwg / 8u, r = nwg % 8u;
   return x * q + (x < r ? x : r) + hw / 8u;
 }
+__device__ __forceinline__ unsigned xcd_linear() { return xcd_linear(gridDim.x); }
 
 // entry of the block that owns workgroup wg of a pass (bisection over start)
 template <typename E>
@@ -212,10 +246,6 @@ __device__ __forceinline__ dim3 tab_tile(const E &e, int pass, unsigned wg) {
 
 }  // namespace codens
 
-// p[e ld + n] = 0 for the ghost entries n of block b within n0..n1, planes
-// e < np (abi.hip)
-__global__ void k_zero_shell(codens::Blk b, long n0, long n1, double *p, long ld, int np);
-void codens_zero_shell(const codens::Blk &b, long n0, long n1, double *p, long ld, int np, hipStream_t st);
 
 // error reporting shared by the entry points (abi.cpp)
 extern "C" void codens_set_error(const char *fmt, ...);

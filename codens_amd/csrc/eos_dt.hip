@@ -12,6 +12,8 @@ using namespace codens;
 
 #define CELL_IJK(b)                                   \
   const dim3 xb = xcd_block();                        \
+  CELL_AT(b, xb)
+#define CELL_AT(b, xb)                                \
   int i = (b).i1 + xb.x * TX + threadIdx.x;     \
   int j = (b).j1 + xb.y * TY + threadIdx.y;     \
   int k = (b).k1 + xb.z;                        \
@@ -66,7 +68,12 @@ __global__ void __launch_bounds__(TX *TY) k_chronos(Blk b, Phys ph, double etal,
                                                     const double *__restrict__ vol,
                                                     const double *__restrict__ cson,
                                                     double *__restrict__ dt) {
-  CELL_IJK(b)
+  const int nz = b.k2 - b.k1;
+  // chronos.f90:110-114 zeroes dt over indc(i1,j1,k1)..indc(i2,j2,k2): the
+  // ghost entries of that range here
+  if (shell_layers(b, nz, b.idx(b.i1, b.j1, b.k1), b.idx(b.i2, b.j2, b.k2), dt, 0, 1)) return;
+  const dim3 xb = xcd_block(false, nz);
+  CELL_AT(b, xb)
   long n = b.idx(i, j, k), m = n - b.npc;
   double simax = fmax(face_s2(sn, b.nnn, m + 1, 0), face_s2(sn, b.nnn, m, 0));
   double sjmax = fmax(face_s2(sn, b.nnn, m + b.nid, 1), face_s2(sn, b.nnn, m, 1));
@@ -158,13 +165,9 @@ extern "C" int codens_chronos(const codens_block *cb, const codens_phys *cp, dou
   }
   Blk b = make_blk(cb);
   hipStream_t st = (hipStream_t)stream;
-  long n0 = b.idx(b.i1, b.j1, b.k1), n1 = b.idx(b.i2, b.j2, b.k2);
-  // chronos.f90:110-114 zeroes dt over indc(i1,j1,k1)..indc(i2,j2,k2): the
-  // ghost entries of that range here, the real cells are written below
-  codens_zero_shell(b, n0, n1, dt, 0, 1, st);
   {
     CodensTimed _tm("chronos", st);
-    hipLaunchKernelGGL(k_chronos, cell_grid(b), dim3(TX, TY), 0, st, b, make_phys(cp), eta, (int)ns, v,
+    hipLaunchKernelGGL(k_chronos, with_shell(b, cell_grid(b)), dim3(TX, TY), 0, st, b, make_phys(cp), eta, (int)ns, v,
                      (long)ldv, mu, mut, sn, vol, cson, dt);
   }
   return codens_check_launch("codens_chronos");

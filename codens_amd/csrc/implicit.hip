@@ -1253,9 +1253,10 @@ __device__ __forceinline__ void update_body(const Blk &b, dim3 tile, double *v, 
   for (int e = 0; e < nvar; e++) v[e * ldv + n] = v[e * ldv + n] + d[e * ldv + n];
 }
 
-__global__ void __launch_bounds__(TX *TY) k_impl_update(Blk b, double *v, long ldv, const double *__restrict__ d,
-                                                        int nvar) {
-  update_body(b, xcd_block(), v, ldv, d, nvar);
+__global__ void __launch_bounds__(TX *TY) k_impl_update(Blk b, double *v, long ldv, double *d, int nvar) {
+  // d = 0 on the ghosts; the last sub-iteration wrote every real cell
+  if (shell_layers(b, b.k2 - b.k1, b.npc, b.npc + b.nnn - 1, d, ldv, 5)) return;
+  update_body(b, xcd_block(false, b.k2 - b.k1), v, ldv, d, nvar);
 }
 
 __global__ void k_zero5(double *d, long ldv, long n0, long n1) {
@@ -1300,9 +1301,7 @@ static int implimf_common(bool eu, const codens_block *cb, const codens_phys *cp
   double *coefe = ws, *diag = ws + 3 * b.nnn, *W = ws + 4 * b.nnn;
   long n0 = b.npc, n1 = b.npc + b.nnn - 1;
   auto tname = [fixed](const char *n) { return fixed ? (const char *)nullptr : n; };
-  // d = 0 on the ghosts; the last sub-iteration writes every real cell
-  if (lmx >= 1) codens_zero_shell(b, n0, n1, d, (long)ldv, 5, st);
-  else hipLaunchKernelGGL(k_zero5, dim3((b.nnn + 255) / 256), dim3(256), 0, st, d, (long)ldv, n0, n1);
+  if (lmx < 1) hipLaunchKernelGGL(k_zero5, dim3((b.nnn + 255) / 256), dim3(256), 0, st, d, (long)ldv, n0, n1);
   dim3 g = cell_grid(b), t(TX, TY);
   {
     CodensTimed _tm(tname("implimf_coef"), st);
@@ -1352,7 +1351,7 @@ static int implimf_common(bool eu, const codens_block *cb, const codens_phys *cp
   }
   {
     CodensTimed _tm(tname("implimf_update"), st);
-    hipLaunchKernelGGL(k_impl_update, g, t, 0, st, b, v, (long)ldv, d, nvar);
+    hipLaunchKernelGGL(k_impl_update, with_shell(b, g), t, 0, st, b, v, (long)ldv, d, nvar);
   }
   return codens_check_launch(what);
 }
@@ -1366,15 +1365,15 @@ int codens_implimf_3d_with(const codens_block *b, const codens_phys *ph, const d
 }
 
 // ---------------------------------------------------------------------------
-// implimf_3d for all blocks of a layout.  Each pass (zero d, coefficients,
-// first sub-iteration, the lmx-1 tiled sub-iterations, update) is one
+// implimf_3d for all blocks of a layout.  Each pass (coefficients, first
+// sub-iteration, the lmx-1 tiled sub-iterations, update) is one
 // flattened launch over every block; a device table gives each block its
 // extents and its first workgroup per pass, and a workgroup runs the
 // per-block kernel's own body on its block's tile.  Block l's coefficients,
 // diagonal and ping-pong increment (9 planes of nnn) start at 9 npc of the
 // workspace.  The sub-iterations of small blocks then share the chip instead
 // of each filling a few CUs.
-enum { IB_ZERO, IB_CELL, IB_SWEEP, IB_COEF, IB_SWEEP2, IB_N };
+enum { IB_ZERO, IB_CELL, IB_SWEEP, IB_COEF, IB_SWEEP2, IB_SHELL, IB_N };
 
 struct ImplEnt {
   Blk b;
@@ -1464,9 +1463,17 @@ k_impl_sweep2_batch(const ImplEnt *__restrict__ tab, int nb, Phys ph, const doub
                   v, ldv, sn_all + 9 * b.npc, c, c + 3 * b.nnn, out_d ? B : A, out_d ? A : B, sx, flag);
 }
 
-__global__ void __launch_bounds__(TX *TY) k_impl_update_batch(const ImplEnt *__restrict__ tab, int nb, double *v,
-                                                              long ldv, const double *__restrict__ d, int nvar) {
-  const unsigned wg = xcd_linear();
+// the update in the first workgroups, d = 0 on the ghosts in those from cells on
+__global__ void __launch_bounds__(TX *TY) k_impl_update_batch(const ImplEnt *__restrict__ tab, int nb, unsigned cells,
+                                                              double *v, long ldv, double *d, int nvar) {
+  if (blockIdx.x >= cells) {
+    const unsigned sh = blockIdx.x - cells;
+    const ImplEnt &E = tab[tab_find(tab, nb, IB_SHELL, sh)];
+    const Blk b = E.b;
+    shell_entries(b, (long)(sh - E.start[IB_SHELL]), b.npc, b.npc + b.nnn - 1, d, ldv, 5);
+    return;
+  }
+  const unsigned wg = xcd_linear(cells);
   const ImplEnt &E = tab[tab_find(tab, nb, IB_CELL, wg)];
   update_body(E.b, tab_tile(E, IB_CELL, wg), v, ldv, d, nvar);
 }
@@ -1523,7 +1530,8 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
                            {cg.x, cg.y, cg.z},
                            {ntx, nty, nkz},
                            {cg.x, cg.y, (unsigned)((b.k2 - b.k1 + E.ks_coef - 1) / E.ks_coef)},
-                           {n2x, n2y, (unsigned)slabs(nz, E.ks_sweep2)}};
+                           {n2x, n2y, (unsigned)slabs(nz, E.ks_sweep2)},
+                           {(unsigned)((shell_count(b) + 256 * SHELL_PER - 1) / (256 * SHELL_PER)), 1, 1}};
     for (int p = 0; p < IB_N; p++) {
       E.start[p] = tot[p];
       E.gx[p] = g[p][0];
@@ -1552,7 +1560,7 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
   const ImplEnt *ct = tab;
   const int nb = nblk;
   const double *fx = ityprk ? ff : u;
-  hipLaunchKernelGGL(k_zero5_batch, dim3(tot[IB_ZERO]), dim3(256), 0, st, ct, nb, d, (long)ldv);
+  if (lmx < 1) hipLaunchKernelGGL(k_zero5_batch, dim3(tot[IB_ZERO]), dim3(256), 0, st, ct, nb, d, (long)ldv);
   {
     CodensTimed _tm("implimf_coef", st);
     hipLaunchKernelGGL(k_impl_coef_batch, dim3(tot[IB_COEF]), dim3(TX, TY), 0, st, ct, nb, ph, (const double *)v,
@@ -1579,8 +1587,8 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
   }
   {
     CodensTimed _tm("implimf_update", st);
-    hipLaunchKernelGGL(k_impl_update_batch, dim3(tot[IB_CELL]), dim3(TX, TY), 0, st, ct, nb, v, (long)ldv,
-                       (const double *)d, 5);
+    hipLaunchKernelGGL(k_impl_update_batch, dim3(tot[IB_CELL] + tot[IB_SHELL]), dim3(TX, TY), 0, st, ct, nb,
+                       tot[IB_CELL], v, (long)ldv, d, 5);
   }
   return codens_check_launch(what);
 }
@@ -1591,7 +1599,8 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
 // d = the FP32 increment widened to FP64, v += d (real cells)
 __global__ void __launch_bounds__(TX *TY) k_impl_update_f32(Blk b, double *v, long ldv, double *d,
                                                             const float *__restrict__ df) {
-  CELL3(b)
+  if (shell_layers(b, b.k2 - b.k1, b.npc, b.npc + b.nnn - 1, d, ldv, 5)) return;  // d = 0 on the ghosts
+  CELL3_AT(b, xcd_block(false, b.k2 - b.k1))
   long n = b.idx(c[0], c[1], c[2]), m = n - b.npc;
 #pragma unroll
   for (int e = 0; e < 5; e++) {
@@ -1626,9 +1635,7 @@ extern "C" int codens_implimf_3d_f32(const codens_block *cb, const codens_phys *
   float *vF = wf, *uF = wf + 5 * nnn, *fF = wf + 10 * nnn, *snF = wf + 15 * nnn, *cF = wf + 24 * nnn;
   float *dgF = cF + 3 * nnn, *dA = wf + 28 * nnn, *dB = wf + 33 * nnn;
   dim3 g1((unsigned)((nnn + 255) / 256)), t1(256);
-  // d = 0 on the ghosts; the update writes every real cell
-  if (lmx >= 1) codens_zero_shell(b, (long)b.npc, (long)(b.npc + nnn - 1), d, (long)ldv, 5, st);
-  else hipLaunchKernelGGL(k_zero5, g1, t1, 0, st, d, (long)ldv, (long)b.npc, (long)(b.npc + nnn - 1));
+  if (lmx < 1) hipLaunchKernelGGL(k_zero5, g1, t1, 0, st, d, (long)ldv, (long)b.npc, (long)(b.npc + nnn - 1));
   dim3 g = cell_grid(b), t(TX, TY);
   {
     CodensTimed _tm("implimf32_coef", st);
@@ -1660,7 +1667,7 @@ extern "C" int codens_implimf_3d_f32(const codens_block *cb, const codens_phys *
   }
   if (lmx > 0) {
     CodensTimed _tm("implimf32_update", st);
-    hipLaunchKernelGGL(k_impl_update_f32, g, t, 0, st, b, v, (long)ldv, d, (const float *)last.p);
+    hipLaunchKernelGGL(k_impl_update_f32, with_shell(b, g), t, 0, st, b, v, (long)ldv, d, (const float *)last.p);
   }
   return codens_check_launch(what);
 }

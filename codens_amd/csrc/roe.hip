@@ -771,7 +771,12 @@ __device__ __forceinline__ void fused_body(const FusedArgs &A, dim3 t) {
 
 template <bool NS, bool LIM>
 __global__ void __launch_bounds__(FT *FT) __attribute__((amdgpu_waves_per_eu(2))) k_residual_fused(FusedArgs A) {
-  fused_body<NS, LIM>(A, xcd_block());
+  const Blk &b = A.b;
+  const int nz = (b.k2 - b.k1 + A.ks - 1) / A.ks;
+  // u = 0 on the entries of indc(i1-1,j1-1,k1-1)..indc(i2,j2,k2) that are not
+  // real cells (sch_roe.f90:110-125)
+  if (shell_layers(b, nz, b.idx(b.i1 - 1, b.j1 - 1, b.k1 - 1), b.idx(b.i2, b.j2, b.k2), A.u, A.ldv, 5)) return;
+  fused_body<NS, LIM>(A, xcd_block(false, nz));
 }
 
 // u = 0 on the entries of indc(i1-1,j1-1,k1-1)..indc(i2,j2,k2) that are not
@@ -851,12 +856,11 @@ static int roe_common(const codens_block *cb, const codens_phys *cp, const coden
     FusedArgs A{b, ph, 0.25 * sc->muscl, sc->xk, v, ldv, ps, ns ? tq : v, sn, R, u, ff, ityprk, ks};
     {
       CodensTimed _tm("roe_fused", st);
+      g = with_shell(b, g);
       if (ns && ilim == 1) hipLaunchKernelGGL((k_residual_fused<true, true>), g, dim3(FT * FT), 0, st, A);
       else if (ns) hipLaunchKernelGGL((k_residual_fused<true, false>), g, dim3(FT * FT), 0, st, A);
       else hipLaunchKernelGGL((k_residual_fused<false, false>), g, dim3(FT * FT), 0, st, A);
     }
-    CodensTimed _tm("roe_zero_ghost", st);
-    codens_zero_shell(b, n0, n1, u, ldv, 5, st);
     return codens_check_launch(what);
   }
   for (int d = 0; d < 3; d++) {
