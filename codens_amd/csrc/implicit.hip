@@ -1041,6 +1041,96 @@ k_impl_sweep2(Blk b, Phys ph, int ntx, int nty, int ks, const double *__restrict
 }
 
 // ---------------------------------------------------------------------------
+// A sub-iteration of a small block.  The tiled kernel's workgroup there waits
+// for its loads three times (the planes below, its own, the one above) with
+// one or two waves on a compute unit, 7 us on 32 x 16 x 8; here eight lanes
+// share a cell and everything is loaded at once: lane 0 of a cell forms its q,
+// lanes 1..6 that of a neighbour and the term of the face to it, then lane e
+// sums equation e in the order of sweep_tile.inc.  The operations are those of
+// the pair kernel, so the bits are those of the other kernels.  A wave holds
+// eight cells of a row, lane = role * 8 + cell.  It computes each q seven
+// times and loads it from the L2, so it pays only while the chip is not full:
+constexpr int SM_CELLS = 8;
+constexpr long SMALL_BLOCK = 16384;  // real cells
+
+template <bool FIRST>
+__global__ void __launch_bounds__(64) k_impl_sweep_small(Blk b, Phys ph, int ityprk, const double *__restrict__ u,
+                                                         const double *__restrict__ ff,
+                                                         const double *__restrict__ v, long ldv,
+                                                         const double *__restrict__ sn,
+                                                         const double *__restrict__ coefe,
+                                                         const double *__restrict__ diag, DView dold, DView dnew) {
+#pragma clang fp contract(off)
+  __shared__ double own[12][SM_CELLS], tnf[5][6][SM_CELLS], dnb[5][6][SM_CELLS], cf[6][SM_CELLS];
+  const int lane = threadIdx.x, c = lane % SM_CELLS, role = lane / SM_CELLS, f = max(role - 1, 0) % 6;
+  const int nx = b.i2 - b.i1, ny = b.j2 - b.j1, nz = b.k2 - b.k1;
+  const int cell = blockIdx.x * SM_CELLS + c;
+  const bool in = cell < nx * ny * nz;
+  const int x = in ? cell : 0;
+  const int ci = x % nx, cj = (x / nx) % ny, ck = x / (nx * ny);
+  const long n = b.idx(b.i1 + ci, b.j1 + cj, b.k1 + ck), m = n - b.npc, nnn = b.nnn;
+  // this lane's cell and face
+  const int d = f / 2;
+  const bool high = f % 2, nb = role >= 1 && role <= 6;
+  const long inc = d == 0 ? 1 : (d == 1 ? b.nid : b.nijd);
+  const int at = d == 0 ? ci : (d == 1 ? cj : ck), len = d == 0 ? nx : (d == 1 ? ny : nz);
+  const bool real = !nb || (high ? at + 1 < len : at > 0);
+  const long nr = nb && real ? (high ? n + inc : n - inc) : n, mf = high ? m + inc : m;
+  const int e = min(role, 4);
+  double V[5], D[5], s[3], q[14];
+#pragma unroll
+  for (int x = 0; x < 5; x++) {
+    V[x] = v[x * ldv + nr];
+    D[x] = FIRST ? -u[x * ldv + nr] : dold.at(x, nr);
+  }
+  const double gr = FIRST ? diag[nr - b.npc] : 1.;
+  if (FIRST && ityprk) {
+#pragma unroll
+    for (int x = 0; x < 5; x++) D[x] = D[x] - ff[x * ldv + nr];
+  }
+#pragma unroll
+  for (int x = 0; x < 3; x++) s[x] = sn[(x * 3 + d) * nnn + mf];
+  const double co = coefe[d * nnn + (real ? mf : m)], uu = u[e * ldv + n], dg = diag[m];
+  const double fv = ityprk ? ff[e * ldv + n] : 0.;
+  if (FIRST) {
+#pragma unroll
+    for (int x = 0; x < 5; x++) D[x] = D[x] / gr;
+  }
+  dflux_q(ph, V, D, q);
+  if (!real) {
+#pragma unroll
+    for (int x = 0; x < 14; x++) q[x] = 0.;
+  }
+  if (role == 0) {
+#pragma unroll
+    for (int x = 0; x < 12; x++) own[x][c] = q[x];
+  }
+  __syncthreads();
+  if (nb) {
+    double tn[5];
+    tn2_fma(q, s, tn, [&](int x) { return own[x][c]; });
+#pragma unroll
+    for (int x = 0; x < 5; x++) {
+      tnf[x][f][c] = tn[x];
+      dnb[x][f][c] = q[q_comp(x)];
+    }
+    cf[f][c] = co;
+  }
+  __syncthreads();
+  if (role < 5 && in) {
+    double w = -uu - fv;
+#pragma unroll
+    for (int x = 0; x < 3; x++) {
+      const int p = x == 0 ? ci : (x == 1 ? cj : ck), l = x == 0 ? nx : (x == 1 ? ny : nz);
+      w = fma(cf[2 * x][c], dnb[e][2 * x][c], fma(0.5, tnf[e][2 * x][c], w));
+      if (p + 1 < l) w = fma(cf[2 * x + 1][c], dnb[e][2 * x + 1][c], w);
+      w = fma(-0.5, tnf[e][2 * x + 1][c], w);
+    }
+    dnew.at(e, n) = w * (1. / dg);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Tile shape of the tiled sub-iteration, per block shape: 64 x 4, 32 x 8 or
 // 16 x 16, all of 256 threads.  Every cell's arithmetic is the same in all,
 // so the increments are identical bit for bit; what differs is how many
@@ -1317,19 +1407,27 @@ static int implimf_common(bool eu, const codens_block *cb, const codens_phys *cp
   }
   DView A = {d, (long)ldv, 0}, B = {W, b.nnn, b.npc};
   int tile = 0;
-  // sub-iteration 1 starts from d = 0: d = -u/diag (k_impl_sweep1); the
-  // others run in pairs, one left over on its own, alternate launches in
-  // reverse tile order; a forced tile shape, the Euler form, or a block where
-  // pairs do not pay (pair_model), runs them one by one.  The launches
-  // alternate between the two buffers, the last one landing in d.
-  const SweepPlan plan = sweep_plan(lmx, !eu && forced_tile() < 0 && pair_model(b));
+  // sub-iteration 1 starts from d = 0: d = -u/diag (k_impl_sweep1, or the
+  // second one on a small block); the others run in pairs, one left over on its
+  // own, alternate launches in reverse tile order; a small block, a forced tile
+  // shape, the Euler form, or a block where pairs do not pay (pair_model),
+  // runs them one by one.  The launches alternate between the two buffers, the
+  // last one landing in d.
+  const long cells = (long)(b.i2 - b.i1) * (b.j2 - b.j1) * (b.k2 - b.k1);
+  const bool choose = !eu && forced_tile() < 0, small = choose && cells <= SMALL_BLOCK;
+  const SweepPlan plan = sweep_plan(lmx, choose && !small && pair_model(b));
   const double *fx = ityprk ? ff : u, *psx = eu ? ps : v;
   for (int s = 0; s < plan.n; s++) {
     DView out = ((plan.n - 1 - s) % 2 == 0) ? A : B;
     DView in = ((plan.n - 1 - s) % 2 == 0) ? B : A;
+    if (s == 0 && small && plan.single > 0) continue;  // formed by the second
     if (s == 0) {
       CodensTimed _tm(tname("implimf_sweep1"), st);
       hipLaunchKernelGGL(k_impl_sweep1<double>, g, t, 0, st, b, (int)ityprk, u, fx, (long)ldv, diag, out);
+    } else if (s <= plan.single && small) {
+      CodensTimed _tm(tname("implimf_sweep"), st);
+      hipLaunchKernelGGL(s == 1 ? k_impl_sweep_small<true> : k_impl_sweep_small<false>, dim3((unsigned)((cells + SM_CELLS - 1) / SM_CELLS)), dim3(64), 0, st, b, ph,
+                         (int)ityprk, u, fx, (const double *)v, (long)ldv, sn, coefe, diag, in, out);
     } else if (s <= plan.single) {
       if (s == 1 && fixed)
         tile = known_tile(b, eu, (int)sizeof(double));

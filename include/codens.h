@@ -619,8 +619,9 @@ int codens_workspace_set(int32_t set);
  * hold the first two: there a forced 16 x 16 takes the lane model's choice
  * between them: launched lanes times each shape's measured time per lane).
  * In mode -1 the FP64 sub-iterations of codens_implimf_3d run two to a
- * launch, one left over alone, on blocks where that is modelled faster; a
- * forced shape runs every one alone.  All give identical results.  *previous (may be NULL) receives the mode in
+ * launch, one left over alone, on blocks where that is modelled faster, and
+ * blocks of at most 16384 cells use a kernel without tiles; a forced shape
+ * runs every one alone.  All give identical results.  *previous (may be NULL) receives the mode in
  * force before the call. */
 int codens_sweep_tile(int32_t mode, int32_t *previous);
 
@@ -639,7 +640,7 @@ int codens_sweep_tile(int32_t mode, int32_t *previous);
 int codens_residual_path(int32_t fused, int32_t *previous);
 
 /* The tile shape used for a block (eu: implimf_eu, fp32: the FP32 form):
- * 0 or 1, or -1 if not chosen yet. */
+ * 0, 1 or 2, or -1 if not chosen yet or none is used. */
 int codens_sweep_tile_of(const codens_block *b, int32_t eu, int32_t fp32, int32_t *tile);
 
 /* ---- Differentiation of the block residual (no counterpart in the

@@ -1,5 +1,6 @@
-"""The FP64 sub-iterations two to a launch against one to a launch: the same
-operations on every cell, so the same bits."""
+"""The FP64 sub-iterations two to a launch, and those of small blocks, against
+the tiled kernel's, one to a launch: the same operations on every cell, so the
+same bits."""
 import numpy as np
 import pytest
 import torch
@@ -83,3 +84,25 @@ def test_batched_pairs_match_singles(lmx, ityprk):
     two, one, launches = pair_launches(abi, call)
     assert launches == 1, "these blocks run in pairs"
     assert np.array_equal(two[0], one[0]) and np.array_equal(two[1], one[1])
+
+
+# eight cells to a wave: fewer, a row's end inside a wave, the largest block
+@pytest.mark.parametrize("dims", [(2, 2, 2), (5, 3, 2), (17, 9, 7), (32, 32, 16), (2, 90, 2)])
+@pytest.mark.parametrize("lmx,ityprk", [(2, 0), (3, 1), (4, 0)])
+def test_small_block_matches_tiles(dims, lmx, ityprk):
+    from codens_amd import abi
+    lay, sn, vol = random_mesh([dims], seed=13)
+    b = lay.blocks[0]
+    f = fields(lay, near=lmx == 3)
+    snb, g = T(sn[9 * b.npc: 9 * (b.npc + b.nnn)]), {k: T(a) for k, a in f.items()}
+
+    def call():
+        v, d = T(f["v"]), T(np.full_like(f["v"], 5.))
+        abi.timing_read("implimf_sweep1", reset=True)
+        abi.implimf_3d(abi.block(b), abi.phys(), g["u"], g["dt"], v, d, g["ff"], g["mu"], g["mut"], lmx, snb,
+                       T(vol), g["ps"], g["c"], ityprk=ityprk)
+        return v.cpu().numpy(), d.cpu().numpy(), abi.timing_read("implimf_sweep1", reset=True)[1]
+
+    here, tiled, _ = pair_launches(abi, call)
+    assert (here[2], tiled[2]) == (0, 1), "the small block's kernel forms the first increment"
+    assert np.array_equal(here[0], tiled[0]) and np.array_equal(here[1], tiled[1])
