@@ -67,6 +67,14 @@ __device__ __forceinline__ double rcp64(double x) {
   return fma(r, e, r);
 }
 
+// x / d, y = rcp64(d): the steps of the compiler's division after its
+// reciprocal, so that quotients of one divisor share that; zeros, infinities
+// and NaN as there
+__device__ __forceinline__ double div_rcp(double x, double d, double y) {
+  const double q = x * y;
+  return __builtin_amdgcn_div_fixup(fma(fma(-d, q, x), y, q), d, x);
+}
+
 // sn(m, d, c) of a block's metric slice (snorm.f90:65-71)
 __device__ inline double snv(const double *__restrict__ sn, long nnn, long m, int d, int c) {
   return sn[((long)c * 3 + d) * nnn + m];
@@ -95,6 +103,59 @@ __device__ inline dim3 xcd_block(bool rev = false) { return xcd_block(rev, gridD
 inline dim3 cell_grid(const Blk &b) {
   int nx = b.i2 - b.i1, ny = b.j2 - b.j1, nz = b.k2 - b.k1;
   return dim3((nx + TX - 1) / TX, (ny + TY - 1) / TY, nz);
+}
+
+// A launch over the real cells and a margin of ghosts around them in storage
+// order, 256 to a workgroup (dim3(TX, TY) or 256): no lane is idle where the
+// row is no multiple of TX, as a third of cell_grid's are on blocks 16 to 96
+// wide (the gradients of the velocity there 20.7 us a block, so 18.0).
+inline dim3 cell_line(const Blk &b, int margin = 0) {
+  const long e = 2 * margin;
+  return dim3((unsigned)(((b.i2 - b.i1 + e) * (b.j2 - b.j1 + e) * (b.k2 - b.k1 + e) + 255) / 256));
+}
+__device__ __forceinline__ bool line_cell(const Blk &b, unsigned wg, int c[3], int margin = 0) {
+  const unsigned e = 2 * margin, nx = b.i2 - b.i1 + e, ny = b.j2 - b.j1 + e, nz = b.k2 - b.k1 + e;
+  const unsigned t = wg * 256u + threadIdx.x + threadIdx.y * TX, row = t / nx, k = row / ny;
+  c[0] = b.i1 - margin + (int)(t - row * nx);
+  c[1] = b.j1 - margin + (int)(row - k * ny);
+  c[2] = b.k1 - margin + (int)k;
+  return k < nz;
+}
+
+// All of a cell's loads are issued before this and used after it: the compiler
+// otherwise spreads them between the divisions to save registers, and the
+// velocity gradients waited for 17 loads one after another.
+__device__ __forceinline__ void loads_issued() { __builtin_amdgcn_sched_barrier(0); }
+
+// plane-relative load: base is uniform (the plane's first entry), off the
+// cell's 32-bit byte offset in the plane, so that the address is a scalar base
+// and one register (a plane of more than 2^29 entries would take a block of
+// more than 2^31).  The empty asm keeps the compiler from folding the uniform
+// part into per-thread 64-bit addresses.
+template <typename T>
+using GPtr = __attribute__((address_space(1))) T *;
+template <typename T>
+__device__ __forceinline__ GPtr<T> gp(T *base, unsigned off) {
+  uint64_t p = (uint64_t)base;
+  asm("" : "+s"(p));
+  return (GPtr<T>)((GPtr<char>)p + off);
+}
+template <typename T>
+__device__ __forceinline__ T ldp(const T *base, unsigned off) {
+  return *gp(base, off);
+}
+// Hides an offset's value from the loop optimiser, which would otherwise keep
+// a 64-bit address per array and thread in registers and advance them all.
+__device__ __forceinline__ unsigned opaque(unsigned x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// Workgroup barrier that orders only the LDS traffic of the plane exchange.
+__device__ inline void lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // The non-real (ghost) entries of a block's storage, in this order: the k
@@ -159,6 +220,7 @@ __host__ __device__ inline long shell_entry(const Blk &b, const Shell &s, long t
 // fused residual of 256 x 128 x 64, whose workgroups fill the chip twice, took
 // 490 us instead of 370.
 constexpr int SHELL_PER = 4;
+inline unsigned shell_wgs(const Blk &b) { return (unsigned)((shell_count(b) + 256 * SHELL_PER - 1) / (256 * SHELL_PER)); }
 inline dim3 with_shell(const Blk &b, dim3 g) {
   const long per = 256L * SHELL_PER * g.x * g.y;
   g.z += (unsigned)((shell_count(b) + per - 1) / per);

@@ -10,14 +10,10 @@
 
 using namespace codens;
 
-#define CELL_IJK(b)                                   \
-  const dim3 xb = xcd_block();                        \
-  CELL_AT(b, xb)
-#define CELL_AT(b, xb)                                \
-  int i = (b).i1 + xb.x * TX + threadIdx.x;     \
-  int j = (b).j1 + xb.y * TY + threadIdx.y;     \
-  int k = (b).k1 + xb.z;                        \
-  if (i >= (b).i2 || j >= (b).j2) return;
+#define CELL_IJK(b)                                \
+  int ijk[3];                                      \
+  if (!line_cell((b), xcd_linear(), ijk)) return;  \
+  const int i = ijk[0], j = ijk[1], k = ijk[2];
 
 // zpres.f90:66-79
 __global__ void __launch_bounds__(TX *TY) k_zpres(Blk b, Phys ph, const double *__restrict__ v, long ldv,
@@ -67,14 +63,16 @@ __global__ void __launch_bounds__(TX *TY) k_chronos(Blk b, Phys ph, double etal,
                                                     const double *__restrict__ sn,
                                                     const double *__restrict__ vol,
                                                     const double *__restrict__ cson,
-                                                    double *__restrict__ dt) {
-  const int nz = b.k2 - b.k1;
+                                                    double *__restrict__ dt, unsigned cells) {
   // chronos.f90:110-114 zeroes dt over indc(i1,j1,k1)..indc(i2,j2,k2): the
-  // ghost entries of that range here
-  if (shell_layers(b, nz, b.idx(b.i1, b.j1, b.k1), b.idx(b.i2, b.j2, b.k2), dt, 0, 1)) return;
-  const dim3 xb = xcd_block(false, nz);
-  CELL_AT(b, xb)
-  long n = b.idx(i, j, k), m = n - b.npc;
+  // ghost entries of that range in the workgroups after those of the cells
+  if (blockIdx.x >= cells) {
+    shell_entries(b, blockIdx.x - cells, b.idx(b.i1, b.j1, b.k1), b.idx(b.i2, b.j2, b.k2), dt, 0, 1);
+    return;
+  }
+  int c[3];
+  if (!line_cell(b, xcd_linear(cells), c)) return;
+  long n = b.idx(c[0], c[1], c[2]), m = n - b.npc;
   double simax = fmax(face_s2(sn, b.nnn, m + 1, 0), face_s2(sn, b.nnn, m, 0));
   double sjmax = fmax(face_s2(sn, b.nnn, m + b.nid, 1), face_s2(sn, b.nnn, m, 1));
   double skmax = fmax(face_s2(sn, b.nnn, m + b.nijd, 2), face_s2(sn, b.nnn, m, 2));
@@ -130,7 +128,7 @@ extern "C" int codens_zpres(const codens_block *cb, const codens_phys *cp, const
   Blk b = make_blk(cb);
   {
     CodensTimed _tm("zpres", (hipStream_t)stream);
-    hipLaunchKernelGGL(k_zpres, cell_grid(b), dim3(TX, TY), 0, (hipStream_t)stream, b, make_phys(cp), v,
+    hipLaunchKernelGGL(k_zpres, cell_line(b), dim3(TX, TY), 0, (hipStream_t)stream, b, make_phys(cp), v,
                      (long)ldv, ps, temp, cson);
   }
   return codens_check_launch("codens_zpres");
@@ -147,7 +145,7 @@ extern "C" int codens_zvismo(const codens_block *cb, const codens_phys *cp, cons
   Blk b = make_blk(cb);
   {
     CodensTimed _tm("zvismo", (hipStream_t)stream);
-    hipLaunchKernelGGL(k_zvismo, cell_grid(b), dim3(TX, TY), 0, (hipStream_t)stream, b, make_phys(cp), temp,
+    hipLaunchKernelGGL(k_zvismo, cell_line(b), dim3(TX, TY), 0, (hipStream_t)stream, b, make_phys(cp), temp,
                      mu, (int *)nbad);
   }
   return codens_check_launch("codens_zvismo");
@@ -167,8 +165,9 @@ extern "C" int codens_chronos(const codens_block *cb, const codens_phys *cp, dou
   hipStream_t st = (hipStream_t)stream;
   {
     CodensTimed _tm("chronos", st);
-    hipLaunchKernelGGL(k_chronos, with_shell(b, cell_grid(b)), dim3(TX, TY), 0, st, b, make_phys(cp), eta, (int)ns, v,
-                     (long)ldv, mu, mut, sn, vol, cson, dt);
+    const unsigned cells = cell_line(b).x;
+    hipLaunchKernelGGL(k_chronos, dim3(cells + shell_wgs(b)), dim3(TX, TY), 0, st, b, make_phys(cp), eta, (int)ns, v,
+                       (long)ldv, mu, mut, sn, vol, cson, dt, cells);
   }
   return codens_check_launch("codens_chronos");
 }
@@ -184,7 +183,7 @@ extern "C" int codens_sch_expli(const codens_block *cb, const double *u, double 
   Blk b = make_blk(cb);
   {
     CodensTimed _tm("sch_expli", (hipStream_t)stream);
-    hipLaunchKernelGGL(k_sch_expli, cell_grid(b), dim3(TX, TY), 0, (hipStream_t)stream, b, u, v, (long)ldv,
+    hipLaunchKernelGGL(k_sch_expli, cell_line(b), dim3(TX, TY), 0, (hipStream_t)stream, b, u, v, (long)ldv,
                      dt, vol);
   }
   return codens_check_launch("codens_sch_expli");
@@ -201,7 +200,7 @@ extern "C" int codens_rk_stage(const codens_block *cb, double alpha, const doubl
   Blk b = make_blk(cb);
   {
     CodensTimed _tm("rk_stage", (hipStream_t)stream);
-    hipLaunchKernelGGL(k_rk_stage, cell_grid(b), dim3(TX, TY), 0, (hipStream_t)stream, b, alpha, v0, u, v,
+    hipLaunchKernelGGL(k_rk_stage, cell_line(b), dim3(TX, TY), 0, (hipStream_t)stream, b, alpha, v0, u, v,
                        (long)ldv, dt, vol, (int)nvar);
   }
   return codens_check_launch("codens_rk_stage");

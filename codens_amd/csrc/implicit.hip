@@ -171,37 +171,6 @@ __device__ inline void face_tn(const DFlux &A, const DFlux &B, double s1, double
   c[2] = (b).k1 + xb.z;                        \
   if (c[0] >= (b).i2 || c[1] >= (b).j2) return;
 
-// plane-relative load: base is uniform (the plane's first entry), off the
-// cell's 32-bit byte offset in the plane, so that the address is a scalar base
-// and one register (a plane of more than 2^29 entries would take a block of
-// more than 2^31).  The empty asm keeps the compiler from folding the uniform
-// part into per-thread 64-bit addresses.
-template <typename T>
-using GPtr = __attribute__((address_space(1))) T *;
-template <typename T>
-__device__ __forceinline__ GPtr<T> gp(T *base, unsigned off) {
-  uint64_t p = (uint64_t)base;
-  asm("" : "+s"(p));
-  return (GPtr<T>)((GPtr<char>)p + off);
-}
-template <typename T>
-__device__ __forceinline__ T ldp(const T *base, unsigned off) {
-  return *gp(base, off);
-}
-// Hides an offset's value from the loop optimiser, which would otherwise keep
-// a 64-bit address per array and thread in registers and advance them all.
-__device__ __forceinline__ unsigned opaque(unsigned x) {
-  asm volatile("" : "+v"(x));
-  return x;
-}
-
-// Workgroup barrier that orders only the LDS traffic of the plane exchange.
-__device__ inline void lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // implimf_3d.f90:113-224: spectral-radius coefficients of the faces and the
 // diagonal; coefe[d] holds the low face of every real cell.  A workgroup
 // owns a TX x TY tile of real cells and marches a slab of up to CK_KS
@@ -1629,7 +1598,7 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
                            {ntx, nty, nkz},
                            {cg.x, cg.y, (unsigned)((b.k2 - b.k1 + E.ks_coef - 1) / E.ks_coef)},
                            {n2x, n2y, (unsigned)slabs(nz, E.ks_sweep2)},
-                           {(unsigned)((shell_count(b) + 256 * SHELL_PER - 1) / (256 * SHELL_PER)), 1, 1}};
+                           {shell_wgs(b), 1, 1}};
     for (int p = 0; p < IB_N; p++) {
       E.start[p] = tot[p];
       E.gx[p] = g[p][0];

@@ -10,15 +10,9 @@
 
 using namespace codens;
 
-#define REAL3(b) REAL3_AT(b, xcd_block())
-// the same, for the tile XB of a block's own grid
-#define REAL3_AT(b, XB)                              \
-  const dim3 xb = (XB);                              \
-  int c[3];                                          \
-  c[0] = (b).i1 + xb.x * TX + threadIdx.x;           \
-  c[1] = (b).j1 + xb.y * TY + threadIdx.y;           \
-  c[2] = (b).k1 + xb.z;                              \
-  if (c[0] >= (b).i2 || c[1] >= (b).j2) return;
+#define REAL3(b)  \
+  int c[3];       \
+  if (!line_cell((b), xcd_linear(), c)) return;
 
 // Workspace of the implicit phase: the half normal velocities uf and the
 // coefficients ce of the faces of the three directions, the increments dw6,
@@ -37,14 +31,6 @@ constexpr int IMPLI_PLANES = 19;
 __host__ __device__ inline ImpliWs impli_ws(double *ws, long nnn) {
   return ImpliWs{ws,           ws + 3 * nnn,  ws + 6 * nnn,  ws + 7 * nnn,  ws + 8 * nnn,
                  ws + 9 * nnn, ws + 10 * nnn, ws + 13 * nnn, ws + 16 * nnn, ws + 6 * nnn};
-}
-
-// x / d, y = rcp64(d): the steps of the compiler's division after its
-// reciprocal, so that quotients of one divisor share that; zeros, infinities
-// and NaN as there
-__device__ __forceinline__ double div_rcp(double x, double d, double y) {
-  const double q = x * y;
-  return __builtin_amdgcn_div_fixup(fma(fma(-d, q, x), y, q), d, x);
 }
 
 // impli2_eqt_3d.f90:113-208: coefficients of every face i1..i2 (resp. j, k)
@@ -628,7 +614,7 @@ extern "C" int codens_met_samut(const codens_block *cb, const double *tc, const 
   }
   Blk b = make_blk(cb);
   double cv1 = tc[7];
-  hipLaunchKernelGGL(k_met_samut, cell_grid(b), dim3(TX, TY), 0, (hipStream_t)stream, b, cv1 * cv1 * cv1, v,
+  hipLaunchKernelGGL(k_met_samut, cell_line(b), dim3(TX, TY), 0, (hipStream_t)stream, b, cv1 * cv1 * cv1, v,
                      (long)ldv, mu, mut);
   return codens_check_launch("codens_met_samut");
 }
@@ -647,7 +633,7 @@ extern "C" int codens_met_kocmut(const codens_block *cb, const double *tc, int32
     if (rc) return rc;
   }
   Blk b = make_blk(cb);
-  hipLaunchKernelGGL(k_met_kocmut, cell_grid(b), dim3(TX, TY), 0, (hipStream_t)stream, b, (int)kwsst, tc[10], v,
+  hipLaunchKernelGGL(k_met_kocmut, cell_line(b), dim3(TX, TY), 0, (hipStream_t)stream, b, (int)kwsst, tc[10], v,
                      (long)ldv, mu, mut, dist, g9);
   return codens_check_launch("codens_met_kocmut");
 }
@@ -661,7 +647,7 @@ extern "C" int codens_met_cut(const codens_block *cb, int32_t which, double epsk
     return CODENS_EINVAL;
   }
   Blk b = make_blk(cb);
-  hipLaunchKernelGGL(k_met_cut, cell_grid(b), dim3(TX, TY), 0, (hipStream_t)stream, b, (int)which, epsk, epse, v,
+  hipLaunchKernelGGL(k_met_cut, cell_line(b), dim3(TX, TY), 0, (hipStream_t)stream, b, (int)which, epsk, epse, v,
                      (long)ldv);
   return codens_check_launch("codens_met_cut");
 }
@@ -729,7 +715,7 @@ extern "C" int codens_met_smkor(const codens_block *cb, const double *tc, double
     return CODENS_EINVAL;
   }
   Blk b = make_blk(cb);
-  hipLaunchKernelGGL(k_met_smkor, cell_grid(b), dim3(TX, TY), 0, (hipStream_t)stream, b, tc[11], tc[10], tc[13],
+  hipLaunchKernelGGL(k_met_smkor, cell_line(b), dim3(TX, TY), 0, (hipStream_t)stream, b, tc[11], tc[10], tc[13],
                      sigmd, v, (long)ldv, fd, g9, tprod, cfke, ts6, ts7);
   return codens_check_launch("codens_met_smkor");
 }
@@ -744,7 +730,7 @@ extern "C" int codens_met_smch(const codens_block *cb, double cke1, double cke2,
     return CODENS_EINVAL;
   }
   Blk b = make_blk(cb);
-  hipLaunchKernelGGL(k_met_smch, cell_grid(b), dim3(TX, TY), 0, (hipStream_t)stream, b, cke1, cke2, utaumin, v,
+  hipLaunchKernelGGL(k_met_smch, cell_line(b), dim3(TX, TY), 0, (hipStream_t)stream, b, cke1, cke2, utaumin, v,
                      (long)ldv, mu, dist, mnpar, utau, tprod, ts6, ts7);
   return codens_check_launch("codens_met_smch");
 }

@@ -6,13 +6,9 @@
 
 using namespace codens;
 
-#define REAL3(b)                                     \
-  const dim3 xb = xcd_block();                       \
-  int c[3];                                          \
-  c[0] = (b).i1 + xb.x * TX + threadIdx.x;           \
-  c[1] = (b).j1 + xb.y * TY + threadIdx.y;           \
-  c[2] = (b).k1 + xb.z;                              \
-  if (c[0] >= (b).i2 || c[1] >= (b).j2) return;
+#define REAL3(b)  \
+  int c[3];       \
+  if (!line_cell((b), xcd_linear(), c)) return;
 
 namespace {
 // constants as codens_menter orders them
@@ -222,13 +218,13 @@ extern "C" int codens_met_smmt(const codens_block *cb, const double *mc, int32_t
   Blk b = make_blk(cb);
   Menter m = make_menter(mc);
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_smmt_blend, cell_grid(b), dim3(TX, TY), 0, st, b, m, (int)kfracom, v, (long)ldv, mu, dist,
+  hipLaunchKernelGGL(k_smmt_blend, cell_line(b), dim3(TX, TY), 0, st, b, m, (int)kfracom, v, (long)ldv, mu, dist,
                      fd, gkgo, frac);
   if (kfracom != 0 && nfaces > 0) {
     rc = mtcorf1_launch(nfaces, face_start, lines, imxclko, mnpar, frac, ldv, st, "codens_met_smmt");
     if (rc) return rc;
   }
-  hipLaunchKernelGGL(k_smmt_sources, cell_grid(b), dim3(TX, TY), 0, st, b, m, v, (long)ldv, mut, tprod, gkgo, frac,
+  hipLaunchKernelGGL(k_smmt_sources, cell_line(b), dim3(TX, TY), 0, st, b, m, v, (long)ldv, mut, tprod, gkgo, frac,
                      (const double *)nullptr, cfke, ts6, ts7);
   return codens_check_launch("codens_met_smmt");
 }
@@ -252,13 +248,13 @@ extern "C" int codens_met_smmtr(const codens_block *cb, const double *mc, int32_
     codens_set_error("codens_met_smmtr: workspace allocation failed");
     return CODENS_EHIP;
   }
-  hipLaunchKernelGGL(k_smmt_blend, cell_grid(b), dim3(TX, TY), 0, st, b, m, 1, v, (long)ldv, mu, dist, fd, gkgo,
+  hipLaunchKernelGGL(k_smmt_blend, cell_line(b), dim3(TX, TY), 0, st, b, m, 1, v, (long)ldv, mu, dist, fd, gkgo,
                      frac);
   if (nfaces > 0) {
     rc = mtcorf1_launch(nfaces, face_start, lines, imxclko, mnpar, frac, ldv, st, "codens_met_smmtr");
     if (rc) return rc;
   }
-  hipLaunchKernelGGL(k_smmt_sources, cell_grid(b), dim3(TX, TY), 0, st, b, m, v, (long)ldv, mut, tprod, gkgo, frac,
+  hipLaunchKernelGGL(k_smmt_sources, cell_line(b), dim3(TX, TY), 0, st, b, m, v, (long)ldv, mut, tprod, gkgo, frac,
                      g9, cfke, ts6, ts7);
   return codens_check_launch("codens_met_smmtr");
 }
@@ -295,7 +291,7 @@ extern "C" int codens_met_komut(const codens_block *cb, double betae, int32_t ko
     if (rc) return rc;
   }
   Blk b = make_blk(cb);
-  hipLaunchKernelGGL(k_komut, cell_grid(b), dim3(TX, TY), 0, (hipStream_t)stream, b, (int)komsst, betae, v,
+  hipLaunchKernelGGL(k_komut, cell_line(b), dim3(TX, TY), 0, (hipStream_t)stream, b, (int)komsst, betae, v,
                      (long)ldv, mu, mut, dist, g9);
   return codens_check_launch("codens_met_komut");
 }
