@@ -229,6 +229,7 @@ inline dim3 with_shell(const Blk &b, dim3 g) {
 __device__ __forceinline__ void shell_entries(const Blk &b, long wg, long n0, long n1, double *p, long ld, int np) {
   const Shell s = make_shell(b);
   const long cnt = s.na + s.nb + s.nc, t0 = wg * 256L * SHELL_PER + threadIdx.x + threadIdx.y * blockDim.x;
+#pragma unroll 1
   for (int x = 0; x < SHELL_PER; x++) {
     const long t = t0 + x * 256L;
     if (t >= cnt) return;

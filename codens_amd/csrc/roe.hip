@@ -535,8 +535,18 @@ __global__ void __launch_bounds__(256) k_gather(Blk b, long n0, long n1, const d
 //
 // Faces on the block's boundary (a = a1, a2) are the physical flux of the
 // ghost state (sch_roe.f90:497-578), read from HBM (they are few).  The
-// FT+1-th face of each row and column (32 per plane) is taken by half a wave,
-// a different wave on each plane, so the extra work is spread over the four.
+// FT+1-th faces of the rows and those of the columns (16 per plane each) are
+// taken by the first lanes of one wave, another on each plane, so the extra
+// work is spread over the four.
+//
+// Two workgroups per compute unit (two waves per SIMD, of 255 registers and 82
+// KB each), bound by the exchange of memory latency against registers: of a
+// plane's time half is arithmetic.  Its loads go out together, before the first
+// one is used, from scalar bases; q(k-1) and the low k face wait in LDS; the
+// barriers order the LDS traffic only.  256 x 128 x 64 with the limiter 371 ->
+// 312 us, 191 x 101 x 47 183 -> 165, unlimited 96 x 64 x 48 53 -> 47, 32 x 16
+// x 8 16.6 -> 14.3.  A face's normal and ratios loaded one face ahead did not
+// fit the registers (39 spilled, 363 us).
 constexpr int FT = 16;       // tile cells per direction (i, j)
 constexpr int FPP = FT + 4;  // pitch of the primitive plane (halo 2)
 constexpr int FQP = FT + 2;  // pitch of the stress plane (halo 1)
@@ -554,15 +564,21 @@ struct FusedArgs {
   int ks;  // k planes per workgroup
 };
 
-// primitive variables of storage entry n: rho, u, v, w (the divisions of
-// pass 0) and p
-__device__ __forceinline__ void fused_prim(const FusedArgs &A, long n, double q[5]) {
-  double r = A.v[n], ir = rcp64(r);
+// primitive variables of a cell, rho, u, v, w (the divisions of pass 0) and p:
+// loaded (byte offset off of the plane whose first storage entry is n0), then
+// formed
+__device__ __forceinline__ void fused_load(const FusedArgs &A, long n0, unsigned off, double x[5]) {
+#pragma unroll
+  for (int e = 0; e < 4; e++) x[e] = ldp(A.v + (e * A.ldv + n0), off);
+  x[4] = ldp(A.ps + n0, off);
+}
+__device__ __forceinline__ void fused_prim(const double x[5], double q[5]) {
+  const double r = x[0], ir = rcp64(r);
   q[0] = r;
-  q[1] = A.v[A.ldv + n] * ir;
-  q[2] = A.v[2 * A.ldv + n] * ir;
-  q[3] = A.v[3 * A.ldv + n] * ir;
-  q[4] = A.ps[n];
+  q[1] = x[1] * ir;
+  q[2] = x[2] * ir;
+  q[3] = x[3] * ir;
+  q[4] = x[4];
 }
 
 // physical flux of the ghost state of boundary face (direction d, storage
@@ -584,22 +600,31 @@ __device__ __forceinline__ void fused_ghost(const FusedArgs &A, int d, bool low,
 template <bool NS, bool LIM>
 __device__ __forceinline__ void fused_body(const FusedArgs &A, dim3 t) {
   const Blk &b = A.b;
+  // whether the own stresses of plane k+1, loaded for the k face, are kept for
+  // the next plane instead of loaded again: without the limiter's ratios that
+  // was slower (96 x 64 x 48: 50.9 us against 46.7)
+  constexpr bool CARRY = NS && LIM;
   __shared__ double P[5][FPP * FPP];
   __shared__ double Q[NS ? 9 : 1][NS ? FQP * FQP : 1];
   __shared__ double Fi[5][(FT + 1) * FT];
   __shared__ double Fj[5][FT * (FT + 1)];
+  __shared__ double C0[5][FT * FT], HL[5][FT * FT];  // q(k-1) and the low k face of the own column
   const int tid = threadIdx.x, tx = tid % FT, ty = tid / FT;
   const int i0 = b.i1 + (int)t.x * FT, j0 = b.j1 + (int)t.y * FT;
   const int kb = b.k1 + (int)t.z * A.ks, ke = min(kb + A.ks, b.k2);
   const int njd = (int)(b.nijd / b.nid), nkd = (int)(b.nnn / b.nijd);
   const int id2 = b.id1 + (int)b.nid - 1, jd2 = b.jd1 + njd - 1, kd2 = b.kd1 + nkd - 1;
   auto cl = [](int x, int lo, int hi) { return min(max(x, lo), hi); };
-  // own column (clamped into the block's storage: cells past the real ones
-  // are the ghost layer, or beyond it, whose values no needed face uses)
+  // byte offset in a plane, clamped into the block's storage (cells past the
+  // real ones are the ghost layer, or beyond it, whose values no needed face
+  // uses), and the index of a plane's first entry in the block, likewise
+  auto in_plane = [&](int i, int j) {
+    return ((unsigned)(cl(i, b.id1, id2) - b.id1) + (unsigned)(cl(j, b.jd1, jd2) - b.jd1) * (unsigned)b.nid) * 8u;
+  };
+  auto plane = [&](int k) { return (long)(cl(k, b.kd1, kd2) - b.kd1) * b.nijd; };
   const int i = i0 + tx, j = j0 + ty;
   const bool cell = i < b.i2 && j < b.j2;
-  const long col = b.idx(cl(i, b.id1, id2), cl(j, b.jd1, jd2), b.kd1);  // entry at k = kd1
-  auto at = [&](int k) { return col + (long)(cl(k, b.kd1, kd2) - b.kd1) * b.nijd; };
+  const unsigned po = in_plane(i, j);
   // halo element of this thread: prims (tid < 128) or stresses (128..191)
   int hii = 0, hjj = 0, hkind = 0;  // kind 1: prim, 2: stress
   if (tid < 64) {
@@ -614,87 +639,117 @@ __device__ __forceinline__ void fused_body(const FusedArgs &A, dim3 t) {
     else { g -= 32; hii = g % FT; hjj = (g / FT) ? FT : -1; }
     hkind = 2;
   }
-  const long hcol = b.idx(cl(i0 + hii, b.id1, id2), cl(j0 + hjj, b.jd1, jd2), b.kd1);
+  const unsigned ph = in_plane(i0 + hii, j0 + hjj);
   const int so = (ty + 2) * FPP + tx + 2, sq = (ty + 1) * FQP + tx + 1;
-  const double z9[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  // own column registers: c0 = q(k-1), cq = q(k), c2 = q(k+1); Hlo = the
-  // low k face of plane k
-  double c0[5], cq[5], c2[5], Hlo[5];
-  fused_prim(A, at(kb - 1), c0);
-  fused_prim(A, at(kb), cq);
-  fused_prim(A, at(kb + 1), c2);
-  // the low face of the slab's first plane
-  if (cell) {
-    const long n = b.idx(i, j, kb), m = n - b.npc;
-    double s0 = snv(A.sn, b.nnn, m, 2, 0), s1 = snv(A.sn, b.nnn, m, 2, 1), s2 = snv(A.sn, b.nnn, m, 2, 2);
-    if (kb == b.k1) {
-      fused_ghost<NS>(A, 2, true, n, b.nijd, s0, s1, s2, Hlo);
-    } else {
-      double q[4][5], rl[5], rh[5], tl[9], tr[9];
-      fused_prim(A, at(kb - 2), q[0]);
+  auto load_tq = [&](long mk, unsigned off, double x[9]) {
 #pragma unroll
-      for (int e = 0; e < 5; e++) { q[1][e] = c0[e]; q[2][e] = cq[e]; q[3][e] = c2[e]; }
-      const long nl = at(kb - 1), nr = at(kb);
+    for (int e = 0; e < 9; e++) x[e] = NS ? ldp(A.tq + (e * A.ldv + b.npc + mk), off) : 0.;
+  };
+  auto load_sn = [&](int d, long mk, unsigned off, double x[3]) {
 #pragma unroll
-      for (int x = 0; x < 9; x++) {
-        tl[x] = NS ? A.tq[x * A.ldv + nl] : 0.;
-        tr[x] = NS ? A.tq[x * A.ldv + nr] : 0.;
-      }
-      const bool lim = LIM && kb <= b.k2 - 2;
+    for (int c = 0; c < 3; c++) x[c] = ldp(A.sn + ((3 * c + d) * b.nnn + mk), off);
+  };
+  // the limiter's ratios of the face and of the next one in direction d
+  auto load_rr = [&](int d, long mk, long inc, unsigned off, bool lim, double rl[5], double rh[5]) {
+#pragma unroll
+    for (int e = 0; e < 5; e++) rl[e] = rh[e] = 0.;
+    if (LIM && lim) {
 #pragma unroll
       for (int e = 0; e < 5; e++) {
-        rl[e] = lim ? A.rr[(10 + e) * b.nnn + m] : 0.;
-        rh[e] = lim ? A.rr[(10 + e) * b.nnn + m + b.nijd] : 0.;
+        rl[e] = ldp(A.rr + ((5 * d + e) * b.nnn + mk), off);
+        rh[e] = ldp(A.rr + ((5 * d + e) * b.nnn + mk + inc), off);
       }
-      muscl_roe_half(A.ph, s0, s1, s2, q, lim, rl, rh, A.cm, A.xk, tl, tr, Hlo);
+    }
+  };
+  // own column registers: cq = q(k), c2 = q(k+1)
+  double cq[5], c2[5];
+  {
+    // the low face of the slab's first plane
+    const long m1 = plane(kb);
+    double x[4][5], s[3], rl[5], rh[5], tl[9], tr[9], c0[5], H[5];
+    const bool lim = LIM && kb <= b.k2 - 2;
+#pragma unroll
+    for (int e = 0; e < 4; e++) fused_load(A, b.npc + plane(kb - 2 + e), po, x[e]);
+    load_sn(2, m1, po, s);
+    load_tq(plane(kb - 1), po, tl);
+    load_tq(m1, po, tr);
+    load_rr(2, m1, b.nijd, po, lim && kb > b.k1, rl, rh);
+    loads_issued();
+    fused_prim(x[1], c0);
+    fused_prim(x[2], cq);
+    fused_prim(x[3], c2);
+    if (cell) {
+      if (kb == b.k1) {
+        fused_ghost<NS>(A, 2, true, b.idx(i, j, kb), b.nijd, s[0], s[1], s[2], H);
+      } else {
+        double q[4][5];
+        fused_prim(x[0], q[0]);
+#pragma unroll
+        for (int e = 0; e < 5; e++) { q[1][e] = c0[e]; q[2][e] = cq[e]; q[3][e] = c2[e]; }
+        muscl_roe_half(A.ph, s[0], s[1], s[2], q, lim, rl, rh, A.cm, A.xk, tl, tr, H);
+      }
+#pragma unroll
+      for (int e = 0; e < 5; e++) HL[e][tid] = H[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 5; e++) C0[e][tid] = c0[e];
+    if (CARRY) {
+#pragma unroll
+      for (int x = 0; x < 9; x++) Q[x][sq] = tr[x];
     }
   }
+  const int wave = tid / 64, lane = tid % 64;
   for (int k = kb; k < ke; k++) {
-    // plane k into LDS: own cell, own stresses, halo element
+    const long mk = plane(k);
+    // plane k into LDS: own cell, own stresses, halo element; every load of it
+    // before the first is used
     {
-      const long nk = at(k);
+      double own[9], halo[NS ? 9 : 5];
+      if (!CARRY) load_tq(mk, po, own);
+      if (hkind == 1) fused_load(A, b.npc + mk, ph, halo);
+      else if (NS && hkind == 2) load_tq(mk, ph, halo);
+      loads_issued();
 #pragma unroll
       for (int e = 0; e < 5; e++) P[e][so] = cq[e];
-      if (NS) {
+      if (NS && !CARRY) {
 #pragma unroll
-        for (int x = 0; x < 9; x++) Q[x][sq] = A.tq[x * A.ldv + nk];
+        for (int x = 0; x < 9; x++) Q[x][sq] = own[x];
       }
-      const long nh = hcol + (long)(cl(k, b.kd1, kd2) - b.kd1) * b.nijd;
       if (hkind == 1) {
         double hv[5];
-        fused_prim(A, nh, hv);
+        fused_prim(halo, hv);
         const int sh = (hjj + 2) * FPP + hii + 2;
 #pragma unroll
         for (int e = 0; e < 5; e++) P[e][sh] = hv[e];
       } else if (NS && hkind == 2) {
         const int sh = (hjj + 1) * FQP + hii + 1;
 #pragma unroll
-        for (int x = 0; x < 9; x++) Q[x][sh] = A.tq[x * A.ldv + nh];
+        for (int x = 0; x < 9; x++) Q[x][sh] = halo[x];
       }
     }
-    __syncthreads();
-    // i and j faces of plane k; the extra (FT+1-th) faces by half of wave
-    // (k - kb) % 4
-    const int wave = tid / 64, lane = tid % 64;
-    const int njob = (wave == (k - kb) % 4 && lane < 2 * FT) ? 3 : 2;
-    for (int job = 0; job < njob; job++) {
-      int d, fx, fy;
-      if (job == 0) { d = 0; fx = tx; fy = ty; }
-      else if (job == 1) { d = 1; fx = tx; fy = ty; }
-      else if (lane < FT) { d = 0; fx = FT; fy = lane; }
-      else { d = 1; fx = lane - FT; fy = FT; }
+    lds_sync();
+    // i and j faces of plane k: the own cell's low face, and the FT+1-th faces
+    // by the first lanes of one wave per direction, another on each plane
+#pragma clang loop unroll(disable)
+    for (int job = 0; job < 4; job++) {
+      const int d = job / 2;  // uniform
+      const bool extra = job % 2;
+      if (extra && wave != (k - kb + 2 * d) % 4) continue;
+      const int fx = extra ? (d == 0 ? FT : lane) : tx, fy = extra ? (d == 0 ? lane : FT) : ty;
       const int fi = i0 + fx, fj = j0 + fy;
-      const bool need = d == 0 ? (fi <= b.i2 && fj < b.j2) : (fi < b.i2 && fj <= b.j2);
+      const bool need = (!extra || lane < FT) && (d == 0 ? fi <= b.i2 && fj < b.j2 : fi < b.i2 && fj <= b.j2);
       if (!need) continue;
       const int a = d == 0 ? fi : fj, a1 = d == 0 ? b.i1 : b.j1, a2 = d == 0 ? b.i2 : b.j2;
       const long inc = d == 0 ? 1 : b.nid;
-      const long n = b.idx(fi, fj, k), m = n - b.npc;
-      double s0 = snv(A.sn, b.nnn, m, d, 0), s1 = snv(A.sn, b.nnn, m, d, 1), s2 = snv(A.sn, b.nnn, m, d, 2);
-      double f[5];
+      const unsigned off = in_plane(fi, fj);
+      double s[3], f[5];
+      load_sn(d, mk, off, s);
       if (a == a1 || a == a2) {
-        fused_ghost<NS>(A, d, a == a1, n, inc, s0, s1, s2, f);
+        fused_ghost<NS>(A, d, a == a1, b.idx(fi, fj, k), inc, s[0], s[1], s[2], f);
       } else {
         double q[4][5], rl[5], rh[5], tl[9], tr[9];
+        const bool lim = LIM && a <= a2 - 2;
+        load_rr(d, mk, inc, off, lim, rl, rh);
         const int dx = d == 0, dy = d == 1;
 #pragma unroll
         for (int s = 0; s < 4; s++) {
@@ -708,13 +763,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs &A, dim3 t) {
           tl[x] = NS ? Q[x][ql] : 0.;
           tr[x] = NS ? Q[x][qr] : 0.;
         }
-        const bool lim = LIM && a <= a2 - 2;
-#pragma unroll
-        for (int e = 0; e < 5; e++) {
-          rl[e] = lim ? A.rr[(5 * d + e) * b.nnn + m] : 0.;
-          rh[e] = lim ? A.rr[(5 * d + e) * b.nnn + m + inc] : 0.;
-        }
-        muscl_roe_half(A.ph, s0, s1, s2, q, lim, rl, rh, A.cm, A.xk, tl, tr, f);
+        muscl_roe_half(A.ph, s[0], s[1], s[2], q, lim, rl, rh, A.cm, A.xk, tl, tr, f);
       }
       if (d == 0) {
 #pragma unroll
@@ -725,47 +774,53 @@ __device__ __forceinline__ void fused_body(const FusedArgs &A, dim3 t) {
       }
     }
     // the k face between planes k and k+1 of the own column
-    double Hhi[5], c3[5];
-    fused_prim(A, at(k + 2), c3);
-    if (cell) {
-      const long n = b.idx(i, j, k + 1), m = n - b.npc;
-      double s0 = snv(A.sn, b.nnn, m, 2, 0), s1 = snv(A.sn, b.nnn, m, 2, 1), s2 = snv(A.sn, b.nnn, m, 2, 2);
-      if (k + 1 == b.k2) {
-        fused_ghost<NS>(A, 2, false, n, b.nijd, s0, s1, s2, Hhi);
-      } else {
-        double q[4][5], rl[5], rh[5], tl[9], tr[9];
+    double Hhi[5], c3[5], tr[9];
+    {
+      const long mn = plane(k + 1);
+      double x[5], s[3], rl[5], rh[5];
+      const bool lim = LIM && k + 1 <= b.k2 - 2;
+      fused_load(A, b.npc + plane(k + 2), po, x);
+      load_sn(2, mn, po, s);
+      load_tq(mn, po, tr);
+      load_rr(2, mn, b.nijd, po, lim, rl, rh);
+      loads_issued();
+      fused_prim(x, c3);
+      if (cell) {
+        if (k + 1 == b.k2) {
+          fused_ghost<NS>(A, 2, false, b.idx(i, j, k + 1), b.nijd, s[0], s[1], s[2], Hhi);
+        } else {
+          double q[4][5], tl[9];
 #pragma unroll
-        for (int e = 0; e < 5; e++) { q[0][e] = c0[e]; q[1][e] = cq[e]; q[2][e] = c2[e]; q[3][e] = c3[e]; }
-        const long nr = at(k + 1);
+          for (int e = 0; e < 5; e++) { q[0][e] = C0[e][tid]; q[1][e] = P[e][so]; q[2][e] = c2[e]; q[3][e] = c3[e]; }
 #pragma unroll
-        for (int x = 0; x < 9; x++) {
-          tl[x] = NS ? Q[x][sq] : 0.;
-          tr[x] = NS ? A.tq[x * A.ldv + nr] : 0.;
+          for (int x = 0; x < 9; x++) tl[x] = NS ? Q[x][sq] : 0.;
+          muscl_roe_half(A.ph, s[0], s[1], s[2], q, lim, rl, rh, A.cm, A.xk, tl, tr, Hhi);
         }
-        const bool lim = LIM && k + 1 <= b.k2 - 2;
-#pragma unroll
-        for (int e = 0; e < 5; e++) {
-          rl[e] = lim ? A.rr[(10 + e) * b.nnn + m] : 0.;
-          rh[e] = lim ? A.rr[(10 + e) * b.nnn + m + b.nijd] : 0.;
-        }
-        muscl_roe_half(A.ph, s0, s1, s2, q, lim, rl, rh, A.cm, A.xk, tl, tr, Hhi);
       }
+#pragma unroll
+      for (int e = 0; e < 5; e++) C0[e][tid] = P[e][so];
     }
-    __syncthreads();
+    lds_sync();
+    if (CARRY) {  // the own stresses of the next plane
+#pragma unroll
+      for (int x = 0; x < 9; x++) Q[x][sq] = tr[x];
+    }
     if (cell) {
-      const long n = b.idx(i, j, k);
 #pragma unroll
       for (int e = 0; e < 5; e++) {
         double r = Fi[e][ty * (FT + 1) + tx + 1] - Fi[e][ty * (FT + 1) + tx];
         r = r + (Fj[e][(ty + 1) * FT + tx] - Fj[e][ty * FT + tx]);
-        r = r + (Hhi[e] - Hlo[e]);
-        A.u[e * A.ldv + n] = r;
-        if (A.ityprk) A.ff[e * A.ldv + n] = A.ff[e * A.ldv + n] - r;
-        Hlo[e] = Hhi[e];
+        r = r + (Hhi[e] - HL[e][tid]);
+        HL[e][tid] = Hhi[e];
+        *gp(A.u + (e * A.ldv + b.npc + mk), po) = r;
+        if (A.ityprk) {
+          const auto ff = gp(A.ff + (e * A.ldv + b.npc + mk), po);
+          *ff = *ff - r;
+        }
       }
     }
 #pragma unroll
-    for (int e = 0; e < 5; e++) { c0[e] = cq[e]; cq[e] = c2[e]; c2[e] = c3[e]; }
+    for (int e = 0; e < 5; e++) { cq[e] = c2[e]; c2[e] = c3[e]; }
   }
 }
 
