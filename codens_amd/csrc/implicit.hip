@@ -713,12 +713,13 @@ __global__ void __launch_bounds__(TXS *TYS) SW_ATTR k_impl_sweep_tiled(Blk b, Ph
 // the last bit of the state into 1e-7 of the next residual).  The term of an
 // i face is formed by the cell above it and passed down a lane.
 //
-// One workgroup per CU (135 KB of LDS, 236 registers, two waves per SIMD).  On
-// 256 x 128 x 64 a pair takes 190 us and moves 660 MB, against 2 x 125 us for
+// One workgroup per CU (135 KB of LDS, 254 registers, two waves per SIMD).  On
+// 256 x 128 x 64 a pair takes 185 us and moves 660 MB, against 2 x 125 us for
 // single sweeps of 674 MB each, at 5.4 TB/s, what a large copy reaches; a pair's
-// waves issue or wait for arithmetic and LDS half of the time.  With workgroup barriers in place of
-// the flags below it took 225 us, with the i and j faces' operands loaded at
-// the top of their plane instead of during the plane below 199 us.
+// waves issue or wait for arithmetic and LDS half of the time.  With workgroup
+// barriers in place of the flags below it took 225 us, with flags that waited
+// for the loads in flight 192, and before that with the i and j faces' operands
+// loaded at the top of their plane instead of during the plane below 199.
 constexpr int S2_TX = 32, S2_TY = 16, S2_NC = S2_TX * S2_TY, S2_OX = S2_TX - 4, S2_OY = S2_TY - 4;
 constexpr int S2_STASH = 5, S2_LDS = (28 + S2_STASH) * S2_NC;
 constexpr int S2_KS = 16;  // k planes per workgroup in the all-blocks launch
@@ -782,15 +783,33 @@ __device__ __forceinline__ void tn2_fma(const double A[14], const double s[3], d
 // component of q that holds d of equation e
 __device__ __forceinline__ constexpr int q_comp(int e) { return e == 0 ? 12 : (e == 4 ? 13 : e - 1); }
 
+// a flag that waves of a workgroup pass to each other (as an LDS access: a
+// volatile access through a generic pointer stays one, and waits for the global
+// loads in flight)
+using LdsFlag = volatile __attribute__((address_space(3))) int;
+
+// gp and ldp without the empty asm, whose scalar operands the pair kernel has no
+// registers for (the opaque offsets suffice there; the fused residual is 2%
+// slower without it)
+template <typename T>
+__device__ __forceinline__ GPtr<T> gp2(T *base, unsigned off) {
+  return (GPtr<T>)((GPtr<char>)(uint64_t)base + off);
+}
+template <typename T>
+__device__ __forceinline__ T ldp2(const T *base, unsigned off) {
+  return *gp2(base, off);
+}
+
 // BATCH: with the bits of the all-blocks launch's single sweeps
 template <bool FF, bool BATCH>
 __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int nty, int ks, const Phys &ph,
                                             const double *__restrict__ u, const double *__restrict__ ff,
                                             const double *__restrict__ v, long ldv, const double *__restrict__ sn,
                                             const double *__restrict__ coefe, const double *__restrict__ diag,
-                                            const DView dold, const DView dnew, double *sx, volatile int *flag) {
+                                            const DView dold, const DView dnew, double *sx, LdsFlag *flag) {
 #pragma clang fp contract(off)
-  const int bx = lg % ntx, by = (lg / ntx) % nty, bz = lg / (ntx * nty);
+  auto scalar = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  const int bx = scalar(lg % ntx), by = scalar((lg / ntx) % nty), bz = scalar(lg / (ntx * nty));
   const int t = threadIdx.x, tx = t % S2_TX, ty = t / S2_TX;
   const int i = b.i1 + bx * S2_OX - 2 + tx, j = b.j1 + by * S2_OY - 2 + ty;
   const int kb = b.k1 + bz * ks, ke = min(kb + ks, b.k2);
@@ -815,8 +834,8 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
   auto load_vd = [&](long m, unsigned off, double V[5], double D[5]) {
 #pragma unroll
     for (int e = 0; e < 5; e++) {
-      V[e] = ldp(v + (e * ldv + b.npc + m), off);
-      D[e] = ldp(dold.p + (e * dold.ld + (b.npc - dold.off) + m), off);
+      V[e] = ldp2(v + (e * ldv + b.npc + m), off);
+      D[e] = ldp2(dold.p + (e * dold.ld + (b.npc - dold.off) + m), off);
     }
   };
   // own slots start as the plane below A's first: q of A there, zero of B
@@ -826,8 +845,8 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
 #pragma unroll
     for (int c = 0; c < 14; c++) q[c] = qn[c] = 0.;
 #pragma unroll
-    for (int c = 0; c < 3; c++) skl[c] = ldp(sn + ((c * 3 + 2) * nnn + mk), pl);
-    ckl = ldp(coefe + (2 * nnn + mk), pl);
+    for (int c = 0; c < 3; c++) skl[c] = ldp2(sn + ((c * 3 + 2) * nnn + mk), pl);
+    ckl = ldp2(coefe + (2 * nnn + mk), pl);
     if (own && ka > b.k1) {
       load_vd(mk - nijd, pl, V, D);
       dflux_q(ph, V, D, q);
@@ -866,19 +885,21 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   };
   struct IJ {
-    double sil[3], sjl[3], sjh[3], cil, cih, cjl, cjh;
+    double sil[3], sjl[3], sjh[3], cil, cih, cjl, cjh, uu[5];
   } o, on;
   auto load_ij = [&](long m, unsigned pl, IJ &o) {
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      o.sil[c] = ldp(sn + (c * 3 * nnn + m), pl);
-      o.sjl[c] = ldp(sn + ((c * 3 + 1) * nnn + m), pl);
-      o.sjh[c] = ldp(sn + ((c * 3 + 1) * nnn + m + b.nid), pl);
+      o.sil[c] = ldp2(sn + (c * 3 * nnn + m), pl);
+      o.sjl[c] = ldp2(sn + ((c * 3 + 1) * nnn + m), pl);
+      o.sjh[c] = ldp2(sn + ((c * 3 + 1) * nnn + m + b.nid), pl);
     }
-    o.cil = ldp(coefe + m, pl);
-    o.cih = ldp(coefe + m, pl + 8u);
-    o.cjl = ldp(coefe + (nnn + m), pl);
-    o.cjh = ldp(coefe + (nnn + m + b.nid), pl);
+    o.cil = ldp2(coefe + m, pl);
+    o.cih = ldp2(coefe + m, pl + 8u);
+    o.cjl = ldp2(coefe + (nnn + m), pl);
+    o.cjh = ldp2(coefe + (nnn + m + b.nid), pl);
+#pragma unroll
+    for (int e = 0; e < 5; e++) o.uu[e] = ldp2(u + (e * ldv + b.npc + m), pl);
   };
   load_ij(mk, opaque(pl0), o);
   for (int k = ka; k <= kz; k++, mk += nijd) {
@@ -886,16 +907,14 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
     const unsigned pl = opaque(pl0);
     // the loads of the plane but its i and j faces', which came with the plane
     // below
-    double skh[3], uu[5], fv[5] = {0., 0., 0., 0., 0.}, Vn[5], Dn[5];
+    double skh[3], fv[5] = {0., 0., 0., 0., 0.}, Vn[5], Dn[5];
 #pragma unroll
-    for (int c = 0; c < 3; c++) skh[c] = ldp(sn + ((c * 3 + 2) * nnn + mk + nijd), pl);
-    const double ckh = kreal ? ldp(coefe + (2 * nnn + mk + nijd), pl) : 0.;
-    const double dg = ldp(diag + mk, pl);
-#pragma unroll
-    for (int e = 0; e < 5; e++) uu[e] = ldp(u + (e * ldv + b.npc + mk), pl);
+    for (int c = 0; c < 3; c++) skh[c] = ldp2(sn + ((c * 3 + 2) * nnn + mk + nijd), pl);
+    const double ckh = kreal ? ldp2(coefe + (2 * nnn + mk + nijd), pl) : 0.;
+    const double dg = ldp2(diag + mk, pl);
     if constexpr (FF) {
 #pragma unroll
-      for (int e = 0; e < 5; e++) fv[e] = ldp(ff + (e * ldv + b.npc + mk), pl);
+      for (int e = 0; e < 5; e++) fv[e] = ldp2(ff + (e * ldv + b.npc + mk), pl);
     }
     if (own && kreal) load_vd(mk + nijd, pl, Vn, Dn);
     double q[14], w[5], tn[5], dlo[5], dhi[5];
@@ -906,7 +925,7 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
 #pragma unroll
       for (int e = 0; e < 5; e++) {
         const double th = lane_above(tn[e]);
-        w[e] = fma(o.cil, Q[q_comp(e) * S2_NC + tl], fma(0.5, tn[e], -uu[e] - fv[e]));
+        w[e] = fma(o.cil, Q[q_comp(e) * S2_NC + tl], fma(0.5, tn[e], -o.uu[e] - fv[e]));
         if (ireal) w[e] = fma(o.cih, Q[q_comp(e) * S2_NC + tr], w[e]);
         w[e] = fma(-0.5, th, w[e]);
       }
@@ -968,7 +987,7 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
     if (BATCH && first(k)) tn2_fma<K1>(q, skl, tk, belowB);
     if (out && k > kb) {
 #pragma unroll
-      for (int e = 0; e < 5; e++) *gp(dnew.p + (e * dnew.ld + (b.npc - dnew.off) + mk - nijd), pl) = dhi[e];
+      for (int e = 0; e < 5; e++) *gp2(dnew.p + (e * dnew.ld + (b.npc - dnew.off) + mk - nijd), pl) = dhi[e];
     }
 #pragma unroll
     for (int c = 0; c < 14; c++) qB[c * S2_NC + t] = q[c];
@@ -990,7 +1009,7 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
     tn2_fma<KF>(q, skl, tk, [&](int) { return 0.; });
 #pragma unroll
     for (int e = 0; e < 5; e++)
-      *gp(dnew.p + (e * dnew.ld + (b.npc - dnew.off) + mk - nijd), opaque(pl0)) =
+      *gp2(dnew.p + (e * dnew.ld + (b.npc - dnew.off) + mk - nijd), opaque(pl0)) =
           fma(-0.5, tk[e], base[e]) * rdb;
   }
 }
@@ -1006,7 +1025,7 @@ k_impl_sweep2(Blk b, Phys ph, int ntx, int nty, int ks, const double *__restrict
   __syncthreads();
   unsigned lg = xcd_linear();
   if (rev) lg = gridDim.x - 1 - lg;
-  sweep2_body<FF, false>(b, (int)lg, ntx, nty, ks, ph, u, ff, v, ldv, sn, coefe, diag, dold, dnew, sx, flag);
+  sweep2_body<FF, false>(b, (int)lg, ntx, nty, ks, ph, u, ff, v, ldv, sn, coefe, diag, dold, dnew, sx, (LdsFlag *)flag);
 }
 
 // ---------------------------------------------------------------------------
@@ -1186,13 +1205,13 @@ Pair pair_of(const Blk &b) {
 
 // Whether a block's sub-iterations run in pairs: the modelled time (us) of a
 // pair against that of two single sweeps.  Measured on MI355X: a step of the
-// pair kernel takes 5.5 us, a step of a single sweep 3.4 us while few of the
+// pair kernel takes 5.3 us, a step of a single sweep 3.4 us while few of the
 // chip's 512 workgroup places are taken and 6.8 us when all are.  Two singles
-// / a pair: 256 x 128 x 64 250 / 190 us, 200 x 120 x 100 370 / 207, 128 x 128
-// x 32 60 / 60, 75 x 61 x 43 45 / 39, 32 x 16 x 8 14 / 19.  In FP32 the sweeps
+// / a pair: 256 x 128 x 64 250 / 185 us, 200 x 120 x 100 370 / 206, 128 x 128
+// x 32 60 / 58, 75 x 61 x 43 45 / 36, 32 x 16 x 8 14 / 19.  In FP32 the sweeps
 // are bound by their arithmetic, of which a pair has half as much again (its
 // tile's rings): singles.
-constexpr double PAIR_STEP = 5.5, ONE_STEP = 6.8;
+constexpr double PAIR_STEP = 5.3, ONE_STEP = 6.8;
 bool pair_model(const Blk &b) {
   const int tile = tile_model(b), tx = tile_tx(tile), ty = tile_ty(tile), nz = b.k2 - b.k1;
   const long txy = (long)((b.i2 - b.i1 + tx - 1) / tx) * ((b.j2 - b.j1 + ty - 1) / ty);
@@ -1527,7 +1546,7 @@ k_impl_sweep2_batch(const ImplEnt *__restrict__ tab, int nb, Phys ph, const doub
   double *c = ws + 9 * b.npc;
   DView A = {d, ldv, 0}, B = {c + 4 * b.nnn, b.nnn, b.npc};
   sweep2_body<FF, true>(b, (int)(wg - E.start[IB_SWEEP2]), (int)E.gx[IB_SWEEP2], (int)E.gy[IB_SWEEP2], E.ks_sweep2, ph, u, ff,
-                  v, ldv, sn_all + 9 * b.npc, c, c + 3 * b.nnn, out_d ? B : A, out_d ? A : B, sx, flag);
+                  v, ldv, sn_all + 9 * b.npc, c, c + 3 * b.nnn, out_d ? B : A, out_d ? A : B, sx, (LdsFlag *)flag);
 }
 
 // the update in the first workgroups, d = 0 on the ghosts in those from cells on
