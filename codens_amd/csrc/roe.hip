@@ -281,12 +281,6 @@ __device__ __forceinline__ void chain_jk_body(const Blk &b, dim3 bi, const doubl
   }
 }
 
-__global__ void __launch_bounds__(64) k_limiter_chain_jk(Blk b, const double *__restrict__ v,
-                                                         const double *__restrict__ uvw,
-                                                         const double *__restrict__ ps, double *__restrict__ R) {
-  chain_jk_body(b, dim3(blockIdx.x, blockIdx.y, blockIdx.z), v, uvw, ps, R);
-}
-
 // Direction i: a lane's line is contiguous in memory, so lanes walking their
 // own lines would touch 64 cache lines per access.  The wave instead moves
 // chunks of CH_C cells of its 64 lines through LDS: coalesced loads (each
@@ -370,10 +364,21 @@ __device__ __forceinline__ void chain_i_body(const Blk &b, dim3 bi, const double
   }
 }
 
-__global__ void __launch_bounds__(64) k_limiter_chain_i(Blk b, const double *__restrict__ v,
-                                                        const double *__restrict__ uvw,
-                                                        const double *__restrict__ ps, double *__restrict__ R) {
-  chain_i_body(b, dim3(blockIdx.x, blockIdx.y, 1), v, uvw, ps, R);
+// All three directions in one launch, the i lines (gi groups of 64 per variable)
+// first: those are bound by the latency of their 64-line chains, the j and k
+// lines (gjk groups per variable and direction) by memory, so each hides under
+// the other (256 x 128 x 64: 49 and 66 us one after the other, 100 together; 191
+// x 101 x 47: 32 and 32, 50).
+__global__ void __launch_bounds__(64) k_limiter_chains(Blk b, unsigned gi, unsigned gjk, const double *__restrict__ v,
+                                                       const double *__restrict__ uvw,
+                                                       const double *__restrict__ ps, double *__restrict__ R) {
+  const unsigned w = blockIdx.x;
+  if (w < 5 * gi) {
+    chain_i_body(b, dim3(w % gi, w / gi, 1), v, uvw, ps, R);
+  } else {
+    const unsigned x = w - 5 * gi, y = x / gjk;
+    chain_jk_body(b, dim3(x % gjk, y % 5, y / 5), v, uvw, ps, R);
+  }
 }
 
 // physical flux . S of a ghost state (sch_roe.f90:497-578)
@@ -898,10 +903,8 @@ static int roe_common(const codens_block *cb, const codens_phys *cp, const coden
     CodensTimed _tm("roe_limiter_chain", st);
     long nl0 = (long)(b.j2 - b.j1) * (b.k2 - b.k1);
     long nl12 = (long)(b.i2 - b.i1) * max(b.k2 - b.k1, b.j2 - b.j1);
-    hipLaunchKernelGGL(k_limiter_chain_i, dim3((unsigned)((nl0 + CH_LINES - 1) / CH_LINES), 5), dim3(64), 0, st, b,
-                       v, uvw, ps, R);
-    hipLaunchKernelGGL(k_limiter_chain_jk, dim3((unsigned)((nl12 + CH_LINES - 1) / CH_LINES), 5, 2), dim3(64), 0, st,
-                       b, v, uvw, ps, R);
+    const unsigned gi = (unsigned)((nl0 + CH_LINES - 1) / CH_LINES), gjk = (unsigned)((nl12 + CH_LINES - 1) / CH_LINES);
+    hipLaunchKernelGGL(k_limiter_chains, dim3(5 * gi + 10 * gjk), dim3(64), 0, st, b, gi, gjk, v, uvw, ps, R);
   }
   long n0 = b.idx(b.i1 - 1, b.j1 - 1, b.k1 - 1), n1 = b.idx(b.i2, b.j2, b.k2);
   if (fused) {
@@ -972,18 +975,18 @@ __global__ void __launch_bounds__(256) k_prim_uvw_batch(const BatchEnt *__restri
   prim_uvw_body(E.b, blockIdx.x - E.start[BP_PRIM], v, ldv, uvw + 3 * E.b.npc);
 }
 
-__global__ void __launch_bounds__(64) k_chain_i_batch(const BatchEnt *__restrict__ tab, int nb,
-                                                      const double *__restrict__ v, const double *__restrict__ uvw,
-                                                      const double *__restrict__ ps, double *R) {
-  const BatchEnt &E = tab[tab_find(tab, nb, BP_CHAIN_I, blockIdx.x)];
-  chain_i_body(E.b, tab_tile(E, BP_CHAIN_I, blockIdx.x), v, uvw + 3 * E.b.npc, ps, R + 15 * E.b.npc);
-}
-
-__global__ void __launch_bounds__(64) k_chain_jk_batch(const BatchEnt *__restrict__ tab, int nb,
-                                                       const double *__restrict__ v, const double *__restrict__ uvw,
-                                                       const double *__restrict__ ps, double *R) {
-  const BatchEnt &E = tab[tab_find(tab, nb, BP_CHAIN_JK, blockIdx.x)];
-  chain_jk_body(E.b, tab_tile(E, BP_CHAIN_JK, blockIdx.x), v, uvw + 3 * E.b.npc, ps, R + 15 * E.b.npc);
+__global__ void __launch_bounds__(64) k_chains_batch(const BatchEnt *__restrict__ tab, int nb, unsigned ni,
+                                                     const double *__restrict__ v, const double *__restrict__ uvw,
+                                                     const double *__restrict__ ps, double *R) {
+  unsigned w = blockIdx.x;
+  if (w < ni) {
+    const BatchEnt &E = tab[tab_find(tab, nb, BP_CHAIN_I, w)];
+    chain_i_body(E.b, tab_tile(E, BP_CHAIN_I, w), v, uvw + 3 * E.b.npc, ps, R + 15 * E.b.npc);
+  } else {
+    w -= ni;
+    const BatchEnt &E = tab[tab_find(tab, nb, BP_CHAIN_JK, w)];
+    chain_jk_body(E.b, tab_tile(E, BP_CHAIN_JK, w), v, uvw + 3 * E.b.npc, ps, R + 15 * E.b.npc);
+  }
 }
 
 __global__ void __launch_bounds__(TX *TY) __attribute__((amdgpu_waves_per_eu(CODENS_FF_WAVES)))
@@ -1148,10 +1151,8 @@ extern "C" int codens_sch_roe_batch(int32_t nblk, const codens_block *blocks, co
   }
   if (ilim == 1) {
     CodensTimed _tm("roe_limiter_chain", st);
-    hipLaunchKernelGGL(k_chain_i_batch, dim3(tot[BP_CHAIN_I]), dim3(64), 0, st, (const BatchEnt *)tab, (int)nblk, v,
-                       (const double *)uvw, ps, R);
-    hipLaunchKernelGGL(k_chain_jk_batch, dim3(tot[BP_CHAIN_JK]), dim3(64), 0, st, (const BatchEnt *)tab, (int)nblk,
-                       v, (const double *)uvw, ps, R);
+    hipLaunchKernelGGL(k_chains_batch, dim3(tot[BP_CHAIN_I] + tot[BP_CHAIN_JK]), dim3(64), 0, st,
+                       (const BatchEnt *)tab, (int)nblk, tot[BP_CHAIN_I], v, (const double *)uvw, ps, R);
   }
   if (fused) {
     const double cm = 0.25 * sc->muscl;
