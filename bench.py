@@ -190,21 +190,18 @@ def main():
     sweep_name = "implimf32_sweep" if fp32 else "implimf_sweep"
     sweep_bytes = SWEEP_BYTES_PER_CELL // 2 if fp32 else SWEEP_BYTES_PER_CELL  # the same 33 values in FP32
     n_timing = max(3, args.steps // 4)
-    # the launches of two sub-iterations at once, where there are any: each
-    # moves what one sub-iteration's does, so that passes over the cells, not
-    # sub-iterations, make the bytes
-    sw2 = kern.get("implimf_sweep2")
+    # two sub-iterations at once (all but the first launch), where there are
+    # any: each launch moves what one sub-iteration's does
+    if "implimf_sweep2" in kern:
+        sweep_name = "implimf_sweep2"
     sw = kern.get(sweep_name, {"avg_us": float("nan"), "launches": nblk * (case.lmax - 1) * n_timing})
     # bytes of all sweep launches over their summed time: the timing stages
     # sweep every cell lmax-1 times, in one launch per block and
     # sub-iteration, or one per sub-iteration when the blocks are batched
-    if sw2:
-        singles = kern[sweep_name]["launches"] if sweep_name in kern else 0
-        passes = sw2["launches"] / (singles + 2 * sw2["launches"]) * (case.lmax - 1) * n_timing
-        sweep_name, sw = "implimf_sweep2", sw2
+    if sweep_name == "implimf_sweep2":
+        cells_per_launch = ncell / (1 if "implicit" in s.batch else nblk)
     else:
-        passes = (case.lmax - 1) * n_timing
-    cells_per_launch = ncell * passes / sw["launches"]
+        cells_per_launch = ncell * (case.lmax - 1) * n_timing / sw["launches"]
     achieved = sweep_bytes * cells_per_launch / (sw["avg_us"] * 1e-6) / 1e9
     out = {
         "metric": "Mcell-updates/s per implicit iter to 1e-8 residual drop; % of HBM roofline",

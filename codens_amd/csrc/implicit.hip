@@ -720,7 +720,10 @@ __global__ void __launch_bounds__(TXS *TYS) SW_ATTR k_impl_sweep_tiled(Blk b, Ph
 // barriers in place of the flags below it took 225 us, with flags that waited
 // for the loads in flight 192, and before that with the i and j faces' operands
 // loaded at the top of their plane instead of during the plane below 199.
-constexpr int S2_TX = 32, S2_TY = 16, S2_NC = S2_TX * S2_TY, S2_OX = S2_TX - 4, S2_OY = S2_TY - 4;
+constexpr int S2_TX = 32, S2_TY = 16, S2_NC = S2_TX * S2_TY;
+// cells that a tile writes; FIRST, where A needs no neighbour, one ring more
+constexpr int s2_ox(bool first) { return S2_TX - (first ? 2 : 4); }
+constexpr int s2_oy(bool first) { return S2_TY - (first ? 2 : 4); }
 constexpr int S2_STASH = 5, S2_LDS = (28 + S2_STASH) * S2_NC;
 constexpr int S2_KS = 16;  // k planes per workgroup in the all-blocks launch
 
@@ -800,8 +803,9 @@ __device__ __forceinline__ T ldp2(const T *base, unsigned off) {
   return *gp2(base, off);
 }
 
-// BATCH: with the bits of the all-blocks launch's single sweeps
-template <bool FF, bool BATCH>
+// BATCH: with the bits of the all-blocks launch's single sweeps.  FIRST: A is
+// sub-iteration 1, which starts from d = 0 and is (-u - ff)/diag.
+template <bool FF, bool BATCH, bool FIRST>
 __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int nty, int ks, const Phys &ph,
                                             const double *__restrict__ u, const double *__restrict__ ff,
                                             const double *__restrict__ v, long ldv, const double *__restrict__ sn,
@@ -811,11 +815,12 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
   auto scalar = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
   const int bx = scalar(lg % ntx), by = scalar((lg / ntx) % nty), bz = scalar(lg / (ntx * nty));
   const int t = threadIdx.x, tx = t % S2_TX, ty = t / S2_TX;
-  const int i = b.i1 + bx * S2_OX - 2 + tx, j = b.j1 + by * S2_OY - 2 + ty;
+  constexpr int RING = FIRST ? 1 : 2;
+  const int i = b.i1 + bx * s2_ox(FIRST) - RING + tx, j = b.j1 + by * s2_oy(FIRST) - RING + ty;
   const int kb = b.k1 + bz * ks, ke = min(kb + ks, b.k2);
   const int ka = max(kb - 1, b.k1), kz = min(ke, b.k2 - 1);  // planes of A
   const bool own = i >= b.i1 && i < b.i2 && j >= b.j1 && j < b.j2;
-  const bool out = own && tx >= 2 && tx < S2_TX - 2 && ty >= 2 && ty < S2_TY - 2;
+  const bool out = own && tx >= RING && tx < S2_TX - RING && ty >= RING && ty < S2_TY - RING;
   const bool ireal = i + 1 < b.i2, jreal = j + 1 < b.j2;
   // offset in a plane of this thread's cell, or of the nearest cell whose low
   // faces exist (the first ghost past the real cells closes their last face)
@@ -825,6 +830,9 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
   // the result is not used)
   const int tl = max(t - 1, 0), tr = min(t + 1, S2_NC - 1), td = max(t - S2_TX, tx), tu = min(t + S2_TX, S2_NC - S2_TX + tx);
   double *const qA = sx, *const qB = sx + 14 * S2_NC, *const stash = sx + 28 * S2_NC + t;
+  // B's q of the plane below (own slot) and of the plane.  A pair meets twice a
+  // plane, so one buffer serves; FIRST meets once and takes qA's as a second
+  double *qP = qB, *qC = FIRST ? qA : qB;
   auto st = [&](int x) -> double & { return stash[x * S2_NC]; };  // V of the plane
   const long nnn = b.nnn, nijd = b.nijd;
   constexpr int KF = BATCH ? K_FACE : 0, K1 = BATCH ? K_FIRST : 0;
@@ -835,7 +843,7 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
 #pragma unroll
     for (int e = 0; e < 5; e++) {
       V[e] = ldp2(v + (e * ldv + b.npc + m), off);
-      D[e] = ldp2(dold.p + (e * dold.ld + (b.npc - dold.off) + m), off);
+      if (!FIRST) D[e] = ldp2(dold.p + (e * dold.ld + (b.npc - dold.off) + m), off);
     }
   };
   // own slots start as the plane below A's first: q of A there, zero of B
@@ -847,13 +855,13 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
 #pragma unroll
     for (int c = 0; c < 3; c++) skl[c] = ldp2(sn + ((c * 3 + 2) * nnn + mk), pl);
     ckl = ldp2(coefe + (2 * nnn + mk), pl);
-    if (own && ka > b.k1) {
+    if (!FIRST && own && ka > b.k1) {
       load_vd(mk - nijd, pl, V, D);
       dflux_q(ph, V, D, q);
     }
     if (own) {
       load_vd(mk, pl, V, D);
-      dflux_q(ph, V, D, qn);
+      if (!FIRST) dflux_q(ph, V, D, qn);
 #pragma unroll
       for (int e = 0; e < 5; e++) st(e) = V[e];
     }
@@ -862,7 +870,7 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
     else tn2_fma<K1>(qn, skl, tkA, below);
 #pragma unroll
     for (int c = 0; c < 14; c++) {
-      qA[c * S2_NC + t] = q[c];
+      if (!FIRST) qA[c * S2_NC + t] = q[c];
       qB[c * S2_NC + t] = 0.;
     }
 #pragma unroll
@@ -873,7 +881,9 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
   // waves of a SIMD then drift apart and one computes while the other waits
   // for its loads.  Every wave runs the same number of phases and raises its
   // flag in each before it waits, so every wait ends.  A row is overwritten
-  // only after its readers have raised the flag of the following phase.
+  // only after its readers have raised the flag of the following phase: a
+  // buffer is written again two phases later (two meetings a plane, or one and
+  // two buffers in turn).
   const int wv = __builtin_amdgcn_readfirstlane(t / 64);
   int phase = 0;
   auto meet = [&]() {
@@ -939,30 +949,35 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
 #pragma unroll
       for (int e = 0; e < 5; e++) w[e] = fma(ckl, dlo[e], fma(0.5, tk[e], fma(-0.5, tn[e], w[e])));
     };
-    // A on plane k
-#pragma unroll
-    for (int e = 0; e < 5; e++) dlo[e] = qA[q_comp(e) * S2_NC + t];  // of the plane below
-#pragma unroll
-    for (int c = 0; c < 14; c++) {
-      q[c] = qn[c];
-      qA[c * S2_NC + t] = q[c];
-      qn[c] = 0.;
-    }
-    meet();
-    faces(qA, tkA);
-    // the plane above, the face between and what its increment adds
-    if (own && kreal) dflux_q(ph, Vn, Dn, qn);
-    auto here = [&](int c) { return q[c]; };
-    tn2_fma<KF>(qn, skh, tkA, here);
-#pragma unroll
-    for (int e = 0; e < 5; e++) {
-      if (kreal) w[e] = fma(ckh, qn[q_comp(e)], w[e]);
-      w[e] = fma(-0.5, tkA[e], w[e]);
-    }
-    if (BATCH && first(k + 1)) tn2_fma<K1>(qn, skh, tkA, here);
     const double rd = 1. / dg;
+    if constexpr (FIRST) {
 #pragma unroll
-    for (int e = 0; e < 5; e++) dhi[e] = w[e] * rd;  // A's increment
+      for (int e = 0; e < 5; e++) dhi[e] = (-o.uu[e] - fv[e]) / dg;
+    } else {
+      // A on plane k
+#pragma unroll
+      for (int e = 0; e < 5; e++) dlo[e] = qA[q_comp(e) * S2_NC + t];  // of the plane below
+#pragma unroll
+      for (int c = 0; c < 14; c++) {
+        q[c] = qn[c];
+        qA[c * S2_NC + t] = q[c];
+        qn[c] = 0.;
+      }
+      meet();
+      faces(qA, tkA);
+      // the plane above, the face between and what its increment adds
+      if (own && kreal) dflux_q(ph, Vn, Dn, qn);
+      auto here = [&](int c) { return q[c]; };
+      tn2_fma<KF>(qn, skh, tkA, here);
+#pragma unroll
+      for (int e = 0; e < 5; e++) {
+        if (kreal) w[e] = fma(ckh, qn[q_comp(e)], w[e]);
+        w[e] = fma(-0.5, tkA[e], w[e]);
+      }
+      if (BATCH && first(k + 1)) tn2_fma<K1>(qn, skh, tkA, here);
+#pragma unroll
+      for (int e = 0; e < 5; e++) dhi[e] = w[e] * rd;  // A's increment
+    }
 #pragma unroll
     for (int c = 0; c < 14; c++) q[c] = 0.;
     if (own) {
@@ -977,11 +992,11 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
     }
     // B: plane k - 1 is complete with the face to plane k
     double tk[5];
-    auto belowB = [&](int c) { return qB[c * S2_NC + t]; };
+    auto belowB = [&](int c) { return qP[c * S2_NC + t]; };
     tn2_fma<KF>(q, skl, tk, belowB);
 #pragma unroll
     for (int e = 0; e < 5; e++) {
-      dlo[e] = qB[q_comp(e) * S2_NC + t];
+      dlo[e] = qP[q_comp(e) * S2_NC + t];
       dhi[e] = fma(-0.5, tk[e], fma(ckl, dhi[e], base[e])) * rdb;
     }
     if (BATCH && first(k)) tn2_fma<K1>(q, skl, tk, belowB);
@@ -990,10 +1005,15 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
       for (int e = 0; e < 5; e++) *gp2(dnew.p + (e * dnew.ld + (b.npc - dnew.off) + mk - nijd), pl) = dhi[e];
     }
 #pragma unroll
-    for (int c = 0; c < 14; c++) qB[c * S2_NC + t] = q[c];
+    for (int c = 0; c < 14; c++) qC[c * S2_NC + t] = q[c];
     load_ij(mk + nijd, pl, on);  // of the plane above (a ghost's past the last: not used)
     meet();
-    faces(qB, tk);
+    faces(qC, tk);
+    if (FIRST) {
+      double *const x = qP;
+      qP = qC;
+      qC = x;
+    }
     o = on;
 #pragma unroll
     for (int e = 0; e < 5; e++) base[e] = w[e];
@@ -1005,7 +1025,7 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
   if (out && ke == b.k2) {  // the block's last plane: its upper face is a ghost's
     double q[14], tk[5];
 #pragma unroll
-    for (int c = 0; c < 14; c++) q[c] = qB[c * S2_NC + t];
+    for (int c = 0; c < 14; c++) q[c] = qP[c * S2_NC + t];
     tn2_fma<KF>(q, skl, tk, [&](int) { return 0.; });
 #pragma unroll
     for (int e = 0; e < 5; e++)
@@ -1014,7 +1034,7 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
   }
 }
 
-template <bool FF>
+template <bool FF, bool FIRST>
 __global__ void __launch_bounds__(S2_NC) __attribute__((amdgpu_waves_per_eu(2)))
 k_impl_sweep2(Blk b, Phys ph, int ntx, int nty, int ks, const double *__restrict__ u, const double *__restrict__ ff,
               const double *__restrict__ v, long ldv, const double *__restrict__ sn, const double *__restrict__ coefe,
@@ -1025,7 +1045,7 @@ k_impl_sweep2(Blk b, Phys ph, int ntx, int nty, int ks, const double *__restrict
   __syncthreads();
   unsigned lg = xcd_linear();
   if (rev) lg = gridDim.x - 1 - lg;
-  sweep2_body<FF, false>(b, (int)lg, ntx, nty, ks, ph, u, ff, v, ldv, sn, coefe, diag, dold, dnew, sx, (LdsFlag *)flag);
+  sweep2_body<FF, false, FIRST>(b, (int)lg, ntx, nty, ks, ph, u, ff, v, ldv, sn, coefe, diag, dold, dnew, sx, (LdsFlag *)flag);
 }
 
 // ---------------------------------------------------------------------------
@@ -1192,9 +1212,9 @@ struct Pair {
   int ntx, nty, ks;
   long wgs, steps;  // workgroups; steps of one after another on a compute unit
 };
-Pair pair_of(const Blk &b) {
-  const int nz = b.k2 - b.k1, ncu = codens_resident_workgroups(1);
-  Pair p{(b.i2 - b.i1 + S2_OX - 1) / S2_OX, (b.j2 - b.j1 + S2_OY - 1) / S2_OY, 1, 0, 0};
+Pair pair_of(const Blk &b, bool first = false) {
+  const int nz = b.k2 - b.k1, ncu = codens_resident_workgroups(1), ox = s2_ox(first), oy = s2_oy(first);
+  Pair p{(b.i2 - b.i1 + ox - 1) / ox, (b.j2 - b.j1 + oy - 1) / oy, 1, 0, 0};
   for (int ks = 1; ks <= nz; ks++) {
     const long w = (long)p.ntx * p.nty * ((nz + ks - 1) / ks);
     const long c = (w + ncu - 1) / ncu * (std::min(ks + 2, nz) + 1);
@@ -1221,13 +1241,15 @@ bool pair_model(const Blk &b) {
   return PAIR_STEP * pair_of(b).steps < 2. * one;
 }
 
-// two sub-iterations in -> out
-void launch_sweep2(const Blk &b, hipStream_t st, Phys ph, int ityprk, const double *u, const double *ff,
+// two sub-iterations in -> out; first: sub-iterations 1 and 2, in not read
+void launch_sweep2(bool first, const Blk &b, hipStream_t st, Phys ph, int ityprk, const double *u, const double *ff,
                    const double *v, long ldv, const double *sn, const double *coefe, const double *diag, DView in,
                    DView out, int rev) {
-  const Pair p = pair_of(b);
-  hipLaunchKernelGGL(ityprk ? k_impl_sweep2<true> : k_impl_sweep2<false>, dim3((unsigned)p.wgs), dim3(S2_NC), 0, st, b,
-                     ph, p.ntx, p.nty, p.ks, u, ff, v, ldv, sn, coefe, diag, in, out, rev);
+  const Pair p = pair_of(b, first);
+  auto *k = first ? (ityprk ? k_impl_sweep2<true, true> : k_impl_sweep2<false, true>)
+                  : (ityprk ? k_impl_sweep2<true, false> : k_impl_sweep2<false, false>);
+  hipLaunchKernelGGL(k, dim3((unsigned)p.wgs), dim3(S2_NC), 0, st, b, ph, p.ntx, p.nty, p.ks, u, ff, v, ldv, sn, coefe,
+                     diag, in, out, rev);
 }
 
 template <bool EU, typename T>
@@ -1272,13 +1294,18 @@ int pick_tile(const Blk &b, hipStream_t st, Phys ph, int ityprk, const T *u, con
 }
 }  // namespace
 
-// Launches of lmx sub-iterations: the first (from d = 0), singles, pairs
+// Launches of lmx sub-iterations: the first (from d = 0), singles, pairs.  In
+// pairs an even number of them begins with a pair too (the FIRST form: on 256 x
+// 128 x 64 139 us, on 200 x 120 x 100 136, against 33 and 42 for k_impl_sweep1 and
+// 131 and 194 for a single sweep).
 struct SweepPlan {
+  bool first2;
   int single, pairs, n;
 };
 static SweepPlan sweep_plan(int lmx, bool pairs) {
-  const int rest = lmx > 1 ? lmx - 1 : 0, np = pairs ? rest / 2 : 0;
-  return {rest - 2 * np, np, lmx > 0 ? 1 + rest - np : 0};
+  const bool first2 = pairs && lmx > 1 && lmx % 2 == 0;
+  const int rest = std::max(0, lmx - (first2 ? 2 : 1)), np = pairs ? rest / 2 : 0;
+  return {first2, rest - 2 * np, np, lmx > 0 ? 1 + rest - np : 0};
 }
 
 static int forced_tile() {
@@ -1409,7 +1436,10 @@ static int implimf_common(bool eu, const codens_block *cb, const codens_phys *cp
     DView out = ((plan.n - 1 - s) % 2 == 0) ? A : B;
     DView in = ((plan.n - 1 - s) % 2 == 0) ? B : A;
     if (s == 0 && small && plan.single > 0) continue;  // formed by the second
-    if (s == 0) {
+    if (s == 0 && plan.first2) {
+      CodensTimed _tm(tname("implimf_sweep1"), st);
+      launch_sweep2(true, b, st, ph, (int)ityprk, u, fx, v, (long)ldv, sn, coefe, diag, in, out, 0);
+    } else if (s == 0) {
       CodensTimed _tm(tname("implimf_sweep1"), st);
       hipLaunchKernelGGL(k_impl_sweep1<double>, g, t, 0, st, b, (int)ityprk, u, fx, (long)ldv, diag, out);
     } else if (s <= plan.single && small) {
@@ -1432,7 +1462,7 @@ static int implimf_common(bool eu, const codens_block *cb, const codens_phys *cp
                                     s % 2);
     } else {
       CodensTimed _tm(tname("implimf_sweep2"), st);
-      launch_sweep2(b, st, ph, (int)ityprk, u, fx, v, (long)ldv, sn, coefe, diag, in, out, s % 2);
+      launch_sweep2(false, b, st, ph, (int)ityprk, u, fx, v, (long)ldv, sn, coefe, diag, in, out, s % 2);
     }
   }
   {
@@ -1459,7 +1489,7 @@ int codens_implimf_3d_with(const codens_block *b, const codens_phys *ph, const d
 // diagonal and ping-pong increment (9 planes of nnn) start at 9 npc of the
 // workspace.  The sub-iterations of small blocks then share the chip instead
 // of each filling a few CUs.
-enum { IB_ZERO, IB_CELL, IB_SWEEP, IB_COEF, IB_SWEEP2, IB_SHELL, IB_N };
+enum { IB_ZERO, IB_CELL, IB_SWEEP, IB_COEF, IB_SWEEP2, IB_FIRST2, IB_SHELL, IB_N };
 
 struct ImplEnt {
   Blk b;
@@ -1531,7 +1561,7 @@ __global__ void __launch_bounds__(SW_TX *SW_TY) k_impl_sweep_batch(const ImplEnt
 }
 
 // two sub-iterations of every block
-template <bool FF>
+template <bool FF, bool FIRST>
 __global__ void __launch_bounds__(S2_NC) __attribute__((amdgpu_waves_per_eu(2)))
 k_impl_sweep2_batch(const ImplEnt *__restrict__ tab, int nb, Phys ph, const double *__restrict__ u,
                     const double *__restrict__ ff, const double *__restrict__ v, long ldv,
@@ -1541,11 +1571,12 @@ k_impl_sweep2_batch(const ImplEnt *__restrict__ tab, int nb, Phys ph, const doub
   if (threadIdx.x < S2_NC / 64) flag[threadIdx.x] = 0;
   __syncthreads();
   const unsigned wg = rev ? gridDim.x - 1 - xcd_linear() : xcd_linear();
-  const ImplEnt &E = tab[tab_find(tab, nb, IB_SWEEP2, wg)];
+  constexpr int PASS = FIRST ? IB_FIRST2 : IB_SWEEP2;
+  const ImplEnt &E = tab[tab_find(tab, nb, PASS, wg)];
   const Blk b = uniform_blk(E.b);
   double *c = ws + 9 * b.npc;
   DView A = {d, ldv, 0}, B = {c + 4 * b.nnn, b.nnn, b.npc};
-  sweep2_body<FF, true>(b, (int)(wg - E.start[IB_SWEEP2]), (int)E.gx[IB_SWEEP2], (int)E.gy[IB_SWEEP2], E.ks_sweep2, ph, u, ff,
+  sweep2_body<FF, true, FIRST>(b, (int)(wg - E.start[PASS]), (int)E.gx[PASS], (int)E.gy[PASS], E.ks_sweep2, ph, u, ff,
                   v, ldv, sn_all + 9 * b.npc, c, c + 3 * b.nnn, out_d ? B : A, out_d ? A : B, sx, (LdsFlag *)flag);
 }
 
@@ -1605,7 +1636,8 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
     E.ks_coef = CK_KS;
     E.ks_sweep = SW_KS;
     const int nz = b.k2 - b.k1, ns2 = slabs(nz, S2_KS);
-    const unsigned n2x = (b.i2 - b.i1 + S2_OX - 1) / S2_OX, n2y = (b.j2 - b.j1 + S2_OY - 1) / S2_OY;
+    auto over = [](int n, int o) { return (unsigned)((n + o - 1) / o); };
+    const unsigned n2x = over(b.i2 - b.i1, s2_ox(false)), n2y = over(b.j2 - b.j1, s2_oy(false));
     E.ks_sweep2 = slabs(nz, ns2);  // even slabs of at most S2_KS planes
     // pairs or singles, for all blocks alike: the steps of each on a chip that
     // is full, as in pair_model
@@ -1617,6 +1649,8 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
                            {ntx, nty, nkz},
                            {cg.x, cg.y, (unsigned)((b.k2 - b.k1 + E.ks_coef - 1) / E.ks_coef)},
                            {n2x, n2y, (unsigned)slabs(nz, E.ks_sweep2)},
+                           {over(b.i2 - b.i1, s2_ox(true)), over(b.j2 - b.j1, s2_oy(true)),
+                            (unsigned)slabs(nz, E.ks_sweep2)},
                            {shell_wgs(b), 1, 1}};
     for (int p = 0; p < IB_N; p++) {
       E.start[p] = tot[p];
@@ -1656,7 +1690,12 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
   const SweepPlan plan = sweep_plan(lmx, pairs);
   for (int s = 0; s < plan.n; s++) {
     const int out_d = (plan.n - 1 - s) % 2 == 0;
-    if (s == 0) {
+    if (s == 0 && plan.first2) {
+      CodensTimed _tm("implimf_sweep1", st);
+      hipLaunchKernelGGL((ityprk ? k_impl_sweep2_batch<true, true> : k_impl_sweep2_batch<false, true>),
+                         dim3(tot[IB_FIRST2]), dim3(S2_NC), 0, st, ct, nb, ph, u, fx, (const double *)v, (long)ldv,
+                         sn_all, ws, d, out_d, 0);
+    } else if (s == 0) {
       CodensTimed _tm("implimf_sweep1", st);
       hipLaunchKernelGGL(k_impl_sweep1_batch, dim3(tot[IB_CELL]), dim3(TX, TY), 0, st, ct, nb, (int)ityprk, u, fx,
                          (long)ldv, ws, d, out_d);
@@ -1666,8 +1705,8 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
                          (int)ityprk, u, fx, (const double *)v, (long)ldv, sn_all, ws, d, out_d, s % 2);
     } else {
       CodensTimed _tm("implimf_sweep2", st);
-      hipLaunchKernelGGL(ityprk ? k_impl_sweep2_batch<true> : k_impl_sweep2_batch<false>, dim3(tot[IB_SWEEP2]),
-                         dim3(S2_NC), 0, st, ct, nb, ph, u, fx, (const double *)v, (long)ldv, sn_all, ws, d, out_d,
+      hipLaunchKernelGGL((ityprk ? k_impl_sweep2_batch<true, false> : k_impl_sweep2_batch<false, false>),
+                         dim3(tot[IB_SWEEP2]), dim3(S2_NC), 0, st, ct, nb, ph, u, fx, (const double *)v, (long)ldv, sn_all, ws, d, out_d,
                          s % 2);
     }
   }

@@ -27,12 +27,14 @@ def fields(lay, near=False):
 
 def pair_launches(abi, call):
     """call() in the default mode, and with one sub-iteration to a launch
-    forced; launches of pairs in the former"""
+    forced; launches of pairs (but a first one) and of single sub-iterations
+    in the former"""
     abi.timing_enable(True)
-    abi.timing_read("implimf_sweep2", reset=True)
+    for name in ("implimf_sweep", "implimf_sweep2"):
+        abi.timing_read(name, reset=True)
     try:
         two = call()
-        launches = abi.timing_read("implimf_sweep2", reset=True)[1]
+        launches = abi.timing_read("implimf_sweep2", reset=True)[1], abi.timing_read("implimf_sweep", reset=True)[1]
         prev = abi.sweep_tile(0)
         try:
             one = call()
@@ -44,11 +46,12 @@ def pair_launches(abi, call):
     return two, one, launches
 
 
-# tiles of 28 x 12 cells and slabs of 1 to 6 planes: whole and partial tiles, one
-# cell past a tile, two planes, a block narrower than the rings
-@pytest.mark.parametrize("dims", [(56, 60, 37), (57, 61, 40), (2, 300, 60), (200, 200, 2), (300, 121, 3),
+# tiles of 28 x 12 cells (30 x 14 of the first pair of an even number) and slabs of
+# 1 to 6 planes: whole and partial tiles, one cell past a tile, two planes, a
+# block narrower than the rings
+@pytest.mark.parametrize("dims", [(56, 60, 37), (57, 61, 40), (60, 70, 37), (61, 57, 40), (2, 300, 60), (200, 200, 2), (300, 121, 3),
                                   (600, 240, 2), (113, 49, 33)])
-@pytest.mark.parametrize("lmx,ityprk", [(3, 0), (4, 1)])
+@pytest.mark.parametrize("lmx,ityprk", [(2, 0), (3, 0), (4, 1)])
 def test_pairs_match_singles(dims, lmx, ityprk):
     from codens_amd import abi
     lay, sn, vol = random_mesh([dims], seed=7)
@@ -63,11 +66,11 @@ def test_pairs_match_singles(dims, lmx, ityprk):
         return v.cpu().numpy(), d.cpu().numpy()
 
     two, one, launches = pair_launches(abi, call)
-    assert launches == 1, "the shape is one that runs in pairs"
+    assert launches == ((lmx - 1) // 2, 0), "the shape is one that runs in pairs"
     assert np.array_equal(two[0], one[0]) and np.array_equal(two[1], one[1])
 
 
-@pytest.mark.parametrize("lmx,ityprk", [(3, 1), (4, 0)])
+@pytest.mark.parametrize("lmx,ityprk", [(2, 1), (3, 1), (4, 0)])
 def test_batched_pairs_match_singles(lmx, ityprk):
     from codens_amd import abi
     lay, sn, vol = random_mesh([(29, 13, 17), (56, 60, 37), (5, 3, 2), (28, 12, 16), (2, 40, 33)], seed=9)
@@ -82,7 +85,7 @@ def test_batched_pairs_match_singles(lmx, ityprk):
         return v.cpu().numpy(), d.cpu().numpy()
 
     two, one, launches = pair_launches(abi, call)
-    assert launches == 1, "these blocks run in pairs"
+    assert launches == ((lmx - 1) // 2, 0), "these blocks run in pairs"
     assert np.array_equal(two[0], one[0]) and np.array_equal(two[1], one[1])
 
 
