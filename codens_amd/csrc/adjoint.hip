@@ -369,18 +369,10 @@ __device__ inline T load_sn(const AdjArgs &a, long m, int d, int c) {
   return ldx<T>(a.sn, a.snd, o);
 }
 
-// real cell of a 1-D launch over the real cells, i fastest
-__device__ inline bool real_cell(const Blk &b, long t, int c[3]) {
-  long nx = b.i2 - b.i1, ny = b.j2 - b.j1, nz = b.k2 - b.k1;
-  if (t >= nx * ny * nz) return false;
-  c[0] = b.i1 + (int)(t % nx);
-  c[1] = b.j1 + (int)((t / nx) % ny);
-  c[2] = b.k1 + (int)(t / (nx * ny));
-  return true;
-}
+
 // face of direction d (along index a1..a2, real transverse range), i fastest
-__device__ inline bool face_of(const Blk &b, int d, long t, int c[3]) {
-  long n0 = b.i2 - b.i1 + (d == 0), n1 = b.j2 - b.j1 + (d == 1), n2 = b.k2 - b.k1 + (d == 2);
+__device__ inline bool face_of(const Blk &b, int d, unsigned t, int c[3]) {
+  const unsigned n0 = b.i2 - b.i1 + (d == 0), n1 = b.j2 - b.j1 + (d == 1), n2 = b.k2 - b.k1 + (d == 2);
   if (t >= n0 * n1 * n2) return false;
   c[0] = b.i1 + (int)(t % n0);
   c[1] = b.j1 + (int)((t / n0) % n1);
@@ -395,7 +387,7 @@ __device__ inline int along(const int c[3], int d) { return c[d]; }
 template <typename T>
 __global__ void __launch_bounds__(256) k_adj_thermo(AdjArgs a) {
   int c[3];
-  if (!real_cell(a.b, blockIdx.x * 256L + threadIdx.x, c)) return;
+  if (!line_cell(a.b, xcd_linear(), c)) return;
   long n = a.b.idx(c[0], c[1], c[2]), m = n - a.b.npc;
   T w[5], p, tt, mu;
   load_v(a, n, w);
@@ -432,24 +424,28 @@ template <typename T>
 __device__ inline T gq(const AdjArgs &a, int q, long m) {
   return q < 3 ? plane<T>(a, P_Q + 1 + q)[m] : plane<T>(a, P_TT)[m];
 }
+__device__ inline const double *gqp(const AdjArgs &a, int q) { return a.ws + (q < 3 ? P_Q + 1 + q : P_TT) * a.b.nnn; }
 
 // Green-Gauss sums of one real cell in zgrad2's accumulation order
-// (directions k, j, i; per direction the interior low face, the interior
-// high face, then the boundary faces), scaled, and the stresses from them.
+// (directions k, j, i; per direction the low face, then the high one),
+// scaled, and the stresses from them (128x64x32 cells: 19 us with the faces'
+// loads behind branches, 15 with a direction's together).
 template <typename T>
 __global__ void __launch_bounds__(256) k_adj_grad(AdjArgs a) {
   int c[3];
-  if (!real_cell(a.b, blockIdx.x * 256L + threadIdx.x, c)) return;
+  if (!line_cell(a.b, xcd_linear(), c)) return;
   const Blk &b = a.b;
   long m = b.idx(c[0], c[1], c[2]) - b.npc;
-  T G[12];
+  T G[12], here[4];
 #pragma unroll
   for (int x = 0; x < 12; x++) G[x] = zro<T>();
+#pragma unroll
+  for (int q = 0; q < 4; q++) here[q] = gq<T>(a, q, m);
+#pragma unroll
   for (int d = 2; d >= 0; d--) {
-    long inc = b.inc(d);
-    int al = c[d], a1 = b.lo(d), a2 = b.hi(d);
-    bool lo_in = al > a1, hi_in = al < a2 - 1;
-    T slo[3], shi[3];
+    const long inc = b.inc(d);
+    const bool lo_in = c[d] > b.lo(d), hi_in = c[d] < b.hi(d) - 1;
+    T slo[3], shi[3], lo[4], hi[4];
 #pragma unroll
     for (int cc = 0; cc < 3; cc++) {
       slo[cc] = load_sn<T>(a, m, d, cc);
@@ -457,33 +453,15 @@ __global__ void __launch_bounds__(256) k_adj_grad(AdjArgs a) {
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      T here = gq<T>(a, q, m);
-      if (lo_in) {
-        T fv = here + gq<T>(a, q, m - inc);
-#pragma unroll
-        for (int cc = 0; cc < 3; cc++) G[3 * q + cc] = G[3 * q + cc] - fv * slo[cc];
-      }
-      if (hi_in) {
-        T fv = gq<T>(a, q, m + inc) + here;
-#pragma unroll
-        for (int cc = 0; cc < 3; cc++) G[3 * q + cc] = G[3 * q + cc] + fv * shi[cc];
-      }
+      lo[q] = gq<T>(a, q, m - inc);
+      hi[q] = gq<T>(a, q, m + inc);
     }
-    if (!lo_in) {
+    loads_issued();
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        T gv = gq<T>(a, q, m - inc);
+    for (int q = 0; q < 4; q++) {
+      const T fl = (lo_in ? here[q] : lo[q]) + lo[q], fh = hi[q] + (hi_in ? here[q] : hi[q]);
 #pragma unroll
-        for (int cc = 0; cc < 3; cc++) G[3 * q + cc] = G[3 * q + cc] - slo[cc] * 2. * gv;
-      }
-    }
-    if (!hi_in) {
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        T gv = gq<T>(a, q, m + inc);
-#pragma unroll
-        for (int cc = 0; cc < 3; cc++) G[3 * q + cc] = G[3 * q + cc] + shi[cc] * 2. * gv;
-      }
+      for (int cc = 0; cc < 3; cc++) G[3 * q + cc] = G[3 * q + cc] - fl * slo[cc] + fh * shi[cc];
     }
   }
   const T c0 = grad_scale(ldx<T>(a.vol, a.vold, m + b.npc));
@@ -566,7 +544,7 @@ __global__ void __launch_bounds__(256) k_adj_faces(AdjArgs a, int d) {
 template <typename T>
 __global__ void __launch_bounds__(256) k_adj_gather(AdjArgs a, double *u, double *ud) {
   int c[3];
-  if (!real_cell(a.b, blockIdx.x * 256L + threadIdx.x, c)) return;
+  if (!line_cell(a.b, xcd_linear(), c)) return;
   const Blk &b = a.b;
   long n = b.idx(c[0], c[1], c[2]), m = n - b.npc;
 #pragma unroll
@@ -762,126 +740,148 @@ __device__ inline MusclW muscl_w(const AdjArgs &a) {
 // launch (nb0, nb1: workgroups of the first two): adjoints of the MUSCL
 // states, of the ghost state on boundary faces, and the metric's.  One
 // writer per entry.  The stresses' adjoints are gathered by k_adjb_tq.
+// Bound by the planes it moves (39 written, 66 read): 128x64x32 cells took
+// 49 us with loads behind branches, a boundary face's one after another (each
+// wave of direction i has some), 44 with all of a face's in one group.
 __global__ void __launch_bounds__(128) k_adjb_faces(AdjArgs a, AdjBar B, unsigned nb0, unsigned nb1) {
-  const int d = blockIdx.x < nb0 ? 0 : (blockIdx.x < nb0 + nb1 ? 1 : 2);
-  const long blk = blockIdx.x - (d == 0 ? 0 : (d == 1 ? nb0 : nb0 + nb1));
+  const unsigned wg = xcd_linear();
+  const int d = wg < nb0 ? 0 : (wg < nb0 + nb1 ? 1 : 2);
+  const long blk = wg - (d == 0 ? 0 : (d == 1 ? nb0 : nb0 + nb1));
   int c[3];
   if (!face_of(a.b, d, blk * 128L + threadIdx.x, c)) return;
   const Blk &b = a.b;
-  const long inc = b.inc(d), m = b.idx(c[0], c[1], c[2]) - b.npc, n = m + b.npc, nnn = b.nnn, ldv = a.ldv;
+  const long inc = b.inc(d), m = b.idx(c[0], c[1], c[2]) - b.npc, nnn = b.nnn, ldv = a.ldv;
   const int al = c[d], a1 = b.lo(d), a2 = b.hi(d);
-  const double *ub = B.ub;
+  const double *ub = B.ub + b.npc;
+  const unsigned mb = 8u * (unsigned)m, ib = 8u * (unsigned)inc;  // byte offsets in a plane
   double s[3], sb[3];
 #pragma unroll
-  for (int cc = 0; cc < 3; cc++) s[cc] = load_sn<double>(a, m, d, cc);
+  for (int cc = 0; cc < 3; cc++) s[cc] = ldp(a.sn + ((long)cc * 3 + d) * nnn, mb);
   double Lb[5] = {0., 0., 0., 0., 0.}, Rb[5] = {0., 0., 0., 0., 0.};
   if (al > a1 && al < a2) {
     // u(m) has -H(m), u(m-inc) has +H(m); H = 0.5 f
-    double fb[5], L[5], R[5], tl[9], tr[9];
-#pragma unroll
-    for (int e = 0; e < 5; e++) fb[e] = 0.5 * (ub[e * ldv + n - inc] - ub[e * ldv + n]);
+    double fb[5], L[5], R[5], tl[9], tr[9], u[2][5], q[4][5];
 #pragma unroll
     for (int e = 0; e < 5; e++) {
-      const double *qp = a.ws + (P_Q + e) * nnn;
-      muscl_lr(a.muscl, a.xk, qp[m - 2 * inc], qp[m - inc], qp[m], qp[m + inc], L[e], R[e]);
+      u[0][e] = ldp(ub + e * ldv, mb - ib);
+      u[1][e] = ldp(ub + e * ldv, mb);
+#pragma unroll
+      for (int x = 0; x < 4; x++) q[x][e] = ldp(a.ws + (P_Q + e) * nnn, mb + (unsigned)(x - 2) * ib);
     }
 #pragma unroll
     for (int x = 0; x < 9; x++) {
-      tl[x] = a.ws[(P_TQ + x) * nnn + m - inc];
-      tr[x] = a.ws[(P_TQ + x) * nnn + m];
+      tl[x] = ldp(a.ws + (P_TQ + x) * nnn, mb - ib);
+      tr[x] = ldp(a.ws + (P_TQ + x) * nnn, mb);
+    }
+    loads_issued();
+#pragma unroll
+    for (int e = 0; e < 5; e++) {
+      fb[e] = 0.5 * (u[0][e] - u[1][e]);
+      muscl_lr(a.muscl, a.xk, q[0][e], q[1][e], q[2][e], q[3][e], L[e], R[e]);
     }
     roe_face_vjp(a.ph, s, L, R, tl, tr, fb, Lb, Rb, sb);
   } else {
     const bool lo = al == a1;
-    const long mg = lo ? m - inc : m;
-    double hb[5], w[5], t[9], wb[5], pb, p = a.ws[(P_Q + 4) * nnn + mg];
+    const unsigned mg = lo ? mb - ib : mb, mh = lo ? mb : mb - ib;
+    double hb[5], w[5], t[9], wb[5], pb, p = ldp(a.ws + (P_Q + 4) * nnn, mg);
 #pragma unroll
-    for (int e = 0; e < 5; e++) hb[e] = lo ? -ub[e * ldv + n] : ub[e * ldv + n - inc];
+    for (int e = 0; e < 5; e++) hb[e] = ldp(ub + e * ldv, mh);
 #pragma unroll
-    for (int e = 0; e < 5; e++) w[e] = a.ws[(P_W + e) * nnn + mg];
+    for (int e = 0; e < 5; e++) w[e] = ldp(a.ws + (P_W + e) * nnn, mg);
 #pragma unroll
-    for (int x = 0; x < 9; x++) t[x] = a.ws[(P_TQ + x) * nnn + mg];
+    for (int x = 0; x < 9; x++) t[x] = ldp(a.ws + (P_TQ + x) * nnn, mg);
+    loads_issued();
+#pragma unroll
+    for (int e = 0; e < 5; e++) hb[e] = lo ? -hb[e] : hb[e];
     phys_flux_vjp(a.ph, w, p, t, s, hb, wb, pb, sb);
 #pragma unroll
-    for (int e = 0; e < 5; e++) bpl(a, B, B_W + e)[mg] = wb[e];
-    bpl(a, B, B_W + 5)[mg] = pb;
+    for (int e = 0; e < 5; e++) *gp(bpl(a, B, B_W + e), mg) = wb[e];
+    *gp(bpl(a, B, B_W + 5), mg) = pb;
   }
 #pragma unroll
   for (int e = 0; e < 5; e++) {
-    bpl(a, B, B_F + 10 * d + e)[m] = Lb[e];
-    bpl(a, B, B_F + 10 * d + 5 + e)[m] = Rb[e];
+    *gp(bpl(a, B, B_F + 10 * d + e), mb) = Lb[e];
+    *gp(bpl(a, B, B_F + 10 * d + 5 + e), mb) = Rb[e];
   }
 #pragma unroll
-  for (int cc = 0; cc < 3; cc++) B.snb[((long)cc * 3 + d) * nnn + m] = sb[cc];
+  for (int cc = 0; cc < 3; cc++) *gp(B.snb + ((long)cc * 3 + d) * nnn, mb) = sb[cc];
 }
 
 // Stresses of a real cell: their adjoints gathered from the cell's six faces
 // (a boundary face's ghost holds a copy of the cell's stresses), then those
-// of the raw gradient sums, of mu and of vol.  A face's flux has
+// of the raw gradient sums, of mu and of vol (26 us with its conditional loads
+// one by one, 18 with a direction's together; 128x64x32 cells).  A face's flux has
 // -(tau S) . (w, u) - q . S against its adjoint (w, f4), with u the velocity
 // of the cell's side: y = -(w + f4 u) is the adjoint of tau S.
 __global__ void __launch_bounds__(256) k_adjb_tq(AdjArgs a, AdjBar B) {
 #pragma clang fp contract(fast)
   int c[3];
-  if (!real_cell(a.b, blockIdx.x * 256L + threadIdx.x, c)) return;
+  if (!line_cell(a.b, xcd_linear(), c)) return;
   const Blk &b = a.b;
   const long m = b.idx(c[0], c[1], c[2]) - b.npc, n = m + b.npc, nnn = b.nnn, ldv = a.ldv;
+  const unsigned mb = 8u * (unsigned)m;  // the cell's byte offset in a plane
   const double *Q = a.ws + (P_Q + 1) * nnn, *W = a.ws + P_W * nnn;
   const double c4m = 0.25 * a.muscl * (1. - a.xk), c4p = 0.25 * a.muscl * (1. + a.xk);
   double ub0[4], u0[3], tb[9];
 #pragma unroll
-  for (int e = 0; e < 4; e++) ub0[e] = B.ub[(e + 1) * ldv + n];
+  for (int e = 0; e < 4; e++) ub0[e] = ldp(B.ub + (e + 1) * ldv + b.npc, mb);
 #pragma unroll
-  for (int x = 0; x < 3; x++) u0[x] = Q[x * nnn + m];
+  for (int x = 0; x < 3; x++) u0[x] = ldp(Q + x * nnn, mb);
 #pragma unroll
   for (int x = 0; x < 9; x++) tb[x] = 0.;
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     const long inc = b.inc(d);
+    const unsigned ib = 8u * (unsigned)inc;
     const bool bnd[2] = {c[d] == b.lo(d), c[d] == b.hi(d) - 1};
-    double um[2][3];  // velocities of the neighbours below and above
-#pragma unroll
-    for (int x = 0; x < 3; x++) {
-      um[0][x] = Q[x * nnn + m - inc];
-      um[1][x] = Q[x * nnn + m + inc];
-    }
+    // of the neighbours below and above: velocities, adjoints of u (a boundary's
+    // are not read), and the faces' normals
+    double um[2][3], un[2][4], s[2][3];
 #pragma unroll
     for (int side = 0; side < 2; side++) {
-      const long off = side ? inc : -inc;
+      const unsigned mo = side ? mb + ib : mb - ib;
+#pragma unroll
+      for (int x = 0; x < 3; x++) um[side][x] = ldp(Q + x * nnn, mo);
+#pragma unroll
+      for (int e = 0; e < 4; e++) un[side][e] = ldp(B.ub + (e + 1) * ldv + b.npc, bnd[side] ? mb : mo);
+#pragma unroll
+      for (int x = 0; x < 3; x++) s[side][x] = ldp(a.sn + ((long)x * 3 + d) * nnn, side ? mo : mb);
+    }
+    loads_issued();
+#pragma unroll
+    for (int side = 0; side < 2; side++) {
       const double sg = side ? 1. : -1.;
-      double s[3], w[4], u[3];
+      double w[4], u[3];
 #pragma unroll
-      for (int x = 0; x < 3; x++) s[x] = load_sn<double>(a, side ? m + inc : m, d, x);
+      for (int e = 0; e < 4; e++) w[e] = bnd[side] ? sg * ub0[e] : 0.5 * sg * (ub0[e] - un[side][e]);
+      // the MUSCL state of the cell's side: extrapolated toward the face
 #pragma unroll
-      for (int e = 0; e < 4; e++)
-        w[e] = bnd[side] ? sg * ub0[e] : 0.5 * sg * (ub0[e] - B.ub[(e + 1) * ldv + n + off]);
-      if (bnd[side]) {
-        const double ir = 1. / W[m + off];
+      for (int x = 0; x < 3; x++) u[x] = u0[x] + c4m * (u0[x] - um[1 - side][x]) + c4p * (um[side][x] - u0[x]);
+      if (bnd[side]) {  // the ghost's
+        const long mg = m + (side ? inc : -inc);
+        const double ir = 1. / W[mg];
 #pragma unroll
-        for (int x = 0; x < 3; x++) u[x] = W[(x + 1) * nnn + m + off] * ir;
-      } else {
-        // the MUSCL state of the cell's side: extrapolated toward the face
-#pragma unroll
-        for (int x = 0; x < 3; x++) u[x] = u0[x] + c4m * (u0[x] - um[1 - side][x]) + c4p * (um[side][x] - u0[x]);
+        for (int x = 0; x < 3; x++) u[x] = W[(x + 1) * nnn + mg] * ir;
       }
       double y[3];
 #pragma unroll
       for (int x = 0; x < 3; x++) y[x] = -(w[x] + w[3] * u[x]);
-      tb[0] += y[0] * s[0];
-      tb[1] += y[0] * s[1] + y[1] * s[0];
-      tb[2] += y[0] * s[2] + y[2] * s[0];
-      tb[3] += y[1] * s[1];
-      tb[4] += y[1] * s[2] + y[2] * s[1];
-      tb[5] += y[2] * s[2];
+      const double *S = s[side];
+      tb[0] += y[0] * S[0];
+      tb[1] += y[0] * S[1] + y[1] * S[0];
+      tb[2] += y[0] * S[2] + y[2] * S[0];
+      tb[3] += y[1] * S[1];
+      tb[4] += y[1] * S[2] + y[2] * S[1];
+      tb[5] += y[2] * S[2];
 #pragma unroll
-      for (int x = 0; x < 3; x++) tb[6 + x] -= w[3] * s[x];
+      for (int x = 0; x < 3; x++) tb[6 + x] -= w[3] * S[x];
     }
   }
   // tq is linear in mu and in the scale c0 of the gradients
   const double mu = a.ws[P_MU * nnn + m], vol = a.vol[n], c0 = grad_scale(vol);
   double tt = 0.;
 #pragma unroll
-  for (int x = 0; x < 9; x++) tt += tb[x] * a.ws[(P_TQ + x) * nnn + m];
+  for (int x = 0; x < 9; x++) tt += tb[x] * ldp(a.ws + (P_TQ + x) * nnn, mb);
   bpl(a, B, B_MU)[m] = tt / mu;
   B.volb[n] = signbit(vol) ? 0. : -tt / (vol + DBL_MIN);
   const double mc = mu * c0, m3 = 2. / 3. * mc, kq = a.ph.cp * (mu / a.ph.pr) * c0;
@@ -889,7 +889,7 @@ __global__ void __launch_bounds__(256) k_adjb_tq(AdjArgs a, AdjBar B) {
                        m3 * (2. * tb[3] - tb[0] - tb[5]), mc * tb[4], m3 * (2. * tb[5] - tb[0] - tb[3]),
                        kq * tb[6], kq * tb[7], kq * tb[8]};
 #pragma unroll
-  for (int x = 0; x < 9; x++) bpl(a, B, B_G + x)[m] = g[x];
+  for (int x = 0; x < 9; x++) *gp(bpl(a, B, B_G + x), mb) = g[x];
 }
 
 // plane (from B_G) of the adjoint of d(quantity q)/d(x_cc)
@@ -903,63 +903,103 @@ static_assert(g_plane(0, 1) == 1 && g_plane(2, 0) == 2 && g_plane(1, 1) == 3 && 
 // faces transposed (onto its own u, v, w, T; onto a boundary face's ghost;
 // onto the metrics of its low faces and of the block's high faces), the MUSCL
 // states' adjoints of the faces that reach the cell, and the thermodynamics
-// onto the conservative state.
+// onto the conservative state.  Bound by its 82 planes: 128x64x32 cells took
+// 51 us with a branch around each conditional load, 45 (4.1 TB/s) with two
+// groups of unconditional loads per direction, the face states' sums formed
+// before the second (48 with all of them at once: 330 registers, one wave).
 __global__ void __launch_bounds__(256) k_adjb_cells(AdjArgs a, AdjBar B) {
 #pragma clang fp contract(fast)
   int c[3];
-  if (!real_cell(a.b, blockIdx.x * 256L + threadIdx.x, c)) return;
+  if (!line_cell(a.b, xcd_linear(), c)) return;
   const Blk &b = a.b;
   const long n = b.idx(c[0], c[1], c[2]), m = n - b.npc, nnn = b.nnn;
+  const unsigned mb = 8u * (unsigned)m;  // the cell's byte offset in a plane
   const MusclW mw = muscl_w(a);
   double g0[9], q0[4], vb[4] = {0., 0., 0., 0.}, qb[5] = {0., 0., 0., 0., 0.};
 #pragma unroll
-  for (int x = 0; x < 9; x++) g0[x] = bpl(a, B, B_G + x)[m];
+  for (int x = 0; x < 9; x++) g0[x] = ldp(bpl(a, B, B_G + x), mb);
 #pragma unroll
-  for (int q = 0; q < 4; q++) q0[q] = gq<double>(a, q, m);
+  for (int q = 0; q < 4; q++) q0[q] = ldp(gqp(a, q), mb);
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     const long inc = b.inc(d);
     const int al = c[d], a1 = b.lo(d), a2 = b.hi(d);
-#pragma unroll
-    for (int side = 0; side < 2; side++) {
-      const bool bnd = side ? al == a2 - 1 : al == a1;
-      const long off = side ? inc : -inc, mf = side ? m + inc : m;
-      double s[3], t[9], sb[3] = {0., 0., 0.};
-#pragma unroll
-      for (int x = 0; x < 3; x++) s[x] = load_sn<double>(a, mf, d, x);
-      // adjoint of the face sums: low cell's less high cell's
-#pragma unroll
-      for (int x = 0; x < 9; x++) {
-        const double gn = bnd ? 0. : bpl(a, B, B_G + x)[m + off];
-        t[x] = side ? g0[x] - gn : gn - g0[x];
-      }
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        double f = 0.;
-#pragma unroll
-        for (int x = 0; x < 3; x++) f += t[g_plane(q, x)] * s[x];
-        if (bnd) bpl(a, B, B_V + q)[m + off] = 2. * f;
-        else vb[q] += f;
-        if (side == 0 || bnd) {
-          const double fv = bnd ? 2. * gq<double>(a, q, m + off) : q0[q] + gq<double>(a, q, m + off);
-#pragma unroll
-          for (int x = 0; x < 3; x++) sb[x] += t[g_plane(q, x)] * fv;
-        }
-      }
-      if (side == 0 || bnd) {
-#pragma unroll
-        for (int x = 0; x < 3; x++) B.snb[((long)x * 3 + d) * nnn + mf] += sb[x];
-      }
-    }
+    const unsigned ib = 8u * (unsigned)inc;
+    const bool bnd[2] = {al == a1, al == a2 - 1};
     // the cell is q1 of its high face, q2 of its low face, q0 of the face
     // after the high one and q3 of the face before the low one
+    double L[3][5], R[3][5];
+    const bool far = al + 2 < a2, near = al - 1 > a1;
 #pragma unroll
     for (int e = 0; e < 5; e++) {
       const double *Lb = bpl(a, B, B_F + 10 * d + e), *Rb = Lb + 5 * nnn;
-      double r = mw.l2 * Lb[m] + mw.r2 * Rb[m] + mw.l1 * Lb[m + inc] + mw.r1 * Rb[m + inc];
-      if (al + 2 < a2) r += mw.l0 * Lb[m + 2 * inc];
-      if (al - 1 > a1) r += mw.r3 * Rb[m - inc];
+      L[0][e] = ldp(Lb, mb);
+      L[1][e] = ldp(Lb, mb + ib);
+      L[2][e] = ldp(Lb, mb + (far ? 2 * ib : 0));
+      R[0][e] = ldp(Rb, mb);
+      R[1][e] = ldp(Rb, mb + ib);
+      R[2][e] = ldp(Rb, mb - (near ? ib : 0));
+    }
+    loads_issued();
+#pragma unroll
+    for (int e = 0; e < 5; e++) {
+      double r = mw.l2 * L[0][e] + mw.r2 * R[0][e] + mw.l1 * L[1][e] + mw.r1 * R[1][e];
+      r += far ? mw.l0 * L[2][e] : 0.;
+      r += near ? mw.r3 * R[2][e] : 0.;
       qb[e] += r;
+      asm volatile("" : "+v"(qb[e]));  // formed here, its loads' registers free for the next ones
+    }
+    const unsigned mh = mb + (bnd[1] ? ib : 0);
+    double s[2][3], gn[2][9], qn[2][4], sb0[3], sb1[3];
+#pragma unroll
+    for (int side = 0; side < 2; side++) {
+      const unsigned mo = side ? mb + ib : mb - ib, mi = bnd[side] ? mb : mo;
+#pragma unroll
+      for (int x = 0; x < 3; x++) s[side][x] = ldp(a.sn + ((long)x * 3 + d) * nnn, side ? mo : mb);
+#pragma unroll
+      for (int x = 0; x < 9; x++) gn[side][x] = ldp(bpl(a, B, B_G + x), mi);
+#pragma unroll
+      for (int q = 0; q < 4; q++) qn[side][q] = ldp(gqp(a, q), mo);
+    }
+#pragma unroll
+    for (int x = 0; x < 3; x++) {
+      sb0[x] = ldp(B.snb + ((long)x * 3 + d) * nnn, mb);
+      sb1[x] = ldp(B.snb + ((long)x * 3 + d) * nnn, mh);
+    }
+    loads_issued();
+#pragma unroll
+    for (int side = 0; side < 2; side++) {
+      const unsigned mo = side ? mb + ib : mb - ib;
+      double t[9], sb[3] = {0., 0., 0.};
+      // adjoint of the face sums: low cell's less high cell's
+#pragma unroll
+      for (int x = 0; x < 9; x++) {
+        const double g = bnd[side] ? 0. : gn[side][x];
+        t[x] = side ? g0[x] - g : g - g0[x];
+      }
+      double f[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        f[q] = 0.;
+#pragma unroll
+        for (int x = 0; x < 3; x++) f[q] += t[g_plane(q, x)] * s[side][x];
+        vb[q] += bnd[side] ? 0. : f[q];
+        const double fv = bnd[side] ? 2. * qn[side][q] : q0[q] + qn[side][q];
+#pragma unroll
+        for (int x = 0; x < 3; x++) sb[x] += t[g_plane(q, x)] * fv;
+      }
+      if (bnd[side]) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) *gp(bpl(a, B, B_V + q), mo) = 2. * f[q];
+      }
+      // a face's by the cell above it, the block's last face by the one below
+      if (side == 0) {
+#pragma unroll
+        for (int x = 0; x < 3; x++) *gp(B.snb + ((long)x * 3 + d) * nnn, mb) = sb0[x] + sb[x];
+      } else if (bnd[1]) {
+#pragma unroll
+        for (int x = 0; x < 3; x++) *gp(B.snb + ((long)x * 3 + d) * nnn, mh) = sb1[x] + sb[x];
+      }
     }
   }
   double w[5];
