@@ -37,52 +37,79 @@ __host__ __device__ inline ImpliWs impli_ws(double *ws, long nnn) {
 // of the real transverse range; the launch covers the cells up to i2, j2, k2.
 // rv = (mu + mut/cmt)/rho of the two cells (zero of a ghost, as in the
 // reference's cleared array) is formed here, its divisions and the velocities'
-// sharing one reciprocal per cell.  22 planes through memory, 3.6 TB/s: 42 us on
-// 130 x 96 x 66, where a pass of its own for rv and one that cleared the work
-// arrays took 29 us more.
-__device__ __forceinline__ void faces_body(const Blk &b, dim3 xb, const double *__restrict__ v, long ldv,
+// sharing one reciprocal per cell.  All loads first and no idle lanes: its 22
+// planes move at 4.7 TB/s, 32 us on 130 x 96 x 66; with tiles of 64 x 4, the
+// loads between the divisions and behind the neighbours' branches it took 42
+// us, and a pass of its own for rv and one that cleared the work arrays 29 more.
+__host__ __device__ __forceinline__ Blk upto_high(Blk b) {
+  b.i2++;
+  b.j2++;
+  b.k2++;
+  return b;
+}
+__device__ __forceinline__ void faces_body(const Blk &b, unsigned wg, const double *__restrict__ v, long ldv,
                                            const double *__restrict__ mu, const double *__restrict__ mut, double cmt,
                                            const double *__restrict__ sn, const double *__restrict__ vol,
                                            const ImpliWs &w) {
   int c[3];
-  c[0] = b.i1 + xb.x * TX + threadIdx.x;
-  c[1] = b.j1 + xb.y * TY + threadIdx.y;
-  c[2] = b.k1 + xb.z;
-  if (c[0] > b.i2 || c[1] > b.j2) return;
-  const double yc = rcp64(cmt);
-  auto cell = [&](long n, bool real, double q[4]) {
-    const double r = v[n], y = rcp64(r);
+  if (!line_cell(upto_high(b), wg, c)) return;
+  const int high = (c[0] == b.i2) + (c[1] == b.j2) + (c[2] == b.k2);
+  if (high > 1) return;
+  const long n = b.idx(c[0], c[1], c[2]), m = n - b.npc, n1 = b.idx(b.i1, b.j1, b.k1);
+  // the cell and its low neighbours: rho, momentum, mu, mut, vol (a ghost has
+  // no mu and mut: those of the first cell are loaded and not used)
+  double z[4][7], s[3][3];
 #pragma unroll
-    for (int e = 0; e < 3; e++) q[e] = div_rcp(v[(1 + e) * ldv + n], r, y);
-    q[3] = real ? div_rcp(mu[n] + div_rcp(mut[n], cmt, yc), r, y) : 0.;
+  for (int x = 0; x < 4; x++) {
+    const long nx = x ? n - b.inc(x - 1) : n;
+#pragma unroll
+    for (int e = 0; e < 4; e++) z[x][e] = v[e * ldv + nx];
+    const int d = x - 1;
+    const long nr = (x ? c[d] > b.lo(d) && (!high || c[d] == b.hi(d)) : !high) ? nx : n1;
+    z[x][4] = mu[nr];
+    z[x][5] = mut[nr];
+    z[x][6] = vol[nx];
+  }
+#pragma unroll
+  for (int d = 0; d < 3; d++)
+#pragma unroll
+    for (int e = 0; e < 3; e++) s[d][e] = snv(sn, b.nnn, m, d, e);
+  loads_issued();
+  const double yc = rcp64(cmt);
+  auto cell = [&](const double z[7], bool real, double q[4]) {
+    const double y = rcp64(z[0]);
+#pragma unroll
+    for (int e = 0; e < 3; e++) q[e] = div_rcp(z[1 + e], z[0], y);
+    const double rv = div_rcp(z[4] + div_rcp(z[5], cmt, yc), z[0], y);
+    q[3] = real ? rv : 0.;
   };
-  const long n = b.idx(c[0], c[1], c[2]), m = n - b.npc;
   double q[4];
-  cell(n, c[0] < b.i2 && c[1] < b.j2 && c[2] < b.k2, q);
+  cell(z[0], !high, q);
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     bool ok = true;
 #pragma unroll
     for (int x = 0; x < 3; x++) ok = ok && c[x] <= b.hi(x) - (x == d ? 0 : 1);
-    if (!ok) continue;
-    const long inc = b.inc(d);
-    double s1 = snv(sn, b.nnn, m, d, 0), s2 = snv(sn, b.nnn, m, d, 1), s3 = snv(sn, b.nnn, m, d, 2);
+    const double s1 = s[d][0], s2 = s[d][1], s3 = s[d][2];
     double cnds = s1 * s1 + s2 * s2 + s3 * s3;
     double l[4];
-    cell(n - inc, c[d] > b.lo(d), l);
+    cell(z[d + 1], c[d] > b.lo(d), l);
     double uu = 0.5 * (q[0] + l[0]), vv = 0.5 * (q[1] + l[1]), ww = 0.5 * (q[2] + l[2]);
     double uf = 0.5 * (uu * s1 + vv * s2 + ww * s3);
-    w.uf[d * b.nnn + m] = uf;
-    w.ce[d * b.nnn + m] = fabs(uf) + (q[3] + l[3]) * cnds / (vol[n] + vol[n - inc]);
+    const double ce = fabs(uf) + (q[3] + l[3]) * cnds / (z[0][6] + z[d + 1][6]);
+    if (ok) {
+      w.uf[d * b.nnn + m] = uf;
+      w.ce[d * b.nnn + m] = ce;
+    }
   }
 }
 
-__global__ void __launch_bounds__(TX *TY) k_impli2_faces(Blk b, const double *__restrict__ v, long ldv,
+__global__ void __launch_bounds__(256) k_impli2_faces(Blk b, const double *__restrict__ v, long ldv,
                                                          const double *__restrict__ mu,
                                                          const double *__restrict__ mut, double cmt,
                                                          const double *__restrict__ sn,
                                                          const double *__restrict__ vol, ImpliWs w) {
-  faces_body(b, xcd_block(), v, ldv, mu, mut, cmt, sn, vol, w);
+  faces_body(b, xcd_linear(), v, ldv, mu, mut, cmt, sn, vol, w);
 }
 
 // One sweep along direction d (impli2_eqt_3d.f90:238-275, 292-329, 346-383)
@@ -115,7 +142,7 @@ __global__ void __launch_bounds__(TX *TY) k_impli2_faces(Blk b, const double *__
 // 32 lines per wave, as few lines as there are then spread over more SIMDs);
 // with the coefficients formed and eliminated again in every sweep, one lane
 // for both equations and the loads a batch of eight steps ahead the two took
-// 20 and 40 us.  The whole phase 454 -> 290 us.
+// 20 and 40 us.  The whole phase 454 -> 280 us.
 constexpr int RT = 16;
 
 // writes val[e] of cell c = (i, j, k) of this thread's tile to the line-major
@@ -390,8 +417,7 @@ extern "C" int codens_impli2_eqt_3d(const codens_block *cb, const double *u, int
   }
   ImpliWs w = impli_ws(ws, b.nnn);
   CodensTimed _tm("impli2_eqt_3d", st);
-  dim3 gf((b.i2 - b.i1 + 1 + TX - 1) / TX, (b.j2 - b.j1 + 1 + TY - 1) / TY, b.k2 - b.k1 + 1);
-  hipLaunchKernelGGL(k_impli2_faces, gf, dim3(TX, TY), 0, st, b, v, (long)ldv, mu, mut, cmt, sn, vol, w);
+  hipLaunchKernelGGL(k_impli2_faces, cell_line(upto_high(b)), dim3(256), 0, st, b, v, (long)ldv, mu, mut, cmt, sn, vol, w);
   dim3 gr((b.i2 - b.i1 + RT - 1) / RT, (b.j2 - b.j1 + RT - 1) / RT, b.k2 - b.k1);
   hipLaunchKernelGGL(k_impli2_diag, gr, dim3(RT * RT), 0, st, b, dt, vol, cfke, u, (long)ldv, w);
   const long most = std::max(n_lines(b, 0), std::max(n_lines(b, 1), n_lines(b, 2)));
@@ -421,7 +447,7 @@ struct TurbEnt {
   unsigned gx[TB_N], gy[TB_N];  // this block's grid, per pass
 };
 
-__global__ void __launch_bounds__(TX *TY) k_impli2_faces_batch(const TurbEnt *__restrict__ tab, int nb,
+__global__ void __launch_bounds__(256) k_impli2_faces_batch(const TurbEnt *__restrict__ tab, int nb,
                                                                const double *__restrict__ v, long ldv,
                                                                const double *__restrict__ mu,
                                                                const double *__restrict__ mut, double cmt,
@@ -430,7 +456,7 @@ __global__ void __launch_bounds__(TX *TY) k_impli2_faces_batch(const TurbEnt *__
   const unsigned wg = xcd_linear();
   const TurbEnt &E = tab[tab_find(tab, nb, TB_FACE, wg)];
   const Blk b = uniform_blk(E.b);
-  faces_body(b, tab_tile(E, TB_FACE, wg), v, ldv, mu, mut, cmt, sn_all + 9 * b.npc, vol,
+  faces_body(b, wg - E.start[TB_FACE], v, ldv, mu, mut, cmt, sn_all + 9 * b.npc, vol,
              impli_ws(ws + IMPLI_PLANES * b.npc, b.nnn));
 }
 
@@ -500,7 +526,7 @@ extern "C" int codens_impli2_eqt_3d_batch(int32_t nblk, const codens_block *bloc
     E.b = b;
     const unsigned ni = b.i2 - b.i1, nj = b.j2 - b.j1, nk = b.k2 - b.k1;
     auto waves = [&](int d, int per) { return (unsigned)((n_lines(b, d) + per - 1) / per); };
-    unsigned g[TB_N][3] = {{(ni + 1 + TX - 1) / TX, (nj + 1 + TY - 1) / TY, nk + 1},
+    unsigned g[TB_N][3] = {{cell_line(upto_high(b)).x, 1, 1},
                            {(ni + RT - 1) / RT, (nj + RT - 1) / RT, nk},
                            {waves(0, 64), 1, 1},
                            {waves(1, 64), 1, 1},
@@ -533,7 +559,7 @@ extern "C" int codens_impli2_eqt_3d_batch(int32_t nblk, const codens_block *bloc
   const TurbEnt *ct = tab;
   const int nb = nblk;
   CodensTimed _tm("impli2_eqt_3d", st);
-  hipLaunchKernelGGL(k_impli2_faces_batch, dim3(tot[TB_FACE]), dim3(TX, TY), 0, st, ct, nb, (const double *)v,
+  hipLaunchKernelGGL(k_impli2_faces_batch, dim3(tot[TB_FACE]), dim3(256), 0, st, ct, nb, (const double *)v,
                      (long)ldv, mu, mut, cmt, sn_all, vol, ws);
   hipLaunchKernelGGL(k_impli2_diag_batch, dim3(tot[TB_RHS]), dim3(RT * RT), 0, st, ct, nb, dt, vol, cfke, u,
                      (long)ldv, ws);
