@@ -270,6 +270,14 @@ __device__ __forceinline__ unsigned xcd_linear(unsigned nwg) {
   return x * q + (x < r ? x : r) + hw / 8u;
 }
 __device__ __forceinline__ unsigned xcd_linear() { return xcd_linear(gridDim.x); }
+// The same within groups of 8 per, each XCD a run of per workgroups of every
+// group: for launches over blocks of unlike cost per workgroup, where an eighth
+// of the whole grid on each XCD leaves some of them done early.
+__device__ __forceinline__ unsigned xcd_grouped(unsigned per) {
+  const unsigned hw = blockIdx.x, g = 8u * per, base = hw - hw % g, left = gridDim.x - base;
+  const unsigned r = hw - base, x = r % 8u, n = left < g ? left : g, q = n / 8u, rem = n % 8u;
+  return base + x * q + (x < rem ? x : rem) + r / 8u;
+}
 
 // entry of the block that owns workgroup wg of a pass (bisection over start)
 template <typename E>
