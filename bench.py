@@ -43,8 +43,8 @@ SWEEP_BYTES_PER_CELL = 8 * (5 + 5 + 5 + 9 + 1 + 3 + 5)  # u, v, d_in, sn, diag, 
 # + 1.0 x WRITE_SIZE (factors from a 512 MiB device copy in the same run),
 # 658,503 KiB = 674.3 MB against 553.6 MB algorithmic (64x4 tiles)
 # (profiles/traffic_wall_ns_256x128x64.md); of two sub-iterations in one
-# launch 645,000 KiB, with the same factors.
-SWEEP_TRAFFIC_BYTES = {"implimf_sweep": 658503 * 1024, "implimf_sweep2": 645000 * 1024}
+# launch 654,303 KiB, with the same factors.
+SWEEP_TRAFFIC_BYTES = {"implimf_sweep": 658503 * 1024, "implimf_sweep2": 654303 * 1024}
 HBM_PEAK_GBS = 8000.0
 
 

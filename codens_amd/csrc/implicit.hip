@@ -1570,7 +1570,9 @@ k_impl_sweep2_batch(const ImplEnt *__restrict__ tab, int nb, Phys ph, const doub
   __shared__ int flag[S2_NC / 64];
   if (threadIdx.x < S2_NC / 64) flag[threadIdx.x] = 0;
   __syncthreads();
-  const unsigned wg = rev ? gridDim.x - 1 - xcd_linear() : xcd_linear();
+  // one workgroup of a compute unit is in flight, so 32 on an XCD: in groups of
+  // those 3.71 ms over 48 blocks of 40M cells, with an eighth of the grid each 3.79
+  const unsigned wg = rev ? gridDim.x - 1 - xcd_grouped(32) : xcd_grouped(32);
   constexpr int PASS = FIRST ? IB_FIRST2 : IB_SWEEP2;
   const ImplEnt &E = tab[tab_find(tab, nb, PASS, wg)];
   const Blk b = uniform_blk(E.b);

@@ -453,7 +453,7 @@ __global__ void __launch_bounds__(256) k_impli2_faces_batch(const TurbEnt *__res
                                                                const double *__restrict__ mut, double cmt,
                                                                const double *__restrict__ sn_all,
                                                                const double *__restrict__ vol, double *ws) {
-  const unsigned wg = xcd_linear();
+  const unsigned wg = xcd_grouped(64);
   const TurbEnt &E = tab[tab_find(tab, nb, TB_FACE, wg)];
   const Blk b = uniform_blk(E.b);
   faces_body(b, wg - E.start[TB_FACE], v, ldv, mu, mut, cmt, sn_all + 9 * b.npc, vol,
@@ -465,7 +465,7 @@ __global__ void __launch_bounds__(RT *RT) k_impli2_diag_batch(const TurbEnt *__r
                                                               const double *__restrict__ vol,
                                                               const double *__restrict__ cfke,
                                                               const double *__restrict__ u, long ldv, double *ws) {
-  const unsigned wg = xcd_linear();
+  const unsigned wg = xcd_grouped(64);
   const TurbEnt &E = tab[tab_find(tab, nb, TB_RHS, wg)];
   const Blk b = uniform_blk(E.b);
   diag_body(b, tab_tile(E, TB_RHS, wg), dt, vol, cfke, u, ldv, impli_ws(ws + IMPLI_PLANES * b.npc, b.nnn));
@@ -486,7 +486,7 @@ __global__ void __launch_bounds__(64) k_impli2_elim_batch(const TurbEnt *__restr
 
 __global__ void __launch_bounds__(RT *RT) k_impli2_rhs_batch(const TurbEnt *__restrict__ tab, int nb, int d,
                                                              const double *__restrict__ u, long ldv, double *ws) {
-  const unsigned wg = xcd_linear();
+  const unsigned wg = xcd_grouped(64);
   const TurbEnt &E = tab[tab_find(tab, nb, TB_RHS, wg)];
   const Blk b = uniform_blk(E.b);
   rhs_body(b, tab_tile(E, TB_RHS, wg), d, u, ldv, impli_ws(ws + IMPLI_PLANES * b.npc, b.nnn));
