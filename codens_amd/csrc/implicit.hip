@@ -1613,7 +1613,7 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
   std::vector<int32_t> key;
   std::vector<std::pair<long, long>> span(nblk);
   unsigned tot[IB_N] = {0};
-  double one = 0., two = 0.;
+  double one = 0., two = 0., longest = 0.;  // one: the fill by singles
   auto slabs = [](int nz, int ks) { return (nz + ks - 1) / ks; };
   for (int l = 0; l < nblk; l++) {
     int rc = codens_check_block(&blocks[l], what);
@@ -1641,10 +1641,12 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
     auto over = [](int n, int o) { return (unsigned)((n + o - 1) / o); };
     const unsigned n2x = over(b.i2 - b.i1, s2_ox(false)), n2y = over(b.j2 - b.j1, s2_oy(false));
     E.ks_sweep2 = slabs(nz, ns2);  // even slabs of at most S2_KS planes
-    // pairs or singles, for all blocks alike: the steps of each on a chip that
-    // is full, as in pair_model
-    one += ONE_STEP / 512. * ntx * nty * slabs(nz, SW_KS) * (SW_KS + 1);
+    // pairs or singles, for all blocks alike, as in pair_model: the steps of
+    // each on a chip that is full, and at least those of the longest workgroup
+    // (three blocks of 12 to 40 cells a side: two singles 58 us, a pair 78)
+    one += ntx * nty * slabs(nz, SW_KS) / 512.;
     two += PAIR_STEP / 256. * n2x * n2y * slabs(nz, E.ks_sweep2) * (E.ks_sweep2 + 3);
+    longest = std::max(longest, PAIR_STEP * (E.ks_sweep2 + 3));
     const unsigned nkz = (unsigned)((b.k2 - b.k1 + E.ks_sweep - 1) / E.ks_sweep);
     unsigned g[IB_N][3] = {{(unsigned)((b.nnn + 255) / 256), 1, 1},
                            {cg.x, cg.y, cg.z},
@@ -1669,7 +1671,8 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
     }
   }
   const long tot_n = span[nblk - 1].second;
-  const bool pairs = forced_tile() < 0 && two < 2. * one;
+  one = std::max(1., one) * (SW_KS + 1) * 0.5 * ONE_STEP * (1. + std::min(1., one));
+  const bool pairs = forced_tile() < 0 && std::max(two, longest) < 2. * one;
   for (int l = 0; l < nblk; l++) key.push_back(ent[l].tile);
   ImplEnt *tab = (ImplEnt *)codens_device_table(1, key, ent.data(), sizeof(ImplEnt) * nblk, st, what);
   if (!tab) return CODENS_EHIP;

@@ -71,9 +71,12 @@ def test_pairs_match_singles(dims, lmx, ityprk):
 
 
 @pytest.mark.parametrize("lmx,ityprk", [(2, 1), (3, 1), (4, 0)])
-def test_batched_pairs_match_singles(lmx, ityprk):
+@pytest.mark.parametrize("full", [False, True])
+def test_batched_pairs_match_singles(lmx, ityprk, full):
+    """Small blocks alone take single sweeps; with a block that fills the chip all run in pairs."""
     from codens_amd import abi
-    lay, sn, vol = random_mesh([(29, 13, 17), (56, 60, 37), (5, 3, 2), (28, 12, 16), (2, 40, 33)], seed=9)
+    dims = [(29, 13, 17), (56, 60, 37), (5, 3, 2), (28, 12, 16), (2, 40, 33)]
+    lay, sn, vol = random_mesh(dims + [(160, 128, 48)] * full, seed=9)
     f = fields(lay)
     g, gsn, gvol = {k: T(a) for k, a in f.items()}, T(sn), T(vol)
     arr = abi.block_array([abi.block(b) for b in lay.blocks])
@@ -85,7 +88,7 @@ def test_batched_pairs_match_singles(lmx, ityprk):
         return v.cpu().numpy(), d.cpu().numpy()
 
     two, one, launches = pair_launches(abi, call)
-    assert launches == ((lmx - 1) // 2, 0), "these blocks run in pairs"
+    assert launches == (((lmx - 1) // 2, 0) if full else (0, lmx - 1))
     assert np.array_equal(two[0], one[0]) and np.array_equal(two[1], one[1])
 
 
