@@ -216,18 +216,38 @@ class Solver:
             fs, lines, ghost, mnpar = self.parko
             abi.met_parko(fs, lines, ghost, mnpar, self.mu, self.dist, 0.075, self.v, stream=s)
 
-        def sources(l, b, s):
+        def gradients(l, b, s):
             abi.teq_gradv(b, self.sn_blk[l], self.vol, self.v, self.g9[l], stream=s)
             abi.met_prod(b, self.mut, self.v, self.g9[l], self.tprod[l], stream=s)
             abi.met_gradtr(b, self.sn_blk[l], self.vol, self.v, self.fd, stream=s)
+
+        def sources(l, b, s):
             if sa:
                 abi.met_smsa(b, t.tc, self.sn_blk[l], self.vol, self.v, self.mu, self.dist, self.g9[l], self.fd,
                              self.cfke, self.ts6, self.ts7, stream=s)
             else:
                 abi.met_smko(b, t.tc, self.v, self.tprod[l], self.cfke, self.ts6, self.ts7, self.cson, stream=s)
             abi.met_flud(b, t.kfludis, t.tc, self.v, self.mu, self.mut, self.fd, stream=s)
-        self._per_block(sources)
-        s = self.stream
+
+        def both(l, b, s):
+            gradients(l, b, s)
+            sources(l, b, s)
+        if sa and self.side:
+            # met_smsa reads fd at the block-local index (met_smsa.f90:216-217),
+            # the first nnn entries of the storage: flux densities of earlier
+            # blocks.  The blocks whose entries a later one reads go first, one
+            # after another, as all do on one stream.
+            read, reach = set(), 0
+            for l, b in reversed(list(enumerate(self.lay.blocks))):
+                if b.npc < reach:
+                    read.add(l)
+                reach = max(reach, b.nnn)
+            self._per_block(gradients)
+            for l in sorted(read):
+                sources(l, self.blocks[l], s)
+            self._per_block(lambda l, b, s: l in read or sources(l, b, s))
+        else:
+            self._per_block(both)
         if self.tq_copy[0].numel():
             abi.met_rbse(self.tq_copy[0], self.tq_copy[1], self.fd, stream=s)
         g, i, r = self.coin
