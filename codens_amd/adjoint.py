@@ -154,17 +154,17 @@ class AdjointProblem:
 
     # -- residual ------------------------------------------------------------
     def residual(self, v, sn_blk, vol):
-        """u(v) of the production kernels (real cells; zero elsewhere)."""
+        """u(v) of the production kernels (real cells; zero elsewhere), a copy
+        that later calls of the solver leave alone."""
         S = self.S
         S.v.copy_(v)
-        S.u = torch.zeros_like(S.v)  # the caller's: sch_roe writes the real cells and zeroes the ghosts
         S.sn_blk = [sn_blk.contiguous()]
         S.vol = vol.contiguous()
         S.thermo()
         S.ghosts()
         S.stresses()
         S.residual()
-        return S.u[:5]
+        return S.u[:5].clone()
 
     def jvp(self, v, sn_blk, vol, vd, snd, vold):
         z = lambda t, like: torch.zeros_like(like) if t is None else t.contiguous()
