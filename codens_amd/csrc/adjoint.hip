@@ -1034,7 +1034,16 @@ __global__ void __launch_bounds__(128) k_adjb_ghost(AdjArgs a, AdjBar B, long nf
   // states reach it (where the block has one)
   const int c[3] = {b.id1 + (int)(mg % b.nid), b.jd1 + (int)((mg / b.nid) % (b.nijd / b.nid)),
                     b.kd1 + (int)(mg / b.nijd)};
-  const int d = (c[2] < b.k1 || c[2] >= b.k2) ? 2 : ((c[1] < b.j1 || c[1] >= b.j2) ? 1 : 0);
+  int d = 0, layers = 0;
+#pragma unroll
+  for (int x = 0; x < 3; x++) {
+    const int out = max(b.lo(x) - c[x], c[x] - b.hi(x) + 1);
+    if (out > 0) {
+      d = x;
+      layers += out;
+    }
+  }
+  if (layers != 1) return;  // an edge's, a corner's or a deeper ghost: no face reads it
   const bool lo = c[d] < b.lo(d);
   const long inc = b.inc(d);
   const MusclW mw = muscl_w(a);
@@ -1065,8 +1074,10 @@ __global__ void __launch_bounds__(128) k_adjb_ghost(AdjArgs a, AdjBar B, long nf
 }
 
 // the entries of vb, snb and volb that no pass writes: snb of every entry
-// (the face pass writes the faces), vb and volb of the ghosts
-__global__ void __launch_bounds__(256) k_adjb_clear(Blk b, long ldv, double *vb, double *snb, double *volb) {
+// (the face pass writes the faces), vb and volb of the ghosts; and the value
+// planes of the ghosts, as neither list need name all of them
+__global__ void __launch_bounds__(256) k_adjb_clear(Blk b, long ldv, double *vb, double *snb, double *volb,
+                                                    double *ws) {
   const long m = blockIdx.x * 256L + threadIdx.x;
   if (m >= b.nnn) return;
 #pragma unroll
@@ -1076,6 +1087,7 @@ __global__ void __launch_bounds__(256) k_adjb_clear(Blk b, long ldv, double *vb,
 #pragma unroll
   for (int e = 0; e < 5; e++) vb[e * ldv + b.npc + m] = 0.;
   volb[b.npc + m] = 0.;
+  for (int p = 0; p < NVPLANE; p++) ws[p * b.nnn + m] = 0.;
 }
 
 __global__ void k_adj_zero(double *p, long cnt) {
@@ -1254,12 +1266,8 @@ extern "C" int codens_adj_residual_vjp(const codens_block *cb, const codens_phys
   a.ws = ws;
   AdjBar B{ws + NVPLANE * nnn, ubar, vbar, snbar, volbar};
   const Blk &b = a.b;
-  const long ni = b.i2 - b.i1, nj = b.j2 - b.j1, nk = b.k2 - b.k1, ncell = ni * nj * nk;
-  // every plane entry that is read is written before, except a ghost that
-  // neither list names
-  if (nwall + nfar < 2 * (ni * nj + nj * nk + ni * nk))
-    hipLaunchKernelGGL(k_adj_zero, dim3(nblk(NVPLANE * nnn, 256)), dim3(256), 0, st, ws, NVPLANE * nnn);
-  hipLaunchKernelGGL(k_adjb_clear, dim3(nblk(nnn, 256)), dim3(256), 0, st, b, (long)ldv, vbar, snbar, volbar);
+  const long ncell = (long)(b.i2 - b.i1) * (b.j2 - b.j1) * (b.k2 - b.k1);
+  hipLaunchKernelGGL(k_adjb_clear, dim3(nblk(nnn, 256)), dim3(256), 0, st, b, (long)ldv, vbar, snbar, volbar, ws);
   forward_chain<double>(a, nwall, wall_ghost, wall_inner, nfar, far_ghost, far_inner, far_nrm, st);
   const unsigned nf0 = nblk(nfaces(b, 0), 128), nf1 = nblk(nfaces(b, 1), 128), nf2 = nblk(nfaces(b, 2), 128);
   hipLaunchKernelGGL(k_adjb_faces, dim3(nf0 + nf1 + nf2), dim3(128), 0, st, a, B, nf0, nf1);

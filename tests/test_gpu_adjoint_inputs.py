@@ -1,5 +1,6 @@
 """The adjoint of the block residual where its inputs are not those of a plain
-gradient call: a solver used between the forward and the reverse sweep."""
+gradient call: a solver used between the forward and the reverse sweep, boundary
+lists that name other ghosts than each boundary face's once."""
 import numpy as np
 import pytest
 
@@ -35,3 +36,64 @@ def test_solver_used_before_backward():
     # two reverse sweeps differ by the order of the ghosts' atomic sums only
     for a, b, s in zip(*grads, scale):
         assert s > 0 and float((a - b).abs().max()) <= 1e-12 * s
+
+
+def fields(case, seed=3):
+    """(state, block metrics, volumes, adjoint of u) on the device"""
+    b = case.layout.blocks[0]
+    rng = np.random.default_rng(seed)
+    dev = lambda a: torch.as_tensor(np.ascontiguousarray(a), device="cuda")
+    v = case.v0 * (1 + 1e-2 * rng.standard_normal(case.v0.shape))
+    return [dev(v), dev(case.sn[9 * b.npc: 9 * (b.npc + b.nnn)]), dev(case.vol),
+            dev(rng.standard_normal((5, case.layout.ip11)))]
+
+
+def add(bcs, ghost, inner):
+    """the boundary lists with further wall ghosts"""
+    wg, wi, *far = bcs
+    i64 = lambda a: torch.as_tensor(np.asarray(a, dtype=np.int64), device="cuda")
+    return (torch.cat([wg, i64(ghost)]), torch.cat([wi, i64(inner)]), *far)
+
+
+def close(a, b, s):
+    """equal to the order of the ghosts' atomic sums, NaN where the other is"""
+    return torch.allclose(a, b, rtol=0., atol=1e-12 * s, equal_nan=True)
+
+
+def test_edge_ghosts_in_the_lists():
+    """Ghosts that no face reads add nothing, whatever the workspace held."""
+    P, case = problem()
+    b = case.layout.blocks[0]
+    args = fields(case)
+    plain, bcs = P.vjp(*args), P.bcs
+    ghost = [b.idx(0, 0, 1), b.idx(b.ii2, 0, 2), b.idx(0, b.jj2, 3), b.idx(2, 0, 0), b.idx(2, b.jj2, b.kk2),
+             b.idx(b.ii2, b.jj2, b.kk2), b.idx(0, 0, 0)]
+    inner = [b.idx(1, 1, 1)] * len(ghost)
+    P.bcs = add(bcs, ghost, inner)
+    P.jvp(*args[:3], 1e20 * args[3], None, None)  # writes the tangents of the named ghosts into the same workspace
+    for x, y in zip(plain, P.vjp(*args)):
+        assert close(y, x, float(x.abs().max()))
+
+
+def test_lists_with_one_ghost_twice():
+    """Lists as long as the boundary that leave a ghost out: the result does not
+    depend on what the workspace held, and is NaN next to the ghost that was
+    given no state."""
+    P, case = problem()
+    args, other = fields(case), fields(case, seed=4)
+    wg, wi, *far = P.bcs
+    wg, wi = wg.clone(), wi.clone()
+    left_out = int(wi[3])
+    full = P.bcs
+    P.bcs = (wg, wi, *far)
+    wg[3], wi[3] = wg[4].clone(), wi[4].clone()
+    out = []
+    for before in (args, other):
+        P.bcs = full
+        P.vjp(*before)
+        P.bcs = (wg, wi, *far)
+        out.append(P.vjp(*args))
+    for a, b in zip(*out):
+        s = float(torch.nan_to_num(a).abs().max())
+        assert close(b, a, s)
+    assert bool(out[0][0][:, left_out].isnan().any())
