@@ -19,7 +19,7 @@
 // the face fluxes, the stresses, the gradients and the thermodynamics (the
 // ghost rules: one Dual pass per input).  Its passes gather: a face's
 // adjoints are stored at the face and summed by the cells that use them, so
-// that only the ghost rules, a surface, scatter with FP64 atomic adds.
+// that only the ghosts, a surface, scatter with FP64 atomic adds.
 //
 // Arithmetic restates oracle_flux.c / oracle_visc.c (sch_roe.f90:322-578,
 // zpres.f90:66-79, zvismo.f90:90-104, clpara.f90:44-58, clnrd.f90:60-134,
@@ -807,20 +807,55 @@ __global__ void __launch_bounds__(128) k_adjb_faces(AdjArgs a, AdjBar B, unsigne
   for (int cc = 0; cc < 3; cc++) *gp(B.snb + ((long)cc * 3 + d) * nnn, mb) = sb[cc];
 }
 
-// Stresses of a real cell: their adjoints gathered from the cell's six faces
-// (a boundary face's ghost holds a copy of the cell's stresses), then those
-// of the raw gradient sums, of mu and of vol (26 us with its conditional loads
-// one by one, 18 with a direction's together; 128x64x32 cells).  A face's flux has
-// -(tau S) . (w, u) - q . S against its adjoint (w, f4), with u the velocity
-// of the cell's side: y = -(w + f4 u) is the adjoint of tau S.
+// A face's flux has -(tau S) . (w, u) - q . S against its adjoint w (four
+// components, momentum and energy), with u the velocity of one side: the part
+// of tb, the adjoint of that side's stresses and heat flux.
+__device__ __forceinline__ void tq_face(const double w[4], const double u[3], const double s[3], bool there,
+                                        double tb[9]) {
+#pragma clang fp contract(fast)
+  double y[3], f4 = there ? w[3] : 0.;  // y: the adjoint of tau S
+#pragma unroll
+  for (int x = 0; x < 3; x++) y[x] = there ? -(w[x] + w[3] * u[x]) : 0.;
+  tb[0] += y[0] * s[0];
+  tb[1] += y[0] * s[1] + y[1] * s[0];
+  tb[2] += y[0] * s[2] + y[2] * s[0];
+  tb[3] += y[1] * s[1];
+  tb[4] += y[1] * s[2] + y[2] * s[1];
+  tb[5] += y[2] * s[2];
+#pragma unroll
+  for (int x = 0; x < 3; x++) tb[6 + x] -= f4 * s[x];
+}
+
+// tq is linear in mu and in the scale c0 of the gradients: from the adjoint tb
+// of cell m's those of the raw gradient sums (g), of mu and of vol
+struct TqBar {
+  double g[9], mu, vol;
+};
+__device__ __forceinline__ TqBar tq_cell(const AdjArgs &a, unsigned mb, long m, const double tb[9]) {
+#pragma clang fp contract(fast)
+  const long nnn = a.b.nnn;
+  const double mu = a.ws[P_MU * nnn + m], vol = a.vol[m + a.b.npc], c0 = grad_scale(vol);
+  double tt = 0.;
+#pragma unroll
+  for (int x = 0; x < 9; x++) tt += tb[x] * ldp(a.ws + (P_TQ + x) * nnn, mb);
+  const double mc = mu * c0, m3 = 2. / 3. * mc, kq = a.ph.cp * (mu / a.ph.pr) * c0;
+  return TqBar{{m3 * (2. * tb[0] - tb[3] - tb[5]), mc * tb[1], mc * tb[2], m3 * (2. * tb[3] - tb[0] - tb[5]),
+                mc * tb[4], m3 * (2. * tb[5] - tb[0] - tb[3]), kq * tb[6], kq * tb[7], kq * tb[8]},
+               tt / mu,
+               signbit(vol) ? 0. : -tt / (vol + DBL_MIN)};
+}
+
+// Stresses of a real cell: their adjoints gathered from the cell's interior
+// faces, then those of what they are made of (26 us with its conditional loads
+// one by one, 18 with a direction's together; 128x64x32 cells).
 __global__ void __launch_bounds__(256) k_adjb_tq(AdjArgs a, AdjBar B) {
 #pragma clang fp contract(fast)
   int c[3];
   if (!line_cell(a.b, xcd_linear(), c)) return;
   const Blk &b = a.b;
-  const long m = b.idx(c[0], c[1], c[2]) - b.npc, n = m + b.npc, nnn = b.nnn, ldv = a.ldv;
+  const long m = b.idx(c[0], c[1], c[2]) - b.npc, nnn = b.nnn, ldv = a.ldv;
   const unsigned mb = 8u * (unsigned)m;  // the cell's byte offset in a plane
-  const double *Q = a.ws + (P_Q + 1) * nnn, *W = a.ws + P_W * nnn;
+  const double *Q = a.ws + (P_Q + 1) * nnn;
   const double c4m = 0.25 * a.muscl * (1. - a.xk), c4p = 0.25 * a.muscl * (1. + a.xk);
   double ub0[4], u0[3], tb[9];
 #pragma unroll
@@ -850,46 +885,75 @@ __global__ void __launch_bounds__(256) k_adjb_tq(AdjArgs a, AdjBar B) {
     loads_issued();
 #pragma unroll
     for (int side = 0; side < 2; side++) {
-      const double sg = side ? 1. : -1.;
       double w[4], u[3];
 #pragma unroll
-      for (int e = 0; e < 4; e++) w[e] = bnd[side] ? sg * ub0[e] : 0.5 * sg * (ub0[e] - un[side][e]);
+      for (int e = 0; e < 4; e++) w[e] = (side ? 0.5 : -0.5) * (ub0[e] - un[side][e]);
       // the MUSCL state of the cell's side: extrapolated toward the face
 #pragma unroll
       for (int x = 0; x < 3; x++) u[x] = u0[x] + c4m * (u0[x] - um[1 - side][x]) + c4p * (um[side][x] - u0[x]);
-      if (bnd[side]) {  // the ghost's
-        const long mg = m + (side ? inc : -inc);
-        const double ir = 1. / W[mg];
-#pragma unroll
-        for (int x = 0; x < 3; x++) u[x] = W[(x + 1) * nnn + mg] * ir;
-      }
-      double y[3];
-#pragma unroll
-      for (int x = 0; x < 3; x++) y[x] = -(w[x] + w[3] * u[x]);
-      const double *S = s[side];
-      tb[0] += y[0] * S[0];
-      tb[1] += y[0] * S[1] + y[1] * S[0];
-      tb[2] += y[0] * S[2] + y[2] * S[0];
-      tb[3] += y[1] * S[1];
-      tb[4] += y[1] * S[2] + y[2] * S[1];
-      tb[5] += y[2] * S[2];
-#pragma unroll
-      for (int x = 0; x < 3; x++) tb[6 + x] -= w[3] * S[x];
+      tq_face(w, u, s[side], !bnd[side], tb);
     }
   }
-  // tq is linear in mu and in the scale c0 of the gradients
-  const double mu = a.ws[P_MU * nnn + m], vol = a.vol[n], c0 = grad_scale(vol);
-  double tt = 0.;
+  const TqBar r = tq_cell(a, mb, m, tb);
+  bpl(a, B, B_MU)[m] = r.mu;
+  B.volb[m + b.npc] = r.vol;
 #pragma unroll
-  for (int x = 0; x < 9; x++) tt += tb[x] * ldp(a.ws + (P_TQ + x) * nnn, mb);
-  bpl(a, B, B_MU)[m] = tt / mu;
-  B.volb[n] = signbit(vol) ? 0. : -tt / (vol + DBL_MIN);
-  const double mc = mu * c0, m3 = 2. / 3. * mc, kq = a.ph.cp * (mu / a.ph.pr) * c0;
-  const double g[9] = {m3 * (2. * tb[0] - tb[3] - tb[5]), mc * tb[1], mc * tb[2],
-                       m3 * (2. * tb[3] - tb[0] - tb[5]), mc * tb[4], m3 * (2. * tb[5] - tb[0] - tb[3]),
-                       kq * tb[6], kq * tb[7], kq * tb[8]};
+  for (int x = 0; x < 9; x++) *gp(bpl(a, B, B_G + x), mb) = r.g[x];
+}
+
+// Whether storage entry m of a block (block-local) is the ghost of a boundary
+// face; then the direction it lies in and whether below the block.  An edge's,
+// a corner's or a deeper ghost is read by no face.
+__device__ __forceinline__ bool face_ghost(const Blk &b, long m, int &d, bool &lo) {
+  const int c[3] = {b.id1 + (int)(m % b.nid), b.jd1 + (int)((m / b.nid) % (b.nijd / b.nid)),
+                    b.kd1 + (int)(m / b.nijd)};
+  int layers = 0;
+  d = 0;
 #pragma unroll
-  for (int x = 0; x < 9; x++) *gp(bpl(a, B, B_G + x), mb) = g[x];
+  for (int x = 0; x < 3; x++) {
+    const int out = max(b.lo(x) - c[x], c[x] - b.hi(x) + 1);
+    if (out > 0) {
+      d = x;
+      layers += out;
+    }
+  }
+  lo = c[d] < b.lo(d);
+  return layers == 1;
+}
+
+// Ghost stresses transposed: a boundary face's go to the cell that the list
+// copies them from.
+__global__ void __launch_bounds__(128) k_adjb_tq_ghost(AdjArgs a, AdjBar B, long nwall, const int64_t *__restrict__ wg,
+                                                       const int64_t *__restrict__ wi, long nfar,
+                                                       const int64_t *__restrict__ fg,
+                                                       const int64_t *__restrict__ fi) {
+#pragma clang fp contract(fast)
+  const long t = blockIdx.x * 128L + threadIdx.x;
+  if (t >= nwall + nfar) return;
+  const Blk &b = a.b;
+  const long nnn = b.nnn, mg = (t < nwall ? wg[t] : fg[t - nwall]) - b.npc;
+  const long mi = (t < nwall ? wi[t] : fi[t - nwall]) - b.npc;
+  int d;
+  bool lo;
+  if (!face_ghost(b, mg, d, lo)) return;
+  const long inc = b.inc(d), mr = lo ? mg + inc : mg - inc, mf = lo ? mr : mg;  // its face's cell, its face
+  double w[4], u[3], s[3], tb[9];
+#pragma unroll
+  for (int e = 0; e < 4; e++) w[e] = (lo ? -1. : 1.) * B.ub[(e + 1) * a.ldv + b.npc + mr];
+  const double ir = 1. / a.ws[P_W * nnn + mg];
+#pragma unroll
+  for (int x = 0; x < 3; x++) {
+    u[x] = a.ws[(P_W + 1 + x) * nnn + mg] * ir;
+    s[x] = a.sn[((long)x * 3 + d) * nnn + mf];
+  }
+#pragma unroll
+  for (int x = 0; x < 9; x++) tb[x] = 0.;
+  tq_face(w, u, s, true, tb);
+  const TqBar r = tq_cell(a, 8u * (unsigned)mi, mi, tb);
+  atomicAdd(bpl(a, B, B_MU) + mi, r.mu);
+  atomicAdd(B.volb + b.npc + mi, r.vol);
+#pragma unroll
+  for (int x = 0; x < 9; x++) atomicAdd(bpl(a, B, B_G + x) + mi, r.g[x]);
 }
 
 // plane (from B_G) of the adjoint of d(quantity q)/d(x_cc)
@@ -1030,21 +1094,11 @@ __global__ void __launch_bounds__(128) k_adjb_ghost(AdjArgs a, AdjBar B, long nf
   const int k = (int)(t / nf);
   const Blk &b = a.b;
   const long mg = g[f] - b.npc, ni = in[f], nnn = b.nnn;
-  // the direction the ghost lies in, and the interior face whose MUSCL
-  // states reach it (where the block has one)
-  const int c[3] = {b.id1 + (int)(mg % b.nid), b.jd1 + (int)((mg / b.nid) % (b.nijd / b.nid)),
-                    b.kd1 + (int)(mg / b.nijd)};
-  int d = 0, layers = 0;
-#pragma unroll
-  for (int x = 0; x < 3; x++) {
-    const int out = max(b.lo(x) - c[x], c[x] - b.hi(x) + 1);
-    if (out > 0) {
-      d = x;
-      layers += out;
-    }
-  }
-  if (layers != 1) return;  // an edge's, a corner's or a deeper ghost: no face reads it
-  const bool lo = c[d] < b.lo(d);
+  // the interior face in the ghost's direction whose MUSCL states reach it
+  // (where the block has one)
+  int d;
+  bool lo;
+  if (!face_ghost(b, mg, d, lo)) return;
   const long inc = b.inc(d);
   const MusclW mw = muscl_w(a);
   double wb[5], qb[5], tb;
@@ -1272,6 +1326,9 @@ extern "C" int codens_adj_residual_vjp(const codens_block *cb, const codens_phys
   const unsigned nf0 = nblk(nfaces(b, 0), 128), nf1 = nblk(nfaces(b, 1), 128), nf2 = nblk(nfaces(b, 2), 128);
   hipLaunchKernelGGL(k_adjb_faces, dim3(nf0 + nf1 + nf2), dim3(128), 0, st, a, B, nf0, nf1);
   hipLaunchKernelGGL(k_adjb_tq, dim3(nblk(ncell, 256)), dim3(256), 0, st, a, B);
+  if (nwall + nfar)
+    hipLaunchKernelGGL(k_adjb_tq_ghost, dim3(nblk(nwall + nfar, 128)), dim3(128), 0, st, a, B, (long)nwall, wall_ghost,
+                       wall_inner, (long)nfar, far_ghost, far_inner);
   hipLaunchKernelGGL(k_adjb_cells, dim3(nblk(ncell, 256)), dim3(256), 0, st, a, B);
   if (nwall)
     hipLaunchKernelGGL(k_adjb_ghost<0>, dim3(nblk(5 * nwall, 128)), dim3(128), 0, st, a, B, (long)nwall, wall_ghost,

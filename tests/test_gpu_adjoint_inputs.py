@@ -1,6 +1,7 @@
 """The adjoint of the block residual where its inputs are not those of a plain
 gradient call: a solver used between the forward and the reverse sweep, boundary
-lists that name other ghosts than each boundary face's once."""
+lists that name other ghosts than each boundary face's once or fill them from
+other cells than the adjacent one."""
 import numpy as np
 import pytest
 
@@ -77,8 +78,8 @@ def test_edge_ghosts_in_the_lists():
 
 def test_lists_with_one_ghost_twice():
     """Lists as long as the boundary that leave a ghost out: the result does not
-    depend on what the workspace held, and is NaN next to the ghost that was
-    given no state."""
+    depend on what the workspace held; the metric's adjoint is NaN on the face of
+    the ghost that was given no state (density 0), the state's finite."""
     P, case = problem()
     args, other = fields(case), fields(case, seed=4)
     wg, wi, *far = P.bcs
@@ -96,4 +97,30 @@ def test_lists_with_one_ghost_twice():
     for a, b in zip(*out):
         s = float(torch.nan_to_num(a).abs().max())
         assert close(b, a, s)
-    assert bool(out[0][0][:, left_out].isnan().any())
+    n = case.layout.ip11
+    assert bool(out[0][1].view(3, 3, n)[:, 1, left_out].isnan().any())
+    assert bool(out[0][0].isfinite().all())
+
+
+def test_ghosts_filled_from_other_cells():
+    """<J xdot, ubar> = <xdot, J^T ubar> with every ghost's values taken from
+    some cell of the block, up to three ghosts from one, some far from their
+    face.  Both sides sum the same products in other orders: 1e-11 of the sum of
+    their absolute values, as for the adjacent cells."""
+    P, case = problem()
+    b, rng = case.layout.blocks[0], np.random.default_rng(8)
+    wg, wi, fg, fi, nrm = P.bcs
+    cells = b.interior()
+    pick = lambda t: torch.as_tensor(rng.choice(cells, t.numel()), device="cuda")
+    P.bcs = (wg, pick(wi), fg, pick(fi), nrm)
+    v, sn, vol, ub = fields(case)
+    ub *= P.real
+    vd, snd, vold, _ = [torch.as_tensor(rng.standard_normal(tuple(x.shape)), device="cuda") * x.abs().max()
+                        for x in (v, sn, vol, ub)]
+    _, ud = P.jvp(v, sn, vol, vd, snd, vold)
+    vb, snb, volb = P.vjp(v, sn, vol, ub)
+    terms = [ud * ub, vd * vb, snd * snb, vold * volb]
+    lhs, rhs = float(terms[0].sum()), sum(float(t.sum()) for t in terms[1:])
+    scale = sum(float(t.abs().sum()) for t in terms)
+    assert np.isfinite(scale) and scale > 0
+    assert abs(lhs - rhs) <= 1e-11 * scale, (lhs, rhs, scale)
