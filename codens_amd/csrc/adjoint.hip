@@ -564,8 +564,8 @@ __global__ void __launch_bounds__(256) k_adj_gather(AdjArgs a, double *u, double
 // faces), W the conservative ghost state and its pressure (5 + 1), V the
 // gradient quantities u, v, w, T of the ghosts (4), G the raw gradient sums
 // (the nine distinct ones: the adjoint of the velocity gradient is
-// symmetric), MU mu.
-constexpr int B_F = 0, B_W = 30, B_V = 36, B_G = 40, B_MU = 49, NBPLANE = 50;
+// symmetric), LM log mu (which stays finite where mu is zero).
+constexpr int B_F = 0, B_W = 30, B_V = 36, B_G = 40, B_LM = 49, NBPLANE = 50;
 
 struct AdjBar {
   double *bw;                 // adjoint planes
@@ -827,9 +827,9 @@ __device__ __forceinline__ void tq_face(const double w[4], const double u[3], co
 }
 
 // tq is linear in mu and in the scale c0 of the gradients: from the adjoint tb
-// of cell m's those of the raw gradient sums (g), of mu and of vol
+// of cell m's those of the raw gradient sums (g), of log mu and of vol
 struct TqBar {
-  double g[9], mu, vol;
+  double g[9], lm, vol;
 };
 __device__ __forceinline__ TqBar tq_cell(const AdjArgs &a, unsigned mb, long m, const double tb[9]) {
 #pragma clang fp contract(fast)
@@ -841,7 +841,7 @@ __device__ __forceinline__ TqBar tq_cell(const AdjArgs &a, unsigned mb, long m, 
   const double mc = mu * c0, m3 = 2. / 3. * mc, kq = a.ph.cp * (mu / a.ph.pr) * c0;
   return TqBar{{m3 * (2. * tb[0] - tb[3] - tb[5]), mc * tb[1], mc * tb[2], m3 * (2. * tb[3] - tb[0] - tb[5]),
                 mc * tb[4], m3 * (2. * tb[5] - tb[0] - tb[3]), kq * tb[6], kq * tb[7], kq * tb[8]},
-               tt / mu,
+               tt,
                signbit(vol) ? 0. : -tt / (vol + DBL_MIN)};
 }
 
@@ -895,7 +895,7 @@ __global__ void __launch_bounds__(256) k_adjb_tq(AdjArgs a, AdjBar B) {
     }
   }
   const TqBar r = tq_cell(a, mb, m, tb);
-  bpl(a, B, B_MU)[m] = r.mu;
+  bpl(a, B, B_LM)[m] = r.lm;
   B.volb[m + b.npc] = r.vol;
 #pragma unroll
   for (int x = 0; x < 9; x++) *gp(bpl(a, B, B_G + x), mb) = r.g[x];
@@ -950,7 +950,7 @@ __global__ void __launch_bounds__(128) k_adjb_tq_ghost(AdjArgs a, AdjBar B, long
   for (int x = 0; x < 9; x++) tb[x] = 0.;
   tq_face(w, u, s, true, tb);
   const TqBar r = tq_cell(a, 8u * (unsigned)mi, mi, tb);
-  atomicAdd(bpl(a, B, B_MU) + mi, r.mu);
+  atomicAdd(bpl(a, B, B_LM) + mi, r.lm);
   atomicAdd(B.volb + b.npc + mi, r.vol);
 #pragma unroll
   for (int x = 0; x < 9; x++) atomicAdd(bpl(a, B, B_G + x) + mi, r.g[x]);
@@ -1070,7 +1070,7 @@ __global__ void __launch_bounds__(256) k_adjb_cells(AdjArgs a, AdjBar B) {
   load_v(a, n, w);
   const double ir = 1. / w[0], T = q0[3];
   double Tb = vb[3];
-  if (a.ph.iflu == 1) Tb += bpl(a, B, B_MU)[m] * a.ws[P_MU * nnn + m] * (1.5 / T - 1. / (T + a.ph.asuth));
+  if (a.ph.iflu == 1) Tb += bpl(a, B, B_LM)[m] * (1.5 / T - 1. / (T + a.ph.asuth));
   const double pb = qb[4] + Tb * a.ph.gam * ir, ep = a.ph.gam1 * pb;
   double r0 = qb[0] - Tb * T * ir;
 #pragma unroll

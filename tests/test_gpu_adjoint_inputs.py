@@ -102,17 +102,10 @@ def test_lists_with_one_ghost_twice():
     assert bool(out[0][0].isfinite().all())
 
 
-def test_ghosts_filled_from_other_cells():
-    """<J xdot, ubar> = <xdot, J^T ubar> with every ghost's values taken from
-    some cell of the block, up to three ghosts from one, some far from their
-    face.  Both sides sum the same products in other orders: 1e-11 of the sum of
-    their absolute values, as for the adjacent cells."""
-    P, case = problem()
-    b, rng = case.layout.blocks[0], np.random.default_rng(8)
-    wg, wi, fg, fi, nrm = P.bcs
-    cells = b.interior()
-    pick = lambda t: torch.as_tensor(rng.choice(cells, t.numel()), device="cuda")
-    P.bcs = (wg, pick(wi), fg, pick(fi), nrm)
+def check_dot_product(P, case, rng):
+    """<J xdot, ubar> = <xdot, J^T ubar> over state, metrics and volumes.  Both
+    sides sum the same products in other orders: 1e-11 of the sum of their
+    absolute values."""
     v, sn, vol, ub = fields(case)
     ub *= P.real
     vd, snd, vold, _ = [torch.as_tensor(rng.standard_normal(tuple(x.shape)), device="cuda") * x.abs().max()
@@ -124,3 +117,23 @@ def test_ghosts_filled_from_other_cells():
     scale = sum(float(t.abs().sum()) for t in terms)
     assert np.isfinite(scale) and scale > 0
     assert abs(lhs - rhs) <= 1e-11 * scale, (lhs, rhs, scale)
+
+
+def test_ghosts_filled_from_other_cells():
+    """Every ghost's values taken from some cell of the block, up to three
+    ghosts from one, some far from their face."""
+    P, case = problem()
+    rng = np.random.default_rng(8)
+    wg, wi, fg, fi, nrm = P.bcs
+    cells = case.layout.blocks[0].interior()
+    pick = lambda t: torch.as_tensor(rng.choice(cells, t.numel()), device="cuda")
+    P.bcs = (wg, pick(wi), fg, pick(fi), nrm)
+    check_dot_product(P, case, rng)
+
+
+@pytest.mark.parametrize("iflu", [0, 1])
+def test_no_viscosity(iflu):
+    """The limit of an infinite Reynolds number: viscosity, stresses and heat
+    flux zero everywhere."""
+    P, case = problem(reynz=np.inf, iflu=iflu)
+    check_dot_product(P, case, np.random.default_rng(9))
