@@ -43,35 +43,40 @@ struct DFluxT {  // mass-flux increment (d of rho u, rho v, rho w) and dF
 using DFlux = DFluxT<double>;
 
 // implimf_3d.f90:434-465 for one cell: dF = F(v + d) - F(v), p(v) from the EOS
-// as zpres.f90:72-73 computes it.  The velocities are formed with one
-// reciprocal of each density instead of the reference's divisions (about
-// 1e-16 relative per value; the sub-iteration result moves by ~3e-14).
-template <typename T>
-__device__ inline DFluxT<T> dflux(const Phys &ph, const T V[5], const T D[5]) {
-  const T gam1 = (T)ph.gam1, pinfl = (T)ph.pinfl;
-  T wi1 = V[0] + D[0], wi2 = V[1] + D[1], wi3 = V[2] + D[2], wi4 = V[3] + D[3], wi5 = V[4] + D[4];
-  T ri = T(1) / wi1, r0 = T(1) / V[0];
-  T ui = wi2 * ri, vi = wi3 * ri, wi = wi4 * ri;
-  T pres = gam1 * (wi5 - T(.5) * wi1 * (ui * ui + vi * vi + wi * wi) - pinfl);
-  T a = V[1] * r0, bb = V[2] * r0, c = V[3] * r0;
-  T rhoe = V[4] - T(0.5) * (V[1] * a + V[2] * bb + V[3] * c);
-  T p = gam1 * (rhoe - pinfl);
-  T fxx = V[1] * a + p, fxy = V[2] * a, fxz = V[3] * a;
-  T fyy = V[2] * bb + p, fyz = V[3] * bb, fzz = V[3] * c + p;
-  T e5 = V[4] + p - pinfl;
-  T fex = e5 * a, fey = e5 * bb, fez = e5 * c;
-  DFluxT<T> r;
-  r.mx = D[1]; r.my = D[2]; r.mz = D[3];
-  r.xx = wi1 * (ui * ui) + pres - fxx;
-  r.xy = wi1 * ui * vi - fxy;
-  r.xz = wi1 * ui * wi - fxz;
-  r.ex = ui * (wi5 + pres - pinfl) - fex;
-  r.yy = wi1 * (vi * vi) + pres - fyy;
-  r.yz = wi1 * vi * wi - fyz;
-  r.ey = vi * (wi5 + pres - pinfl) - fey;
-  r.zz = wi1 * (wi * wi) + pres - fzz;
-  r.ez = wi * (wi5 + pres - pinfl) - fez;
-  return r;
+// as zpres.f90:72-73 computes it, as the 14-vector of the sub-iterations: the
+// mass-flux increments (d of rho u, rho v, rho w), the nine dF (xx xy xz yy yz
+// zz, energy x y z), d of rho and of rho E.  The velocities are formed with one
+// reciprocal of each density instead of the reference's divisions (about 1e-16
+// relative per value; the sub-iteration result moves by ~3e-14).
+//
+// Here and in the face sums the fused multiply-adds are written out, so that
+// every kernel that runs sub-iterations rounds alike and gives the same bits:
+// left to the compiler, the all-blocks kernel fused other products of the k
+// faces than the per-block one.
+__device__ __forceinline__ void dflux_q(const Phys &ph, const double V[5], const double D[5], double q[14]) {
+#pragma clang fp contract(off)
+  const double w0 = V[0] + D[0], w1 = V[1] + D[1], w2 = V[2] + D[2], w3 = V[3] + D[3], w4 = V[4] + D[4];
+  const double ri = 1. / w0, r0 = 1. / V[0];
+  const double u = w1 * ri, v = w2 * ri, w = w3 * ri;
+  const double kn = fma(w, w, fma(u, u, v * v));
+  const double xn = fma(-(0.5 * w0), kn, w4) - ph.pinfl, pn = ph.gam1 * xn;
+  const double a = V[1] * r0, b = V[2] * r0, c = V[3] * r0;
+  const double k0 = fma(V[3], c, fma(V[1], a, V[2] * b));
+  const double x0 = fma(-0.5, k0, V[4]) - ph.pinfl, p = ph.gam1 * x0;
+  const double e5 = fma(ph.gam1, x0, V[4]) - ph.pinfl, en = fma(ph.gam1, xn, w4) - ph.pinfl;
+  const double wu = w0 * u, wv = w0 * v;
+  q[0] = D[1]; q[1] = D[2]; q[2] = D[3];
+  q[3] = fma(w0, u * u, pn) - fma(V[1], a, p);
+  q[4] = fma(wu, v, -(V[2] * a));
+  q[5] = fma(wu, w, -(V[3] * a));
+  q[6] = fma(w0, v * v, pn) - fma(V[2], b, p);
+  q[7] = fma(wv, w, -(V[3] * b));
+  q[8] = fma(w0, w * w, pn) - fma(V[3], c, p);
+  q[9] = fma(u, en, -(e5 * a));
+  q[10] = fma(v, en, -(e5 * b));
+  q[11] = fma(w, en, -(e5 * c));
+  q[12] = D[0];
+  q[13] = D[4];
 }
 
 // The same increment dF = F(v + d) - F(v) in difference form, for the FP32
@@ -115,14 +120,6 @@ __device__ inline DFluxT<T> dflux_delta(const Phys &ph, const T V[5], const T D[
   return r;
 }
 
-// dF of the sub-iterations: the reference's form in FP64, the difference
-// form in FP32
-template <typename T>
-__device__ inline DFluxT<T> dflux_sweep(const Phys &ph, const T V[5], const T D[5]) {
-  if constexpr (sizeof(T) == sizeof(float)) return dflux_delta<T>(ph, V, D);
-  else return dflux<T>(ph, V, D);
-}
-
 // implimf_eu.f90:289-312 for one cell: dF from the momenta with
 // wi1 = 1/(rho + d1), the base flux with the caller's pressure p, and the z
 // energy increment without its w factor, as the reference has it.
@@ -150,15 +147,6 @@ __device__ inline DFlux dflux_eu(const Phys &ph, const double V[5], const double
   r.zz = wi1 * (wi * wi) + pres - fzz;
   r.ez = wi1 * h - fez;
   return r;
-}
-
-// tn of a face (implimf_3d.f90:276-292): half-sum of both cells' increments . S
-__device__ inline void face_tn(const DFlux &A, const DFlux &B, double s1, double s2, double s3, double tn[5]) {
-  tn[0] = 0.5 * (A.mx + B.mx) * s1 + 0.5 * (A.my + B.my) * s2 + 0.5 * (A.mz + B.mz) * s3;
-  tn[1] = 0.5 * (A.xx + B.xx) * s1 + 0.5 * (A.xy + B.xy) * s2 + 0.5 * (A.xz + B.xz) * s3;
-  tn[2] = 0.5 * (A.xy + B.xy) * s1 + 0.5 * (A.yy + B.yy) * s2 + 0.5 * (A.yz + B.yz) * s3;
-  tn[3] = 0.5 * (A.xz + B.xz) * s1 + 0.5 * (A.yz + B.yz) * s2 + 0.5 * (A.zz + B.zz) * s3;
-  tn[4] = 0.5 * (A.ex + B.ex) * s1 + 0.5 * (A.ey + B.ey) * s2 + 0.5 * (A.ez + B.ez) * s3;
 }
 
 #define CELL3(b) CELL3_AT(b, xcd_block())
@@ -513,43 +501,33 @@ struct Q14T {
 };
 using Q14 = Q14T<double>;
 
-template <typename T, class DIN>
-__device__ inline void q_of(const Phys &ph, const T *__restrict__ v, long ldv, const DIN &d, long n, Q14T<T> &Q) {
+template <typename T>
+__device__ inline void q_set(const DFluxT<T> &F, const T D[5], Q14T<T> &Q) {
+  Q.q[0] = F.mx; Q.q[1] = F.my; Q.q[2] = F.mz;
+  Q.q[3] = F.xx; Q.q[4] = F.xy; Q.q[5] = F.xz; Q.q[6] = F.yy; Q.q[7] = F.yz; Q.q[8] = F.zz;
+  Q.q[9] = F.ex; Q.q[10] = F.ey; Q.q[11] = F.ez;
+  Q.q[12] = D[0]; Q.q[13] = D[4];
+}
+
+// the 14-vector of a cell: the reference's form in FP64, the difference form
+// in FP32, implimf_eu's own flux increments (with the caller's p)
+template <bool EU, typename T>
+__device__ inline void q_form(const Phys &ph, const T V[5], const T D[5], double p, Q14T<T> &Q) {
+  if constexpr (EU) q_set<T>(dflux_eu(ph, V, D, p), D, Q);
+  else if constexpr (sizeof(T) == sizeof(float)) q_set<T>(dflux_delta<T>(ph, V, D), D, Q);
+  else dflux_q(ph, V, D, Q.q);
+}
+
+template <bool EU, typename T, class DIN>
+__device__ inline void q_model(const Phys &ph, const T *__restrict__ v, long ldv, const DIN &d,
+                               const double *__restrict__ ps, long n, Q14T<T> &Q) {
   T V[5], D[5];
 #pragma unroll
   for (int e = 0; e < 5; e++) {
     V[e] = v[e * ldv + n];
     D[e] = d.at(e, n);
   }
-  DFluxT<T> F = dflux_sweep<T>(ph, V, D);
-  Q.q[0] = F.mx; Q.q[1] = F.my; Q.q[2] = F.mz;
-  Q.q[3] = F.xx; Q.q[4] = F.xy; Q.q[5] = F.xz; Q.q[6] = F.yy; Q.q[7] = F.yz; Q.q[8] = F.zz;
-  Q.q[9] = F.ex; Q.q[10] = F.ey; Q.q[11] = F.ez;
-  Q.q[12] = D[0]; Q.q[13] = D[4];
-}
-
-// the same 14-vector for implimf_eu (its own flux increments, caller's p)
-template <class DIN>
-__device__ inline void q_of_eu(const Phys &ph, const double *__restrict__ v, long ldv, const DIN &d,
-                               const double *__restrict__ ps, long n, Q14 &Q) {
-  double V[5], D[5];
-#pragma unroll
-  for (int e = 0; e < 5; e++) {
-    V[e] = v[e * ldv + n];
-    D[e] = d.at(e, n);
-  }
-  DFlux F = dflux_eu(ph, V, D, ps[n]);
-  Q.q[0] = F.mx; Q.q[1] = F.my; Q.q[2] = F.mz;
-  Q.q[3] = F.xx; Q.q[4] = F.xy; Q.q[5] = F.xz; Q.q[6] = F.yy; Q.q[7] = F.yz; Q.q[8] = F.zz;
-  Q.q[9] = F.ex; Q.q[10] = F.ey; Q.q[11] = F.ez;
-  Q.q[12] = D[0]; Q.q[13] = D[4];
-}
-
-template <bool EU, typename T, class DIN>
-__device__ inline void q_model(const Phys &ph, const T *__restrict__ v, long ldv, const DIN &d,
-                               const double *__restrict__ ps, long n, Q14T<T> &Q) {
-  if constexpr (EU) q_of_eu(ph, v, ldv, d, ps, n, Q);
-  else q_of<T, DIN>(ph, v, ldv, d, n, Q);
+  q_form<EU, T>(ph, V, D, EU ? ps[n] : 0., Q);
 }
 
 template <typename T>
@@ -584,15 +562,8 @@ __device__ inline void vd_q(const Phys &ph, const VD<T> &x, bool real, Q14T<T> &
     q_zero(Q);
     return;
   }
-  DFluxT<T> F;
-  if constexpr (EU) F = dflux_eu(ph, x.V, x.D, x.p);
-  else F = dflux_sweep<T>(ph, x.V, x.D);
-  Q.q[0] = F.mx; Q.q[1] = F.my; Q.q[2] = F.mz;
-  Q.q[3] = F.xx; Q.q[4] = F.xy; Q.q[5] = F.xz; Q.q[6] = F.yy; Q.q[7] = F.yz; Q.q[8] = F.zz;
-  Q.q[9] = F.ex; Q.q[10] = F.ey; Q.q[11] = F.ez;
-  Q.q[12] = x.D[0]; Q.q[13] = x.D[4];
+  q_form<EU, T>(ph, x.V, x.D, x.p, Q);
 }
-
 
 // d of component e from the 14-vector
 template <typename T>
@@ -600,15 +571,25 @@ __device__ inline T q_d(const T *q, int e) {
   return e == 0 ? q[12] : (e == 4 ? q[13] : q[e - 1]);
 }
 
-// tn of a face between cells A and B (implimf_3d.f90:276-292)
-template <typename T>
-__device__ inline void q_tn(const T *A, const T *B, T s1, T s2, T s3, T tn[5]) {
-  const T h = T(0.5);
-  tn[0] = h * (A[0] + B[0]) * s1 + h * (A[1] + B[1]) * s2 + h * (A[2] + B[2]) * s3;
-  tn[1] = h * (A[3] + B[3]) * s1 + h * (A[4] + B[4]) * s2 + h * (A[5] + B[5]) * s3;
-  tn[2] = h * (A[4] + B[4]) * s1 + h * (A[6] + B[6]) * s2 + h * (A[7] + B[7]) * s3;
-  tn[3] = h * (A[5] + B[5]) * s1 + h * (A[7] + B[7]) * s2 + h * (A[8] + B[8]) * s3;
-  tn[4] = h * (A[9] + B[9]) * s1 + h * (A[10] + B[10]) * s2 + h * (A[11] + B[11]) * s3;
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return fma(a, b, c); }
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return fmaf(a, b, c); }
+
+// Twice the face term tn (implimf_3d.f90:276-292), component by component, q
+// of the other cell taken by get(c).  The half is exact and goes into the fused
+// multiply-add that uses the term.
+__host__ __device__ constexpr int tn_comp(int e, int x) {
+  constexpr int C[5][3] = {{0, 1, 2}, {3, 4, 5}, {4, 6, 7}, {5, 7, 8}, {9, 10, 11}};
+  return C[e][x];
+}
+template <typename T, class Get>
+__device__ __forceinline__ void tn2_fma(const T A[14], const T s[3], T tn[5], Get get) {
+#pragma clang fp contract(off)
+  T x[12];
+#pragma unroll
+  for (int c = 0; c < 12; c++) x[c] = A[c] + get(c);
+#pragma unroll
+  for (int e = 0; e < 5; e++)
+    tn[e] = fma_t(x[tn_comp(e, 2)], s[2], fma_t(x[tn_comp(e, 0)], s[0], x[tn_comp(e, 1)] * s[1]));
 }
 
 // First sub-iteration: d and dF are zero, so d = -(u (+ff)) / diag.
@@ -635,18 +616,13 @@ __global__ void __launch_bounds__(TX *TY) k_impl_sweep1(Blk b, int ityprk, const
 
 constexpr int SW_PL = (SW_TY + 2) * (SW_TX + 2);  // LDS plane stride between the 14 components
 
-// face term of the face between the LDS cells a (own side) and o (other side),
-// components read straight from LDS: tn = 0.5 (q_a + q_o) . S
+// twice the term of the face between the LDS cells a (own side) and o (other
+// side), components read straight from LDS
 template <int P, typename T>
-__device__ inline T lds_tn(const T *a, const T *o, int e, T s1, T s2, T s3) {
-  const T h = T(0.5);
-  switch (e) {
-    case 0: return h * (a[0] + o[0]) * s1 + h * (a[P] + o[P]) * s2 + h * (a[2 * P] + o[2 * P]) * s3;
-    case 1: return h * (a[3 * P] + o[3 * P]) * s1 + h * (a[4 * P] + o[4 * P]) * s2 + h * (a[5 * P] + o[5 * P]) * s3;
-    case 2: return h * (a[4 * P] + o[4 * P]) * s1 + h * (a[6 * P] + o[6 * P]) * s2 + h * (a[7 * P] + o[7 * P]) * s3;
-    case 3: return h * (a[5 * P] + o[5 * P]) * s1 + h * (a[7 * P] + o[7 * P]) * s2 + h * (a[8 * P] + o[8 * P]) * s3;
-    default: return h * (a[9 * P] + o[9 * P]) * s1 + h * (a[10 * P] + o[10 * P]) * s2 + h * (a[11 * P] + o[11 * P]) * s3;
-  }
+__device__ __forceinline__ T lds_tn2(const T *a, const T *o, int e, const T s[3]) {
+#pragma clang fp contract(off)
+  const int x = tn_comp(e, 0) * P, y = tn_comp(e, 1) * P, z = tn_comp(e, 2) * P;
+  return fma_t(a[z] + o[z], s[2], fma_t(a[x] + o[x], s[0], (a[y] + o[y]) * s[1]));
 }
 template <int P, typename T>
 __device__ inline T lds_d(const T *a, int e) {
@@ -667,6 +643,7 @@ __device__ __forceinline__ void sweep_body(const Blk b, int lg, int ntx, int nty
                                            const T *__restrict__ sn, const T *__restrict__ coefe,
                                            const T *__restrict__ diag, const DIN dold, const TView<T> dnew,
                                            T *sq) {
+#pragma clang fp contract(off)
   constexpr int PL = (TYS + 2) * (TXS + 2), HALO = 2 * TXS + 2 * TYS;
   static_assert(HALO <= TXS * TYS, "one halo cell per thread at most");
 #include "sweep_tile.inc"
@@ -682,6 +659,7 @@ __global__ void __launch_bounds__(TXS *TYS) SW_ATTR k_impl_sweep_tiled(Blk b, Ph
                                                                    const T *__restrict__ coefe,
                                                                    const T *__restrict__ diag, TView<T> dold,
                                                                    TView<T> dnew, int rev) {
+#pragma clang fp contract(off)
   // XCD-aware tile order: the hardware deals workgroups to the 8 XCDs round
   // robin; give each XCD a contiguous run of tiles so that j/k neighbours
   // share its L2.  rev runs each XCD's tiles in reverse: alternate
@@ -707,10 +685,9 @@ __global__ void __launch_bounds__(TXS *TYS) SW_ATTR k_impl_sweep_tiled(Blk b, Ph
 // reciprocal per cell to the next plane.  A's and B's 14-vectors of a plane lie
 // in LDS buffers of their own; a wave holds two rows.
 //
-// Every cell's operations are those of sweep_tile.inc in the same order, the
-// fused multiply-adds that the compiler forms there written out, so that a
-// pair gives the bits of two single sweeps (the minmod chains turn a change of
-// the last bit of the state into 1e-7 of the next residual).  The term of an
+// Every cell's operations are those of sweep_tile.inc in the same order, so
+// that a pair gives the bits of two single sweeps (the minmod chains turn a
+// change of the last bit of the state into 1e-7 of the next residual).  The term of an
 // i face is formed by the cell above it and passed down a lane.
 //
 // One workgroup per CU (135 KB of LDS, 254 registers, two waves per SIMD).  On
@@ -734,55 +711,6 @@ __device__ __forceinline__ double lane_above(double x) {
   return __hiloint2double(hi, lo);
 }
 
-// dflux with its fused multiply-adds written out
-__device__ __forceinline__ void dflux_q(const Phys &ph, const double V[5], const double D[5], double q[14]) {
-#pragma clang fp contract(off)
-  const double w0 = V[0] + D[0], w1 = V[1] + D[1], w2 = V[2] + D[2], w3 = V[3] + D[3], w4 = V[4] + D[4];
-  const double ri = 1. / w0, r0 = 1. / V[0];
-  const double u = w1 * ri, v = w2 * ri, w = w3 * ri;
-  const double kn = fma(w, w, fma(u, u, v * v));
-  const double xn = fma(-(0.5 * w0), kn, w4) - ph.pinfl, pn = ph.gam1 * xn;
-  const double a = V[1] * r0, b = V[2] * r0, c = V[3] * r0;
-  const double k0 = fma(V[3], c, fma(V[1], a, V[2] * b));
-  const double x0 = fma(-0.5, k0, V[4]) - ph.pinfl, p = ph.gam1 * x0;
-  const double e5 = fma(ph.gam1, x0, V[4]) - ph.pinfl, en = fma(ph.gam1, xn, w4) - ph.pinfl;
-  const double wu = w0 * u, wv = w0 * v;
-  q[0] = D[1]; q[1] = D[2]; q[2] = D[3];
-  q[3] = fma(w0, u * u, pn) - fma(V[1], a, p);
-  q[4] = fma(wu, v, -(V[2] * a));
-  q[5] = fma(wu, w, -(V[3] * a));
-  q[6] = fma(w0, v * v, pn) - fma(V[2], b, p);
-  q[7] = fma(wv, w, -(V[3] * b));
-  q[8] = fma(w0, w * w, pn) - fma(V[3], c, p);
-  q[9] = fma(u, en, -(e5 * a));
-  q[10] = fma(v, en, -(e5 * b));
-  q[11] = fma(w, en, -(e5 * c));
-  q[12] = D[0];
-  q[13] = D[4];
-}
-
-// Twice q_tn, with its fused multiply-adds written out: component by
-// component, q of the other cell taken by get(c).  The half is exact and goes
-// into the fused multiply-add that uses the term.  Of the first two products
-// of component e the first is the fused one, or the second if e is in SECOND.
-// The compiler fuses the second one in the all-blocks kernel's k faces and
-// nowhere else: in K_FACE on the upper face of a plane (which the plane above
-// takes over), in K_FIRST on the lower face of the first plane of a slab.
-constexpr int K_FACE = 1 << 2 | 1 << 3 | 1 << 4, K_FIRST = 1 << 1;
-template <int SECOND = 0, class Get>
-__device__ __forceinline__ void tn2_fma(const double A[14], const double s[3], double tn[5], Get get) {
-#pragma clang fp contract(off)
-  constexpr int C[5][3] = {{0, 1, 2}, {3, 4, 5}, {4, 6, 7}, {5, 7, 8}, {9, 10, 11}};
-  double x[12];
-#pragma unroll
-  for (int c = 0; c < 12; c++) x[c] = A[c] + get(c);
-#pragma unroll
-  for (int e = 0; e < 5; e++) {
-    const double a = x[C[e][0]], b = x[C[e][1]];
-    tn[e] = fma(x[C[e][2]], s[2], SECOND >> e & 1 ? fma(b, s[1], a * s[0]) : fma(a, s[0], b * s[1]));
-  }
-}
-
 // component of q that holds d of equation e
 __device__ __forceinline__ constexpr int q_comp(int e) { return e == 0 ? 12 : (e == 4 ? 13 : e - 1); }
 
@@ -803,9 +731,8 @@ __device__ __forceinline__ T ldp2(const T *base, unsigned off) {
   return *gp2(base, off);
 }
 
-// BATCH: with the bits of the all-blocks launch's single sweeps.  FIRST: A is
-// sub-iteration 1, which starts from d = 0 and is (-u - ff)/diag.
-template <bool FF, bool BATCH, bool FIRST>
+// FIRST: A is sub-iteration 1, which starts from d = 0 and is (-u - ff)/diag.
+template <bool FF, bool FIRST>
 __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int nty, int ks, const Phys &ph,
                                             const double *__restrict__ u, const double *__restrict__ ff,
                                             const double *__restrict__ v, long ldv, const double *__restrict__ sn,
@@ -835,8 +762,6 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
   double *qP = qB, *qC = FIRST ? qA : qB;
   auto st = [&](int x) -> double & { return stash[x * S2_NC]; };  // V of the plane
   const long nnn = b.nnn, nijd = b.nijd;
-  constexpr int KF = BATCH ? K_FACE : 0, K1 = BATCH ? K_FIRST : 0;
-  auto first = [&](int k) { return (k - b.k1) % SW_KS == 0; };  // of a slab of the single sweeps
   double qn[14], tkA[5], base[5], skl[3], ckl, rdb = 0.;  // qn: q of A's next plane
   long mk = (long)(ka - b.kd1) * nijd;
   auto load_vd = [&](long m, unsigned off, double V[5], double D[5]) {
@@ -865,9 +790,7 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
 #pragma unroll
       for (int e = 0; e < 5; e++) st(e) = V[e];
     }
-    auto below = [&](int c) { return q[c]; };
-    if (BATCH && !first(ka)) tn2_fma<KF>(qn, skl, tkA, below);
-    else tn2_fma<K1>(qn, skl, tkA, below);
+    tn2_fma(qn, skl, tkA, [&](int c) { return q[c]; });
 #pragma unroll
     for (int c = 0; c < 14; c++) {
       if (!FIRST) qA[c * S2_NC + t] = q[c];
@@ -967,14 +890,12 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
       faces(qA, tkA);
       // the plane above, the face between and what its increment adds
       if (own && kreal) dflux_q(ph, Vn, Dn, qn);
-      auto here = [&](int c) { return q[c]; };
-      tn2_fma<KF>(qn, skh, tkA, here);
+      tn2_fma(qn, skh, tkA, [&](int c) { return q[c]; });
 #pragma unroll
       for (int e = 0; e < 5; e++) {
         if (kreal) w[e] = fma(ckh, qn[q_comp(e)], w[e]);
         w[e] = fma(-0.5, tkA[e], w[e]);
       }
-      if (BATCH && first(k + 1)) tn2_fma<K1>(qn, skh, tkA, here);
 #pragma unroll
       for (int e = 0; e < 5; e++) dhi[e] = w[e] * rd;  // A's increment
     }
@@ -992,14 +913,12 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
     }
     // B: plane k - 1 is complete with the face to plane k
     double tk[5];
-    auto belowB = [&](int c) { return qP[c * S2_NC + t]; };
-    tn2_fma<KF>(q, skl, tk, belowB);
+    tn2_fma(q, skl, tk, [&](int c) { return qP[c * S2_NC + t]; });
 #pragma unroll
     for (int e = 0; e < 5; e++) {
       dlo[e] = qP[q_comp(e) * S2_NC + t];
       dhi[e] = fma(-0.5, tk[e], fma(ckl, dhi[e], base[e])) * rdb;
     }
-    if (BATCH && first(k)) tn2_fma<K1>(q, skl, tk, belowB);
     if (out && k > kb) {
 #pragma unroll
       for (int e = 0; e < 5; e++) *gp2(dnew.p + (e * dnew.ld + (b.npc - dnew.off) + mk - nijd), pl) = dhi[e];
@@ -1026,7 +945,7 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
     double q[14], tk[5];
 #pragma unroll
     for (int c = 0; c < 14; c++) q[c] = qP[c * S2_NC + t];
-    tn2_fma<KF>(q, skl, tk, [&](int) { return 0.; });
+    tn2_fma(q, skl, tk, [&](int) { return 0.; });
 #pragma unroll
     for (int e = 0; e < 5; e++)
       *gp2(dnew.p + (e * dnew.ld + (b.npc - dnew.off) + mk - nijd), opaque(pl0)) =
@@ -1045,7 +964,7 @@ k_impl_sweep2(Blk b, Phys ph, int ntx, int nty, int ks, const double *__restrict
   __syncthreads();
   unsigned lg = xcd_linear();
   if (rev) lg = gridDim.x - 1 - lg;
-  sweep2_body<FF, false, FIRST>(b, (int)lg, ntx, nty, ks, ph, u, ff, v, ldv, sn, coefe, diag, dold, dnew, sx, (LdsFlag *)flag);
+  sweep2_body<FF, FIRST>(b, (int)lg, ntx, nty, ks, ph, u, ff, v, ldv, sn, coefe, diag, dold, dnew, sx, (LdsFlag *)flag);
 }
 
 // ---------------------------------------------------------------------------
@@ -1578,7 +1497,7 @@ k_impl_sweep2_batch(const ImplEnt *__restrict__ tab, int nb, Phys ph, const doub
   const Blk b = uniform_blk(E.b);
   double *c = ws + 9 * b.npc;
   DView A = {d, ldv, 0}, B = {c + 4 * b.nnn, b.nnn, b.npc};
-  sweep2_body<FF, true, FIRST>(b, (int)(wg - E.start[PASS]), (int)E.gx[PASS], (int)E.gy[PASS], E.ks_sweep2, ph, u, ff,
+  sweep2_body<FF, FIRST>(b, (int)(wg - E.start[PASS]), (int)E.gx[PASS], (int)E.gy[PASS], E.ks_sweep2, ph, u, ff,
                   v, ldv, sn_all + 9 * b.npc, c, c + 3 * b.nnn, out_d ? B : A, out_d ? A : B, sx, (LdsFlag *)flag);
 }
 
