@@ -714,10 +714,9 @@ __device__ __forceinline__ double lane_above(double x) {
 // component of q that holds d of equation e
 __device__ __forceinline__ constexpr int q_comp(int e) { return e == 0 ? 12 : (e == 4 ? 13 : e - 1); }
 
-// a flag that waves of a workgroup pass to each other (as an LDS access: a
-// volatile access through a generic pointer stays one, and waits for the global
-// loads in flight)
-using LdsFlag = volatile __attribute__((address_space(3))) int;
+// a flag that waves of a workgroup pass to each other (an LDS pointer: an access
+// through a generic one waits for the global loads in flight too)
+using LdsFlag = __attribute__((address_space(3))) int;
 
 // gp and ldp without the empty asm, whose scalar operands the pair kernel has no
 // registers for (the opaque offsets suffice there; the fused residual is 2%
@@ -806,15 +805,17 @@ __device__ __forceinline__ void sweep2_body(const Blk &b, int lg, int ntx, int n
   // flag in each before it waits, so every wait ends.  A row is overwritten
   // only after its readers have raised the flag of the following phase: a
   // buffer is written again two phases later (two meetings a plane, or one and
-  // two buffers in turn).
+  // two buffers in turn).  The flags are relaxed atomics, so that the fences
+  // around them order the rows.
   const int wv = __builtin_amdgcn_readfirstlane(t / 64);
   int phase = 0;
+  auto raised = [&](int w) { return __hip_atomic_load(flag + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
   auto meet = [&]() {
     phase++;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    flag[wv] = phase;
-    if (wv > 0) while (flag[wv - 1] < phase) __builtin_amdgcn_s_sleep(0);
-    if (wv < S2_NC / 64 - 1) while (flag[wv + 1] < phase) __builtin_amdgcn_s_sleep(0);
+    __hip_atomic_store(flag + wv, phase, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (wv > 0) while (raised(wv - 1) < phase) __builtin_amdgcn_s_sleep(0);
+    if (wv < S2_NC / 64 - 1) while (raised(wv + 1) < phase) __builtin_amdgcn_s_sleep(0);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   };
   struct IJ {
