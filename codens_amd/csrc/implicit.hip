@@ -421,6 +421,14 @@ k_impl_coef_tiled(Blk b, Phys ph, const double *__restrict__ v, long ldv,
   coef_tiled_body<T>(b, xcd_block(), ph, v, ldv, mu, mut, dt, vol, cson, sn, dtpas, kfmg, coefe, diag, ks, S, F);
 }
 
+// The next slab depth after x with fewer slabs in nz planes (of the depths with
+// the same number of slabs the smallest takes the fewest steps, and there are
+// at most 2 sqrt(nz) numbers), nz + 1 after the last
+static int next_slab(int nz, int x) {
+  const int slabs = (nz + x - 1) / x;
+  return slabs > 1 ? (nz + slabs - 2) / (slabs - 1) : nz + 1;
+}
+
 // Slab depth of k_impl_coef_tiled on the tiles g.x x g.y: of four workgroups
 // per compute unit, the fewest steps over their rounds (a slab of ks planes
 // takes ks + 1)
@@ -428,7 +436,7 @@ static int coef_slab(const Blk &b, dim3 g) {
   const int nz = b.k2 - b.k1, places = codens_resident_workgroups(4);
   int ks = 1;
   long best = 0;
-  for (int x = 1; x <= nz; x++) {
+  for (int x = 1; x <= nz; x = next_slab(nz, x)) {
     const long c = ((long)g.x * g.y * ((nz + x - 1) / x) + places - 1) / places * (x + 1);
     if (x == 1 || c < best) { ks = x; best = c; }
   }
@@ -1135,7 +1143,7 @@ struct Pair {
 Pair pair_of(const Blk &b, bool first = false) {
   const int nz = b.k2 - b.k1, ncu = codens_resident_workgroups(1), ox = s2_ox(first), oy = s2_oy(first);
   Pair p{(b.i2 - b.i1 + ox - 1) / ox, (b.j2 - b.j1 + oy - 1) / oy, 1, 0, 0};
-  for (int ks = 1; ks <= nz; ks++) {
+  for (int ks = 1; ks <= nz; ks = next_slab(nz, ks)) {
     const long w = (long)p.ntx * p.nty * ((nz + ks - 1) / ks);
     const long c = (w + ncu - 1) / ncu * (std::min(ks + 2, nz) + 1);
     if (ks == 1 || c < p.steps) { p.ks = ks; p.wgs = w; p.steps = c; }
