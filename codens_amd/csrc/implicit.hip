@@ -15,6 +15,7 @@
 #include <algorithm>
 
 #include <array>
+#include <cmath>
 #include <map>
 #include <mutex>
 
@@ -1152,20 +1153,42 @@ Pair pair_of(const Blk &b, bool first = false) {
 }
 
 // Whether a block's sub-iterations run in pairs: the modelled time (us) of a
-// pair against that of two single sweeps.  Measured on MI355X: a step of the
-// pair kernel takes 5.3 us, a step of a single sweep 3.4 us while few of the
-// chip's 512 workgroup places are taken and 6.8 us when all are.  Two singles
-// / a pair: 256 x 128 x 64 250 / 185 us, 200 x 120 x 100 370 / 206, 128 x 128
-// x 32 60 / 58, 75 x 61 x 43 45 / 36, 32 x 16 x 8 14 / 19.  In FP32 the sweeps
-// are bound by their arithmetic, of which a pair has half as much again (its
-// tile's rings): singles.
-constexpr double PAIR_STEP = 5.3, ONE_STEP = 6.8;
+// pair against that of two single sweeps.  Measured on MI355X over 310 block
+// shapes of 2 to 300 cells a side: a step of the pair kernel takes 4.4 to 5.2 us
+// (less on blocks of fewer rows than its tile).  A single sweep's workgroup
+// takes 3.4 us a plane and 4 to start, and the launch fills the chip's places in
+// rounds, of which a partly filled last one takes 0.9 of a full one at most;
+// where the places are full of active lanes the memory limits, with idle lanes
+// 0.4 of that.  Two singles / a pair:
+//   256 x 128 x 64 245 / 174 us, 200 x 120 x 100 367 / 192, 128 x 128 x 32 58 / 52,
+//   75 x 61 x 43 41 / 33, 48 x 40 x 36 19 / 24, 16 x 16 x 400 19 / 33,
+//   4 x 64 x 400 47 / 60
+// (the pair kernel's tiles of 28 x 12 cells leave most of their lanes idle on
+// the last two).  Of the 310 shapes the rule runs 6 in pairs where that is
+// slower by more than 2% (14% at most), and 13 singly (29% at most).
+constexpr double PAIR_STEP = 4.8;
+
+// A single sweep whose workgroups (of planes planes) would fill the chip's
+// places `fill` times, a share `active` of their lanes on cells
+double single_model(double fill, double planes, double active) {
+  const double rounds = fill <= 1. ? 1. : std::min(std::ceil(fill), fill + 0.9);
+  const double latency = rounds * (3.4 * planes + 4.);
+  const double memory = std::max(1., fill) * (planes + 1.) * 2.8 * (0.8 + 1.2 * active * std::min(1., fill));
+  return std::max(latency, memory);
+}
+
 bool pair_model(const Blk &b) {
-  const int tile = tile_model(b), tx = tile_tx(tile), ty = tile_ty(tile), nz = b.k2 - b.k1;
-  const long txy = (long)((b.i2 - b.i1 + tx - 1) / tx) * ((b.j2 - b.j1 + ty - 1) / ty);
-  const int ks = slab_depth(txy, nz, SW_KS);
-  const double fill = txy * ((nz + ks - 1) / ks) / 512.;
-  const double one = std::max(1., fill) * (ks + 1) * 0.5 * ONE_STEP * (1. + std::min(1., fill));
+  const int nx = b.i2 - b.i1, ny = b.j2 - b.j1, nz = b.k2 - b.k1;
+  const double places = codens_resident_workgroups(2);
+  double one = 0.;  // with the shape that takes least
+  for (int t = 0; t < N_SWEEP_TILES; t++) {
+    const int tx = tile_tx(t), ty = tile_ty(t);
+    const long txy = (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
+    const int ks = slab_depth(txy, nz, SW_KS);
+    const double wgs = (double)txy * ((nz + ks - 1) / ks);
+    const double x = single_model(wgs / places, ks, (double)nx * ny * nz / (wgs * ks * tx * ty));
+    if (t == 0 || x < one) one = x;
+  }
   return PAIR_STEP * pair_of(b).steps < 2. * one;
 }
 
@@ -1541,7 +1564,8 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
   std::vector<int32_t> key;
   std::vector<std::pair<long, long>> span(nblk);
   unsigned tot[IB_N] = {0};
-  double one = 0., two = 0., longest = 0.;  // one: the fill by singles
+  double one_wgs = 0., lanes = 0., cells = 0., two = 0., longest = 0.;
+  int deepest = 0;
   auto slabs = [](int nz, int ks) { return (nz + ks - 1) / ks; };
   for (int l = 0; l < nblk; l++) {
     int rc = codens_check_block(&blocks[l], what);
@@ -1569,12 +1593,16 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
     auto over = [](int n, int o) { return (unsigned)((n + o - 1) / o); };
     const unsigned n2x = over(b.i2 - b.i1, s2_ox(false)), n2y = over(b.j2 - b.j1, s2_oy(false));
     E.ks_sweep2 = slabs(nz, ns2);  // even slabs of at most S2_KS planes
-    // pairs or singles, for all blocks alike, as in pair_model: the steps of
-    // each on a chip that is full, and at least those of the longest workgroup
-    // (three blocks of 12 to 40 cells a side: two singles 58 us, a pair 78)
-    one += ntx * nty * slabs(nz, SW_KS) / 512.;
-    two += PAIR_STEP / 256. * n2x * n2y * slabs(nz, E.ks_sweep2) * (E.ks_sweep2 + 3);
-    longest = std::max(longest, PAIR_STEP * (E.ks_sweep2 + 3));
+    // pairs or singles, for all blocks alike, as in pair_model: the steps of a
+    // pair on a chip that is full, and at least those of the longest workgroup
+    // (three blocks of 12 to 40 cells a side: two singles 55 us, a pair 77)
+    const double wgs = (double)ntx * nty * slabs(nz, SW_KS);
+    one_wgs += wgs;
+    lanes += (double)ntx * nty * nz * SW_TX * SW_TY;
+    cells += (double)(b.i2 - b.i1) * (b.j2 - b.j1) * nz;
+    deepest = std::max(deepest, std::min(SW_KS, nz));
+    two += (double)n2x * n2y * slabs(nz, E.ks_sweep2) * (E.ks_sweep2 + 2);
+    longest = std::max(longest, E.ks_sweep2 + 2.);
     const unsigned nkz = (unsigned)((b.k2 - b.k1 + E.ks_sweep - 1) / E.ks_sweep);
     unsigned g[IB_N][3] = {{(unsigned)((b.nnn + 255) / 256), 1, 1},
                            {cg.x, cg.y, cg.z},
@@ -1599,8 +1627,10 @@ extern "C" int codens_implimf_3d_batch(int32_t nblk, const codens_block *blocks,
     }
   }
   const long tot_n = span[nblk - 1].second;
-  one = std::max(1., one) * (SW_KS + 1) * 0.5 * ONE_STEP * (1. + std::min(1., one));
-  const bool pairs = forced_tile() < 0 && std::max(two, longest) < 2. * one;
+  const double fill = one_wgs / codens_resident_workgroups(2);
+  const double one = single_model(fill, fill <= 1. ? deepest : lanes / (SW_TX * SW_TY) / one_wgs, cells / lanes);
+  const bool pairs =
+      forced_tile() < 0 && PAIR_STEP * std::max(two / codens_resident_workgroups(1), longest) < 2. * one;
   for (int l = 0; l < nblk; l++) key.push_back(ent[l].tile);
   ImplEnt *tab = (ImplEnt *)codens_device_table(1, key, ent.data(), sizeof(ImplEnt) * nblk, st, what);
   if (!tab) return CODENS_EHIP;

@@ -40,8 +40,41 @@ def host_time(f):
     return best
 
 
+def pair_launches(f):
+    """the number of pairs of sub-iterations (but a first one) that a call launches"""
+    from codens_amd import abi
+    abi.timing_enable(True)
+    try:
+        abi.timing_read("implimf_sweep2", reset=True)
+        f()
+        return abi.timing_read("implimf_sweep2", reset=True)[1]
+    finally:
+        abi.timing_enable(False)
+
+
 def test_host_time_of_long_blocks():
     """The slab depths are found in about the square root of the plane count:
     a block of 40,000 planes takes the host no more than 3 times what one of 40
     takes (6 times with a look at every depth)."""
     assert host_time(call([(2, 2, 40000)])) <= 3. * host_time(call([(64, 64, 40)]))
+
+
+# measured on MI355X, two single sub-iterations / a pair (us)
+@pytest.mark.parametrize("dims,pairs", [((16, 16, 400), False),  # 19 / 33
+                                        ((4, 64, 400), False),  # 47 / 60
+                                        ((3, 63, 128), False), ((5, 231, 17), False), ((8, 30, 202), False),
+                                        ((2, 2, 12000), False),  # 128 / 180
+                                        ((40, 40, 20), False), ((24, 24, 64), False),
+                                        ((20, 20, 2000), True),  # 139 / 90
+                                        ((17, 33, 300), True), ((65, 33, 129), True), ((130, 96, 66), True)])
+def test_pairs_where_they_are_faster(dims, pairs):
+    assert bool(pair_launches(call([dims]))) == pairs
+
+
+@pytest.mark.parametrize("dims,pairs", [([(16, 16, 192)] * 16, False),  # 136 / 176
+                                        ([(28, 12, 64)] * 16, False),  # 61 / 86
+                                        ([(4, 4, 3000)] * 3, False), ([(12, 17, 40), (25, 33, 18), (37, 14, 22)], False),
+                                        ([(16, 192, 16)] * 32, True),  # 273 / 171
+                                        ([(56, 24, 32)] * 32, True)])  # 168 / 102
+def test_batched_pairs_where_they_are_faster(dims, pairs):
+    assert bool(pair_launches(call(dims, batched=True))) == pairs
