@@ -98,6 +98,30 @@ TIMED_KERNELS = ("implimf_sweep", "implimf_sweep2", "implimf_sweep1", "implimf_c
                  "chronos", "zpres", "zvismo")
 
 
+def pair_cells(s):
+    """Real cells of each block of a solver whose implicit phase, called for
+    the block alone, runs sub-iterations in pairs (on copies of the state)."""
+    from codens_amd import abi
+    c, v, d, out = s.case, s.v.clone(), s.d.clone(), []
+    abi.timing_enable(True)
+    abi.timing_read("implimf_sweep2", reset=True)
+    for b, cb, sn in zip(s.lay.blocks, s.blocks, s.sn_blk):
+        abi.implimf_3d(cb, s.ph, s.u, s.dt, v, d, s.ff, s.mu, s.mut, c.lmax, sn, s.vol, s.ps, s.cson, stream=s.stream)
+        if abi.timing_read("implimf_sweep2", reset=True)[1]:
+            out.append(b.ncells)
+    abi.timing_enable(False)
+    return out
+
+
+def cells_per_sweep_launch(pairs, launches, stages, ncell, lmax, batched):
+    """Mean real cells of a launch of the dominant sweep kernel.  pairs: the
+    cells of the blocks that run in pairs (None: the kernel is the single
+    sweep, which then sweeps every cell lmax - 1 times a stage)."""
+    if pairs is None:
+        return ncell * (lmax - 1) * stages / launches
+    return ncell if batched else sum(pairs) / len(pairs)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -192,16 +216,14 @@ def main():
     n_timing = max(3, args.steps // 4)
     # two sub-iterations at once (all but the first launch), where there are
     # any: each launch moves what one sub-iteration's does
+    pairs = None
     if "implimf_sweep2" in kern:
         sweep_name = "implimf_sweep2"
+        pairs = [] if "implicit" in s.batch else pair_cells(s)
     sw = kern.get(sweep_name, {"avg_us": float("nan"), "launches": nblk * (case.lmax - 1) * n_timing})
-    # bytes of all sweep launches over their summed time: the timing stages
-    # sweep every cell lmax-1 times, in one launch per block and
-    # sub-iteration, or one per sub-iteration when the blocks are batched
-    if sweep_name == "implimf_sweep2":
-        cells_per_launch = ncell / (1 if "implicit" in s.batch else nblk)
-    else:
-        cells_per_launch = ncell * (case.lmax - 1) * n_timing / sw["launches"]
+    # bytes of all sweep launches over their summed time: one launch per block
+    # that takes the kernel, or one for all when the blocks are batched
+    cells_per_launch = cells_per_sweep_launch(pairs, sw["launches"], n_timing, ncell, case.lmax, "implicit" in s.batch)
     achieved = sweep_bytes * cells_per_launch / (sw["avg_us"] * 1e-6) / 1e9
     out = {
         "metric": "Mcell-updates/s per implicit iter to 1e-8 residual drop; % of HBM roofline",
