@@ -92,6 +92,8 @@ def cpu_allcores(case, stages, sample=None):
 
 
 # kernels (or launch groups) timed with HIP events on the launch stream
+# (implimf_sweep1: the first of the sub-iterations' launches, in pairs the first
+# two of an even number)
 TIMED_KERNELS = ("implimf_sweep", "implimf_sweep2", "implimf_sweep1", "implimf_coef", "implimf_update",
                  "implimf32_sweep", "implimf32_sweep1", "implimf32_coef", "implimf32_update", "roe_prim",
                  "roe_limiter_chain", "roe_face_flux", "roe_gather", "roe_fused", "roe_zero_ghost", "zvisqc",
@@ -219,7 +221,7 @@ def main():
     pairs = None
     if "implimf_sweep2" in kern:
         sweep_name = "implimf_sweep2"
-        pairs = [] if "implicit" in s.batch else pair_cells(s)
+        pairs = [] if "implicit" in s.batch else pair_cells(s) if nblk > 1 else [ncell]
     sw = kern.get(sweep_name, {"avg_us": float("nan"), "launches": nblk * (case.lmax - 1) * n_timing})
     # bytes of all sweep launches over their summed time: one launch per block
     # that takes the kernel, or one for all when the blocks are batched

@@ -922,7 +922,8 @@ __device__ __forceinline__ bool face_ghost(const Blk &b, long m, int &d, bool &l
 }
 
 // Ghost stresses transposed: a boundary face's go to the cell that the list
-// copies them from.
+// copies them from, 11 atomic adds a ghost (10 us for the 28,672 of 128x64x32;
+// gathered by the adjacent cell they cost nothing, but the lists may name others).
 __global__ void __launch_bounds__(128) k_adjb_tq_ghost(AdjArgs a, AdjBar B, long nwall, const int64_t *__restrict__ wg,
                                                        const int64_t *__restrict__ wi, long nfar,
                                                        const int64_t *__restrict__ fg,

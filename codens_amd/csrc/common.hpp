@@ -57,8 +57,8 @@ inline Phys make_phys(const codens_phys *p) {
 // squares the relative error, so two steps end within an ulp).  Five VALU
 // instructions in place of the eleven of a correctly rounded division.  On
 // 2^24 random operands of exponents -1000..1000 it equals the correctly
-// rounded 1/x on every one; it is not meant for 0, infinities or operands
-// whose reciprocal is subnormal.
+// rounded 1/x on every one; a few operands next to 1 round the other way.  It
+// is not meant for 0, infinities or operands whose reciprocal is subnormal.
 __device__ __forceinline__ double rcp64(double x) {
   double r = __builtin_amdgcn_rcp(x);
   double e = fma(-x, r, 1.);
@@ -69,7 +69,10 @@ __device__ __forceinline__ double rcp64(double x) {
 
 // x / d, y = rcp64(d): the steps of the compiler's division after its
 // reciprocal, so that quotients of one divisor share that; zeros, infinities
-// and NaN as there
+// and NaN as there.  Without that division's scaling: for divisors of exponents
+// -1020..1020 and quotients and dividends that are zero or above 1e-290, which
+// densities, volumes and the lines' diagonals and what they divide are.  A
+// smaller dividend may round the other way; a divisor beyond gives NaN or 0.
 __device__ __forceinline__ double div_rcp(double x, double d, double y) {
   const double q = x * y;
   return __builtin_amdgcn_div_fixup(fma(fma(-d, q, x), y, q), d, x);
@@ -248,9 +251,11 @@ __device__ __forceinline__ bool shell_layers(const Blk &b, int z0, long n0, long
 // grid of tiles_xy i-j tiles has at least 512 workgroups (two per compute
 // unit of MI355X's 256) or the slab is one plane.  A deeper slab re-reads
 // fewer planes below its first; a small block needs more workgroups to fill
-// the chip.  The coefficient and sub-iteration kernels form a slab's first
-// plane with the functions that form the planes they carry, so their values
-// do not depend on the depth (their all-blocks launches keep full slabs).
+// the chip.  The coefficient and sub-iteration kernels round a slab's first
+// plane as the planes they carry (contraction off, the fused multiply-adds
+// written out), so their values do not depend on the depth: their all-blocks
+// launches keep full slabs, and the coefficients of a block on its own take
+// any depth (coef_slab).
 // The fused residual forms the k face below a slab in other code than the
 // faces it carries, which may round it differently (a few ulp): its
 // all-blocks launch gives each block the per-block depth.

@@ -162,8 +162,8 @@ __device__ inline DFlux dflux_eu(const Phys &ph, const double V[5], const double
 
 // implimf_3d.f90:113-224: spectral-radius coefficients of the faces and the
 // diagonal; coefe[d] holds the low face of every real cell.  A workgroup
-// owns a TX x TY tile of real cells and marches a slab of up to CK_KS
-// k-planes (fewer on small blocks, slab_depth), so that each face is
+// owns a TX x TY tile of real cells and marches a slab of k-planes (of
+// coef_slab's depth, CK_KS in the all-blocks launch), so that each face is
 // evaluated once.  Per plane, the velocity, sound speed, rv and
 // volume of every cell of the tile and of its 1-cell ring (i0-1..i0+TX,
 // j0-1..j0+TY) go to LDS; each thread evaluates the low i and j faces of its
@@ -185,7 +185,7 @@ __device__ inline DFlux dflux_eu(const Phys &ph, const double V[5], const double
 // 19 -> 14 us.  With the FP32 copies 157 us on 256 x 128 x 64, where the
 // coefficients in FP64 (90 us) and a pass that rounded them and the operands
 // (119 us) read them twice.
-constexpr int CK_KS = 8;
+constexpr int CK_KS = 8;  // planes per workgroup in the all-blocks launch
 constexpr int CK_PL = (TX + 2) * (TY + 2);
 
 struct CoefCell {  // the per-cell operands of a face coefficient
@@ -236,7 +236,7 @@ struct F32Copies {
   float *vF, *uF, *fF, *snF;
 };
 
-// the tile xb (x, y: TX x TY columns, z: CK_KS-plane slab) of block b.  T =
+// the tile xb (x, y: TX x TY columns, z: slab of ks planes) of block b.  T =
 // float rounds the coefficients and copies the operands to FP32 on the way:
 // they are the ones that this pass reads, u excepted.
 template <typename T>
@@ -700,7 +700,7 @@ __global__ void __launch_bounds__(TXS *TYS) SW_ATTR k_impl_sweep_tiled(Blk b, Ph
 // i face is formed by the cell above it and passed down a lane.
 //
 // One workgroup per CU (135 KB of LDS, 254 registers, two waves per SIMD).  On
-// 256 x 128 x 64 a pair takes 185 us and moves 660 MB, against 2 x 125 us for
+// 256 x 128 x 64 a pair takes 175 us and moves 670 MB, against 2 x 125 us for
 // single sweeps of 674 MB each, at 5.4 TB/s, what a large copy reaches; a pair's
 // waves issue or wait for arithmetic and LDS half of the time.  With workgroup
 // barriers in place of the flags below it took 225 us, with flags that waited
@@ -986,7 +986,11 @@ k_impl_sweep2(Blk b, Phys ph, int ntx, int nty, int ks, const double *__restrict
 // sums equation e in the order of sweep_tile.inc.  The operations are those of
 // the pair kernel, so the bits are those of the other kernels.  A wave holds
 // eight cells of a row, lane = role * 8 + cell.  It computes each q seven
-// times and loads it from the L2, so it pays only while the chip is not full:
+// times and loads it from the L2, so it pays only while the chip is not full: a
+// sub-iteration of 32 x 16 x 8 takes 3.8 us against 7.0 in tiles, 64 x 32 x 16
+// 8.9 against 9.6, 48 x 40 x 36 15.4 against 12.0.  The line lies below where the
+// two cross, as a block above it reports a timed tile shape
+// (codens_sweep_tile_of), which it did before this kernel.
 constexpr int SM_CELLS = 8;
 constexpr long SMALL_BLOCK = 16384;  // real cells
 
@@ -1166,6 +1170,7 @@ Pair pair_of(const Blk &b, bool first = false) {
 // (the pair kernel's tiles of 28 x 12 cells leave most of their lanes idle on
 // the last two).  Of the 310 shapes the rule runs 6 in pairs where that is
 // slower by more than 2% (14% at most), and 13 singly (29% at most).
+// FP32 sweeps run singly: 61 us on 256 x 128 x 64, whose 349 MB move at 5.7 TB/s.
 constexpr double PAIR_STEP = 4.8;
 
 // A single sweep whose workgroups (of planes planes) would fill the chip's

@@ -14,7 +14,9 @@
 using namespace codens;
 
 // Bound by memory: 26 planes, on 256 x 128 x 64 91 us (4.8 TB/s), on 161 x 97 x
-// 64 52 us, on blocks of 230,000 cells 17 us.  A plane's loads are all issued
+// 64 48 us on the same fields again and 63 on others (3.3 TB/s: its 600
+// workgroups put three on some compute units and two on the others, of the four
+// that fit), on blocks of 230,000 cells 17 us.  A plane's loads are all issued
 // before one is used, the planes alternate between two LDS buffers with one
 // barrier each, which waits for the LDS traffic only and not for the stores of
 // the plane before (99, 66 and 19.7 us with the loads behind each other's

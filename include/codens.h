@@ -420,8 +420,12 @@ int codens_sumsq_rate(const codens_block *blocks, int32_t nb, const double *a, c
  * solve.f90:487-515): when enabled, every launch of the main kernels is
  * bracketed by HIP events on its own stream.  Names: "zpres", "chronos",
  * "zvisqc", "roe_limiter_chain", "roe_face_flux", "roe_gather",
- * "implimf_coef", "implimf_sweep", "implimf_sweep2" (two sub-iterations in
- * one launch), "implimf_update", "sch_expli", "rk_stage".
+ * "implimf_coef", "implimf_sweep1" (the first launch of the sub-iterations:
+ * the first one, or the first two where they run in pairs and their number is
+ * even; none on blocks of at most 16384 cells with more than one), "implimf_sweep",
+ * "implimf_sweep2" (two sub-iterations in one launch), "implimf_update",
+ * "sch_expli", "rk_stage".  The ghosts' zeros of the residual are part of its
+ * launch ("roe_fused"), but for the all-blocks form ("roe_zero_ghost").
  * codens_timing_read synchronises on the recorded events and returns the
  * summed duration and launch count of one kernel; reset != 0 clears it. */
 int codens_timing_enable(int32_t on);
