@@ -175,13 +175,16 @@ class AdjointProblem:
 
     def vjp(self, v, sn_blk, vol, ubar):
         # the call overwrites every entry of a one-block layout (planes past
-        # the fifth aside) and reads ubar on the real cells only
+        # the fifth aside) and reads 5 x ip11 doubles of ubar, on the real cells
+        ub = ubar[:5]
+        if ub.shape != (5, v.shape[-1]) or ub.dtype != torch.float64 or not ub.is_contiguous():
+            ub = torch.empty((5, v.shape[-1]), dtype=torch.float64, device=v.device).copy_(ub)
         vb = torch.empty_like(v, memory_format=torch.contiguous_format)
         vb[5:] = 0.
         snb = torch.empty_like(sn_blk, memory_format=torch.contiguous_format)
         volb = torch.empty_like(vol, memory_format=torch.contiguous_format)
         abi.adj_residual_vjp(self.blk, self.ph, self.sc, v.contiguous(), sn_blk.contiguous(), vol.contiguous(),
-                             self.winf, self.bcs, ubar[:5].contiguous(), vb[:5], snb, volb)
+                             self.winf, self.bcs, ub, vb[:5], snb, volb)
         return vb, snb, volb
 
     # -- the step and the objective -----------------------------------------
