@@ -184,7 +184,9 @@ __device__ inline DFlux dflux_eu(const Phys &ph, const double V[5], const double
 // slabs of 8 in two rounds, the second half empty, took 133 us; 75 x 61 x 43
 // 19 -> 14 us.  With the FP32 copies 157 us on 256 x 128 x 64, where the
 // coefficients in FP64 (90 us) and a pass that rounded them and the operands
-// (119 us) read them twice.
+// (119 us) read them twice.  Blocks of 2 to 4 cells in i leave nearly all lanes
+// idle and lose by it: with one sub-iteration 2 x 300 x 200 178 us, 157 in two
+// passes, 4 x 64 x 400 89 and 90.
 constexpr int CK_KS = 8;  // planes per workgroup in the all-blocks launch
 constexpr int CK_PL = (TX + 2) * (TY + 2);
 
