@@ -182,7 +182,7 @@ __device__ inline DFlux dflux_eu(const Phys &ph, const double V[5], const double
 // cannot do without, where loads one after another behind the divisions that
 // used the first of them, per-thread 64-bit addresses (127 registers) and
 // slabs of 8 in two rounds, the second half empty, took 133 us; 75 x 61 x 43
-// 19 -> 14 us.  With the FP32 copies 157 us on 256 x 128 x 64, where the
+// 19 -> 14 us.  With the FP32 copies 147 us on 256 x 128 x 64, where the
 // coefficients in FP64 (90 us) and a pass that rounded them and the operands
 // (119 us) read them twice.  Blocks of 2 to 4 cells in i leave nearly all lanes
 // idle and lose by it: with one sub-iteration 2 x 300 x 200 178 us, 157 in two
